@@ -22,7 +22,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libmccl_hip.so")
 
-HIP_SOURCES = ["runtime.hip", "fold.hip", "topk.hip", "sparse.hip", "cast.hip"]
+HIP_SOURCES = ["runtime.hip", "fold.hip", "topk.hip", "topk_resident.hip", "sparse.hip", "cast.hip"]
 
 # -ffp-contract=off: every fold is one IEEE operation per element, never an FMA.
 # packed-fp32-ops is switched off for all device code.

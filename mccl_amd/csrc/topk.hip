@@ -10,10 +10,11 @@
 // (NaN patterns sort above infinity), so selection is an exact radix select on
 // that key.  All buckets of a gradient run in the same launches.
 //
-// SINGLE-PASS PATH (one pass over the gradient, 12 B/element of HBM traffic, two
-// launches; default for buckets of 2^18 elements and more): see the section
-// "single-pass path" below.
-// EXACT PATH (any input; small buckets and topk_path = 1; six launches):
+// RESIDENT PATH (topk_resident.hip; one launch): buckets of up to 2 M elements.
+// SINGLE-PASS PATH (one pass over the gradient, 12 B/element of HBM traffic, two launches):
+// larger buckets and many buckets at a time; see the section "single-pass path" below.
+// EXACT PATH (any input; six launches): large buckets with large ratios, many small buckets,
+// and topk_path = 1 (choose_path has the rule and its measurements).
 //   [pass A]   residual <- grad + residual, histogram of key[30:20]
 //   refine x2  histograms of key[19:10], key[9:0] among prefix matches
 //   count      per 4096-element tile: #(key > T), #(key == T)
@@ -22,120 +23,15 @@
 //   Each kernel first derives the previous round's pick from the finished
 //   histogram (every block redundantly; the result is identical), so no
 //   separate pick launches are needed.
-#include "common.hip.h"
-#include "runtime.h"
+#include "topk_common.hip.h"
 
 #include <atomic>
+#include <cmath>
 #include <vector>
 
 namespace mcclhip {
 
 namespace {
-
-constexpr int kTile = 4096;    // exact path: elements per compaction tile
-constexpr int kBins0 = 2048;   // key[30:20]
-constexpr int kBinsR = 1024;   // key[19:10], key[9:0]
-constexpr int kHistWords = kBins0 + 2 * kBinsR;
-constexpr int kStateWords = 32;
-constexpr uint32_t kDense = 0xFFFFFFFFu;  // tile count: more candidates than slots, read the residual range itself
-constexpr uint64_t kFastMinBucket = 1u << 18;
-
-// per-bucket state words
-enum {
-    // single-pass path: the candidate window, published by its sample block with ONE 16-byte store
-    S_LO_KEY = 0,         // candidates have key >= this
-    S_HI_KEY = 1,         // keys >= this fall into the top coarse bin
-    S_THAT = 2,           // predicted threshold key; the streaming blocks store 0.0f for keys >= this
-    S_READY = 3,          // the call's epoch number once the other three are valid; 0 after the call
-    S_P0 = 4, S_R0 = 5,   // exact path: key prefix / picks still to place after round 0
-    S_P1 = 6, S_R1 = 7,   // after round 1
-    S_T = 8, S_NEED = 9,  // exact threshold key, number of keys == T that are taken
-    S_ISTAR = 10,         // single-pass path: ties are taken while index <= this
-    S_OK = 11,            // single-pass path: 1 when the window selection succeeded for this bucket
-    S_EXACT_HIST = 12,    // 1 when hist round 0 holds the full histogram
-    S_TIMEOUT = 13,       // single-pass path: a block gave up waiting (result invalid, payload header poisoned)
-    S_BARF = 16           // 16..19: barriers of the exact selection inside the select launch
-};
-
-struct Geometry {
-    uint64_t n_total;
-    uint64_t bucket_elems;
-    uint32_t nbuckets;
-    uint32_t tiles;    // exact-path tiles per (full) bucket
-    uint32_t k_full;   // k of a bucket with bucket_elems elements
-    uint32_t k_last;   // k of the last bucket
-    uint32_t listed;   // single-pass path: 1 when the buckets are separate buffers (see Buckets)
-    uint32_t ftiles;   // single-pass path: streaming tiles allotted per bucket
-    uint32_t lcapb;    // single-pass path: capacity of one coarse bin's list (entries)
-};
-
-struct Workspace {
-    // zeroed at the start of every exact-path call; the single-pass path zeroes what it uses itself
-    uint32_t* hist;         // [nbuckets][kHistWords]
-    uint32_t* state;        // [nbuckets][kStateWords]
-    // scratch, written before read
-    uint32_t* tile_gt;      // [nbuckets][tiles]
-    uint32_t* tile_eq;      // [nbuckets][tiles]
-    uint32_t* blk_above;    // [nbuckets][64] exact selection inside the select launch: keys above the threshold per group
-    uint32_t* blk_eq;       // [nbuckets][64] ... keys equal to the threshold per group
-    // single-pass path
-    uint32_t* tile_cnt;     // [nbuckets][ftiles] candidates in the tile's slots, or kDense
-    uint64_t* slots;        // [nbuckets][ftiles][128] (bits << 32) | index, index order
-    uint32_t* grp_cnt;      // [nbuckets][64][kCntStride] finished tiles per group (first word of each 256 bytes)
-    uint32_t* gsuf;         // [nbuckets][128 bins][64 groups] a group's candidates in the bins above bin j
-    uint32_t* bin_fill;     // [nbuckets][128] the bucket's candidates per coarse window bin (= entries of the bin's list)
-    uint64_t* blist;        // [nbuckets][63][lcapb] the window's candidates by coarse bin, any order
-    int* status;            // caller's device word (may be null): receives MCCL_HIP_ERR_TIMEOUT when a block gives up
-};
-
-__device__ __forceinline__ uint64_t bucket_count(const Geometry& g, uint32_t b) {
-    const uint64_t start = (uint64_t)b * g.bucket_elems;
-    const uint64_t left = g.n_total - start;
-    return left < g.bucket_elems ? left : g.bucket_elems;
-}
-__device__ __forceinline__ uint32_t bucket_k(const Geometry& g, uint32_t b) {
-    return b + 1 == g.nbuckets ? g.k_last : g.k_full;
-}
-__device__ __forceinline__ uint32_t key_of(float v) { return f2u(v) & 0x7FFFFFFFu; }
-
-// Where the buckets of a single-pass call live.  Uniform layout: the buckets are
-// consecutive ranges of one gradient (mccl_hip_topk_compress).  Listed layout
-// (Geometry::listed): every bucket is a buffer of its own with its own length
-// (mccl_hip_topk_compress_list); g.bucket_elems is then the longest bucket.
-constexpr uint32_t kMaxListed = MCCL_HIP_TOPK_LIST_MAX;
-struct Buckets {
-    const float* grad;
-    float* residual;
-    uint8_t* wire;
-    uint64_t wire_stride;
-    const float* lgrad[kMaxListed];
-    float* lresidual[kMaxListed];
-    uint8_t* lwire[kMaxListed];
-    uint32_t lcount[kMaxListed];
-    uint32_t lk[kMaxListed];
-};
-// The kernels index the table by bucket number.  Indexing the by-value parameter would make
-// the compiler copy all of it to per-lane scratch memory first (2 KiB per lane, and a launch
-// that sets up scratch starts several microseconds later); the kernels read it where it
-// already lies instead, in the kernel-argument segment, through scalar loads.  Buckets is
-// therefore the FIRST parameter of every kernel that takes one.
-typedef const __attribute__((address_space(4))) Buckets* BucketsArg;
-__device__ __forceinline__ BucketsArg buckets_arg() { return (BucketsArg)__builtin_amdgcn_kernarg_segment_ptr(); }
-__device__ __forceinline__ uint64_t bucket_count(const Geometry& g, BucketsArg bk, uint32_t b) {
-    return g.listed ? (uint64_t)bk->lcount[b] : bucket_count(g, b);
-}
-__device__ __forceinline__ uint32_t bucket_k(const Geometry& g, BucketsArg bk, uint32_t b) {
-    return g.listed ? bk->lk[b] : bucket_k(g, b);
-}
-__device__ __forceinline__ const float* bucket_grad(const Geometry& g, BucketsArg bk, uint32_t b) {
-    return g.listed ? bk->lgrad[b] : bk->grad + (uint64_t)b * g.bucket_elems;
-}
-__device__ __forceinline__ float* bucket_residual(const Geometry& g, BucketsArg bk, uint32_t b) {
-    return g.listed ? bk->lresidual[b] : bk->residual + (uint64_t)b * g.bucket_elems;
-}
-__device__ __forceinline__ uint32_t* bucket_wire(const Geometry& g, BucketsArg bk, uint32_t b) {
-    return (uint32_t*)(g.listed ? bk->lwire[b] : bk->wire + (uint64_t)b * bk->wire_stride);
-}
 
 __global__ __launch_bounds__(kBlock) void k_zero_words(uint32_t* p, uint64_t n) {
     // n is a multiple of 4 and p is 16-byte aligned (see carve())
@@ -495,63 +391,6 @@ __global__ __launch_bounds__(kBlock) void k_topk_emit(float* residual, Geometry 
     }
 }
 
-// ---- what blocks of one launch use to talk to each other ----------------------------------
-__device__ __forceinline__ uint32_t ld_agent(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_agent(uint32_t* p, uint32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Histogram add called by all lanes of a wavefront (m: this lane has a key).  When all
-// keys of the wavefront fall into one bin - zeros, constants: the inputs that reach the
-// dense-region and exact paths - one lane adds the count; 64 adds to one LDS address
-// would serialise.
-__device__ __forceinline__ void wave_hist_add(uint32_t* lh, bool m, uint32_t bin) {
-    const uint64_t act = __ballot(m);
-    if (!act) return;
-    const int first = __ffsll((long long)act) - 1;
-    const uint32_t fb = (uint32_t)__shfl((int)bin, first, kWave);
-    if (__ballot(m && bin == fb) == act) {
-        if ((int)(threadIdx.x & (kWave - 1)) == first) atomicAdd(&lh[fb], (uint32_t)__popcll(act));
-    } else if (m) {
-        atomicAdd(&lh[bin], 1u);
-    }
-}
-
-// All threads of the block call it.  Returns false when the wait timed out.
-// Everything blocks hand to each other goes through agent-scope stores, atomics
-// and loads (they bypass the per-XCD L2 copies), so the barrier needs no cache
-// write-back or invalidate: each wavefront only waits until its own stores and
-// atomics have been acknowledged before the block's arrival is counted.  (Whole-
-// cache fences here, repeated by a thousand polling blocks, made the kernel ten
-// times slower.)
-__device__ __forceinline__ bool bucket_barrier(uint32_t* counter, uint32_t parties, uint32_t* flag /* LDS */,
-                                               uint64_t limit_ticks) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        uint64_t t0 = 0;
-        uint32_t ok = 1, polls = 0;
-        while (ld_agent(counter) < parties) {
-            __builtin_amdgcn_s_sleep(8);
-            if ((++polls & 63u) == 0) {  // look at the clock now and then
-                const uint64_t now = (uint64_t)wall_clock64();
-                if (t0 == 0) t0 = now;
-                else if (now - t0 > limit_ticks) {
-                    ok = 0;
-                    break;
-                }
-            }
-        }
-        *flag = ok;
-    }
-    __syncthreads();
-    return *flag != 0;
-}
-
-
 // ================================ single-pass path ==================================
 // Two launches.
 //
@@ -623,38 +462,10 @@ constexpr int kGroups = 64;                   // at most this many groups of til
 constexpr int kCntStride = 64;                // words between two groups' arrival counters: 256 bytes, so that the
                                               // arrivals of a bucket's tiles spread over memory channels
 constexpr int kHeld = 7;                      // tiles per wavefront whose slots a bin / select block keeps in registers
-constexpr int kFSample = 8192;                // sampled elements per bucket
 constexpr int kSelBuckets = 16;               // buckets per k_topk_select launch: 1024 blocks, all resident
-constexpr uint32_t kPoisonK = 0xFFFFFFFFu;    // payload header of a bucket whose selection was abandoned
 constexpr uint32_t kGaveUp = 0xFFFFFFFEu;     // a wavefront's count: its wait for the sample timed out
 static_assert(kFVecs == 4, "the streaming role is written for four vectors per lane");
 
-__device__ __forceinline__ uint64_t ld_agent64(const uint64_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// 16-byte streaming store written through to memory (agent scope): a later 4-byte
-// repair of the same line by a block on another XCD must not be overwritten by a
-// delayed write-back of this one.  A store of more than 8 bytes reads its data
-// registers over the following cycles: the compiler keeps the next vector
-// instruction from overwriting them for stores it emits itself, not for this one,
-// hence the wait states inside the statement.
-__device__ __forceinline__ void store_through(float* p, u4a v) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
-}
-
-// The window of a bucket, one 16-byte store and one 16-byte load: the four words change together.
-__device__ __forceinline__ void store16_agent(uint32_t* p, u4a v) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
-}
-// (waits for every earlier load of the wavefront as well: they complete in order)
-__device__ __forceinline__ u4a load16_agent(const uint32_t* p) {
-    u4a v;
-    asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(p) : "memory");
-    return v;
-}
 // The kCoarse - 1 bins below the top one divide [lo, hi) evenly: bin = ((key - lo) * mul) >> 32.
 __device__ __forceinline__ uint32_t window_mul(uint32_t lo, uint32_t hi) {
     const uint32_t range = hi - lo;  // key - lo < range for every key below hi
@@ -708,36 +519,9 @@ __device__ __forceinline__ bool wait_word(const uint32_t* p, uint32_t want, uint
     return true;
 }
 
-// Waits until the bucket's window is published (S_READY == epoch); called by a whole wavefront
-// or a single thread.  win[3] = 0 when the wait timed out.
-__device__ __forceinline__ u4a wait_window(const uint32_t* st, uint32_t epoch, uint64_t limit_ticks) {
-    uint64_t t0 = 0;
-    uint32_t polls = 0;
-    for (;;) {
-        u4a v = load16_agent(st + S_LO_KEY);
-        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)v[3]) == epoch) {
-            v[3] = 1u;
-            return v;
-        }
-        __builtin_amdgcn_s_sleep(16);
-        if ((++polls & 63u) == 0) {
-            const uint64_t now = (uint64_t)wall_clock64();
-            if (t0 == 0) t0 = now;
-            else if (now - t0 > limit_ticks) {
-                v[3] = 0u;
-                return v;
-            }
-        }
-    }
-}
-
 struct StreamLds {
     union {
-        struct {  // sample block
-            uint32_t lh[3][kBinsR] __attribute__((aligned(16)));
-            uint32_t wsum[3][kBlock / kWave];
-            uint32_t res[3][2];
-        } s;
+        SampleLds<kBlock> s;  // sample block
         struct {  // streaming block
             uint64_t stage[kFWaves][kWave];  // a wavefront's candidates, (bits << 32) | index, in index order
             uint32_t wcnt[kFWaves];
@@ -762,182 +546,26 @@ struct SelectLds {
     uint32_t flag;
 };
 
-// ---- sample ------------------------------------------------------------------------
-// For NR ranks at once: the bin in which a top-down scan of histogram h[z] reaches rank[z],
-// and how many of the rank's elements fall inside that bin.  Thread t owns the PER bins below
-// BINS - PER t (16-byte LDS reads).  res[z] = {bin, left}; bin = BINS when the histogram holds
-// fewer than rank[z] elements or rank[z] == 0.  SHARED: all ranks are read off h[0].  Called
-// by all threads of the block.
-template <int BINS, int NR, bool SHARED = false>
-__device__ __forceinline__ void sample_pick(const uint32_t* const (&h)[NR], const uint32_t (&rank)[NR],
-                                            uint32_t (*wsum)[kBlock / kWave], uint32_t (*res)[2]) {
-    constexpr int PER = BINS / kBlock;
-    constexpr int NH = SHARED ? 1 : NR;  // histograms actually scanned
-    static_assert(PER % 4 == 0, "16-byte LDS reads");
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    uint32_t c[NH][PER], sum[NH], inc[NH];  // c[z][j]: bin BINS - 1 - PER t - j
-#pragma unroll
-    for (int z = 0; z < NH; z++) {
-        const u4a* row = (const u4a*)&h[z][BINS - PER * (threadIdx.x + 1)];
-        sum[z] = 0;
-#pragma unroll
-        for (int v4 = 0; v4 < PER / 4; v4++) {
-            const u4a x = row[PER / 4 - 1 - v4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                c[z][v4 * 4 + q] = x[3 - q];
-                sum[z] += x[3 - q];
-            }
-        }
-        inc[z] = wave_inclusive_scan(sum[z]);
-        if (lane == kWave - 1) wsum[z][wave] = inc[z];
-    }
-    if (threadIdx.x < NR) { res[threadIdx.x][0] = BINS; res[threadIdx.x][1] = 0; }
-    __syncthreads();
-    uint32_t above0[NH];
-#pragma unroll
-    for (int z = 0; z < NH; z++) {
-        above0[z] = inc[z] - sum[z];
-#pragma unroll
-        for (int i = 0; i < kBlock / kWave; i++)
-            if (i < wave) above0[z] += wsum[z][i];
-    }
-#pragma unroll
-    for (int z = 0; z < NR; z++) {
-        constexpr int zz_shared = 0;
-        const int zh = SHARED ? zz_shared : z;
-        uint32_t above = above0[zh];
-#pragma unroll
-        for (int j = 0; j < PER; j++) {
-            if (above < rank[z] && rank[z] <= above + c[zh][j]) {
-                res[z][0] = (uint32_t)(BINS - 1 - PER * (int)threadIdx.x - j);
-                res[z][1] = rank[z] - above;
-            }
-            above += c[zh][j];
-        }
-    }
-    __syncthreads();
-}
-
-// Radix-selects (11 + 10 key bits) three ranks of the sample, whose keys stay in registers:
-// upper and lower end of the candidate window, 6 sigma of the sampling noise away from the
-// expected rank of the k-th largest key, and the predicted threshold.  Clears what the
-// launches accumulate into, then publishes the window and the epoch with one store.
+// The bucket's candidate window; clears what the launches accumulate into, then publishes the
+// window and the epoch with one store.
 __device__ __forceinline__ void fused_sample(BucketsArg bk, const Geometry& g, const Workspace& w, uint32_t b,
                                              uint32_t epoch, StreamLds& L) {
     const FusedGeo fg = fused_geo(g, bk, b);
-    const uint64_t bn = fg.bn;
-    const float* gp = bucket_grad(g, bk, b);
-    const float* rp = bucket_residual(g, bk, b);
-    const uint64_t nvec = bn / 4;
-    constexpr int SV = kFSample / 4;     // sampled vectors
-    constexpr int PV = SV / kBlock;      // vectors per thread; their 4 * PV keys stay in registers
-    // sampled in runs of 8 vectors (one 128-byte line per array), runs evenly spread
-    const uint32_t nsv = nvec < (uint64_t)SV ? (uint32_t)(nvec & ~7ull) : (uint32_t)SV;
-    const uint64_t stride = nsv ? (nvec / (nsv / 8)) : 8;  // vectors between run starts (>= 8)
-    u4a gv[PV], rv[PV];
-#pragma unroll
-    for (int j = 0; j < PV; j++) {
-        const uint32_t i = (uint32_t)j * kBlock + threadIdx.x;
-        const uint32_t ii = i < nsv ? i : 0;
-        const uint64_t v = (uint64_t)(ii >> 3) * stride + (ii & 7);
-        gv[j] = nsv ? *(const u4u4*)(gp + v * 4) : u4a{0u, 0u, 0u, 0u};
-        rv[j] = nsv ? *(const u4u4*)(rp + v * 4) : u4a{0u, 0u, 0u, 0u};
-    }
-    // while the loads are under way: clear what the launches accumulate into (the
-    // acknowledgements are back long before the window is published)
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
-    if (threadIdx.x < kGroups) st_agent(w.grp_cnt + ((uint64_t)b * kGroups + threadIdx.x) * kCntStride, 0u);
-    if (threadIdx.x < kCoarse) st_agent(w.bin_fill + (uint64_t)b * kCoarse + threadIdx.x, 0u);
-    if (threadIdx.x == 0) {
-        st_agent(st + S_OK, 0u);
-        st_agent(st + S_TIMEOUT, 0u);
-        st_agent(st + S_BARF, 0u); st_agent(st + S_BARF + 1, 0u); st_agent(st + S_BARF + 2, 0u); st_agent(st + S_BARF + 3, 0u);
-    }
-    uint32_t* const h0 = &L.s.lh[0][0];  // round 0 uses 2048 bins: lh[0] and lh[1] are adjacent
-    {
-        const u4a z = {0u, 0u, 0u, 0u};
-        for (int i = threadIdx.x; i < 3 * kBinsR / 4; i += kBlock) ((u4a*)h0)[i] = z;
-    }
-    uint32_t key[PV][4];
-#pragma unroll
-    for (int j = 0; j < PV; j++) {
-        // an element past the sample gets the key 0xFFFFFFFF, which no histogram counts
-        const bool have = (uint32_t)j * kBlock + threadIdx.x < nsv;
-#pragma unroll
-        for (int q = 0; q < 4; q++) key[j][q] = have ? key_of(u2f(gv[j][q]) + u2f(rv[j][q])) : 0xFFFFFFFFu;
-    }
-    const uint32_t S = nsv * 4;
-    const float ks = (float)fg.k * (float)S / (float)bn;
-    const float margin = 6.0f * sqrtf(ks) + 16.0f;
-    // ranks: 0 upper end of the window, 1 lower end, 2 the predicted threshold itself
-    constexpr int NR = 3;
-    uint32_t rank[NR];
-    rank[0] = ks - margin >= 1.0f ? (uint32_t)(ks - margin) : 0u;  // 0: no upper end
-    rank[1] = (uint32_t)(ks + margin) + 1u;                       // > S: no lower end
-    rank[2] = ks >= 1.0f ? (uint32_t)ks : 1u;
-    const bool active[NR] = {rank[0] >= 1u && rank[0] <= S, rank[1] <= S, rank[2] <= S};
-    uint32_t prefix[NR];
-    __syncthreads();
-    // round 0: key[30:20], one histogram for all ranks
-#pragma unroll
-    for (int j = 0; j < PV; j++)
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-            if (key[j][q] != 0xFFFFFFFFu) atomicAdd(&h0[key[j][q] >> 20], 1u);
-    __syncthreads();
-    {
-        const uint32_t* const hs[NR] = {h0, h0, h0};
-        const uint32_t want[NR] = {active[0] ? rank[0] : 0u, active[1] ? rank[1] : 0u, active[2] ? rank[2] : 0u};
-        sample_pick<kBins0, NR, true>(hs, want, L.s.wsum, L.s.res);
-    }
-#pragma unroll
-    for (int z = 0; z < NR; z++) {
-        prefix[z] = L.s.res[z][0] << 20;
-        rank[z] = L.s.res[z][1];
-    }
-    __syncthreads();
-    // round 1: key[19:10] among the keys that share a rank's first digit
-    {
-        const u4a z = {0u, 0u, 0u, 0u};
-        for (int i = threadIdx.x; i < 3 * kBinsR / 4; i += kBlock) ((u4a*)h0)[i] = z;
-    }
-    __syncthreads();
-    // (three comparisons per key; the few keys that share a rank's first digit take the branch)
-    const uint32_t d0 = active[0] ? prefix[0] >> 20 : 0xFFFFFFFFu, d1 = active[1] ? prefix[1] >> 20 : 0xFFFFFFFFu,
-                   d2 = active[2] ? prefix[2] >> 20 : 0xFFFFFFFFu;
-#pragma unroll
-    for (int j = 0; j < PV; j++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint32_t kq = key[j][q], d = kq >> 20;
-            if (d == d0 || d == d1 || d == d2) {
-                const uint32_t bin = (kq >> 10) & (kBinsR - 1);
-                if (d == d0) atomicAdd(&L.s.lh[0][bin], 1u);
-                if (d == d1) atomicAdd(&L.s.lh[1][bin], 1u);
-                if (d == d2) atomicAdd(&L.s.lh[2][bin], 1u);
-            }
+    const SampleWindow win = sample_window<kBlock>(bucket_grad(g, bk, b), bucket_residual(g, bk, b), fg.bn, fg.k, L.s, [&] {
+        // (the acknowledgements are back long before the window is published)
+        if (threadIdx.x < kGroups) st_agent(w.grp_cnt + ((uint64_t)b * kGroups + threadIdx.x) * kCntStride, 0u);
+        if (threadIdx.x < kCoarse) st_agent(w.bin_fill + (uint64_t)b * kCoarse + threadIdx.x, 0u);
+        if (threadIdx.x == 0) {
+            st_agent(st + S_OK, 0u);
+            st_agent(st + S_TIMEOUT, 0u);
+            st_agent(st + S_BARF, 0u); st_agent(st + S_BARF + 1, 0u); st_agent(st + S_BARF + 2, 0u); st_agent(st + S_BARF + 3, 0u);
         }
-    __syncthreads();
-    {
-        const uint32_t* const hs[NR] = {L.s.lh[0], L.s.lh[1], L.s.lh[2]};
-        const uint32_t want[NR] = {active[0] ? rank[0] : 0u, active[1] ? rank[1] : 0u, active[2] ? rank[2] : 0u};
-        sample_pick<kBinsR, NR>(hs, want, L.s.wsum, L.s.res);
-    }
+    });
     if (threadIdx.x == 0) {
-#pragma unroll
-        for (int z = 0; z < NR; z++) prefix[z] |= (L.s.res[z][0] & (uint32_t)(kBinsR - 1)) << 10;
-        const uint32_t lo = active[1] ? prefix[1] : 0u;
-        uint32_t hi = active[0] ? (prefix[0] | 0x3FFu) : 0x7FFFFFFFu;  // upper end of the window: rounded up
-        if (hi < lo) hi = lo;
-        // predicted threshold: middle of its 1024-key cell; never below lo: every pre-zeroed
-        // element must be a listed candidate
-        uint32_t that = active[2] ? (prefix[2] | 0x200u) : 0x7FFFFFFFu;
-        if (that < lo) that = lo;
         // every store above must have arrived before the window is published
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        store16_agent(st + S_LO_KEY, u4a{lo, hi, that, epoch});
+        store16_agent(st + S_LO_KEY, u4a{win.lo, win.hi, win.that, epoch});
     }
     // off the critical path: the histograms of the exact selection, should the select launch need it
     for (int i = threadIdx.x; i < kHistWords; i += kBlock) w.hist[(uint64_t)b * kHistWords + i] = 0u;
@@ -1046,15 +674,6 @@ struct GroupTiles {
     }
 };
 __device__ __forceinline__ uint32_t key64(uint64_t e) { return (uint32_t)(e >> 32) & 0x7FFFFFFFu; }
-
-__device__ __forceinline__ void fused_give_up(const Workspace& w, uint32_t* st, uint32_t* out) {
-    if (threadIdx.x == 0) {
-        st_agent(st + S_TIMEOUT, 1u);
-        if (w.status) st_agent((uint32_t*)w.status, (uint32_t)MCCL_HIP_ERR_TIMEOUT);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        st_agent(out, kPoisonK);
-    }
-}
 
 // ---- bin block -----------------------------------------------------------------------------
 __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, const Workspace& w, uint32_t b,
@@ -1597,7 +1216,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
         {
             const uint32_t* const hists[1] = {lh};
             const uint32_t wants[1] = {want};
-            sample_pick<kBinsR, 1>(hists, wants, L.wsum, L.res);
+            sample_pick<kBinsR, 1, kBlock>(hists, wants, L.wsum, L.res);
         }
         const uint32_t bin = L.res[0][0], left = L.res[0][1];
         __syncthreads();  // res is rewritten by the next round
@@ -1742,7 +1361,8 @@ uint64_t workspace_words(const Geometry& g) {
     return zeroed_words(g) + 2 * align4((uint64_t)g.nbuckets * g.tiles) + 2 * align4((uint64_t)g.nbuckets * kGroups) +
            align4((uint64_t)g.nbuckets * g.ftiles) + align4((uint64_t)g.nbuckets * g.ftiles * kTileSlots * 2) +
            align4((uint64_t)g.nbuckets * kGroups * kCntStride) + align4((uint64_t)g.nbuckets * kCoarse * kGroups) +
-           align4((uint64_t)g.nbuckets * kCoarse) + align4((uint64_t)g.nbuckets * (kCoarse - 1) * g.lcapb * 2);
+           align4((uint64_t)g.nbuckets * kCoarse) + align4((uint64_t)g.nbuckets * (kCoarse - 1) * g.lcapb * 2) +
+           (g.bucket_elems <= kRMaxBucket ? (uint64_t)g.nbuckets * kRWords : 0);
 }
 
 Workspace carve(void* base, const Geometry& g) {
@@ -1759,7 +1379,8 @@ Workspace carve(void* base, const Geometry& g) {
     w.grp_cnt = p;     p += align4((uint64_t)g.nbuckets * kGroups * kCntStride);
     w.gsuf = p;       p += align4((uint64_t)g.nbuckets * kGroups * kCoarse);
     w.bin_fill = p;    p += align4((uint64_t)g.nbuckets * kCoarse);
-    w.blist = (uint64_t*)p;
+    w.blist = (uint64_t*)p;  p += align4((uint64_t)g.nbuckets * (kCoarse - 1) * g.lcapb * 2);
+    w.rmem = p;
     w.status = nullptr;
     return w;
 }
@@ -1792,13 +1413,51 @@ bool make_geometry(uint64_t n_total, uint64_t bucket_elems, double ratio, Geomet
 // it is not this call's number; zero is what a finished call leaves behind).
 std::atomic<uint32_t> g_epoch{0x5EED0001u};
 
-// The two launches of the single-pass path.  False when the grid would not fit.
-bool launch_single_pass(const Buckets& bk, const Geometry& g, const Workspace& w, hipStream_t st) {
+uint32_t next_epoch() {
+    uint32_t e = ++g_epoch;
+    if (e == 0) e = ++g_epoch;
+    return e;
+}
+
+enum Path { kPathExact, kPathStream, kPathResident };
+
+// Which kernels a call takes (tuning key "topk_path": 1, 2, 3 fix it).  `counts`: the buckets'
+// lengths when they are listed, else null.  Measured per call, us:
+//   resident up to 512 blocks, as many as the GPU holds at once: one launch against two or six
+//     (65,536 elements: 15 against 28 exact; 1 M: 24.5 against 26 streaming; 8 x 262,144: 26 against
+//     29 streaming).  Beyond, its blocks wait their turn and its barriers lie open (16 x 262,144: 54
+//     against 37 streaming; 64 x 131,072: 99 against 84 exact) - except for buckets of a few blocks
+//     (1500 x 16,384: 167 against 187 exact) ...
+//   ... and where the streaming path's tiles run out of candidate slots (128 per 4096 elements, more
+//     than 3 % inside the sampled window: ratios above about 0.015).  Its tiles are then read again
+//     as a whole (5 %, 2 M elements: 145 us against 30 resident; 6.5 M: 448 against 144 exact; from
+//     eight buckets on that latency is shared: 14 x 6.5 M 826 against 905 exact).
+Path choose_path(const Geometry& g, const uint64_t* counts) {
+    const bool fits = g.bucket_elems <= kRMaxBucket;
+    const uint64_t stream_blocks = (uint64_t)g.nbuckets * ((uint64_t)g.ftiles + kGroups + 1) + kGroups;
+    const bool streams = stream_blocks < 0x7FFFFFFFull;
+    const int path = tuning().topk_path;
+    if (path == 1 && !counts) return kPathExact;
+    if (path == 2 && streams) return kPathStream;
+    if (path == 3 && fits) return kPathResident;
+    const int vecs = resident_vecs(g.bucket_elems);
+    const uint64_t per = (uint64_t)vecs * kFTile;
+    uint64_t blocks = 0;
+    if (counts) for (uint32_t b = 0; b < g.nbuckets; b++) blocks += (counts[b] + per - 1) / per;
+    else blocks = (g.n_total + per - 1) / per;
+    // expected share of a bucket inside the sampled window (see sample_window)
+    const double ks = (double)g.k_full / (double)g.bucket_elems * kFSample;
+    const bool dense = (ks + 6.0 * std::sqrt(ks) + 16.0) / kFSample > (double)kTileSlots / kFTile;
+    if (fits && (blocks <= 512 || g.bucket_elems <= 4 * per || (dense && (vecs == 4 || counts)))) return kPathResident;
+    if (counts) return streams ? kPathStream : (fits ? kPathResident : kPathExact);
+    return streams && g.bucket_elems >= kFastMinBucket && (!dense || (!fits && g.nbuckets >= 8)) ? kPathStream : kPathExact;
+}
+
+// The two launches of the single-pass path.
+void launch_single_pass(const Buckets& bk, const Geometry& g, const Workspace& w, hipStream_t st) {
     // the streaming launch: a sample block per bucket, then per bucket its tiles and 64 bin blocks
     const uint64_t blocks = (uint64_t)g.nbuckets * ((uint64_t)g.ftiles + kGroups + 1) + kGroups;
-    if (blocks >= 0x7FFFFFFFull) return false;
-    uint32_t epoch = ++g_epoch;
-    if (epoch == 0) epoch = ++g_epoch;
+    const uint32_t epoch = next_epoch();
     // 100 MHz ticks a block may wait before it gives up
     const uint64_t lim = (uint64_t)tuning().topk_barrier_ms * 100000ull;
     // blocks that are resident from the start of the launch: they wait for the sample blocks
@@ -1816,6 +1475,18 @@ bool launch_single_pass(const Buckets& bk, const Geometry& g, const Workspace& w
     for (uint32_t b0 = 0; b0 < g.nbuckets; b0 += kSelBuckets) {
         const uint32_t nb = g.nbuckets - b0 < (uint32_t)kSelBuckets ? g.nbuckets - b0 : (uint32_t)kSelBuckets;
         k_topk_select<<<dim3(kGroups, nb), kBlock, 0, st>>>(bk, g, w, b0, lim);
+    }
+}
+
+// False when the call has to take the exact path.
+bool launch_by_path(Path path, const Buckets& bk, const Geometry& g, const Workspace& w, hipStream_t st) {
+    if (path == kPathExact) return false;
+    if (path == kPathStream) {
+        launch_single_pass(bk, g, w, st);
+    } else {
+        const uint32_t epoch = next_epoch();
+        launch_resident(bk, g, w, epoch, tuning().topk_stall_test ? ~epoch : epoch,
+                        (uint64_t)tuning().topk_barrier_ms * 100000ull, st);
     }
     return true;
 }
@@ -1864,24 +1535,19 @@ int mccl_hip_topk_compress(const float* grad, float* residual, uint64_t n_total,
     void* aligned = (void*)(((uintptr_t)workspace + 15) & ~(uintptr_t)15);
     Workspace w = carve(aligned, g);
     w.status = status;
-    const int path = tuning().topk_path;  // 0 auto, 1 exact path only, 2 single-pass path at any size
-    bool fast = path == 2 || (path == 0 && g.bucket_elems >= kFastMinBucket);
-
+    const Path path = choose_path(g, nullptr);
     const uint64_t cap = (uint64_t)device_info().num_cus * (uint64_t)tuning().fold_blocks_per_cu;
     const uint64_t nvec = g.bucket_elems / 4;
     const uint64_t bx = (cap + g.nbuckets - 1) / g.nbuckets;
     const uint64_t need_r = (nvec + kBlock * 4 - 1) / (kBlock * 4);
     const uint32_t bx_r = clamp_u32(bx < need_r ? bx : need_r, 1, 65535);
     const uint32_t bx_t = clamp_u32(bx < g.tiles ? bx : g.tiles, 1, 65535);
-    if (fast) {
-        Buckets bk = {};
-        bk.grad = grad;
-        bk.residual = residual;
-        bk.wire = (uint8_t*)wire;
-        bk.wire_stride = wire_stride;
-        fast = launch_single_pass(bk, g, w, st);
-    }
-    if (!fast) {
+    Buckets bk = {};
+    bk.grad = grad;
+    bk.residual = residual;
+    bk.wire = (uint8_t*)wire;
+    bk.wire_stride = wire_stride;
+    if (!launch_by_path(path, bk, g, w, st)) {
         const uint64_t zw = zeroed_words(g);
         k_zero_words<<<clamp_u32((zw / 4 + kBlock - 1) / kBlock, 1, cap), kBlock, 0, st>>>(w.hist, zw);
         const uint64_t need_a = (nvec + kBlock * 2 - 1) / (kBlock * 2);
@@ -1936,7 +1602,7 @@ int mccl_hip_topk_compress_list(const float* const* host_grads, float* const* ho
     void* aligned = (void*)(((uintptr_t)workspace + 15) & ~(uintptr_t)15);
     Workspace w = carve(aligned, g);
     w.status = status;
-    if (!launch_single_pass(bk, g, w, (hipStream_t)stream)) return MCCL_HIP_ERR_ARG;
+    if (!launch_by_path(choose_path(g, host_counts), bk, g, w, (hipStream_t)stream)) return MCCL_HIP_ERR_ARG;
     return launch_status();
 }
 

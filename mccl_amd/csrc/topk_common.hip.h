@@ -1,0 +1,430 @@
+// What the two top-k kernel families (topk.hip: streaming, topk_resident.hip: resident) share:
+// the call's geometry, workspace and bucket table, and how blocks of one launch talk to each other.
+#pragma once
+
+#include "common.hip.h"
+#include "runtime.h"
+
+namespace mcclhip {
+
+constexpr int kTile = 4096;    // exact path: elements per compaction tile
+constexpr int kBins0 = 2048;   // key[30:20]
+constexpr int kBinsR = 1024;   // key[19:10], key[9:0]
+constexpr int kHistWords = kBins0 + 2 * kBinsR;
+constexpr int kStateWords = 32;
+constexpr uint32_t kDense = 0xFFFFFFFFu;  // tile count: more candidates than slots, read the residual range itself
+constexpr uint64_t kFastMinBucket = 1u << 18;
+constexpr uint32_t kPoisonK = 0xFFFFFFFFu;    // payload header of a bucket whose selection was abandoned
+// resident path (topk_resident.hip): per-bucket scratch, in words
+constexpr int kRList = 1024;                  // elements of the picked bin that are ranked as a list
+constexpr uint64_t kRMaxBlocks = 128;         // blocks of one bucket
+constexpr uint64_t kRMaxBucket = kRMaxBlocks * 1024 * 4 * 4;  // 2,097,152 elements
+constexpr uint32_t kRRow = 2048 + 64;         // one round's histogram: 2048 bins, the count above them, padding
+constexpr uint32_t kRBars = 6;                // barriers: at most four rounds and the list / ties
+constexpr uint32_t kRBar = 4 * kRRow;         // their counters, 256 bytes apart, then the list's fill counter
+constexpr uint32_t kRZeroWords = kRBar + 64 * (kRBars + 1);   // cleared by the lead block
+constexpr uint32_t kRCnt = kRZeroWords;       // per block: elements above the bin, inside the bin
+constexpr uint32_t kRListAt = kRCnt + 2 * (uint32_t)kRMaxBlocks;
+constexpr uint32_t kRWords = kRListAt + 2 * kRList;
+constexpr int kFSample = 8192;                // sampled elements per bucket
+
+// per-bucket state words
+enum {
+    // single-pass path: the candidate window, published by its sample block with ONE 16-byte store
+    S_LO_KEY = 0,         // candidates have key >= this
+    S_HI_KEY = 1,         // keys >= this fall into the top coarse bin
+    S_THAT = 2,           // predicted threshold key; the streaming blocks store 0.0f for keys >= this
+    S_READY = 3,          // the call's epoch number once the other three are valid; 0 after the call
+    S_P0 = 4, S_R0 = 5,   // exact path: key prefix / picks still to place after round 0
+    S_P1 = 6, S_R1 = 7,   // after round 1
+    S_T = 8, S_NEED = 9,  // exact threshold key, number of keys == T that are taken
+    S_ISTAR = 10,         // single-pass path: ties are taken while index <= this
+    S_OK = 11,            // single-pass path: 1 when the window selection succeeded for this bucket
+    S_EXACT_HIST = 12,    // 1 when hist round 0 holds the full histogram
+    S_TIMEOUT = 13,       // single-pass path: a block gave up waiting (result invalid, payload header poisoned)
+    S_BARF = 16           // 16..19: barriers of the exact selection inside the select launch
+};
+
+struct Geometry {
+    uint64_t n_total;
+    uint64_t bucket_elems;
+    uint32_t nbuckets;
+    uint32_t tiles;    // exact-path tiles per (full) bucket
+    uint32_t k_full;   // k of a bucket with bucket_elems elements
+    uint32_t k_last;   // k of the last bucket
+    uint32_t listed;   // single-pass path: 1 when the buckets are separate buffers (see Buckets)
+    uint32_t ftiles;   // single-pass path: streaming tiles allotted per bucket
+    uint32_t lcapb;    // single-pass path: capacity of one coarse bin's list (entries)
+};
+
+struct Workspace {
+    // zeroed at the start of every exact-path call; the single-pass path zeroes what it uses itself
+    uint32_t* hist;         // [nbuckets][kHistWords]
+    uint32_t* state;        // [nbuckets][kStateWords]
+    // scratch, written before read
+    uint32_t* tile_gt;      // [nbuckets][tiles]
+    uint32_t* tile_eq;      // [nbuckets][tiles]
+    uint32_t* blk_above;    // [nbuckets][64] exact selection inside the select launch: keys above the threshold per group
+    uint32_t* blk_eq;       // [nbuckets][64] ... keys equal to the threshold per group
+    // single-pass path
+    uint32_t* tile_cnt;     // [nbuckets][ftiles] candidates in the tile's slots, or kDense
+    uint64_t* slots;        // [nbuckets][ftiles][128] (bits << 32) | index, index order
+    uint32_t* grp_cnt;      // [nbuckets][64][kCntStride] finished tiles per group (first word of each 256 bytes)
+    uint32_t* gsuf;         // [nbuckets][128 bins][64 groups] a group's candidates in the bins above bin j
+    uint32_t* bin_fill;     // [nbuckets][128] the bucket's candidates per coarse window bin (= entries of the bin's list)
+    uint64_t* blist;        // [nbuckets][63][lcapb] the window's candidates by coarse bin, any order
+    uint32_t* rmem;         // [nbuckets][kRWords] resident path
+    int* status;            // caller's device word (may be null): receives MCCL_HIP_ERR_TIMEOUT when a block gives up
+};
+
+__device__ __forceinline__ uint64_t bucket_count(const Geometry& g, uint32_t b) {
+    const uint64_t start = (uint64_t)b * g.bucket_elems;
+    const uint64_t left = g.n_total - start;
+    return left < g.bucket_elems ? left : g.bucket_elems;
+}
+__device__ __forceinline__ uint32_t bucket_k(const Geometry& g, uint32_t b) {
+    return b + 1 == g.nbuckets ? g.k_last : g.k_full;
+}
+__device__ __forceinline__ uint32_t key_of(float v) { return f2u(v) & 0x7FFFFFFFu; }
+
+// Where the buckets of a single-pass call live.  Uniform layout: the buckets are
+// consecutive ranges of one gradient (mccl_hip_topk_compress).  Listed layout
+// (Geometry::listed): every bucket is a buffer of its own with its own length
+// (mccl_hip_topk_compress_list); g.bucket_elems is then the longest bucket.
+constexpr uint32_t kMaxListed = MCCL_HIP_TOPK_LIST_MAX;
+struct Buckets {
+    const float* grad;
+    float* residual;
+    uint8_t* wire;
+    uint64_t wire_stride;
+    const float* lgrad[kMaxListed];
+    float* lresidual[kMaxListed];
+    uint8_t* lwire[kMaxListed];
+    uint32_t lcount[kMaxListed];
+    uint32_t lk[kMaxListed];
+};
+// The kernels index the table by bucket number.  Indexing the by-value parameter would make
+// the compiler copy all of it to per-lane scratch memory first (2 KiB per lane, and a launch
+// that sets up scratch starts several microseconds later); the kernels read it where it
+// already lies instead, in the kernel-argument segment, through scalar loads.  Buckets is
+// therefore the FIRST parameter of every kernel that takes one.
+typedef const __attribute__((address_space(4))) Buckets* BucketsArg;
+__device__ __forceinline__ BucketsArg buckets_arg() { return (BucketsArg)__builtin_amdgcn_kernarg_segment_ptr(); }
+__device__ __forceinline__ uint64_t bucket_count(const Geometry& g, BucketsArg bk, uint32_t b) {
+    return g.listed ? (uint64_t)bk->lcount[b] : bucket_count(g, b);
+}
+__device__ __forceinline__ uint32_t bucket_k(const Geometry& g, BucketsArg bk, uint32_t b) {
+    return g.listed ? bk->lk[b] : bucket_k(g, b);
+}
+__device__ __forceinline__ const float* bucket_grad(const Geometry& g, BucketsArg bk, uint32_t b) {
+    return g.listed ? bk->lgrad[b] : bk->grad + (uint64_t)b * g.bucket_elems;
+}
+__device__ __forceinline__ float* bucket_residual(const Geometry& g, BucketsArg bk, uint32_t b) {
+    return g.listed ? bk->lresidual[b] : bk->residual + (uint64_t)b * g.bucket_elems;
+}
+__device__ __forceinline__ uint32_t* bucket_wire(const Geometry& g, BucketsArg bk, uint32_t b) {
+    return (uint32_t*)(g.listed ? bk->lwire[b] : bk->wire + (uint64_t)b * bk->wire_stride);
+}
+
+
+int resident_vecs(uint64_t n);
+void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t epoch, uint32_t published,
+                     uint64_t limit_ticks, hipStream_t st);
+
+// ---- what blocks of one launch use to talk to each other ----------------------------------
+__device__ __forceinline__ uint32_t ld_agent(const uint32_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent(uint32_t* p, uint32_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Histogram add called by all lanes of a wavefront (m: this lane has a key).  When all
+// keys of the wavefront fall into one bin - zeros, constants: the inputs that reach the
+// dense-region and exact paths - one lane adds the count; 64 adds to one LDS address
+// would serialise.
+__device__ __forceinline__ void wave_hist_add(uint32_t* lh, bool m, uint32_t bin) {
+    const uint64_t act = __ballot(m);
+    if (!act) return;
+    const int first = __ffsll((long long)act) - 1;
+    const uint32_t fb = (uint32_t)__shfl((int)bin, first, kWave);
+    if (__ballot(m && bin == fb) == act) {
+        if ((int)(threadIdx.x & (kWave - 1)) == first) atomicAdd(&lh[fb], (uint32_t)__popcll(act));
+    } else if (m) {
+        atomicAdd(&lh[bin], 1u);
+    }
+}
+
+// All threads of the block call it.  Returns false when the wait timed out.
+// Everything blocks hand to each other goes through agent-scope stores, atomics
+// and loads (they bypass the per-XCD L2 copies), so the barrier needs no cache
+// write-back or invalidate: each wavefront only waits until its own stores and
+// atomics have been acknowledged before the block's arrival is counted.  (Whole-
+// cache fences here, repeated by a thousand polling blocks, made the kernel ten
+// times slower.)
+__device__ __forceinline__ bool bucket_barrier(uint32_t* counter, uint32_t parties, uint32_t* flag /* LDS */,
+                                               uint64_t limit_ticks) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint64_t t0 = 0;
+        uint32_t ok = 1, polls = 0;
+        while (ld_agent(counter) < parties) {
+            __builtin_amdgcn_s_sleep(8);
+            if ((++polls & 63u) == 0) {  // look at the clock now and then
+                const uint64_t now = (uint64_t)wall_clock64();
+                if (t0 == 0) t0 = now;
+                else if (now - t0 > limit_ticks) {
+                    ok = 0;
+                    break;
+                }
+            }
+        }
+        *flag = ok;
+    }
+    __syncthreads();
+    return *flag != 0;
+}
+
+
+__device__ __forceinline__ uint64_t ld_agent64(const uint64_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// 16-byte streaming store written through to memory (agent scope): a later 4-byte
+// repair of the same line by a block on another XCD must not be overwritten by a
+// delayed write-back of this one.  A store of more than 8 bytes reads its data
+// registers over the following cycles: the compiler keeps the next vector
+// instruction from overwriting them for stores it emits itself, not for this one,
+// hence the wait states inside the statement.
+__device__ __forceinline__ void store_through(float* p, u4a v) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
+}
+
+// The window of a bucket, one 16-byte store and one 16-byte load: the four words change together.
+__device__ __forceinline__ void store16_agent(uint32_t* p, u4a v) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
+}
+// (waits for every earlier load of the wavefront as well: they complete in order)
+__device__ __forceinline__ u4a load16_agent(const uint32_t* p) {
+    u4a v;
+    asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(v) : "v"(p) : "memory");
+    return v;
+}
+// Waits until the bucket's window is published (S_READY == epoch); called by a whole wavefront
+// or a single thread.  win[3] = 0 when the wait timed out.
+__device__ __forceinline__ u4a wait_window(const uint32_t* st, uint32_t epoch, uint64_t limit_ticks) {
+    uint64_t t0 = 0;
+    uint32_t polls = 0;
+    for (;;) {
+        u4a v = load16_agent(st + S_LO_KEY);
+        if ((uint32_t)__builtin_amdgcn_readfirstlane((int)v[3]) == epoch) {
+            v[3] = 1u;
+            return v;
+        }
+        __builtin_amdgcn_s_sleep(16);
+        if ((++polls & 63u) == 0) {
+            const uint64_t now = (uint64_t)wall_clock64();
+            if (t0 == 0) t0 = now;
+            else if (now - t0 > limit_ticks) {
+                v[3] = 0u;
+                return v;
+            }
+        }
+    }
+}
+
+// ---- sample ------------------------------------------------------------------------
+template <int THREADS>
+struct SampleLds {
+    uint32_t lh[3][kBinsR] __attribute__((aligned(16)));
+    uint32_t wsum[3][THREADS / kWave];
+    uint32_t res[3][2];
+};
+
+// For NR ranks at once: the bin in which a top-down scan of histogram h[z] reaches rank[z],
+// and how many of the rank's elements fall inside that bin.  Thread t owns the PER bins below
+// BINS - PER t (vector LDS reads).  res[z] = {bin, left}; bin = BINS when the histogram holds
+// fewer than rank[z] elements or rank[z] == 0.  SHARED: all ranks are read off h[0].  Called
+// by all threads of the block.
+template <int BINS, int NR, int THREADS, bool SHARED = false>
+__device__ __forceinline__ void sample_pick(const uint32_t* const (&h)[NR], const uint32_t (&rank)[NR],
+                                            uint32_t (*wsum)[THREADS / kWave], uint32_t (*res)[2]) {
+    constexpr int PER = BINS / THREADS;
+    constexpr int RW = PER % 4 == 0 ? 4 : PER;  // bins per LDS read
+    constexpr int NH = SHARED ? 1 : NR;       // histograms actually scanned
+    static_assert(PER % RW == 0, "whole vectors");
+    typedef uint32_t Row __attribute__((ext_vector_type(RW)));
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = threadIdx.x / kWave;
+    uint32_t c[NH][PER], sum[NH], inc[NH];  // c[z][j]: bin BINS - 1 - PER t - j
+#pragma unroll
+    for (int z = 0; z < NH; z++) {
+        const Row* row = (const Row*)&h[z][BINS - PER * (threadIdx.x + 1)];
+        sum[z] = 0;
+#pragma unroll
+        for (int v = 0; v < PER / RW; v++) {
+            const Row x = row[PER / RW - 1 - v];
+#pragma unroll
+            for (int q = 0; q < RW; q++) {
+                c[z][v * RW + q] = x[RW - 1 - q];
+                sum[z] += x[RW - 1 - q];
+            }
+        }
+        inc[z] = wave_inclusive_scan(sum[z]);
+        if (lane == kWave - 1) wsum[z][wave] = inc[z];
+    }
+    if (threadIdx.x < NR) { res[threadIdx.x][0] = BINS; res[threadIdx.x][1] = 0; }
+    __syncthreads();
+    uint32_t above0[NH];
+#pragma unroll
+    for (int z = 0; z < NH; z++) {
+        above0[z] = inc[z] - sum[z];
+#pragma unroll
+        for (int i = 0; i < THREADS / kWave; i++)
+            if (i < wave) above0[z] += wsum[z][i];
+    }
+#pragma unroll
+    for (int z = 0; z < NR; z++) {
+        const int zh = SHARED ? 0 : z;
+        uint32_t above = above0[zh];
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            if (above < rank[z] && rank[z] <= above + c[zh][j]) {
+                res[z][0] = (uint32_t)(BINS - 1 - PER * (int)threadIdx.x - j);
+                res[z][1] = rank[z] - above;
+            }
+            above += c[zh][j];
+        }
+    }
+    __syncthreads();
+}
+
+// Candidate window of a bucket from 8192 evenly spread elements of grad + residual, whose keys stay
+// in registers: radix select (11 + 10 key bits) of three ranks - upper and lower end of the window,
+// 6 sigma of the sampling noise away from the expected rank of the k-th largest key, and the
+// predicted threshold.  Called by all THREADS threads of a block; the result is valid in thread 0.
+// `under_way()` runs while the sample's loads are under way.
+struct SampleWindow {
+    uint32_t lo, hi, that;
+};
+template <int THREADS, class UnderWay>
+__device__ __forceinline__ SampleWindow sample_window(const float* gp, const float* rp, uint64_t bn, uint32_t k,
+                                                      SampleLds<THREADS>& L, UnderWay&& under_way) {
+    const uint64_t nvec = bn / 4;
+    constexpr int SV = kFSample / 4;     // sampled vectors
+    constexpr int PV = SV / THREADS;     // vectors per thread; their 4 * PV keys stay in registers
+    // sampled in runs of 8 vectors (one 128-byte line per array), runs evenly spread
+    const uint32_t nsv = nvec < (uint64_t)SV ? (uint32_t)(nvec & ~7ull) : (uint32_t)SV;
+    const uint64_t stride = nsv ? (nvec / (nsv / 8)) : 8;  // vectors between run starts (>= 8)
+    u4a gv[PV], rv[PV];
+#pragma unroll
+    for (int j = 0; j < PV; j++) {
+        const uint32_t i = (uint32_t)j * THREADS + threadIdx.x;
+        const uint32_t ii = i < nsv ? i : 0;
+        const uint64_t v = (uint64_t)(ii >> 3) * stride + (ii & 7);
+        gv[j] = nsv ? *(const u4u4*)(gp + v * 4) : u4a{0u, 0u, 0u, 0u};
+        rv[j] = nsv ? *(const u4u4*)(rp + v * 4) : u4a{0u, 0u, 0u, 0u};
+    }
+    under_way();
+    uint32_t* const h0 = &L.lh[0][0];  // round 0 uses 2048 bins: lh[0] and lh[1] are adjacent
+    {
+        const u4a z = {0u, 0u, 0u, 0u};
+        for (int i = threadIdx.x; i < 3 * kBinsR / 4; i += THREADS) ((u4a*)h0)[i] = z;
+    }
+    uint32_t key[PV][4];
+#pragma unroll
+    for (int j = 0; j < PV; j++) {
+        // an element past the sample gets the key 0xFFFFFFFF, which no histogram counts
+        const bool have = (uint32_t)j * THREADS + threadIdx.x < nsv;
+#pragma unroll
+        for (int q = 0; q < 4; q++) key[j][q] = have ? key_of(u2f(gv[j][q]) + u2f(rv[j][q])) : 0xFFFFFFFFu;
+    }
+    const uint32_t S = nsv * 4;
+    const float ks = (float)k * (float)S / (float)bn;
+    const float margin = 6.0f * sqrtf(ks) + 16.0f;
+    // ranks: 0 upper end of the window, 1 lower end, 2 the predicted threshold itself
+    constexpr int NR = 3;
+    uint32_t rank[NR];
+    // A k-th largest key expected among the sample's first few (small ratios) leaves no margin
+    // above it: the sample's largest key is the upper end then, and a threshold above it (probability
+    // e^-ks) fails the window.  Without an upper end the bins would span every float above lo.
+    rank[0] = ks - margin >= 1.0f ? (uint32_t)(ks - margin) : (ks >= 3.0f ? 1u : 0u);  // 0: no upper end
+    rank[1] = (uint32_t)(ks + margin) + 1u;                       // > S: no lower end
+    rank[2] = ks >= 1.0f ? (uint32_t)ks : 1u;
+    const bool active[NR] = {rank[0] >= 1u && rank[0] <= S, rank[1] <= S, rank[2] <= S};
+    uint32_t prefix[NR];
+    __syncthreads();
+    // round 0: key[30:20], one histogram for all ranks
+#pragma unroll
+    for (int j = 0; j < PV; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (key[j][q] != 0xFFFFFFFFu) atomicAdd(&h0[key[j][q] >> 20], 1u);
+    __syncthreads();
+    {
+        const uint32_t* const hs[NR] = {h0, h0, h0};
+        const uint32_t want[NR] = {active[0] ? rank[0] : 0u, active[1] ? rank[1] : 0u, active[2] ? rank[2] : 0u};
+        sample_pick<kBins0, NR, THREADS, true>(hs, want, L.wsum, L.res);
+    }
+#pragma unroll
+    for (int z = 0; z < NR; z++) {
+        prefix[z] = L.res[z][0] << 20;
+        rank[z] = L.res[z][1];
+    }
+    __syncthreads();
+    // round 1: key[19:10] among the keys that share a rank's first digit
+    {
+        const u4a z = {0u, 0u, 0u, 0u};
+        for (int i = threadIdx.x; i < 3 * kBinsR / 4; i += THREADS) ((u4a*)h0)[i] = z;
+    }
+    __syncthreads();
+    // (three comparisons per key; the few keys that share a rank's first digit take the branch)
+    const uint32_t d0 = active[0] ? prefix[0] >> 20 : 0xFFFFFFFFu, d1 = active[1] ? prefix[1] >> 20 : 0xFFFFFFFFu,
+                   d2 = active[2] ? prefix[2] >> 20 : 0xFFFFFFFFu;
+#pragma unroll
+    for (int j = 0; j < PV; j++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint32_t kq = key[j][q], d = kq >> 20;
+            if (d == d0 || d == d1 || d == d2) {
+                const uint32_t bin = (kq >> 10) & (kBinsR - 1);
+                if (d == d0) atomicAdd(&L.lh[0][bin], 1u);
+                if (d == d1) atomicAdd(&L.lh[1][bin], 1u);
+                if (d == d2) atomicAdd(&L.lh[2][bin], 1u);
+            }
+        }
+    __syncthreads();
+    {
+        const uint32_t* const hs[NR] = {L.lh[0], L.lh[1], L.lh[2]};
+        const uint32_t want[NR] = {active[0] ? rank[0] : 0u, active[1] ? rank[1] : 0u, active[2] ? rank[2] : 0u};
+        sample_pick<kBinsR, NR, THREADS>(hs, want, L.wsum, L.res);
+    }
+    SampleWindow win = {0u, 0x7FFFFFFFu, 0x7FFFFFFFu};
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int z = 0; z < NR; z++) prefix[z] |= (L.res[z][0] & (uint32_t)(kBinsR - 1)) << 10;
+        win.lo = active[1] ? prefix[1] : 0u;
+        win.hi = active[0] ? (prefix[0] | 0x3FFu) : 0x7FFFFFFFu;  // upper end of the window: rounded up
+        if (win.hi < win.lo) win.hi = win.lo;
+        // predicted threshold: middle of its 1024-key cell; never below lo: every pre-zeroed
+        // element must be a listed candidate
+        win.that = active[2] ? (prefix[2] | 0x200u) : 0x7FFFFFFFu;
+        if (win.that < win.lo) win.that = win.lo;
+    }
+    return win;
+}
+
+__device__ __forceinline__ void fused_give_up(const Workspace& w, uint32_t* st, uint32_t* out) {
+    if (threadIdx.x == 0) {
+        st_agent(st + S_TIMEOUT, 1u);
+        if (w.status) st_agent((uint32_t*)w.status, (uint32_t)MCCL_HIP_ERR_TIMEOUT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        st_agent(out, kPoisonK);
+    }
+}
+
+}  // namespace mcclhip

@@ -1,0 +1,507 @@
+// Top-k compress of buckets that fit the register file: one launch, one pass over memory.
+//
+// Semantics and ordering as in topk.hip (csrc/compression/TopKCompression.cpp:38-120).
+//
+// A bucket is cut into blocks of 4096 * V consecutive elements; a block loads grad and residual
+// once and keeps its sums in registers until the bucket's threshold is known, then writes residual
+// and payload once.  The threshold is found by radix selection over the key's bits: a round
+// histograms the keys inside the current key range into 2048 bins in LDS, the blocks add theirs into
+// the bucket's histogram in memory, meet at a counter barrier and all pick the same bin.  When the
+// picked bin holds at most kRList elements they are gathered into one list, which every block ranks
+// by itself; otherwise the next round splits the bin, down to a single key whose ties are taken in
+// index order.  The first round covers a window around the threshold taken from a sample (large
+// buckets; the rounds restart on the full key range if it misleads) or every key (small ones); a
+// one-block bucket needs no memory but its own.  Any ratio and any distribution takes this path:
+// nothing depends on how the keys are spread.
+//
+// What bounds it is latency, not bandwidth: for one bucket of 65,536 elements (1.3 MB of traffic)
+// launch 3 us, load 1.3, two rounds of 0.8 + 1.3 (barrier) + 1, list 1.3 + 1.5 (barrier), rank and
+// scan 1.5, store 0.5.  Against the six launches of the exact path: 4096 elements 7.4 us (25.5),
+// 65,537 17.4 (27.7), 262,144 19.0 (25.4 on the two-launch path), 1 M 23.5 (26.7); at a ratio of
+// 5 % 1 M elements 24.7 us (84.9) and 2 M 30.4 (144).
+//
+// The blocks of a bucket wait for one another, so they have to be resident together.  At 64
+// registers, 25 KiB of LDS and 1024 threads two blocks fit a CU, 64 an XCD; a bucket has at most 128 blocks,
+// 16 per XCD.  Every XCD dispatches its share of a grid in grid order, so only the newest bucket
+// of a launch can be incompletely dispatched on it, with at most 15 blocks that wait: the four
+// hardware queues of a process can have four such launches under way and still leave a slot.
+#include "topk_common.hip.h"
+
+#include <type_traits>
+
+namespace mcclhip {
+
+namespace {
+
+constexpr int kRThreads = 1024;
+constexpr int kRWaves = kRThreads / kWave;
+constexpr int kRBins = 2048;       // bins of one round
+constexpr int kRRank = 96;          // a list longer than this is split before it is ranked
+static_assert(kRBins == 2 * kRThreads, "a thread owns two bins");
+constexpr uint32_t kRSampleMin = 1u << 18;  // buckets of this many elements start from a sampled window
+
+template <int V>
+struct ResidentLds {
+    // a round's histogram, [kRBins] = keys above the range; later the block's picks, one bit per element
+    uint32_t lh[kRBins + 4] __attribute__((aligned(16)));
+    union {
+        struct {
+            uint64_t list[kRList];             // the picked bin's elements
+            uint64_t sub[kRList];              // ... those of one bin of the list
+        };
+        uint32_t pre[kRThreads * 4 * V / 32];   // picks before each 32 elements
+        SampleLds<kRThreads> s;
+    };
+    uint32_t scratch[kRWaves];
+    uint32_t pick[3];                          // bin, picks left inside it, elements inside it
+    uint32_t win[4];
+    uint32_t flag, count, base;
+    uint64_t cut;
+};
+
+// Exclusive scan of one value per thread over the block; smem: kRWaves words.  (The sums of the
+// wavefronts are scanned by a wavefront's lanes: sixteen of them read one by one would take sixteen
+// registers.)
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* smem, uint32_t* total) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const uint32_t inc = wave_inclusive_scan(v);
+    if (lane == kWave - 1) smem[wave] = inc;
+    __syncthreads();
+    const uint32_t s = lane < kRWaves ? smem[lane] : 0u;
+    const uint32_t sums = wave_inclusive_scan(s);
+    __syncthreads();
+    *total = (uint32_t)__builtin_amdgcn_readlane((int)sums, kWave - 1);
+    return (uint32_t)__builtin_amdgcn_readlane((int)(sums - s), wave) + inc - v;
+}
+__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* smem) {
+    uint32_t total;
+    block_scan(v, smem, &total);
+    return total;
+}
+
+// Counting bins from the top, in which the running count reaches r: res = {bin, picks left inside it,
+// elements inside it}.  `two` = bins 2046 - 2 t and 2047 - 2 t of thread t, `above` = elements above
+// all bins.  Returns the elements in all bins; res is untouched when they do not reach r.
+__device__ __forceinline__ uint32_t pick_bin2(u2a two, uint32_t above, uint32_t r, uint32_t* scratch, uint32_t* res) {
+    uint32_t total;
+    uint32_t run = block_scan(two[0] + two[1], scratch, &total) + above;
+#pragma unroll
+    for (int q = 1; q >= 0; q--) {
+        if (run < r && r <= run + two[q]) {
+            res[0] = 2 * (kRThreads - 1 - threadIdx.x) + q;
+            res[1] = r - run;
+            res[2] = two[q];
+        }
+        run += two[q];
+    }
+    __syncthreads();
+    return total;
+}
+
+// All threads of the block; every store and atomic of the block has arrived when it is counted.
+__device__ __forceinline__ bool resident_barrier(uint32_t* counter, uint32_t parties, uint32_t* flag, uint64_t limit_ticks) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint64_t t0 = 0;
+        uint32_t ok = 1, polls = 0;
+        while (ld_agent(counter) < parties) {
+            __builtin_amdgcn_s_sleep(1);
+            if ((++polls & 255u) == 0) {
+                const uint64_t now = (uint64_t)wall_clock64();
+                if (t0 == 0) t0 = now;
+                else if (now - t0 > limit_ticks) {
+                    ok = 0;
+                    break;
+                }
+            }
+        }
+        *flag = ok;
+    }
+    __syncthreads();
+    return *flag != 0;
+}
+
+// grid: x = 0 the bucket's lead block, then its blocks; y = bucket.
+template <int V>
+__global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometry g, Workspace w, uint32_t epoch,
+                                                                uint32_t published, uint64_t limit_ticks) {
+    constexpr uint32_t PER = kRThreads * 4 * V;  // elements of a block
+    const BucketsArg bk = buckets_arg();
+    __shared__ ResidentLds<V> L;
+    const uint32_t b = blockIdx.y;
+    const uint64_t bn = bucket_count(g, bk, b);
+    const uint32_t nblk = (uint32_t)((bn + PER - 1) / PER);
+    uint32_t* st = w.state + (uint64_t)b * kStateWords;
+    uint32_t* const mem = w.rmem + (uint64_t)b * kRWords;
+    float* const rbase = bucket_residual(g, bk, b);
+    const float* const gbase = bucket_grad(g, bk, b);
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const uint32_t k = bucket_k(g, bk, b);
+    if (blockIdx.x == 0) {
+        // ---- lead block: clears what the others add into and publishes the first round's key range
+        if (nblk == 1) return;
+        auto clear = [&] {
+            for (uint32_t i = threadIdx.x; i < kRZeroWords / 4; i += kRThreads) store16_agent(mem + i * 4, u4a{0u, 0u, 0u, 0u});
+            if (threadIdx.x == 0) {
+                st_agent(st + S_OK, 0u);
+                st_agent(st + S_TIMEOUT, 0u);
+            }
+        };
+        SampleWindow win = {0u, 0x7FFFFFFFu, 0u};
+        if (bn >= kRSampleMin) win = sample_window<kRThreads>(gbase, rbase, bn, k, L.s, clear);
+        else clear();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0) store16_agent(st + S_LO_KEY, u4a{win.lo, win.hi, 0u, published});
+        return;
+    }
+    const uint32_t x = blockIdx.x - 1;
+    if (x >= nblk) return;
+    const uint64_t b0 = (uint64_t)x * PER;                       // the block's first element
+    const uint32_t e0 = (uint32_t)wave * (256 * V) + 4 * lane;   // this lane's first element, from b0; vector u is 256 u further
+    const bool full = b0 + PER <= bn;
+    uint32_t* out = bucket_wire(g, bk, b);
+
+    // ---- load: grad + residual, once ----------------------------------------------------------
+    u4a a[V];
+    {
+        // wave-uniform bases: the lanes only differ by a 32-bit offset
+        const float* gp = gbase + b0 + (uint32_t)wave * (256 * V);
+        const float* rp = rbase + b0 + (uint32_t)wave * (256 * V);
+        const uint32_t l4 = 4 * lane;
+        const uint32_t left = full ? PER : (uint32_t)(bn - b0);
+        auto load = [&](auto whole) {
+            constexpr bool WHOLE = decltype(whole)::value;
+            u4a rv[V];
+#pragma unroll
+            for (int u = 0; u < V; u++) {
+                a[u] = rv[u] = u4a{0u, 0u, 0u, 0u};
+                if (WHOLE || e0 + 256 * u + 4 <= left) {
+                    a[u] = __builtin_nontemporal_load((const u4u4*)(gp + 256 * u + l4));
+                    rv[u] = __builtin_nontemporal_load((const u4u4*)(rp + 256 * u + l4));
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < V; u++) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) a[u][q] = f2u(u2f(a[u][q]) + u2f(rv[u][q]));
+                if constexpr (!WHOLE) {
+                    // Elements past the bucket's end count as +0.0 at indices above every real one: a zero
+                    // key is the smallest, and ties go to the lower index, so they are never picked.
+                    const uint32_t e = e0 + 256 * u;
+                    if (e < left && e + 4 > left) {  // the bucket's partial vector
+#pragma unroll
+                        for (int q = 0; q < 3; q++)
+                            if (e + q < left) a[u][q] = f2u(gp[256 * u + l4 + q] + rp[256 * u + l4 + q]);
+                    }
+                }
+            }
+        };
+        if (full) load(std::true_type{});
+        else load(std::false_type{});
+    }
+    // Vector u of the lane.  Every pass over the elements starts each vector with a value the compiler
+    // knows nothing about: it would otherwise carry derived values (keys, comparisons) of all the
+    // vectors from one pass to the next, in registers that are not there.
+    auto vec = [&](int u) -> u4a {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" : "+v"(a[u]));
+        return a[u];
+    };
+    auto give_up = [&] { fused_give_up(w, st, out); };
+
+    // ---- rounds -----------------------------------------------------------------------------------
+    uint32_t base = 0, span = 0x80000000u;  // keys base .. base + span - 1
+    bool window = false;
+    if (nblk > 1) {
+        if (threadIdx.x == 0) {
+            const u4a wn = wait_window(st, epoch, limit_ticks);
+            L.win[0] = wn[0]; L.win[1] = wn[1]; L.win[3] = wn[3];
+        }
+        __syncthreads();
+        if (!L.win[3]) {
+            give_up();
+            return;
+        }
+        base = L.win[0];
+        span = L.win[1] - L.win[0] + 1;
+        window = span != 0x80000000u;
+    }
+    uint32_t r = k;         // picks still to place among the keys of the range and above it
+    bool first = true;      // the keys above the range are not accounted for in r yet
+    uint32_t bar = 0, sh, bin, m, row = 0;
+    for (;;) {
+        sh = 32 - __clz(span - 1);
+        if (span == 1) sh = 0;
+        sh = sh > 11 ? sh - 11 : 0;
+        for (int i = threadIdx.x; i < (kRBins + 4) / 4; i += kRThreads) ((u4a*)L.lh)[i] = u4a{0u, 0u, 0u, 0u};
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < V; u++) {
+            const u4a v = vec(u);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const uint32_t d = (v[q] & 0x7FFFFFFFu) - base;
+                if ((int)d >= 0) atomicAdd(&L.lh[d < span ? d >> sh : (uint32_t)kRBins], 1u);
+            }
+        }
+        __syncthreads();
+        // two bins per thread, counted from the top: thread 0 owns the highest two
+        u2a all = ((const u2a*)L.lh)[kRThreads - 1 - threadIdx.x];
+        uint32_t above = first ? L.lh[kRBins] : 0u;
+        if (nblk > 1) {
+            uint32_t* const gh = mem + row * kRRow;
+            for (uint32_t i = threadIdx.x; i <= (uint32_t)kRBins; i += kRThreads) {
+                const uint32_t c = L.lh[i];
+                if (c) __hip_atomic_fetch_add(gh + i, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (!resident_barrier(mem + kRBar + 64 * bar, nblk, &L.flag, limit_ticks)) {
+                give_up();
+                return;
+            }
+            bar++;
+            row++;
+            const uint64_t two = ld_agent64((const uint64_t*)gh + (kRThreads - 1 - threadIdx.x));
+            above = first ? ld_agent(gh + kRBins) : 0u;
+            all = u2a{(uint32_t)two, (uint32_t)(two >> 32)};
+        }
+        const uint32_t total = pick_bin2(all, above, r, L.scratch, L.pick);
+        if (window && first && (r <= above || r > above + total)) {  // the sample misled: every key, from the start
+            base = 0;
+            span = 0x80000000u;
+            window = false;
+            continue;
+        }
+        bin = L.pick[0];
+        r = L.pick[1];
+        m = L.pick[2];
+        first = false;
+        base += bin << sh;
+        const uint32_t left = span - (bin << sh);
+        span = left < (1u << sh) ? left : 1u << sh;
+        if (m <= (uint32_t)kRList || span == 1) break;
+        __syncthreads();
+    }
+
+    // ---- the picked bin -----------------------------------------------------------------------------
+    const bool tied = m > (uint32_t)kRList;  // one key, more often than the list holds: ties by index
+    const uint32_t eq = L.lh[bin];           // this block's elements in the bin
+    uint32_t gt;                             // ... and above it
+    {
+        const u2a own = ((const u2a*)L.lh)[threadIdx.x];
+        uint32_t s = threadIdx.x == 0 ? L.lh[kRBins] : 0u;
+#pragma unroll
+        for (int q = 0; q < 2; q++) s += 2 * threadIdx.x + q > bin ? own[q] : 0u;
+        gt = block_sum(s, L.scratch);
+    }
+    uint32_t T, istar, before;  // picks: key > T, or key == T and index <= istar; picks of earlier blocks
+    {
+        uint64_t* const cnts = (uint64_t*)(mem + kRCnt);
+        if (threadIdx.x == 0) {
+            L.count = 0;
+            if (nblk > 1) {
+                st_agent64(cnts + x, ((uint64_t)gt << 32) | eq);
+                if (!tied && eq)
+                    L.base = __hip_atomic_fetch_add(mem + kRBar + 64 * kRBars, eq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        __syncthreads();
+        if (!tied && eq) {  // block-uniform
+#pragma unroll
+            for (int u = 0; u < V; u++) {
+                const u4a v = vec(u);
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const uint32_t key = v[q] & 0x7FFFFFFFu;
+                    if (key - base < span) {
+                        const uint32_t i = atomicAdd(&L.count, 1u);
+                        // larger is picked earlier: key, then lower index
+                        if (i < (uint32_t)kRList) L.list[i] = ((uint64_t)key << 32) | (uint32_t)~((uint32_t)b0 + e0 + 256 * u + q);
+                    }
+                }
+            }
+            __syncthreads();
+            if (nblk > 1) {
+                uint64_t* gl = (uint64_t*)(mem + kRListAt) + L.base;
+                for (uint32_t i = threadIdx.x; i < eq && L.base + i < (uint32_t)kRList; i += kRThreads) st_agent64(gl + i, L.list[i]);
+            }
+        }
+        uint32_t gt_before = 0, eq_before = 0;
+        if (nblk > 1) {
+            if (!resident_barrier(mem + kRBar + 64 * bar, nblk, &L.flag, limit_ticks)) {
+                give_up();
+                return;
+            }
+            const uint64_t c = threadIdx.x < x ? ld_agent64(cnts + threadIdx.x) : 0ull;
+            static_assert(kRList <= kRThreads, "one entry per thread");
+            if (!tied && threadIdx.x < m) L.list[threadIdx.x] = ld_agent64((const uint64_t*)(mem + kRListAt) + threadIdx.x);
+            gt_before = block_sum((uint32_t)(c >> 32), L.scratch);
+            if (tied) eq_before = block_sum((uint32_t)c, L.scratch);
+        }
+        if (!tied) {
+            // The r-th largest entry.  A long list is split once more first: 2048 bins over its key range,
+            // and only the bin that holds the entry is ranked, by counting for each of its entries the larger
+            // ones (1024 entries ranked that way take 10 us, a few dozen less than one).
+            const uint64_t me = threadIdx.x < m ? L.list[threadIdx.x] : 0ull;
+            const uint64_t* ranked = L.list;
+            uint32_t rm = m, rr = r;
+            bool in = threadIdx.x < m;
+            if (m > (uint32_t)kRRank && span > 1) {  // block-uniform
+                sh = 32 - __clz(span - 1);
+                sh = sh > 11 ? sh - 11 : 0;
+                ((u2a*)L.lh)[threadIdx.x] = u2a{0u, 0u};
+                if (threadIdx.x == 0) L.count = 0;
+                __syncthreads();
+                const uint32_t mybin = ((uint32_t)(me >> 32) - base) >> sh;
+                if (in) atomicAdd(&L.lh[mybin], 1u);
+                __syncthreads();
+                pick_bin2(((const u2a*)L.lh)[kRThreads - 1 - threadIdx.x], 0u, r, L.scratch, L.pick);
+                in = in && mybin == L.pick[0];
+                if (in) L.sub[atomicAdd(&L.count, 1u)] = me;
+                rr = L.pick[1];
+                rm = L.pick[2];
+                ranked = L.sub;
+                __syncthreads();
+            }
+            if (in) {
+                uint32_t rank = 0;
+#pragma unroll 4
+                for (uint32_t j = 0; j < rm; j++) rank += ranked[j] > me ? 1u : 0u;
+                if (rank == rr - 1) L.cut = me;
+            }
+            __syncthreads();
+            const uint64_t cut = L.cut;
+            T = (uint32_t)(cut >> 32);
+            istar = ~(uint32_t)cut;
+            const uint32_t mine = threadIdx.x < m && me >= cut && ~(uint32_t)me < (uint32_t)b0 ? 1u : 0u;
+            before = gt_before + block_sum(mine, L.scratch);
+        } else {
+            T = base;
+            const uint32_t quota = r > eq_before ? (r - eq_before < eq ? r - eq_before : eq) : 0u;
+            before = gt_before + (eq_before < r ? eq_before : r);
+            istar = 0xFFFFFFFFu;
+            if (quota == 0) {
+                T = base + 1;
+            } else if (quota < eq) {
+                // the one block in which the ties run out: the quota-th of its equal keys, from a bit per element
+                __syncthreads();
+                if (threadIdx.x < PER / 32) L.lh[threadIdx.x] = 0;
+                __syncthreads();
+#pragma unroll
+                for (int u = 0; u < V; u++) {
+                    const u4a v = vec(u);
+                    uint32_t nib = 0;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) nib |= ((v[q] & 0x7FFFFFFFu) == base ? 1u : 0u) << q;
+                    const uint32_t e = e0 + 256 * u;
+                    if (nib) atomicOr(&L.lh[e >> 5], nib << (e & 31));
+                }
+                __syncthreads();
+                uint32_t bitsleft = threadIdx.x < PER / 32 ? L.lh[threadIdx.x] : 0u, tot;
+                const uint32_t c = __popc(bitsleft);
+                const uint32_t run = block_scan(c, L.scratch, &tot);
+                if (run < quota && quota <= run + c) {
+                    for (uint32_t n = quota - run; n > 1; n--) bitsleft &= bitsleft - 1;
+                    L.flag = (uint32_t)b0 + 32 * threadIdx.x + (uint32_t)__ffs((int)bitsleft) - 1u;
+                }
+                __syncthreads();
+                istar = L.flag;
+            }
+        }
+    }
+
+    // ---- picks: a bit per element, prefix sums over words of 32, then residual and payload ------
+    constexpr uint32_t WORDS = PER / 32;
+    static_assert(WORDS <= kRThreads && WORDS <= kRBins, "one word per thread");
+    __syncthreads();
+    if (threadIdx.x < WORDS) L.lh[threadIdx.x] = 0;
+    __syncthreads();
+    uint32_t nibs = 0;
+#pragma unroll
+    for (int u = 0; u < V; u++) {
+        const u4a v = vec(u);
+        const uint32_t e = e0 + 256 * u;
+        uint32_t nib = 0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint32_t key = v[q] & 0x7FFFFFFFu;
+            nib |= (key >= T + ((uint32_t)b0 + e + q > istar ? 1u : 0u) ? 1u : 0u) << q;
+        }
+        nibs |= nib << (4 * u);
+        if (nib) atomicOr(&L.lh[e >> 5], nib << (e & 31));
+    }
+    __syncthreads();
+    {
+        uint32_t total;
+        const uint32_t run = block_scan(threadIdx.x < WORDS ? __popc(L.lh[threadIdx.x]) : 0u, L.scratch, &total);
+        if (threadIdx.x < WORDS) L.pre[threadIdx.x] = before + run;
+    }
+    __syncthreads();
+    float* const rp = rbase + b0 + (uint32_t)wave * (256 * V);
+    const uint32_t l4 = 4 * lane;
+    const uint32_t left = full ? PER : (uint32_t)(bn - b0);
+#pragma unroll
+    for (int u = 0; u < V; u++) {
+        const u4a v = vec(u);
+        const uint32_t e = e0 + 256 * u;
+        const uint32_t nib = (nibs >> (4 * u)) & 15u;
+        u4a z;
+#pragma unroll
+        for (int q = 0; q < 4; q++) z[q] = nib >> q & 1u ? 0u : v[q];
+        if (e + 4 <= left) __builtin_nontemporal_store(z, (u4u4*)(rp + 256 * u + l4));
+        else if (e < left) {
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+                if (e + q < left) rp[256 * u + l4 + q] = u2f(z[q]);
+        }
+        if (nib) {
+            uint32_t pos = L.pre[e >> 5] + __popc(L.lh[e >> 5] & ((1u << (e & 31)) - 1u));
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                if ((nib >> q & 1u) && pos < k) {  // (pos < k whatever the scratch memory held)
+                    const u2a pr = {(uint32_t)b0 + e + q, v[q]};
+                    *(u2a4*)(out + 1 + 2 * (uint64_t)pos) = pr;
+                    pos++;
+                }
+            }
+        }
+    }
+    if (x == 0 && threadIdx.x == 0) {
+        st[S_T] = T;
+        st[S_ISTAR] = istar;
+        st[S_READY] = 0u;  // a replay of a captured launch carries the same epoch
+        if (nblk == 1) st[S_TIMEOUT] = 0u;
+        st[S_OK] = 1u;
+        if (nblk == 1 || !ld_agent(st + S_TIMEOUT)) out[0] = k;
+    }
+}
+
+template <int V>
+void launch(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t epoch, uint32_t published,
+            uint64_t limit, hipStream_t st) {
+    constexpr uint64_t per = (uint64_t)kRThreads * 4 * V;
+    const uint32_t gx = (uint32_t)((g.bucket_elems + per - 1) / per) + 1;
+    k_topk_resident<V><<<dim3(gx, g.nbuckets), kRThreads, 0, st>>>(bk, g, w, epoch, published, limit);
+}
+
+}  // namespace
+
+// Vectors per thread for buckets of up to n elements.  The barriers cost more with more blocks, the
+// passes over a block's elements with more vectors; measured (one bucket, 1 %): 200,000 elements
+// 17.9 / 19.8 / 28.1 us with 1 / 2 / 4 vectors, 524,288 elements 22.4 / 20.6 / 21.2 us.
+int resident_vecs(uint64_t n) { return n <= 64 * 4096 ? 1 : n <= 64 * 8192 ? 2 : 4; }
+
+void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t epoch, uint32_t published,
+                     uint64_t limit_ticks, hipStream_t st) {
+    switch (resident_vecs(g.bucket_elems)) {
+        case 1: launch<1>(bk, g, w, epoch, published, limit_ticks, st); break;
+        case 2: launch<2>(bk, g, w, epoch, published, limit_ticks, st); break;
+        default: launch<4>(bk, g, w, epoch, published, limit_ticks, st); break;
+    }
+}
+
+}  // namespace mcclhip
