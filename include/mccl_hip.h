@@ -41,6 +41,7 @@ extern "C" {
 #define MCCL_HIP_ERR_WORKSPACE (-8) /* workspace smaller than mccl_hip_topk_workspace_bytes()       */
 #define MCCL_HIP_ERR_TIMEOUT (-9)   /* fence wait exceeded its limit (csrc/metal/EventSync.mm:37-71) */
 #define MCCL_HIP_ERR_POINTER (-10)  /* the bytes are not memory a kernel on the current GPU can reach */
+#define MCCL_HIP_ERR_ORDER (-11)    /* mccl_hip_topk_decompress_sorted: indices do not ascend      */
 
 /* ---- element types (at::ScalarType values) ------------------------------ */
 #define MCCL_HIP_U8 0
@@ -222,6 +223,15 @@ int mccl_hip_topk_path_report(const void* workspace, uint64_t n_total, uint64_t 
  * skipped.  status may be NULL. */
 int mccl_hip_topk_decompress(const void* wire, uint64_t wire_bytes, float* dense, uint64_t count,
                              int* status, void* stream);
+
+/* mccl_hip_topk_decompress for payloads whose indices ascend strictly (what
+ * compress emits), in one launch.  `status` (required; device memory or pinned
+ * host memory, zeroed by the caller) receives what mccl_hip_topk_decompress
+ * would report, or MCCL_HIP_ERR_ORDER when the indices do not ascend; unless it
+ * stays 0 the contents of dense are unspecified, and a caller that has to accept
+ * such payloads calls mccl_hip_topk_decompress. */
+int mccl_hip_topk_decompress_sorted(const void* wire, uint64_t wire_bytes, float* dense, uint64_t count,
+                                    int* status, void* stream);
 
 /* Decompress + accumulate of `ws` ranks' payloads into one dense buffer, the
  * sparse equivalent of decompressing every peer's payload and folding the

@@ -93,21 +93,33 @@ at::Tensor& TopKCompressor::residual_for(uint64_t stable_id, size_t count) {
     return error_buffers_[stable_id];
 }
 
-// The device word the compress launches report a give-up through (a block of the single-pass
-// path that waited too long for another block of its launch).  The launches are asynchronous,
-// so the word is looked at by the calls that wait for the stream anyway: decompress() and
-// check_compress_status().  Caller holds mu_.
+namespace {
+// One int in pinned host memory: kernels write it where it lies, the host reads it after a stream
+// wait with no copy of its own (a device word costs a copy kernel and a second wait per read).
+at::Tensor pinned_word() {
+    return at::zeros({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+}
+int read_word(const at::Tensor& t) { return *static_cast<const volatile int*>(t.data_ptr<int>()); }
+
+void wait_for_current_stream() {
+    throw_on_status(mccl_hip_sync(c10::hip::getCurrentHIPStream().stream()), "TopK stream wait");
+}
+}  // namespace
+
+// The word the compress launches report a give-up through (a block of a launch that waited too
+// long for another block of it).  The launches are asynchronous, so the word is looked at by the
+// calls that wait for the stream anyway: decompress() and check_compress_status().  Caller holds mu_.
 int* TopKCompressor::compress_status() {
-    if (!compress_status_.defined())
-        compress_status_ = at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(at::kCUDA));
+    if (!compress_status_.defined()) compress_status_ = pinned_word();
     return compress_status_.data_ptr<int>();
 }
 
+// The current stream has been waited for.
 void TopKCompressor::throw_if_compress_failed() {
     if (!compress_status_.defined()) return;
-    const int st = compress_status_.item<int>();
+    const int st = read_word(compress_status_);
     if (st == 0) return;
-    compress_status_.zero_();
+    *compress_status_.data_ptr<int>() = 0;
     if (st == MCCL_HIP_ERR_TIMEOUT)
         throw TimeoutError("TopK compress: a block gave up waiting for another block of its launch; "
                            "the payloads of that call are invalid");
@@ -116,6 +128,8 @@ void TopKCompressor::throw_if_compress_failed() {
 
 void TopKCompressor::check_compress_status() {
     std::lock_guard<std::mutex> lock(mu_);
+    if (!compress_status_.defined()) return;
+    wait_for_current_stream();
     throw_if_compress_failed();
 }
 
@@ -216,22 +230,29 @@ std::vector<at::Tensor> TopKCompressor::compress_many(const std::vector<at::Tens
 }
 
 // csrc/compression/TopKCompression.cpp:122-152.  The reference validates while
-// it scatters and throws; here the kernel reports through a device flag that
-// is read back once the stream has drained (the call is synchronous, as the
-// reference's is).
+// it scatters and throws; here the kernel reports through a word in host memory
+// that is read once the stream has drained (the call is synchronous, as the
+// reference's is).  A payload that does not ascend, or that breaks a rule, is
+// expanded (again) by the kernels that take pairs in any order.
 void TopKCompressor::decompress(const void* src, size_t compressed_size, void* dst, size_t nbytes,
                                 at::ScalarType dtype) {
     MCCL_CHECK(dtype == at::kFloat, "TopK decompression currently supports float32 only");
     const size_t count = nbytes / sizeof(float);
     std::lock_guard<std::mutex> lock(mu_);
     metal_kernels_init();
-    if (!status_.defined()) status_ = at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(at::kCUDA));
-    status_.zero_();
-    const int rc = mccl_hip_topk_decompress(src, compressed_size, static_cast<float*>(dst), count,
-                                            status_.data_ptr<int>(), c10::hip::getCurrentHIPStream().stream());
-    if (rc == MCCL_HIP_ERR_SIZE) throw MCCLError("TopK decompress: size mismatch");
-    throw_on_status(rc, "TopK decompress");
-    const int st = status_.item<int>();
+    if (!status_.defined()) status_ = pinned_word();
+    int* const word = status_.data_ptr<int>();
+    void* const stream = c10::hip::getCurrentHIPStream().stream();
+    auto expand = [&](auto fn) {
+        *word = 0;
+        const int rc = fn(src, compressed_size, static_cast<float*>(dst), count, word, stream);
+        if (rc == MCCL_HIP_ERR_SIZE) throw MCCLError("TopK decompress: size mismatch");
+        throw_on_status(rc, "TopK decompress");
+        wait_for_current_stream();
+        return read_word(status_);
+    };
+    int st = count ? expand(mccl_hip_topk_decompress_sorted) : MCCL_HIP_ERR_ORDER;
+    if (st != 0) st = expand(mccl_hip_topk_decompress);
     throw_if_compress_failed();
     if (st == MCCL_HIP_ERR_SIZE) throw MCCLError("TopK decompress: size mismatch");
     if (st == MCCL_HIP_ERR_INDEX) throw MCCLError("TopK decompress: index out of bounds");

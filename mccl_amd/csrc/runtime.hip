@@ -79,6 +79,7 @@ const char* mccl_hip_strerror(int code) {
         case MCCL_HIP_ERR_WORKSPACE: return "workspace too small";
         case MCCL_HIP_ERR_TIMEOUT: return "fence wait timed out";
         case MCCL_HIP_ERR_POINTER: return "pointer is not GPU-accessible memory";
+        case MCCL_HIP_ERR_ORDER: return "payload indices do not ascend";
         default: return "unknown error";
     }
 }

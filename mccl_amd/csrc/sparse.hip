@@ -60,6 +60,77 @@ __global__ __launch_bounds__(kBlock) void k_scatter(const uint32_t* wire, uint32
     }
 }
 
+// ---- decompress of an ascending payload in one launch ---------------------------------
+// A block owns a tile of the dense buffer: zeroed in LDS, given the pairs that fall inside it,
+// written once.  It finds its pairs without a search: every block reads the same kSamples evenly
+// spaced indices, counts those below its first element (s) and below its end (u), and takes the
+// strides from sample s - 1 up to sample u - its own pairs and a few neighbours'.  Two dependent
+// round trips (samples, pairs) and the stores; fill and scatter are two launches and write the
+// picked lines twice.  6,553,600 elements, 65,536 pairs: 6.1 us in the kernel against 5.9 + 3.2 and
+// the launch between them.
+// Whether the payload ascends is checked on the way, by all blocks together: samples ascend, and
+// every block checks the adjacent pairs of its strides and the one that links them to the next
+// stride; the last strides of a block are the first of the next one (u of a tile is s of the next),
+// so every adjacent pair is looked at by somebody.
+constexpr int kDecTile = 8192;
+constexpr int kDecSamples = kBlock;      // one per thread
+constexpr uint32_t kDecMaxStride = 4096;  // beyond (over a million pairs) fill and scatter are as fast
+
+__global__ __launch_bounds__(kBlock) void k_decompress_sorted(const uint32_t* wire, uint32_t k, uint32_t stride, float* dense,
+                                                              uint64_t count, int* status) {
+    __shared__ __attribute__((aligned(16))) float tile[kDecTile];
+    __shared__ uint32_t samp[kDecSamples + 1];
+    __shared__ uint32_t below[2];
+    const uint64_t t0 = (uint64_t)blockIdx.x * kDecTile;
+    const uint64_t t1 = t0 + kDecTile < count ? t0 + kDecTile : count;
+    const uint32_t* const pairs = wire + 1;
+    const uint64_t mypos = (uint64_t)threadIdx.x * stride;
+    const uint32_t have_k = wire[0];
+    const uint32_t mine = mypos < k ? pairs[2 * mypos] : 0xFFFFFFFFu;
+#pragma unroll
+    for (int i = 0; i < kDecTile / (4 * kBlock); i++) ((u4a*)tile)[i * kBlock + threadIdx.x] = u4a{0u, 0u, 0u, 0u};
+    if (threadIdx.x < 2) below[threadIdx.x] = 0;
+    if (threadIdx.x == 0) samp[kDecSamples] = 0xFFFFFFFFu;
+    samp[threadIdx.x] = mine;
+    if (have_k != k) {  // the same in every lane of the grid
+        if (blockIdx.x == 0 && threadIdx.x == 0) *status = MCCL_HIP_ERR_SIZE;
+        return;
+    }
+    __syncthreads();
+    int bad = 0;
+    if (mypos + stride < k && mine >= samp[threadIdx.x + 1]) bad = MCCL_HIP_ERR_ORDER;
+    // (a position past the payload reads 0xFFFFFFFF and counts as beyond every element)
+    const uint64_t ms = __ballot(mypos < k && mine < t0), mu = __ballot(mypos < k && mine < t1);
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        if (ms) atomicAdd(&below[0], (uint32_t)__popcll(ms));
+        if (mu) atomicAdd(&below[1], (uint32_t)__popcll(mu));
+    }
+    __syncthreads();
+    const uint64_t s = below[0], u = t1 == count ? kDecSamples : below[1];  // the last tile takes what is left
+    const uint64_t p0 = (s ? s - 1 : 0) * stride;
+    uint64_t p1 = u * stride;
+    if (p1 > k) p1 = k;
+    for (uint64_t p = p0 + threadIdx.x; p < p1; p += kBlock) {
+        const u2a pr = *(const u2a4*)(pairs + 2 * p);
+        const uint32_t next = p + 1 < k ? pairs[2 * (p + 1)] : 0xFFFFFFFFu;
+        if (p + 1 < k && pr[0] >= next) bad = MCCL_HIP_ERR_ORDER;
+        if (pr[0] >= count) bad = bad ? bad : MCCL_HIP_ERR_INDEX;
+        const uint64_t off = (uint64_t)pr[0] - t0;
+        if (off < t1 - t0) tile[off] = u2f(pr[1]);
+    }
+    if (bad) *status = bad;
+    __syncthreads();
+    float* const out = dense + t0;
+    const uint32_t len = (uint32_t)(t1 - t0);
+    if (len == (uint32_t)kDecTile) {
+#pragma unroll
+        for (int i = 0; i < kDecTile / (4 * kBlock); i++)
+            *(u4u4*)(out + 4 * (i * kBlock + threadIdx.x)) = ((const u4a*)tile)[i * kBlock + threadIdx.x];
+    } else {
+        for (uint32_t i = threadIdx.x; i < len; i += kBlock) out[i] = tile[i];
+    }
+}
+
 struct WirePtrs {
     const uint8_t* w[MCCL_HIP_MAX_WORLD];
 };
@@ -701,6 +772,23 @@ int mccl_hip_topk_decompress(const void* wire, uint64_t wire_bytes, float* dense
     }
     k_scatter<<<clamp_u32((k64 + kBlock - 1) / kBlock, 1, cap), kBlock, 0, st>>>(
         (const uint32_t*)wire, (uint32_t)k64, dense, count, status);
+    return launch_status();
+}
+
+int mccl_hip_topk_decompress_sorted(const void* wire, uint64_t wire_bytes, float* dense, uint64_t count,
+                                    int* status, void* stream) {
+    if (!wire || !dense || !status || ((uintptr_t)wire & 3)) return MCCL_HIP_ERR_ARG;
+    if (count == 0 || count > 0xFFFFFFFFull) return MCCL_HIP_ERR_ARG;
+    if (wire_bytes < 4 || ((wire_bytes - 4) & 7)) return MCCL_HIP_ERR_SIZE;
+    const uint64_t k = (wire_bytes - 4) / 8;
+    if (k > 0xFFFFFFFFull) return MCCL_HIP_ERR_SIZE;
+    int rc = mccl_hip_init();
+    if (rc) return rc;
+    const uint64_t stride = k ? (k + kDecSamples - 1) / kDecSamples : 1;
+    if (stride > kDecMaxStride)
+        return mccl_hip_topk_decompress(wire, wire_bytes, dense, count, status, stream);
+    k_decompress_sorted<<<(uint32_t)((count + kDecTile - 1) / kDecTile), kBlock, 0, (hipStream_t)stream>>>(
+        (const uint32_t*)wire, (uint32_t)k, (uint32_t)stride, dense, count, status);
     return launch_status();
 }
 

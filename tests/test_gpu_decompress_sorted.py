@@ -1,0 +1,79 @@
+"""TopKCompressor.decompress (one launch for ascending payloads, the order-free kernels behind it)
+against the oracle at the edges of its tiles (8192 elements) and of its 256 samples, for spread,
+clustered, unordered and repeated indices, and for indices past the end."""
+import ctypes as ct
+
+import numpy as np
+import pytest
+import torch
+import torch.distributed  # noqa: F401
+
+import oracle
+from oracle import F32
+from tests._gpu_util import DEV, to_np, bits
+
+pytestmark = pytest.mark.gpu
+
+
+def _payload(idx, val):
+    w = np.empty(1 + 2 * idx.size, np.uint32)
+    w[0] = idx.size
+    w[1::2] = idx
+    w[2::2] = val.view(np.uint32)
+    return w.view(np.uint8)
+
+
+def _status(wire, n):
+    from mccl_amd import _lib
+    dense = torch.full((n,), 3.0, device=DEV)
+    st = torch.zeros(1, dtype=torch.int32, device=DEV)
+    rc = _lib.load().mccl_hip_topk_decompress_sorted(ct.c_void_p(wire.data_ptr()), wire.numel(), ct.c_void_p(dense.data_ptr()), n,
+                                                    ct.c_void_p(st.data_ptr()), None)
+    torch.cuda.synchronize()
+    return rc, int(st), dense
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (8191, 1), (8192, 8192), (8193, 255), (8193, 256), (16_385, 257),
+                                 (70_001, 700), (1_000_003, 10_000), (3_000_001, 150_001)])
+def test_ascending_payloads(n, k):
+    from mccl_amd import _C
+    rng = np.random.default_rng(n + k)
+    comp = _C.TopKCompressor(min(1.0, (k + 0.5) / n))
+    spread = np.sort(rng.choice(n, k, replace=False)).astype(np.uint32)
+    for idx in (spread, np.arange(k, dtype=np.uint32), np.arange(n - k, n, dtype=np.uint32)):
+        w = _payload(idx, rng.standard_normal(k).astype(np.float32))
+        want, rc = oracle.topk_decompress(w, n)
+        assert rc == 0
+        dw = torch.from_numpy(w).to(DEV)
+        rc, st, dense = _status(dw, n)
+        assert (rc, st) == (0, 0) and np.array_equal(bits(to_np(dense, F32)), bits(want))
+        assert np.array_equal(bits(to_np(comp.decompress(dw, n), F32)), bits(want))
+
+
+@pytest.mark.parametrize("k", [2, 300, 20_000])
+def test_unordered_payloads_take_the_other_kernels(k):
+    from mccl_amd import _C
+    n = 100_003
+    rng = np.random.default_rng(k)
+    comp = _C.TopKCompressor(min(1.0, (k + 0.5) / n))
+    idx = np.sort(rng.choice(n, k, replace=False)).astype(np.uint32)
+    val = rng.standard_normal(k).astype(np.float32)
+    for at in {0, (k - 1) // 2, k - 2}:
+        sw = idx.copy()
+        sw[at], sw[at + 1] = idx[at + 1], idx[at]     # one pair of neighbours exchanged
+        rep = idx.copy()
+        rep[at + 1] = idx[at]                         # one index twice, with the same value
+        same = val.copy()
+        same[at + 1] = val[at]
+        for i, v in ((sw, val), (rep, same)):
+            w = _payload(i, v)
+            want, _ = oracle.topk_decompress(w, n)
+            dw = torch.from_numpy(w).to(DEV)
+            assert _status(dw, n)[1] == -11
+            assert np.array_equal(bits(to_np(comp.decompress(dw, n), F32)), bits(want))
+    w = torch.from_numpy(_payload(idx, val)).to(DEV)
+    assert _status(w, int(idx[-1]))[1] == oracle.ERR_INDEX
+    with pytest.raises(RuntimeError, match="index out of bounds"):
+        comp.decompress(w, int(idx[-1]))
+    w[:4] = 0
+    assert _status(w, n)[1] == oracle.ERR_SIZE
