@@ -2,11 +2,9 @@
 // applies to every inbound chunk, the AVG scale, the fused add+scale, and the
 // W-way fold in ring-step order.
 //
-// All of them are HBM-bound streaming kernels: 256-thread blocks, every lane
-// moves 16 bytes per access (global_load/store_dwordx4), a few independent
-// accesses per operand are issued before the first use, and the grid is sized
-// to keep every CU's wave slots full.  The destination is peeled to 16-byte
-// alignment; sources are read with element alignment only, because chunk views
+// All of them are HBM-bound streaming kernels: every lane moves 16 bytes per
+// access (global_load/store_dwordx4), one tile per block in address order.
+// The destination is peeled to 16-byte alignment; sources are read with element alignment only, because chunk views
 // start at arbitrary element offsets (csrc/backend/ProcessGroupMCCL.cpp:1735-1741).
 //
 // Arithmetic follows the reference's CPU folds (csrc/metal/AccelerateOps.mm):
@@ -22,12 +20,18 @@ namespace mcclhip {
 
 namespace {
 
-// Vectors in flight per thread and operand.  Measured on MI355X over 96.5 M elements (fraction
-// of the 8 TB/s peak): the binary folds are fastest with one (fold 0.81 against 0.78 with four,
-// scale 0.86 against 0.77: a 1024-element tile per block keeps the set of tiles in flight one
-// narrow address front); the ring fold with one for three ranks (0.76 against 0.73), eight for
-// six and seven ranks (0.71 against 0.70) and four otherwise.
-constexpr int kUnroll = 1;
+// Binary fold of two 96.5 M-element fp32 arrays that no cache holds: 176 us, 6.58 TB/s of 12 B/element
+// (217 us with 256-thread blocks, a 64-bit index per lane and a grid capped at 65,536 blocks); the
+// folds of a ring step as one list of 120: 178 us (223).
+// Threads per block of the binary folds.  One wavefront per block, one 16-byte vector per lane and
+// operand: the set of tiles in flight is one narrow address front, and what a wavefront executes
+// beside its three memory instructions is kept to a handful of scalar ones - a block of this size
+// moves 3 KiB, so every further instruction shows.  Measured on a bare dst += src over 402 MB
+// arrays: 178 / 181 / 187 / 190 us with 64 / 128 / 256 / 1024 threads, 185 and 193 with two and
+// four vectors per lane.
+constexpr int kFoldBlock = 64;
+// Vectors in flight per thread and rank buffer of the ring fold: one for three ranks (0.76 of the
+// 8 TB/s peak against 0.73), eight for six and seven ranks (0.71 against 0.70), four otherwise.
 constexpr int ring_unroll(int ws) { return ws == 3 ? 1 : ((ws == 6 || ws == 7) ? 8 : 4); }
 
 template <bool NT>
@@ -40,6 +44,9 @@ __device__ __forceinline__ u4a load_vec_u(const void* p) {
     if constexpr (ES == 4) {
         if constexpr (NT) return __builtin_nontemporal_load((const u4u4*)p);
         else return *(const u4u4*)p;
+    } else if constexpr (ES == 1) {
+        if constexpr (NT) return __builtin_nontemporal_load((const u4u1*)p);
+        else return *(const u4u1*)p;
     } else {
         if constexpr (NT) return __builtin_nontemporal_load((const u4u2*)p);
         else return *(const u4u2*)p;
@@ -85,92 +92,7 @@ __device__ __forceinline__ void fold_elem(void* dst, const void* src, uint64_t i
     }
 }
 
-// ---- binary fold / scale / fused ----------------------------------------------
-// Layout: [head scalars][nvec 16-byte vectors][tail scalars]; head makes the
-// destination 16-byte aligned.
-// block `block` of `nblocks` takes its share of one fold
-template <int DT, int OP, int KIND, bool NT>
-__device__ __forceinline__ void fold2_block(void* dst, const void* src, uint64_t n, float scale, uint32_t head,
-                                            uint64_t nvec, uint32_t block, uint32_t nblocks) {
-    constexpr int ES = ElemInfo<DT>::size;
-    constexpr int EPV = ElemInfo<DT>::per_vec;
-    u4a* dv = (u4a*)((char*)dst + (uint64_t)head * ES);
-    const char* sv = (const char*)src + (uint64_t)head * ES;
-    const uint64_t tile = (uint64_t)kBlock * kUnroll;
-    for (uint64_t base = (uint64_t)block * tile; base < nvec; base += (uint64_t)nblocks * tile) {
-        u4a d[kUnroll], s[kUnroll];
-        if (base + tile <= nvec) {
-#pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                uint64_t idx = base + (uint64_t)u * kBlock + threadIdx.x;
-                d[u] = load_vec_a<NT>(dv + idx);
-                if constexpr (KIND != 2) s[u] = load_vec_u<ES, NT>(sv + idx * 16);
-                else s[u] = d[u];
-            }
-#pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                uint64_t idx = base + (uint64_t)u * kBlock + threadIdx.x;
-                u4a r;
-#pragma unroll
-                for (int q = 0; q < 4; q++) r[q] = fold_dword<DT, OP, KIND>(d[u][q], s[u][q], scale);
-                store_vec_a<NT>(dv + idx, r);
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < kUnroll; u++) {
-                uint64_t idx = base + (uint64_t)u * kBlock + threadIdx.x;
-                if (idx < nvec) {
-                    u4a dd = load_vec_a<NT>(dv + idx);
-                    u4a ss = dd;
-                    if constexpr (KIND != 2) ss = load_vec_u<ES, NT>(sv + idx * 16);
-                    u4a r;
-#pragma unroll
-                    for (int q = 0; q < 4; q++) r[q] = fold_dword<DT, OP, KIND>(dd[q], ss[q], scale);
-                    store_vec_a<NT>(dv + idx, r);
-                }
-            }
-        }
-    }
-    // scalar head and tail (fewer than EPV elements each)
-    const uint64_t g = (uint64_t)block * kBlock + threadIdx.x;
-    if (g < head) fold_elem<DT, OP, KIND>(dst, src, g, scale);
-    const uint64_t tail = head + nvec * EPV;
-    if (g < (uint64_t)EPV && tail + g < n) fold_elem<DT, OP, KIND>(dst, src, tail + g, scale);
-}
-
-template <int DT, int OP, int KIND, bool NT>
-__global__ __launch_bounds__(kBlock) void k_fold2(void* dst, const void* src, uint64_t n,
-                                                  float scale, uint32_t head, uint64_t nvec) {
-    fold2_block<DT, OP, KIND, NT>(dst, src, n, scale, head, nvec, blockIdx.x, gridDim.x);
-}
-
-// ---- a list of independent binary folds in one launch ---------------------------
-// blockIdx.y = fold, blockIdx.x strides over that fold's vectors.  The table is read where
-// the launch put it, in the kernel-argument segment, through scalar loads (indexing the
-// by-value parameter would make the compiler copy it to per-lane scratch memory first): it
-// is therefore the only parameter.
-constexpr int kFoldBatch = 128;  // folds per launch
-struct FoldBatch {
-    void* dst[kFoldBatch];
-    const void* src[kFoldBatch];
-    uint64_t n[kFoldBatch];
-};
-template <int DT, int OP, bool NT>
-__global__ __launch_bounds__(kBlock) void k_fold2_batch(FoldBatch) {
-    typedef const __attribute__((address_space(4))) FoldBatch* Arg;
-    const Arg fb = (Arg)__builtin_amdgcn_kernarg_segment_ptr();
-    constexpr int ES = ElemInfo<DT>::size;
-    constexpr int EPV = ElemInfo<DT>::per_vec;
-    void* dst = fb->dst[blockIdx.y];
-    const void* src = fb->src[blockIdx.y];
-    const uint64_t n = fb->n[blockIdx.y];
-    uint64_t head = ((16 - ((uintptr_t)dst & 15)) & 15) / ES;
-    if (head > n) head = n;
-    const uint64_t nvec = (n - head) / EPV;
-    fold2_block<DT, OP, 0, NT>(dst, src, n, 1.0f, (uint32_t)head, nvec, blockIdx.x, gridDim.x);
-}
-
-// ---- integral types (DDP metadata, counters): plain grid-stride ---------------
+// ---- integral types (DDP metadata, counters) ------------------------------------
 // Wrap-around arithmetic, bool folded as raw uint8
 // (csrc/metal/AccelerateOps.mm:206-236, csrc/metal/shaders.metal:554-731).
 template <typename T, int OP>
@@ -181,20 +103,113 @@ __device__ __forceinline__ T fold_int(T d, T s) {
     else if constexpr (OP == kMin) return s < d ? s : d;
     else return s > d ? s : d;
 }
+
+// ---- element kinds of a binary fold: 16 bytes and one element -----------------------
+template <int DT, int OP, int KIND>
+struct FoldFloat {
+    static constexpr int size = ElemInfo<DT>::size;
+    static constexpr bool needs_src = KIND != 2;
+    static __device__ __forceinline__ u4a vec(u4a d, u4a s, float scale) {
+        u4a r;
+#pragma unroll
+        for (int q = 0; q < 4; q++) r[q] = fold_dword<DT, OP, KIND>(d[q], s[q], scale);
+        return r;
+    }
+    static __device__ __forceinline__ void elem(char* d, const char* s, float scale) {
+        fold_elem<DT, OP, KIND>(d, s, 0, scale);
+    }
+};
 template <typename T, int OP>
-__global__ __launch_bounds__(kBlock) void k_fold2_int(T* dst, const T* src, uint64_t n) {
-    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kBlock)
-        dst[i] = fold_int<T, OP>(dst[i], src[i]);
+struct FoldInt {
+    static constexpr int size = sizeof(T);
+    static constexpr bool needs_src = true;
+    static __device__ __forceinline__ u4a vec(u4a d, u4a s, float) {
+        constexpr int N = 16 / sizeof(T);
+        typedef T V __attribute__((ext_vector_type(N)));
+        const V dv = __builtin_bit_cast(V, d), sv = __builtin_bit_cast(V, s);
+        V r;
+#pragma unroll
+        for (int i = 0; i < N; i++) r[i] = fold_int<T, OP>(dv[i], sv[i]);
+        return __builtin_bit_cast(u4a, r);
+    }
+    static __device__ __forceinline__ void elem(char* d, const char* s, float) {
+        *(T*)d = fold_int<T, OP>(*(const T*)d, *(const T*)s);
+    }
+};
+
+// ---- binary fold / scale / fused ----------------------------------------------
+// Layout: [head scalars][nvec 16-byte vectors][tail scalars]; head makes the destination 16-byte
+// aligned; `dst` and `src` point at the body.  The launch computes it (fold_span), so that a
+// wavefront starts with its addresses at hand.
+struct __attribute__((aligned(32))) FoldSpan {
+    char* dst;
+    const char* src;
+    uint64_t nvec;
+    uint16_t head, tail;  // elements, fewer than 16 bytes each
+    uint32_t pad;
+};
+
+template <int ES, bool NT>
+__device__ __forceinline__ u4a load_src(const void* p) {
+    return load_vec_u<(ES == 2 ? 2 : (ES == 1 ? 1 : 4)), NT>(p);
 }
-template <typename T, int OP>
-__global__ __launch_bounds__(kBlock) void k_fold2_batch_int(FoldBatch) {
+
+// Block `block` of `nblocks` of one fold.
+template <class F, bool NT>
+__device__ __forceinline__ void fold_span_block(char* dst, const char* src, uint64_t nvec, uint32_t head, uint32_t tail,
+                                                float scale, uint32_t block, uint32_t nblocks) {
+    const uint32_t off = threadIdx.x * 16u;
+    uint64_t v = (uint64_t)block * kFoldBlock;
+    // (the launch gives a block one round unless the grid is capped)
+    for (; v + kFoldBlock <= nvec; v += (uint64_t)nblocks * kFoldBlock) {
+        char* const dp = dst + v * 16;
+        const u4a d = load_vec_a<NT>((const u4a*)(dp + off));
+        u4a s = d;
+        if constexpr (F::needs_src) s = load_src<F::size, NT>(src + v * 16 + off);
+        store_vec_a<NT>((u4a*)(dp + off), F::vec(d, s, scale));
+    }
+    if (v < nvec && threadIdx.x < nvec - v) {
+        char* const dp = dst + v * 16;
+        const u4a d = load_vec_a<NT>((const u4a*)(dp + off));
+        u4a s = d;
+        if constexpr (F::needs_src) s = load_src<F::size, NT>(src + v * 16 + off);
+        store_vec_a<NT>((u4a*)(dp + off), F::vec(d, s, scale));
+    }
+    if (block + 1 == nblocks && (head | tail)) {  // scalars: at most 15 in front of the body, 15 behind it
+        const uint32_t t = threadIdx.x;
+        constexpr uint32_t EPV = 16 / F::size;
+        if (t < head) {
+            const int64_t o = -(int64_t)((head - t) * F::size);
+            F::elem(dst + o, F::needs_src ? src + o : nullptr, scale);
+        } else if (t >= EPV && t - EPV < tail) {
+            const uint64_t o = nvec * 16 + (uint64_t)(t - EPV) * F::size;
+            F::elem(dst + o, F::needs_src ? src + o : nullptr, scale);
+        }
+    }
+}
+
+template <class F, bool NT>
+__global__ __launch_bounds__(kFoldBlock) void k_fold2(char* dst, const char* src, uint64_t nvec, uint32_t head,
+                                                      uint32_t tail, float scale) {
+    fold_span_block<F, NT>(dst, src, nvec, head, tail, scale, blockIdx.x, gridDim.x);
+}
+
+// ---- a list of independent binary folds in one launch ---------------------------
+// blockIdx.y = fold, blockIdx.x strides over that fold's vectors.  The table is read where
+// the launch put it, in the kernel-argument segment, one 32-byte scalar load per block (indexing
+// the by-value parameter would make the compiler copy it to per-lane scratch memory first): it
+// is therefore the only parameter.
+constexpr int kFoldBatch = 120;  // folds per launch: the kernel arguments stay below 4 KiB
+struct FoldBatch {
+    FoldSpan f[kFoldBatch];
+};
+template <class F, bool NT>
+__global__ __launch_bounds__(kFoldBlock) void k_fold2_batch(FoldBatch) {
     typedef const __attribute__((address_space(4))) FoldBatch* Arg;
     const Arg fb = (Arg)__builtin_amdgcn_kernarg_segment_ptr();
-    T* dst = (T*)fb->dst[blockIdx.y];
-    const T* src = (const T*)fb->src[blockIdx.y];
-    const uint64_t n = fb->n[blockIdx.y];
-    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kBlock)
-        dst[i] = fold_int<T, OP>(dst[i], src[i]);
+    const uint32_t y = blockIdx.y;
+    fold_span_block<F, NT>(fb->f[y].dst, fb->f[y].src, fb->f[y].nvec, fb->f[y].head, fb->f[y].tail, 1.0f, blockIdx.x,
+                           gridDim.x);
 }
 
 // T(float(x) * scale): int32 rounds half away from zero, int64 / uint8 truncate
@@ -382,113 +397,107 @@ __global__ __launch_bounds__(kBlock) void k_ring_fold(void* out, RingPtrs ptrs, 
 
 // ---- launch helpers -----------------------------------------------------------
 
-// One tile per block wherever possible: measured on MI355X, 16 K short-lived blocks
-// in address order stream faster (6.38 TB/s for the binary fold) than a persistent
-// grid of 2 K blocks striding through the array (6.20 TB/s).  The cap only bounds
-// the grid for very large arrays; the kernels stride when it applies.
+// Blocks for `work_tiles` tiles: one tile per block in address order; the cap only bounds the grid
+// for very large arrays (the kernels stride when it applies).
 uint32_t stream_blocks(uint64_t work_tiles) {
     const uint64_t cap = (uint64_t)device_info().num_cus * (uint64_t)tuning().fold_blocks_per_cu;
     return clamp_u32(work_tiles, 1, cap);
 }
 
+FoldSpan fold_span(void* dst, const void* src, uint64_t n, int es) {
+    uint64_t head = ((16 - ((uintptr_t)dst & 15)) & 15) / es;
+    if (head > n) head = n;
+    FoldSpan f;
+    f.dst = (char*)dst + head * es;
+    f.src = src ? (const char*)src + head * es : nullptr;
+    f.nvec = (n - head) * es / 16;
+    f.head = (uint16_t)head;
+    f.tail = (uint16_t)(n - head - f.nvec * 16 / es);
+    f.pad = 0;
+    return f;
+}
+
+template <class F>
+int launch_fold2_f(void* dst, const void* src, uint64_t n, float scale, hipStream_t st) {
+    const FoldSpan f = fold_span(dst, src, n, F::size);
+    const uint32_t blocks = stream_blocks((f.nvec + kFoldBlock - 1) / kFoldBlock);
+    if (tuning().nontemporal)
+        k_fold2<F, true><<<blocks, kFoldBlock, 0, st>>>(f.dst, f.src, f.nvec, f.head, f.tail, scale);
+    else
+        k_fold2<F, false><<<blocks, kFoldBlock, 0, st>>>(f.dst, f.src, f.nvec, f.head, f.tail, scale);
+    return launch_status();
+}
 template <int DT, int OP, int KIND>
 int launch_fold2_t(void* dst, const void* src, uint64_t n, float scale, hipStream_t st) {
-    constexpr int ES = ElemInfo<DT>::size;
-    constexpr int EPV = ElemInfo<DT>::per_vec;
-    uint64_t head = ((16 - ((uintptr_t)dst & 15)) & 15) / ES;
-    if (head > n) head = n;
-    const uint64_t nvec = (n - head) / EPV;
-    const uint64_t tile = (uint64_t)kBlock * kUnroll;
-    const uint32_t blocks = stream_blocks((nvec + tile - 1) / tile);
-    if (tuning().nontemporal)
-        k_fold2<DT, OP, KIND, true><<<blocks, kBlock, 0, st>>>(dst, src, n, scale, (uint32_t)head, nvec);
-    else
-        k_fold2<DT, OP, KIND, false><<<blocks, kBlock, 0, st>>>(dst, src, n, scale, (uint32_t)head, nvec);
-    return launch_status();
+    return launch_fold2_f<FoldFloat<DT, OP, KIND>>(dst, src, n, scale, st);
 }
 
-template <int DT>
-int launch_fold2_dt(void* dst, const void* src, uint64_t n, int opi, hipStream_t st) {
-    switch (opi) {
-        case kAdd: return launch_fold2_t<DT, kAdd, 0>(dst, src, n, 1.0f, st);
-        case kMul: return launch_fold2_t<DT, kMul, 0>(dst, src, n, 1.0f, st);
-        case kMin: return launch_fold2_t<DT, kMin, 0>(dst, src, n, 1.0f, st);
-        default: return launch_fold2_t<DT, kMax, 0>(dst, src, n, 1.0f, st);
-    }
-}
-
-template <typename T>
-int launch_fold2_int(void* dst, const void* src, uint64_t n, int opi, hipStream_t st) {
-    const uint32_t blocks = stream_blocks((n + kBlock - 1) / kBlock);
-    switch (opi) {
-        case kAdd: k_fold2_int<T, kAdd><<<blocks, kBlock, 0, st>>>((T*)dst, (const T*)src, n); break;
-        case kMul: k_fold2_int<T, kMul><<<blocks, kBlock, 0, st>>>((T*)dst, (const T*)src, n); break;
-        case kMin: k_fold2_int<T, kMin><<<blocks, kBlock, 0, st>>>((T*)dst, (const T*)src, n); break;
-        default: k_fold2_int<T, kMax><<<blocks, kBlock, 0, st>>>((T*)dst, (const T*)src, n); break;
-    }
-    return launch_status();
-}
-
-// One launch per kFoldBatch folds.  x covers the longest fold of the launch (shorter folds' surplus
-// blocks leave at once), capped so that the whole grid stays within the streaming kernels' bound.
-template <class Launch>
-int launch_batches(void* const* dsts, const void* const* srcs, const uint64_t* counts, uint32_t nfolds,
-                   uint64_t elems_per_block, Launch&& launch) {
+// One launch per kFoldBatch folds.  Every fold gets as many blocks as the longest one needs (shorter
+// folds' surplus blocks leave at once), but at most twice the average: the folds of a ring step are
+// alike, and in a ragged list a grid cut to the longest fold would consist of surplus blocks.
+template <class F>
+int launch_fold2_batch_f(void* const* dsts, const void* const* srcs, const uint64_t* counts, uint32_t nfolds,
+                         hipStream_t st) {
     const uint64_t cap = (uint64_t)device_info().num_cus * (uint64_t)tuning().fold_blocks_per_cu;
+    const bool nt = tuning().nontemporal != 0;
     FoldBatch fb;
     uint32_t m = 0;
-    uint64_t longest = 0;
+    uint64_t longest = 0, sum = 0;  // blocks
     auto flush = [&]() {
         if (m == 0) return;
-        for (uint32_t i = m; i < (uint32_t)kFoldBatch; i++) { fb.dst[i] = nullptr; fb.src[i] = nullptr; fb.n[i] = 0; }
-        const uint64_t want = (longest + elems_per_block - 1) / elems_per_block;
-        launch(fb, dim3(clamp_u32(want, 1, cap / m > 0 ? cap / m : 1), m, 1));
+        for (uint32_t i = m; i < (uint32_t)kFoldBatch; i++) fb.f[i] = FoldSpan{};
+        const uint64_t most = 2 * ((sum + m - 1) / m) + 1;
+        const dim3 grid(clamp_u32(longest < most ? longest : most, 1, cap / m > 0 ? cap / m : 1), m, 1);
+        if (nt) k_fold2_batch<F, true><<<grid, kFoldBlock, 0, st>>>(fb);
+        else k_fold2_batch<F, false><<<grid, kFoldBlock, 0, st>>>(fb);
         m = 0;
-        longest = 0;
+        longest = sum = 0;
     };
     for (uint32_t i = 0; i < nfolds; i++) {
         if (counts[i] == 0) continue;
-        fb.dst[m] = dsts[i];
-        fb.src[m] = srcs[i];
-        fb.n[m] = counts[i];
-        longest = counts[i] > longest ? counts[i] : longest;
+        fb.f[m] = fold_span(dsts[i], srcs[i], counts[i], F::size);
+        const uint64_t blocks = (fb.f[m].nvec + kFoldBlock - 1) / kFoldBlock;
+        longest = blocks > longest ? blocks : longest;
+        sum += blocks;
         if (++m == (uint32_t)kFoldBatch) flush();
     }
     flush();
     return launch_status();
 }
 
-template <int DT, int OP>
-int launch_fold2_batch_t(void* const* dsts, const void* const* srcs, const uint64_t* counts, uint32_t nfolds,
-                         hipStream_t st) {
-    const uint64_t per_block = (uint64_t)kBlock * kUnroll * ElemInfo<DT>::per_vec;
-    const bool nt = tuning().nontemporal != 0;
-    return launch_batches(dsts, srcs, counts, nfolds, per_block, [&](const FoldBatch& fb, dim3 grid) {
-        if (nt) k_fold2_batch<DT, OP, true><<<grid, kBlock, 0, st>>>(fb);
-        else k_fold2_batch<DT, OP, false><<<grid, kBlock, 0, st>>>(fb);
-    });
-}
-template <int DT>
-int launch_fold2_batch_dt(void* const* dsts, const void* const* srcs, const uint64_t* counts, uint32_t nfolds,
-                          int opi, hipStream_t st) {
-    switch (opi) {
-        case kAdd: return launch_fold2_batch_t<DT, kAdd>(dsts, srcs, counts, nfolds, st);
-        case kMul: return launch_fold2_batch_t<DT, kMul>(dsts, srcs, counts, nfolds, st);
-        case kMin: return launch_fold2_batch_t<DT, kMin>(dsts, srcs, counts, nfolds, st);
-        default: return launch_fold2_batch_t<DT, kMax>(dsts, srcs, counts, nfolds, st);
+// Calls fn(F{}) with the fold kind of an element type and op.
+template <class Fn>
+int with_fold_kind(int dtype, int opi, Fn&& fn) {
+#define MCCLHIP_KINDS(K)                                       \
+    switch (opi) {                                             \
+        case kAdd: return fn(K(kAdd){});                       \
+        case kMul: return fn(K(kMul){});                       \
+        case kMin: return fn(K(kMin){});                       \
+        default: return fn(K(kMax){});                         \
     }
-}
-template <typename T>
-int launch_fold2_batch_int(void* const* dsts, const void* const* srcs, const uint64_t* counts, uint32_t nfolds,
-                           int opi, hipStream_t st) {
-    return launch_batches(dsts, srcs, counts, nfolds, kBlock, [&](const FoldBatch& fb, dim3 grid) {
-        switch (opi) {
-            case kAdd: k_fold2_batch_int<T, kAdd><<<grid, kBlock, 0, st>>>(fb); break;
-            case kMul: k_fold2_batch_int<T, kMul><<<grid, kBlock, 0, st>>>(fb); break;
-            case kMin: k_fold2_batch_int<T, kMin><<<grid, kBlock, 0, st>>>(fb); break;
-            default: k_fold2_batch_int<T, kMax><<<grid, kBlock, 0, st>>>(fb); break;
-        }
-    });
+#define MCCLHIP_K_F32(OP) FoldFloat<MCCL_HIP_F32, OP, 0>
+#define MCCLHIP_K_F16(OP) FoldFloat<MCCL_HIP_F16, OP, 0>
+#define MCCLHIP_K_BF16(OP) FoldFloat<MCCL_HIP_BF16, OP, 0>
+#define MCCLHIP_K_I32(OP) FoldInt<int32_t, OP>
+#define MCCLHIP_K_I64(OP) FoldInt<int64_t, OP>
+#define MCCLHIP_K_U8(OP) FoldInt<uint8_t, OP>
+    switch (dtype) {
+        case MCCL_HIP_F32: MCCLHIP_KINDS(MCCLHIP_K_F32)
+        case MCCL_HIP_F16: MCCLHIP_KINDS(MCCLHIP_K_F16)
+        case MCCL_HIP_BF16: MCCLHIP_KINDS(MCCLHIP_K_BF16)
+        case MCCL_HIP_I32: MCCLHIP_KINDS(MCCLHIP_K_I32)
+        case MCCL_HIP_I64: MCCLHIP_KINDS(MCCLHIP_K_I64)
+        case MCCL_HIP_BOOL:
+        case MCCL_HIP_U8: MCCLHIP_KINDS(MCCLHIP_K_U8)
+        default: return MCCL_HIP_ERR_DTYPE;
+    }
+#undef MCCLHIP_KINDS
+#undef MCCLHIP_K_F32
+#undef MCCLHIP_K_F16
+#undef MCCLHIP_K_BF16
+#undef MCCLHIP_K_I32
+#undef MCCLHIP_K_I64
+#undef MCCLHIP_K_U8
 }
 
 template <typename T>
@@ -569,16 +578,7 @@ int mccl_hip_fold2(void* dst, const void* src, uint64_t n, int dtype, int op, vo
     int rc = mccl_hip_init();
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
-    switch (dtype) {
-        case MCCL_HIP_F32: return launch_fold2_dt<MCCL_HIP_F32>(dst, src, n, opi, st);
-        case MCCL_HIP_F16: return launch_fold2_dt<MCCL_HIP_F16>(dst, src, n, opi, st);
-        case MCCL_HIP_BF16: return launch_fold2_dt<MCCL_HIP_BF16>(dst, src, n, opi, st);
-        case MCCL_HIP_I32: return launch_fold2_int<int32_t>(dst, src, n, opi, st);
-        case MCCL_HIP_I64: return launch_fold2_int<int64_t>(dst, src, n, opi, st);
-        case MCCL_HIP_BOOL:
-        case MCCL_HIP_U8: return launch_fold2_int<uint8_t>(dst, src, n, opi, st);
-        default: return MCCL_HIP_ERR_DTYPE;
-    }
+    return with_fold_kind(dtype, opi, [&](auto f) { return launch_fold2_f<decltype(f)>(dst, src, n, 1.0f, st); });
 }
 
 int mccl_hip_fold2_batch(void* const* host_dsts, const void* const* host_srcs, const uint64_t* host_counts,
@@ -614,14 +614,9 @@ int mccl_hip_fold2_batch(void* const* host_dsts, const void* const* host_srcs, c
     int rc = mccl_hip_init();
     if (rc) return rc;
     hipStream_t st = (hipStream_t)stream;
-    switch (dtype) {
-        case MCCL_HIP_F32: return launch_fold2_batch_dt<MCCL_HIP_F32>(host_dsts, host_srcs, host_counts, nfolds, opi, st);
-        case MCCL_HIP_F16: return launch_fold2_batch_dt<MCCL_HIP_F16>(host_dsts, host_srcs, host_counts, nfolds, opi, st);
-        case MCCL_HIP_BF16: return launch_fold2_batch_dt<MCCL_HIP_BF16>(host_dsts, host_srcs, host_counts, nfolds, opi, st);
-        case MCCL_HIP_I32: return launch_fold2_batch_int<int32_t>(host_dsts, host_srcs, host_counts, nfolds, opi, st);
-        case MCCL_HIP_I64: return launch_fold2_batch_int<int64_t>(host_dsts, host_srcs, host_counts, nfolds, opi, st);
-        default: return launch_fold2_batch_int<uint8_t>(host_dsts, host_srcs, host_counts, nfolds, opi, st);
-    }
+    return with_fold_kind(dtype, opi, [&](auto f) {
+        return launch_fold2_batch_f<decltype(f)>(host_dsts, host_srcs, host_counts, nfolds, st);
+    });
 }
 
 int mccl_hip_scale(void* buf, uint64_t n, int dtype, float scale, void* stream) {

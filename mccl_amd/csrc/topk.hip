@@ -1536,7 +1536,7 @@ int mccl_hip_topk_compress(const float* grad, float* residual, uint64_t n_total,
     Workspace w = carve(aligned, g);
     w.status = status;
     const Path path = choose_path(g, nullptr);
-    const uint64_t cap = (uint64_t)device_info().num_cus * (uint64_t)tuning().fold_blocks_per_cu;
+    const uint64_t cap = (uint64_t)device_info().num_cus * (uint64_t)(tuning().fold_blocks_per_cu < 256 ? tuning().fold_blocks_per_cu : 256);
     const uint64_t nvec = g.bucket_elems / 4;
     const uint64_t bx = (cap + g.nbuckets - 1) / g.nbuckets;
     const uint64_t need_r = (nvec + kBlock * 4 - 1) / (kBlock * 4);
