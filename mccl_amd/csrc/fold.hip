@@ -30,9 +30,17 @@ namespace {
 // arrays: 178 / 181 / 187 / 190 us with 64 / 128 / 256 / 1024 threads, 185 and 193 with two and
 // four vectors per lane.
 constexpr int kFoldBlock = 64;
-// Vectors in flight per thread and rank buffer of the ring fold: one for three ranks (0.76 of the
-// 8 TB/s peak against 0.73), eight for six and seven ranks (0.71 against 0.70), four otherwise.
-constexpr int ring_unroll(int ws) { return ws == 3 ? 1 : ((ws == 6 || ws == 7) ? 8 : 4); }
+// Blocks go to the XCDs in turn, and tiles start where the destination's address is a multiple of
+// 1 KiB and rows of tiles at multiples of 8 KiB (kGroupVecs vectors): an XCD always works on the same
+// eighth of every 8 KiB, and no wavefront ends inside a cache line.  Chunks that start anywhere
+// else: ring fold of 8 ranks, chunks of 819,204 elements 638 us with tiles that start with the chunk,
+// 597 with tiles on 1 KiB, 579 with rows on 8 KiB.
+constexpr int kXcds = 8;
+constexpr int kGroupVecs = kXcds * kFoldBlock;
+// Vectors per lane and rank buffer of the ring fold, in one-wavefront blocks as well: one where the
+// world size is known at compile time (all ranks' loads are in flight together; two cost 2-3 % from
+// two to eight ranks), four where the ranks come one after the other.
+constexpr int ring_unroll(int ws) { return ws == 0 ? 4 : 1; }
 
 template <bool NT>
 __device__ __forceinline__ u4a load_vec_a(const u4a* p) {
@@ -55,6 +63,17 @@ __device__ __forceinline__ u4a load_vec_u(const void* p) {
 template <bool NT>
 __device__ __forceinline__ void store_vec_a(u4a* p, u4a v) {
     if constexpr (NT) __builtin_nontemporal_store(v, p);
+    else *p = v;
+}
+
+// The ring fold's output: written through the XCD's L2 (agent scope) and left to the memory-side
+// cache, which gathers it into longer write bursts between the reads.  8 ranks, 386 MB per rank:
+// 566 us against 582 with a streaming store (bare kernel, rotating buffers).  (A store of
+// more than 8 bytes reads its registers over the following cycles: the wait states keep what
+// follows the statement from overwriting them.)
+template <bool NT>
+__device__ __forceinline__ void store_ring(u4a* p, u4a v) {
+    if constexpr (NT) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
     else *p = v;
 }
 
@@ -138,15 +157,16 @@ struct FoldInt {
 };
 
 // ---- binary fold / scale / fused ----------------------------------------------
-// Layout: [head scalars][nvec 16-byte vectors][tail scalars]; head makes the destination 16-byte
-// aligned; `dst` and `src` point at the body.  The launch computes it (fold_span), so that a
-// wavefront starts with its addresses at hand.
+// Layout: [head scalars][16-byte vectors][tail scalars]; head makes the destination 16-byte aligned.
+// `lead` vectors of the first tile group lie in front of the body, and `dst`, `src` and `nvec` count
+// from the group's start.  The launch computes all of it (fold_span), so that a wavefront starts
+// with its addresses at hand.
 struct __attribute__((aligned(32))) FoldSpan {
     char* dst;
     const char* src;
     uint64_t nvec;
     uint16_t head, tail;  // elements, fewer than 16 bytes each
-    uint32_t pad;
+    uint32_t lead;        // vectors of the first tile group that lie in front of the body
 };
 
 template <int ES, bool NT>
@@ -157,29 +177,24 @@ __device__ __forceinline__ u4a load_src(const void* p) {
 // Block `block` of `nblocks` of one fold.
 template <class F, bool NT>
 __device__ __forceinline__ void fold_span_block(char* dst, const char* src, uint64_t nvec, uint32_t head, uint32_t tail,
-                                                float scale, uint32_t block, uint32_t nblocks) {
-    const uint32_t off = threadIdx.x * 16u;
-    uint64_t v = (uint64_t)block * kFoldBlock;
+                                                uint32_t lead, float scale, uint32_t block, uint32_t nblocks) {
+    const uint32_t t = threadIdx.x;
+    auto fold_vec = [&](uint64_t v) {
+        char* const dp = dst + v * 16;
+        const u4a d = load_vec_a<NT>((const u4a*)(dp + t * 16u));
+        u4a s = d;
+        if constexpr (F::needs_src) s = load_src<F::size, NT>(src + v * 16 + t * 16u);
+        store_vec_a<NT>((u4a*)(dp + t * 16u), F::vec(d, s, scale));
+    };
     // (the launch gives a block one round unless the grid is capped)
-    for (; v + kFoldBlock <= nvec; v += (uint64_t)nblocks * kFoldBlock) {
-        char* const dp = dst + v * 16;
-        const u4a d = load_vec_a<NT>((const u4a*)(dp + off));
-        u4a s = d;
-        if constexpr (F::needs_src) s = load_src<F::size, NT>(src + v * 16 + off);
-        store_vec_a<NT>((u4a*)(dp + off), F::vec(d, s, scale));
-    }
-    if (v < nvec && threadIdx.x < nvec - v) {
-        char* const dp = dst + v * 16;
-        const u4a d = load_vec_a<NT>((const u4a*)(dp + off));
-        u4a s = d;
-        if constexpr (F::needs_src) s = load_src<F::size, NT>(src + v * 16 + off);
-        store_vec_a<NT>((u4a*)(dp + off), F::vec(d, s, scale));
+    for (uint64_t v = (uint64_t)block * kFoldBlock; v < nvec; v += (uint64_t)nblocks * kFoldBlock) {
+        if (v >= lead && v + kFoldBlock <= nvec) fold_vec(v);  // (uniform)
+        else if (v + t >= lead && v + t < nvec) fold_vec(v);
     }
     if (block + 1 == nblocks && (head | tail)) {  // scalars: at most 15 in front of the body, 15 behind it
-        const uint32_t t = threadIdx.x;
         constexpr uint32_t EPV = 16 / F::size;
         if (t < head) {
-            const int64_t o = -(int64_t)((head - t) * F::size);
+            const int64_t o = (int64_t)lead * 16 - (int64_t)((head - t) * F::size);
             F::elem(dst + o, F::needs_src ? src + o : nullptr, scale);
         } else if (t >= EPV && t - EPV < tail) {
             const uint64_t o = nvec * 16 + (uint64_t)(t - EPV) * F::size;
@@ -190,8 +205,8 @@ __device__ __forceinline__ void fold_span_block(char* dst, const char* src, uint
 
 template <class F, bool NT>
 __global__ __launch_bounds__(kFoldBlock) void k_fold2(char* dst, const char* src, uint64_t nvec, uint32_t head,
-                                                      uint32_t tail, float scale) {
-    fold_span_block<F, NT>(dst, src, nvec, head, tail, scale, blockIdx.x, gridDim.x);
+                                                      uint32_t tail, uint32_t lead, float scale) {
+    fold_span_block<F, NT>(dst, src, nvec, head, tail, lead, scale, blockIdx.x, gridDim.x);
 }
 
 // ---- a list of independent binary folds in one launch ---------------------------
@@ -208,8 +223,8 @@ __global__ __launch_bounds__(kFoldBlock) void k_fold2_batch(FoldBatch) {
     typedef const __attribute__((address_space(4))) FoldBatch* Arg;
     const Arg fb = (Arg)__builtin_amdgcn_kernarg_segment_ptr();
     const uint32_t y = blockIdx.y;
-    fold_span_block<F, NT>(fb->f[y].dst, fb->f[y].src, fb->f[y].nvec, fb->f[y].head, fb->f[y].tail, 1.0f, blockIdx.x,
-                           gridDim.x);
+    fold_span_block<F, NT>(fb->f[y].dst, fb->f[y].src, fb->f[y].nvec, fb->f[y].head, fb->f[y].tail, fb->f[y].lead,
+                           1.0f, blockIdx.x, gridDim.x);
 }
 
 // T(float(x) * scale): int32 rounds half away from zero, int64 / uint8 truncate
@@ -231,63 +246,84 @@ struct RingPtrs {
     const void* in[2 * MCCL_HIP_MAX_WORLD];
 };
 
-// blockIdx.y = bucket * nchunks + chunk.  Each block row folds one chunk of one
-// bucket, so the first rank of the fold is uniform over the block.
+// How a call is cut: computed by the launch, so that a block starts with multiplications only.
+struct RingCut {
+    uint64_t n_total, bucket_elems;
+    uint64_t ce_full, ce_last;  // elements per chunk in a full bucket and in the last one
+    uint32_t nbuckets, chunked;
+};
+
+// blockIdx = (tile, chunk, bucket).  A row of blocks folds one chunk of one bucket, so the first
+// rank of the fold is uniform over the block.
+// Measured over 96.5 M fp32 elements per rank, 25 MiB buckets, buffers that no cache holds (TB/s, against
+// 256-thread blocks with up to eight vectors per lane and rank whose tiles began with the chunk):
+// W = 2: 6.6 (6.2), 3: 6.5 (6.2), 4: 6.4 (6.0), 5: 6.3 (6.0), 6: 6.3 (5.7), 7: 6.2 (5.6), 8: 6.2 (5.9);
+// bf16 W = 4: 6.5 (6.1), W = 8: 6.4 (5.9).  What bounds it is HBM with reads and writes mixed; the wait
+// for the rank pointers behind the computation of the cut was worth 4 % at W = 8.
 // WSC > 0 fixes the world size at compile time, so the rank loop unrolls and
 // all WSC * ring_unroll(WSC) loads of a thread are in flight together; WSC == 0 reads
 // it at run time.
 template <int DT, int OP, bool NT, int WSC>
-__global__ __launch_bounds__(kBlock) void k_ring_fold(void* out, RingPtrs ptrs, int ws_rt,
-                                                      uint64_t n_total, uint64_t bucket_elems,
-                                                      int schedule, uint32_t nchunks, float scale,
-                                                      int apply_scale, int stepwise) {
+__global__ __launch_bounds__(kFoldBlock) void k_ring_fold(void* out, RingPtrs ptrs, RingCut cut, int ws_rt, float scale,
+                                                          int apply_scale, int stepwise) {
     constexpr int ES = ElemInfo<DT>::size;
     constexpr int EPV = ElemInfo<DT>::per_vec;
     constexpr int U = ring_unroll(WSC);
     const int ws = WSC > 0 ? WSC : ws_rt;
-    const uint32_t bucket = blockIdx.y / nchunks;
-    const uint32_t c = blockIdx.y - bucket * nchunks;
-    const uint64_t bstart = (uint64_t)bucket * bucket_elems;
-    const uint64_t bn = (n_total - bstart) < bucket_elems ? (n_total - bstart) : bucket_elems;
-    const uint64_t ce = (bn + nchunks - 1) / nchunks;
-    const uint64_t cstart = (uint64_t)c * ce;
-    if (cstart >= bn) return;
-    const uint64_t len = (bn - cstart) < ce ? (bn - cstart) : ce;
-    const uint64_t e0 = bstart + cstart;  // first element of the chunk in every buffer
-    const int first = (schedule == MCCL_HIP_RING_CHUNKED) ? (int)(((c + 1) >> 1) % (uint32_t)ws)
-                                                          : (int)(c % (uint32_t)ws);
-
-    char* o = (char*)out + e0 * ES;
-    uint64_t head = ((16 - ((uintptr_t)o & 15)) & 15) / ES;
-    if (head > len) head = len;
-    const uint64_t nvec = (len - head) / EPV;
-    const uint64_t voff = (e0 + head) * ES;  // byte offset of the vector body
-    u4a* ov = (u4a*)((char*)out + voff);
-
-    const uint64_t tile = (uint64_t)kBlock * U;
+    const uint32_t bucket = blockIdx.z, c = blockIdx.y;
+    // basic: c < ws; chunked: (c + 1) / 2 <= ws
+    const int half = (int)((c + 1) >> 1);
+    const int first = cut.chunked ? (half == ws ? 0 : half) : (int)c;
     const void* rp[WSC > 0 ? WSC : 1];  // rank buffers in fold order (compile-time world sizes)
     if constexpr (WSC > 0) {
 #pragma unroll
         for (int j = 0; j < WSC; j++) rp[j] = ptrs.in[first + j];
     }
+    const uint64_t bstart = (uint64_t)bucket * cut.bucket_elems;
+    const bool last = bucket + 1 == cut.nbuckets;
+    const uint64_t bn = last ? cut.n_total - bstart : cut.bucket_elems;
+    const uint64_t ce = last ? cut.ce_last : cut.ce_full;
+    const uint64_t cstart = (uint64_t)c * ce;
+    const uint64_t rest = cstart < bn ? bn - cstart : 0;
+    const uint64_t len = rest < ce ? rest : ce;
+    const uint64_t e0 = bstart + cstart;  // first element of the chunk in every buffer
+
+    char* o = (char*)out + e0 * ES;
+    uint64_t head = ((16 - ((uintptr_t)o & 15)) & 15) / ES;
+    if (head > len) head = len;
+    const uint64_t nvec = (len - head) / EPV;
+    // a row's tiles start at a tile group of the output's addresses: `lead` vectors lie in front of the chunk
+    const uint32_t lead = (uint32_t)(((uintptr_t)o + head * ES) >> 4) & (kGroupVecs - 1);
+    const uint64_t voff = (e0 + head) * ES - lead * 16u;  // byte offset of the first tile
+
+    const uint64_t tile = (uint64_t)kFoldBlock * U;
     auto rank_ptr = [&](int j, int r) -> const char* {
         if constexpr (WSC > 0) return (const char*)rp[j];
         else return (const char*)ptrs.in[r];
     };
-    for (uint64_t base = (uint64_t)blockIdx.x * tile; base < nvec; base += (uint64_t)gridDim.x * tile) {
+    const uint64_t base = (uint64_t)blockIdx.x * tile;
+    // (the pointers' load is under way while the cut is computed, not started behind the branch)
+    if constexpr (WSC > 0) {
+#pragma unroll
+        for (int j = 0; j < WSC; j++) asm volatile("" : "+s"(rp[j]));
+    }
+    if (nvec && base + tile > lead && base < nvec + lead) {
+        // byte offsets from the tile's start; outside the chunk its first or last vector is folded and not stored
+        const uint32_t end = (uint32_t)(nvec + lead - base < tile ? nvec + lead - base : tile);
+        const uint32_t begin = base < lead ? (uint32_t)(lead - base) : 0u;
+        uint32_t off[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t i = (uint32_t)u * kFoldBlock + threadIdx.x;
+            off[u] = (i < begin ? begin : (i < end ? i : end - 1)) * 16u;
+        }
         if constexpr (DT == MCCL_HIP_F32) {
             float acc[U][4];
-            uint64_t idx[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                idx[u] = base + (uint64_t)u * kBlock + threadIdx.x;
-                if (idx[u] >= nvec) idx[u] = nvec - 1;  // clamp: recomputes a valid vector, store is guarded
-            }
             {
-                const char* p = rank_ptr(0, first) + voff;
+                const char* p = rank_ptr(0, first) + voff + base * 16;
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    u4a v = load_vec_u<ES, NT>(p + idx[u] * 16);
+                    u4a v = load_vec_u<ES, NT>(p + off[u]);
 #pragma unroll
                     for (int q = 0; q < 4; q++) acc[u][q] = u2f(v[q]);
                 }
@@ -296,10 +332,10 @@ __global__ __launch_bounds__(kBlock) void k_ring_fold(void* out, RingPtrs ptrs, 
 #pragma unroll
             for (int j = 1; j < ws; j++) {
                 r = (r + 1 == ws) ? 0 : r + 1;
-                const char* p = rank_ptr(j, r) + voff;
+                const char* p = rank_ptr(j, r) + voff + base * 16;
                 u4a v[U];
 #pragma unroll
-                for (int u = 0; u < U; u++) v[u] = load_vec_u<ES, NT>(p + idx[u] * 16);
+                for (int u = 0; u < U; u++) v[u] = load_vec_u<ES, NT>(p + off[u]);
 #pragma unroll
                 for (int u = 0; u < U; u++)
 #pragma unroll
@@ -310,21 +346,15 @@ __global__ __launch_bounds__(kBlock) void k_ring_fold(void* out, RingPtrs ptrs, 
                 u4a rv;
 #pragma unroll
                 for (int q = 0; q < 4; q++) rv[q] = f2u(apply_scale ? acc[u][q] * scale : acc[u][q]);
-                if (base + (uint64_t)u * kBlock + threadIdx.x < nvec) store_vec_a<NT>(ov + idx[u], rv);
+                if (off[u] == (uint32_t)(u * kFoldBlock + threadIdx.x) * 16u) store_ring<NT>((u4a*)((char*)out + voff + base * 16 + off[u]), rv);
             }
         } else {
             float acc[U][8];
-            uint64_t idx[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                idx[u] = base + (uint64_t)u * kBlock + threadIdx.x;
-                if (idx[u] >= nvec) idx[u] = nvec - 1;
-            }
             {
-                const char* p = rank_ptr(0, first) + voff;
+                const char* p = rank_ptr(0, first) + voff + base * 16;
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    u4a v = load_vec_u<ES, NT>(p + idx[u] * 16);
+                    u4a v = load_vec_u<ES, NT>(p + off[u]);
 #pragma unroll
                     for (int q = 0; q < 4; q++) {
                         acc[u][2 * q] = widen16<DT>(v[q] & 0xFFFFu);
@@ -336,10 +366,10 @@ __global__ __launch_bounds__(kBlock) void k_ring_fold(void* out, RingPtrs ptrs, 
 #pragma unroll
             for (int j = 1; j < ws; j++) {
                 r = (r + 1 == ws) ? 0 : r + 1;
-                const char* p = rank_ptr(j, r) + voff;
+                const char* p = rank_ptr(j, r) + voff + base * 16;
                 u4a v[U];
 #pragma unroll
-                for (int u = 0; u < U; u++) v[u] = load_vec_u<ES, NT>(p + idx[u] * 16);
+                for (int u = 0; u < U; u++) v[u] = load_vec_u<ES, NT>(p + off[u]);
 #pragma unroll
                 for (int u = 0; u < U; u++)
 #pragma unroll
@@ -363,13 +393,14 @@ __global__ __launch_bounds__(kBlock) void k_ring_fold(void* out, RingPtrs ptrs, 
                     float hi = apply_scale ? acc[u][2 * q + 1] * scale : acc[u][2 * q + 1];
                     rv[q] = narrow16<DT>(lo) | (narrow16<DT>(hi) << 16);
                 }
-                if (base + (uint64_t)u * kBlock + threadIdx.x < nvec) store_vec_a<NT>(ov + idx[u], rv);
+                if (off[u] == (uint32_t)(u * kFoldBlock + threadIdx.x) * 16u) store_ring<NT>((u4a*)((char*)out + voff + base * 16 + off[u]), rv);
             }
         }
     }
 
     // scalar head and tail of the chunk
-    const uint64_t g = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (blockIdx.x != 0 || (head == 0 && nvec * EPV == len)) return;
+    const uint64_t g = threadIdx.x;
     const uint64_t tail = head + nvec * EPV;
     uint64_t i = len;  // element (relative to the chunk) this thread folds, if any
     if (g < head) i = g;
@@ -407,13 +438,14 @@ uint32_t stream_blocks(uint64_t work_tiles) {
 FoldSpan fold_span(void* dst, const void* src, uint64_t n, int es) {
     uint64_t head = ((16 - ((uintptr_t)dst & 15)) & 15) / es;
     if (head > n) head = n;
+    const uint64_t body = (n - head) * es / 16;
     FoldSpan f;
-    f.dst = (char*)dst + head * es;
-    f.src = src ? (const char*)src + head * es : nullptr;
-    f.nvec = (n - head) * es / 16;
     f.head = (uint16_t)head;
-    f.tail = (uint16_t)(n - head - f.nvec * 16 / es);
-    f.pad = 0;
+    f.tail = (uint16_t)(n - head - body * 16 / es);
+    f.lead = body ? (uint32_t)(((uintptr_t)dst + head * es) >> 4) & (kGroupVecs - 1) : 0u;
+    f.dst = (char*)dst + head * es - f.lead * 16u;
+    f.src = src ? (const char*)src + head * es - f.lead * 16u : nullptr;
+    f.nvec = body ? body + f.lead : 0;
     return f;
 }
 
@@ -422,9 +454,9 @@ int launch_fold2_f(void* dst, const void* src, uint64_t n, float scale, hipStrea
     const FoldSpan f = fold_span(dst, src, n, F::size);
     const uint32_t blocks = stream_blocks((f.nvec + kFoldBlock - 1) / kFoldBlock);
     if (tuning().nontemporal)
-        k_fold2<F, true><<<blocks, kFoldBlock, 0, st>>>(f.dst, f.src, f.nvec, f.head, f.tail, scale);
+        k_fold2<F, true><<<blocks, kFoldBlock, 0, st>>>(f.dst, f.src, f.nvec, f.head, f.tail, f.lead, scale);
     else
-        k_fold2<F, false><<<blocks, kFoldBlock, 0, st>>>(f.dst, f.src, f.nvec, f.head, f.tail, scale);
+        k_fold2<F, false><<<blocks, kFoldBlock, 0, st>>>(f.dst, f.src, f.nvec, f.head, f.tail, f.lead, scale);
     return launch_status();
 }
 template <int DT, int OP, int KIND>
@@ -447,7 +479,9 @@ int launch_fold2_batch_f(void* const* dsts, const void* const* srcs, const uint6
         if (m == 0) return;
         for (uint32_t i = m; i < (uint32_t)kFoldBatch; i++) fb.f[i] = FoldSpan{};
         const uint64_t most = 2 * ((sum + m - 1) / m) + 1;
-        const dim3 grid(clamp_u32(longest < most ? longest : most, 1, cap / m > 0 ? cap / m : 1), m, 1);
+        uint64_t gx = longest < most ? longest : most;
+        if (m > 1) gx = (gx + kXcds - 1) / kXcds * kXcds;  // every fold starts on the same XCD
+        const dim3 grid(clamp_u32(gx, 1, cap / m > 0 ? cap / m : 1), m, 1);
         if (nt) k_fold2_batch<F, true><<<grid, kFoldBlock, 0, st>>>(fb);
         else k_fold2_batch<F, false><<<grid, kFoldBlock, 0, st>>>(fb);
         m = 0;
@@ -514,19 +548,21 @@ int launch_ring_t(void* out, const RingPtrs& ptrs, int ws, uint64_t n_total, uin
     constexpr int EPV = ElemInfo<DT>::per_vec;
     const uint64_t bn = bucket_elems < n_total ? bucket_elems : n_total;
     const uint64_t ce = (bn + nchunks - 1) / nchunks;
-    const uint64_t tile_vecs = (uint64_t)kBlock * ring_unroll(ws >= 2 && ws <= 8 ? ws : 0);
-    const uint64_t tiles = (ce / EPV + tile_vecs - 1) / tile_vecs;
-    const uint64_t rows = (uint64_t)nchunks * nbuckets;
+    const uint64_t tile_vecs = (uint64_t)kFoldBlock * ring_unroll(ws >= 2 && ws <= 8 ? ws : 0);
+    const uint64_t group = 16 * kGroupVecs;
+    const bool on_groups = ((uintptr_t)out | (ce * ElemInfo<DT>::size) | (bucket_elems * ElemInfo<DT>::size)) % group == 0;
+    uint64_t tiles = (ce / EPV + (on_groups ? 0 : kGroupVecs - 1) + tile_vecs - 1) / tile_vecs;
+    if (nchunks * nbuckets > 1) tiles = (tiles + kXcds - 1) / kXcds * kXcds;  // every row starts on the same XCD
     // One tile per block, x fastest: blocks are dispatched in address order, so
     // the set of tiles in flight is one contiguous front per rank buffer.  A
     // persistent grid looping inside each chunk row scatters the front over all
     // rows and costs about 13 % of the bandwidth on MI355X.
-    uint64_t per_row = tiles < 1 ? 1 : tiles;
-    if (per_row > 0x7FFFFFFFull) per_row = 0x7FFFFFFFull;
-    dim3 grid((uint32_t)per_row, (uint32_t)rows, 1);
+    if (tiles > 0xFFFFFFFFull / kFoldBlock) return MCCL_HIP_ERR_ARG;  // more than 2^32 threads in a row: a chunk of 68 GB
+    const RingCut cut = {n_total, bucket_elems, ce, (n_total - (nbuckets - 1) * bucket_elems + nchunks - 1) / nchunks,
+                         nbuckets, schedule == MCCL_HIP_RING_CHUNKED ? 1u : 0u};
+    dim3 grid((uint32_t)(tiles < 1 ? 1 : tiles), nchunks, nbuckets);
 #define MCCLHIP_RING_LAUNCH(NT, WSC)                                                                  \
-    k_ring_fold<DT, OP, NT, WSC><<<grid, kBlock, 0, st>>>(out, ptrs, ws, n_total, bucket_elems, schedule, \
-                                                          nchunks, scale, apply_scale, stepwise)
+    k_ring_fold<DT, OP, NT, WSC><<<grid, kFoldBlock, 0, st>>>(out, ptrs, cut, ws, scale, apply_scale, stepwise)
     const bool nt = tuning().nontemporal != 0;
     switch (ws) {
         // world sizes 2..8 have an unrolled instance each: all loads of a thread are in flight
