@@ -12,6 +12,7 @@
 #include "../../../include/mccl_hip.h"
 #include "Compression.hpp"
 #include "Errors.hpp"
+#include "FastCalls.hpp"
 #include "HipKernels.hpp"
 #include "Options.hpp"
 #include "RingDriver.hpp"
@@ -66,6 +67,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.attr("__version__") = "0.5.0";
     m.attr("__protocol_version__") = 5;
     m.attr("__hip_abi_version__") = mccl_hip_abi_version();
+    mccl::add_fast_calls(m.ptr());
 
     py::enum_<mccl::CompressionMode>(m, "CompressionMode")
         .value("NONE", mccl::CompressionMode::NONE)

@@ -10,7 +10,7 @@ import sysconfig
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(os.path.dirname(HERE))
 OBJ = os.path.join(PKG, "build", "ext")
-SOURCES = ["HipKernels.cpp", "Compression.cpp", "RingDriver.cpp", "Registration.cpp"]
+SOURCES = ["HipKernels.cpp", "Compression.cpp", "RingDriver.cpp", "FastCalls.cpp", "Registration.cpp"]
 
 
 def target() -> str:

@@ -14,7 +14,9 @@
 #include "common.hip.h"
 #include "runtime.h"
 
+#include <algorithm>
 #include <type_traits>
+#include <vector>
 
 namespace mcclhip {
 
@@ -636,16 +638,31 @@ int mccl_hip_fold2_batch(void* const* host_dsts, const void* const* host_srcs, c
         if (!host_dsts[i] || !host_srcs[i] || host_counts[i] > MCCL_HIP_MAX_ELEMS) return MCCL_HIP_ERR_ARG;
     }
     // the folds of one call run in no particular order: a destination may not overlap any other
-    // fold's destination or source
+    // fold's destination or source.  Destinations in address order that do not overlap their
+    // neighbours overlap none; a source then has to be compared with those it reaches into.
+    struct Range {
+        uintptr_t lo, hi;
+        uint32_t fold;
+    };
+    std::vector<Range> d;
+    d.reserve(nfolds);
+    bool sorted = true;
     for (uint32_t i = 0; i < nfolds; i++) {
         if (host_counts[i] == 0) continue;
-        const uintptr_t d0 = (uintptr_t)host_dsts[i], d1 = d0 + host_counts[i] * (uint64_t)es;
-        for (uint32_t j = 0; j < nfolds; j++) {
-            if (j == i || host_counts[j] == 0) continue;
-            const uint64_t bytes = host_counts[j] * (uint64_t)es;
-            const uintptr_t a0 = (uintptr_t)host_dsts[j], b0 = (uintptr_t)host_srcs[j];
-            if ((d0 < a0 + bytes && a0 < d1) || (d0 < b0 + bytes && b0 < d1)) return MCCL_HIP_ERR_ARG;
-        }
+        const uintptr_t lo = (uintptr_t)host_dsts[i];
+        if (!d.empty() && lo < d.back().lo) sorted = false;
+        d.push_back({lo, lo + host_counts[i] * (uint64_t)es, i});
+    }
+    if (!sorted) std::sort(d.begin(), d.end(), [](const Range& a, const Range& b) { return a.lo < b.lo; });
+    for (size_t i = 1; i < d.size(); i++)
+        if (d[i].lo < d[i - 1].hi) return MCCL_HIP_ERR_ARG;
+    for (uint32_t i = 0; i < nfolds; i++) {
+        if (host_counts[i] == 0) continue;
+        const uintptr_t lo = (uintptr_t)host_srcs[i], hi = lo + host_counts[i] * (uint64_t)es;
+        // the first destination that ends behind the source's start, and those after it
+        auto it = std::partition_point(d.begin(), d.end(), [&](const Range& r) { return r.hi <= lo; });
+        for (; it != d.end() && it->lo < hi; ++it)
+            if (it->fold != i) return MCCL_HIP_ERR_ARG;
     }
     int rc = mccl_hip_init();
     if (rc) return rc;

@@ -7,6 +7,7 @@ computes on the host.
 from __future__ import annotations
 
 import ctypes as C
+import os
 from typing import Optional, Sequence
 
 import torch
@@ -21,6 +22,40 @@ _DTYPE_CODE = {
     torch.uint8: 0, torch.int32: 3, torch.int64: 4, torch.float16: 5,
     torch.float32: 6, torch.bool: 11, torch.bfloat16: 15,
 }
+
+
+class _Unbound:
+    """Stands in for the extension until the first call, which binds it."""
+
+    def __getattr__(self, name):
+        global _native
+        _native = _bind_native()
+        return getattr(_native, name)
+
+
+class _Checked:
+    """No extension: every call goes through the checks below."""
+
+    def __getattr__(self, name):
+        return lambda *args: False
+
+
+def _bind_native():
+    if os.environ.get("MCCL_HIP_LIBRARY"):   # the extension is linked to the library beside it
+        return _Checked()
+    _lib.load()
+    try:
+        import torch.distributed  # noqa: F401  (registers the c10d types the extension builds on)
+        from . import _C
+    except ImportError:
+        return _Checked()
+    return _C
+
+
+# Well-formed calls are checked and launched in one C call (mccl_amd/csrc/ext/FastCalls.cpp), which
+# returns False, with nothing done, for everything else; that goes through the checks below and
+# through ctypes, and raises what is wrong with it.
+_native = _Unbound()
 
 
 def dtype_code(t: torch.Tensor) -> int:
@@ -51,6 +86,8 @@ def _dev(t: torch.Tensor, what: str, dtype: Optional[torch.dtype] = None, min_nu
 
 
 def fold2(dst: torch.Tensor, src: torch.Tensor, op: int = SUM) -> torch.Tensor:
+    if _native._fast_fold2(dst, src, op):
+        return dst
     _dev(dst, "dst"); _dev(src, "src")
     if dst.shape != src.shape or dst.dtype != src.dtype:
         raise ValueError("shape / dtype mismatch")
@@ -63,6 +100,8 @@ def fold2_batch(dsts: Sequence[torch.Tensor], srcs: Sequence[torch.Tensor], op: 
     """dsts[i] (op)= srcs[i] for every i, in one launch per 128 folds.  The folds run in no
     particular order: a destination may not overlap any other fold's destination or source
     (the library refuses such a list)."""
+    if _native._fast_fold2_batch(dsts, srcs, op):
+        return
     if len(dsts) != len(srcs):
         raise ValueError("as many sources as destinations")
     if not dsts:
@@ -84,6 +123,8 @@ def scale(buf: torch.Tensor, s: float) -> torch.Tensor:
 
 
 def fold2_scale(dst: torch.Tensor, src: torch.Tensor, s: float) -> torch.Tensor:
+    if _native._fast_fold2_scale(dst, src, s):
+        return dst
     _dev(dst, "dst"); _dev(src, "src")
     if dst.shape != src.shape or dst.dtype != src.dtype:
         raise ValueError("shape / dtype mismatch")
@@ -99,6 +140,9 @@ def _ptrs(tensors: Sequence[torch.Tensor]):
 def ring_fold(out: torch.Tensor, ins: Sequence[torch.Tensor], op: int = SUM,
               schedule: int = RING_BASIC, bucket_elems: Optional[int] = None,
               scale_by: Optional[float] = None, stepwise: bool = False) -> torch.Tensor:
+    if isinstance(out, torch.Tensor) and _native._fast_ring_fold(out, ins, op, schedule, bucket_elems or max(out.numel(), 1),
+                                                                 scale_by, int(stepwise)):
+        return out
     _dev(out, "out")
     for t in ins:
         _dev(t, "in")
@@ -140,6 +184,9 @@ def topk_compress(grad: torch.Tensor, residual: torch.Tensor, ratio: float,
                   status: Optional[torch.Tensor] = None):
     """Returns (wire uint8 tensor [nbuckets * stride], stride). residual is updated.
     status: int32 device tensor of one element that receives ERR_TIMEOUT (caller zeroes it)."""
+    if wire is not None and bucket_elems and _native._fast_topk_compress(grad, residual, ratio, bucket_elems, wire, workspace,
+                                                                         wire_stride, status):
+        return wire, wire_stride
     _dev(grad, "grad"); _dev(residual, "residual")
     if grad.dtype != torch.float32 or residual.dtype != torch.float32:
         raise _lib.MCCLHipError(-2, "TopK compression currently supports float32 only")
@@ -242,6 +289,8 @@ def sparse_accumulate(acc: torch.Tensor, wires: Sequence[torch.Tensor], wire_str
                       bucket_elems: Optional[int] = None, scale_by: Optional[float] = None,
                       status: Optional[torch.Tensor] = None, workspace="auto") -> torch.Tensor:
     """workspace: "auto" allocates the scratch, None selects the scratch-free kernel."""
+    if bucket_elems and _native._fast_sparse_accumulate(acc, wires, wire_stride, bucket_elems, scale_by, status, workspace):
+        return acc
     _dev(acc, "acc", torch.float32)
     n = acc.numel()
     be = bucket_elems or max(n, 1)
