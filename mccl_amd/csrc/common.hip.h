@@ -23,6 +23,15 @@ typedef uint32_t u2a4 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t u2u2 __attribute__((ext_vector_type(2), aligned(2)));
 typedef uint32_t u4u1 __attribute__((ext_vector_type(4), aligned(1)));
 
+// 16-byte store at agent scope: written through the XCD's L2 and kept by the memory-side cache.  A
+// store of more than 8 bytes reads its data registers over the following cycles: the compiler
+// keeps the next vector instruction from overwriting them for stores it emits itself, not for
+// this one, hence the wait states inside the statement (without them lanes 12-15 of a row stored
+// the next value moved into the register now and then).
+__device__ __forceinline__ void store16_agent(void* p, u4a v) {
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
+}
+
 enum { kAdd = 0, kMul = 1, kMin = 2, kMax = 3 };
 
 // Maps a c10d reduce-op code to the kernel op set; -1 when unsupported.

@@ -62,20 +62,14 @@ __device__ __forceinline__ u4a load_vec_u(const void* p) {
         else return *(const u4u2*)p;
     }
 }
+// The folds' output: streaming loads, but stores that stay in the memory-side cache (256 MB), which
+// gathers them into longer write bursts between the reads and still holds them for the next call.
+// Binary fold in place, against streaming stores, three buffer pairs in turn: 2 M elements 4.1 us
+// (5.0), 6.5 M 11.0 (12.9), 13 M 20.1 (24.7), 20 M 29.8 (38.5), 26 M 47.9 (47.2), 96.5 M 174.7 (174);
+// loads without the hint are 10-40 % slower from 13 M on.  Ring fold, 8 ranks of 96.5 M: 566 (582).
 template <bool NT>
-__device__ __forceinline__ void store_vec_a(u4a* p, u4a v) {
-    if constexpr (NT) __builtin_nontemporal_store(v, p);
-    else *p = v;
-}
-
-// The ring fold's output: written through the XCD's L2 (agent scope) and left to the memory-side
-// cache, which gathers it into longer write bursts between the reads.  8 ranks, 386 MB per rank:
-// 566 us against 582 with a streaming store (bare kernel, rotating buffers).  (A store of
-// more than 8 bytes reads its registers over the following cycles: the wait states keep what
-// follows the statement from overwriting them.)
-template <bool NT>
-__device__ __forceinline__ void store_ring(u4a* p, u4a v) {
-    if constexpr (NT) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
+__device__ __forceinline__ void store_out(u4a* p, u4a v) {
+    if constexpr (NT) store16_agent(p, v);
     else *p = v;
 }
 
@@ -186,7 +180,7 @@ __device__ __forceinline__ void fold_span_block(char* dst, const char* src, uint
         const u4a d = load_vec_a<NT>((const u4a*)(dp + t * 16u));
         u4a s = d;
         if constexpr (F::needs_src) s = load_src<F::size, NT>(src + v * 16 + t * 16u);
-        store_vec_a<NT>((u4a*)(dp + t * 16u), F::vec(d, s, scale));
+        store_out<NT>((u4a*)(dp + t * 16u), F::vec(d, s, scale));
     };
     // (the launch gives a block one round unless the grid is capped)
     for (uint64_t v = (uint64_t)block * kFoldBlock; v < nvec; v += (uint64_t)nblocks * kFoldBlock) {
@@ -348,7 +342,7 @@ __global__ __launch_bounds__(kFoldBlock) void k_ring_fold(void* out, RingPtrs pt
                 u4a rv;
 #pragma unroll
                 for (int q = 0; q < 4; q++) rv[q] = f2u(apply_scale ? acc[u][q] * scale : acc[u][q]);
-                if (off[u] == (uint32_t)(u * kFoldBlock + threadIdx.x) * 16u) store_ring<NT>((u4a*)((char*)out + voff + base * 16 + off[u]), rv);
+                if (off[u] == (uint32_t)(u * kFoldBlock + threadIdx.x) * 16u) store_out<NT>((u4a*)((char*)out + voff + base * 16 + off[u]), rv);
             }
         } else {
             float acc[U][8];
@@ -395,7 +389,7 @@ __global__ __launch_bounds__(kFoldBlock) void k_ring_fold(void* out, RingPtrs pt
                     float hi = apply_scale ? acc[u][2 * q + 1] * scale : acc[u][2 * q + 1];
                     rv[q] = narrow16<DT>(lo) | (narrow16<DT>(hi) << 16);
                 }
-                if (off[u] == (uint32_t)(u * kFoldBlock + threadIdx.x) * 16u) store_ring<NT>((u4a*)((char*)out + voff + base * 16 + off[u]), rv);
+                if (off[u] == (uint32_t)(u * kFoldBlock + threadIdx.x) * 16u) store_out<NT>((u4a*)((char*)out + voff + base * 16 + off[u]), rv);
             }
         }
     }

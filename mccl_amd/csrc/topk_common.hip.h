@@ -196,18 +196,12 @@ __device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
 }
 // 16-byte streaming store written through to memory (agent scope): a later 4-byte
 // repair of the same line by a block on another XCD must not be overwritten by a
-// delayed write-back of this one.  A store of more than 8 bytes reads its data
-// registers over the following cycles: the compiler keeps the next vector
-// instruction from overwriting them for stores it emits itself, not for this one,
-// hence the wait states inside the statement.
+// delayed write-back of this one.  (The wait states: see store16_agent.)
 __device__ __forceinline__ void store_through(float* p, u4a v) {
     asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
 }
 
-// The window of a bucket, one 16-byte store and one 16-byte load: the four words change together.
-__device__ __forceinline__ void store16_agent(uint32_t* p, u4a v) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
-}
+// A bucket's window is one store16_agent and one load16_agent: the four words change together.
 // (waits for every earlier load of the wavefront as well: they complete in order)
 __device__ __forceinline__ u4a load16_agent(const uint32_t* p) {
     u4a v;
