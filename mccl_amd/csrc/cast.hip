@@ -11,8 +11,9 @@
 // without setting the quiet bit.  The tuning key "fp16_portable" selects that
 // behaviour, for bit-identical results with such a build.
 //
-// Both kernels stream with one tile per block in address order.  Narrowing
-// handles 8 elements per lane (two 16-byte loads, one 16-byte store).
+// Both kernels stream with one tile per block in address order.  A lane owns
+// 4 consecutive elements (16 bytes one side, 8 the other), or two such groups a
+// block apart; every access of a wavefront covers consecutive addresses.
 #include "common.hip.h"
 #include "runtime.h"
 
@@ -54,61 +55,74 @@ __device__ __forceinline__ uint32_t widen_transport(uint32_t h) {
     return PORTABLE ? f16_to_f32_portable(h) : f2u(widen_f16(h));
 }
 
-template <bool PORTABLE>
-__global__ __launch_bounds__(kBlock) void k_cast_f32_f16(const float* __restrict__ src, uint16_t* __restrict__ dst,
-                                                         uint64_t n) {
-    const uint64_t ngrp = n / 8;  // groups of 8 elements
-    for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < ngrp; i += (uint64_t)gridDim.x * kBlock) {
-        const u4a a = __builtin_nontemporal_load((const u4u4*)(src + i * 8));
-        const u4a b = __builtin_nontemporal_load((const u4u4*)(src + i * 8 + 4));
-        u4a o;
-        o[0] = narrow_transport<PORTABLE>(a[0]) | (narrow_transport<PORTABLE>(a[1]) << 16);
-        o[1] = narrow_transport<PORTABLE>(a[2]) | (narrow_transport<PORTABLE>(a[3]) << 16);
-        o[2] = narrow_transport<PORTABLE>(b[0]) | (narrow_transport<PORTABLE>(b[1]) << 16);
-        o[3] = narrow_transport<PORTABLE>(b[2]) | (narrow_transport<PORTABLE>(b[3]) << 16);
-        __builtin_nontemporal_store(o, (u4u2*)(dst + i * 8));
+// Measured with three buffer pairs in turn, us for 1.6 M / 6.5 M / 26 M / 96.5 M elements (6 B each):
+//   narrowing  two groups, one wavefront per block      3.0   6.4  22.2  87.8
+//              one group                                3.2   7.3  23.7  84.2
+//              8 elements per lane, 256 threads           -   8.2     -  93.2
+//   widening   two groups, one wavefront per block      3.0   6.6  22.5  91.6
+//              one group, four wavefronts               3.1   7.0  23.3  85.9
+//              two groups, four wavefronts, streamed      -   7.4     -  94.3
+// Streaming loads throughout, and stores that stay in the memory-side cache, where whoever takes
+// the payload reads them.  From kCastLarge elements on neither side fits there, and the shapes of
+// the right-hand column win.
+constexpr uint64_t kCastLarge = 48u << 20;
+
+template <bool PORTABLE, int THREADS, int GROUPS>
+__global__ __launch_bounds__(THREADS) void k_cast_f32_f16(const float* __restrict__ src, uint16_t* __restrict__ dst, uint64_t n) {
+    const uint64_t nquad = n / 4;
+    uint64_t q0 = (uint64_t)blockIdx.x * (THREADS * GROUPS);
+    for (; q0 < nquad; q0 += (uint64_t)gridDim.x * (THREADS * GROUPS)) {
+        const float* sp = src + q0 * 4;
+        uint16_t* dp = dst + q0 * 4;
+        u4a v[GROUPS];
+#pragma unroll
+        for (int j = 0; j < GROUPS; j++)
+            if (q0 + j * THREADS + threadIdx.x < nquad) v[j] = __builtin_nontemporal_load((const u4u4*)(sp + 4 * (j * THREADS + threadIdx.x)));
+#pragma unroll
+        for (int j = 0; j < GROUPS; j++)
+            if (q0 + j * THREADS + threadIdx.x < nquad)
+                store8_agent(dp + 4 * (j * THREADS + threadIdx.x),
+                             u2a{narrow_transport<PORTABLE>(v[j][0]) | (narrow_transport<PORTABLE>(v[j][1]) << 16),
+                                 narrow_transport<PORTABLE>(v[j][2]) | (narrow_transport<PORTABLE>(v[j][3]) << 16)});
     }
-    const uint64_t g = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (g < 8 && ngrp * 8 + g < n) dst[ngrp * 8 + g] = (uint16_t)narrow_transport<PORTABLE>(f2u(src[ngrp * 8 + g]));
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) dst[nquad * 4 + threadIdx.x] = (uint16_t)narrow_transport<PORTABLE>(f2u(src[nquad * 4 + threadIdx.x]));
 }
 
-// Widening writes twice what it reads, so the layout follows the stores: a lane
-// owns 4 consecutive elements (one 8-byte load, one 16-byte store) and a wave's
-// store covers 1 KiB of consecutive addresses; kWidenQuads such groups per lane,
-// a block apart, keep several loads in flight (measured on the 96.5 M-element
-// gradient: 1 group 6.11, 2 groups 6.24, 4 groups 5.84, 8 groups 5.50 TB/s).
-constexpr int kWidenQuads = 2;
-
-template <bool PORTABLE>
-__global__ __launch_bounds__(kBlock) void k_cast_f16_f32(const uint16_t* __restrict__ src, float* __restrict__ dst,
-                                                         uint64_t n) {
+template <bool PORTABLE, int THREADS, int GROUPS>
+__global__ __launch_bounds__(THREADS) void k_cast_f16_f32(const uint16_t* __restrict__ src, float* __restrict__ dst, uint64_t n) {
     const uint64_t nquad = n / 4;
-    for (uint64_t base = (uint64_t)blockIdx.x * (kBlock * kWidenQuads); base < nquad;
-         base += (uint64_t)gridDim.x * (kBlock * kWidenQuads)) {
-        u2a h[kWidenQuads];
+    uint64_t q0 = (uint64_t)blockIdx.x * (THREADS * GROUPS);
+    for (; q0 < nquad; q0 += (uint64_t)gridDim.x * (THREADS * GROUPS)) {
+        const uint16_t* sp = src + q0 * 4;
+        float* dp = dst + q0 * 4;
+        u2a h[GROUPS];
 #pragma unroll
-        for (int j = 0; j < kWidenQuads; j++) {
-            const uint64_t q = base + (uint64_t)j * kBlock + threadIdx.x;
-            if (q < nquad) h[j] = __builtin_nontemporal_load((const u2u2*)(src + q * 4));
-        }
+        for (int j = 0; j < GROUPS; j++)
+            if (q0 + j * THREADS + threadIdx.x < nquad) h[j] = __builtin_nontemporal_load((const u2u2*)(sp + 4 * (j * THREADS + threadIdx.x)));
 #pragma unroll
-        for (int j = 0; j < kWidenQuads; j++) {
-            const uint64_t q = base + (uint64_t)j * kBlock + threadIdx.x;
-            if (q < nquad) {
-                u4a o;
-                o[0] = widen_transport<PORTABLE>(h[j][0] & 0xFFFFu); o[1] = widen_transport<PORTABLE>(h[j][0] >> 16);
-                o[2] = widen_transport<PORTABLE>(h[j][1] & 0xFFFFu); o[3] = widen_transport<PORTABLE>(h[j][1] >> 16);
-                __builtin_nontemporal_store(o, (u4u4*)(dst + q * 4));
-            }
-        }
+        for (int j = 0; j < GROUPS; j++)
+            if (q0 + j * THREADS + threadIdx.x < nquad)
+                store16_agent(dp + 4 * (j * THREADS + threadIdx.x),
+                              u4a{widen_transport<PORTABLE>(h[j][0] & 0xFFFFu), widen_transport<PORTABLE>(h[j][0] >> 16),
+                                  widen_transport<PORTABLE>(h[j][1] & 0xFFFFu), widen_transport<PORTABLE>(h[j][1] >> 16)});
     }
-    const uint64_t g = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (g < 4 && nquad * 4 + g < n) dst[nquad * 4 + g] = u2f(widen_transport<PORTABLE>(src[nquad * 4 + g]));
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) dst[nquad * 4 + threadIdx.x] = u2f(widen_transport<PORTABLE>(src[nquad * 4 + threadIdx.x]));
 }
 
 uint32_t cast_blocks(uint64_t n, uint64_t per_block) {
     const uint64_t cap = (uint64_t)device_info().num_cus * (uint64_t)tuning().fold_blocks_per_cu;
     return clamp_u32((n + per_block - 1) / per_block, 1, cap);
+}
+
+template <bool PORTABLE>
+void launch_narrow(const float* src, uint16_t* dst, uint64_t n, hipStream_t st) {
+    if (n < kCastLarge) k_cast_f32_f16<PORTABLE, 64, 2><<<cast_blocks(n, 8 * 64), 64, 0, st>>>(src, dst, n);
+    else k_cast_f32_f16<PORTABLE, 64, 1><<<cast_blocks(n, 4 * 64), 64, 0, st>>>(src, dst, n);
+}
+template <bool PORTABLE>
+void launch_widen(const uint16_t* src, float* dst, uint64_t n, hipStream_t st) {
+    if (n < kCastLarge) k_cast_f16_f32<PORTABLE, 64, 2><<<cast_blocks(n, 8 * 64), 64, 0, st>>>(src, dst, n);
+    else k_cast_f16_f32<PORTABLE, 256, 1><<<cast_blocks(n, 4 * 256), 256, 0, st>>>(src, dst, n);
 }
 
 }  // namespace
@@ -123,10 +137,8 @@ int mccl_hip_cast_f32_to_f16(const float* src, void* dst, uint64_t n, void* stre
     if (!src || !dst || n > MCCL_HIP_MAX_ELEMS || ((uintptr_t)src & 3) || ((uintptr_t)dst & 1)) return MCCL_HIP_ERR_ARG;
     int rc = mccl_hip_init();
     if (rc) return rc;
-    if (tuning().fp16_portable)
-        k_cast_f32_f16<true><<<cast_blocks(n, 8 * kBlock), kBlock, 0, (hipStream_t)stream>>>(src, (uint16_t*)dst, n);
-    else
-        k_cast_f32_f16<false><<<cast_blocks(n, 8 * kBlock), kBlock, 0, (hipStream_t)stream>>>(src, (uint16_t*)dst, n);
+    if (tuning().fp16_portable) launch_narrow<true>(src, (uint16_t*)dst, n, (hipStream_t)stream);
+    else launch_narrow<false>(src, (uint16_t*)dst, n, (hipStream_t)stream);
     return launch_status();
 }
 
@@ -135,10 +147,8 @@ int mccl_hip_cast_f16_to_f32(const void* src, float* dst, uint64_t n, void* stre
     if (!src || !dst || n > MCCL_HIP_MAX_ELEMS || ((uintptr_t)dst & 3) || ((uintptr_t)src & 1)) return MCCL_HIP_ERR_ARG;
     int rc = mccl_hip_init();
     if (rc) return rc;
-    if (tuning().fp16_portable)
-        k_cast_f16_f32<true><<<cast_blocks(n, 4 * kBlock * kWidenQuads), kBlock, 0, (hipStream_t)stream>>>((const uint16_t*)src, dst, n);
-    else
-        k_cast_f16_f32<false><<<cast_blocks(n, 4 * kBlock * kWidenQuads), kBlock, 0, (hipStream_t)stream>>>((const uint16_t*)src, dst, n);
+    if (tuning().fp16_portable) launch_widen<true>((const uint16_t*)src, dst, n, (hipStream_t)stream);
+    else launch_widen<false>((const uint16_t*)src, dst, n, (hipStream_t)stream);
     return launch_status();
 }
 
