@@ -1424,7 +1424,7 @@ enum Path { kPathExact, kPathStream, kPathResident };
 // Which kernels a call takes (tuning key "topk_path": 1, 2, 3 fix it).  `counts`: the buckets'
 // lengths when they are listed, else null.  Measured per call, us:
 //   resident up to 512 blocks, as many as the GPU holds at once: one launch against two or six
-//     (65,536 elements: 15 against 28 exact; 1 M: 24.5 against 26 streaming; 8 x 262,144: 26 against
+//     (65,536 elements: 15 against 28 exact; 1 M: 22 against 26 streaming; 8 x 262,144: 26 against
 //     29 streaming).  Beyond, its blocks wait their turn and its barriers lie open (16 x 262,144: 54
 //     against 37 streaming; 64 x 131,072: 99 against 84 exact) - except for buckets of a few blocks
 //     (1500 x 16,384: 167 against 187 exact) ...
@@ -1440,7 +1440,7 @@ Path choose_path(const Geometry& g, const uint64_t* counts) {
     if (path == 1 && !counts) return kPathExact;
     if (path == 2 && streams) return kPathStream;
     if (path == 3 && fits) return kPathResident;
-    const int vecs = resident_vecs(g.bucket_elems);
+    const int vecs = resident_vecs(g.bucket_elems, g.nbuckets);
     const uint64_t per = (uint64_t)vecs * kFTile;
     uint64_t blocks = 0;
     if (counts) for (uint32_t b = 0; b < g.nbuckets; b++) blocks += (counts[b] + per - 1) / per;

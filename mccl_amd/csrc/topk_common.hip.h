@@ -19,11 +19,15 @@ constexpr uint32_t kPoisonK = 0xFFFFFFFFu;    // payload header of a bucket whos
 constexpr int kRList = 1024;                  // elements of the picked bin that are ranked as a list
 constexpr uint64_t kRMaxBlocks = 128;         // blocks of one bucket
 constexpr uint64_t kRMaxBucket = kRMaxBlocks * 1024 * 4 * 4;  // 2,097,152 elements
-constexpr uint32_t kRRow = 2048 + 64;         // one round's histogram: 2048 bins, the count above them, padding
+constexpr uint32_t kRSampleMin = 1u << 18;    // buckets of this many elements start from a sampled window
+constexpr uint32_t kRRow = 2048 + 64;         // one round's histogram: its bins, the count above them, padding
+constexpr uint32_t kRRows = 4;                // a windowed round, three on the full key range (11 + 11 + 9 bits)
 constexpr uint32_t kRBars = 6;                // barriers: at most four rounds and the list / ties
-constexpr uint32_t kRBar = 4 * kRRow;         // their counters, 256 bytes apart, then the list's fill counter
-constexpr uint32_t kRZeroWords = kRBar + 64 * (kRBars + 1);   // cleared by the lead block
-constexpr uint32_t kRCnt = kRZeroWords;       // per block: elements above the bin, inside the bin
+constexpr uint32_t kRBarLines = 8;            // counters of a barrier, 256 bytes apart
+constexpr uint32_t kRBarWords = 64 * kRBarLines;
+constexpr uint32_t kRFill = kRBars * kRBarWords;   // after the barriers: the list's fill counter
+constexpr uint32_t kRRow0 = kRFill + 64;
+constexpr uint32_t kRCnt = kRRow0 + kRRows * kRRow;           // per block: elements above the bin, inside the bin
 constexpr uint32_t kRListAt = kRCnt + 2 * (uint32_t)kRMaxBlocks;
 constexpr uint32_t kRWords = kRListAt + 2 * kRList;
 constexpr int kFSample = 8192;                // sampled elements per bucket
@@ -127,7 +131,7 @@ __device__ __forceinline__ uint32_t* bucket_wire(const Geometry& g, BucketsArg b
 }
 
 
-int resident_vecs(uint64_t n);
+int resident_vecs(uint64_t n, uint32_t nbuckets);
 void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t epoch, uint32_t published,
                      uint64_t limit_ticks, hipStream_t st);
 
@@ -210,6 +214,7 @@ __device__ __forceinline__ u4a load16_agent(const uint32_t* p) {
 }
 // Waits until the bucket's window is published (S_READY == epoch); called by a whole wavefront
 // or a single thread.  win[3] = 0 when the wait timed out.
+template <int SLEEP = 16>
 __device__ __forceinline__ u4a wait_window(const uint32_t* st, uint32_t epoch, uint64_t limit_ticks) {
     uint64_t t0 = 0;
     uint32_t polls = 0;
@@ -219,7 +224,7 @@ __device__ __forceinline__ u4a wait_window(const uint32_t* st, uint32_t epoch, u
             v[3] = 1u;
             return v;
         }
-        __builtin_amdgcn_s_sleep(16);
+        __builtin_amdgcn_s_sleep(SLEEP);
         if ((++polls & 63u) == 0) {
             const uint64_t now = (uint64_t)wall_clock64();
             if (t0 == 0) t0 = now;
@@ -232,8 +237,13 @@ __device__ __forceinline__ u4a wait_window(const uint32_t* st, uint32_t epoch, u
 }
 
 // ---- sample ------------------------------------------------------------------------
+// The first round's histogram is kept in copies, by lane, a few banks apart: gradients share few
+// exponents, and lanes that add to one LDS word take turns (8192 keys: 1.6 to 2.4 us with one copy).
 template <int THREADS>
 struct SampleLds {
+    static constexpr int kCopies = THREADS >= 1024 ? 4 : 1;
+    static constexpr int kCopy = kBins0 + 8;  // words
+    uint32_t h0[kCopies * kCopy] __attribute__((aligned(16)));
     uint32_t lh[3][kBinsR] __attribute__((aligned(16)));
     uint32_t wsum[3][THREADS / kWave];
     uint32_t res[3][2];
@@ -243,8 +253,8 @@ struct SampleLds {
 // and how many of the rank's elements fall inside that bin.  Thread t owns the PER bins below
 // BINS - PER t (vector LDS reads).  res[z] = {bin, left}; bin = BINS when the histogram holds
 // fewer than rank[z] elements or rank[z] == 0.  SHARED: all ranks are read off h[0].  Called
-// by all threads of the block.
-template <int BINS, int NR, int THREADS, bool SHARED = false>
+// by all threads of the block.  COPIES: every histogram is the sum of that many, STRIDE words apart.
+template <int BINS, int NR, int THREADS, bool SHARED = false, int COPIES = 1, int STRIDE = 0>
 __device__ __forceinline__ void sample_pick(const uint32_t* const (&h)[NR], const uint32_t (&rank)[NR],
                                             uint32_t (*wsum)[THREADS / kWave], uint32_t (*res)[2]) {
     constexpr int PER = BINS / THREADS;
@@ -253,7 +263,7 @@ __device__ __forceinline__ void sample_pick(const uint32_t* const (&h)[NR], cons
     static_assert(PER % RW == 0, "whole vectors");
     typedef uint32_t Row __attribute__((ext_vector_type(RW)));
     const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     uint32_t c[NH][PER], sum[NH], inc[NH];  // c[z][j]: bin BINS - 1 - PER t - j
 #pragma unroll
     for (int z = 0; z < NH; z++) {
@@ -261,7 +271,9 @@ __device__ __forceinline__ void sample_pick(const uint32_t* const (&h)[NR], cons
         sum[z] = 0;
 #pragma unroll
         for (int v = 0; v < PER / RW; v++) {
-            const Row x = row[PER / RW - 1 - v];
+            Row x = row[PER / RW - 1 - v];
+#pragma unroll
+            for (int d = 1; d < COPIES; d++) x += row[PER / RW - 1 - v + d * (STRIDE / RW)];
 #pragma unroll
             for (int q = 0; q < RW; q++) {
                 c[z][v * RW + q] = x[RW - 1 - q];
@@ -276,10 +288,8 @@ __device__ __forceinline__ void sample_pick(const uint32_t* const (&h)[NR], cons
     uint32_t above0[NH];
 #pragma unroll
     for (int z = 0; z < NH; z++) {
-        above0[z] = inc[z] - sum[z];
-#pragma unroll
-        for (int i = 0; i < THREADS / kWave; i++)
-            if (i < wave) above0[z] += wsum[z][i];
+        const uint32_t s = lane < THREADS / kWave ? wsum[z][lane] : 0u;
+        above0[z] = inc[z] - sum[z] + (uint32_t)__builtin_amdgcn_readlane((int)(wave_inclusive_scan(s) - s), wave);
     }
 #pragma unroll
     for (int z = 0; z < NR; z++) {
@@ -324,11 +334,13 @@ __device__ __forceinline__ SampleWindow sample_window(const float* gp, const flo
         rv[j] = nsv ? *(const u4u4*)(rp + v * 4) : u4a{0u, 0u, 0u, 0u};
     }
     under_way();
-    uint32_t* const h0 = &L.lh[0][0];  // round 0 uses 2048 bins: lh[0] and lh[1] are adjacent
+    constexpr int COPIES = SampleLds<THREADS>::kCopies, COPY = SampleLds<THREADS>::kCopy;
     {
         const u4a z = {0u, 0u, 0u, 0u};
-        for (int i = threadIdx.x; i < 3 * kBinsR / 4; i += THREADS) ((u4a*)h0)[i] = z;
+        static_assert(offsetof(SampleLds<THREADS>, lh) == sizeof(L.h0), "cleared as one");
+        for (int i = threadIdx.x; i < (COPIES * COPY + 3 * kBinsR) / 4; i += THREADS) ((u4a*)L.h0)[i] = z;
     }
+    uint32_t* const h0 = L.h0 + (threadIdx.x % COPIES) * COPY;
     uint32_t key[PV][4];
 #pragma unroll
     for (int j = 0; j < PV; j++) {
@@ -360,22 +372,16 @@ __device__ __forceinline__ SampleWindow sample_window(const float* gp, const flo
             if (key[j][q] != 0xFFFFFFFFu) atomicAdd(&h0[key[j][q] >> 20], 1u);
     __syncthreads();
     {
-        const uint32_t* const hs[NR] = {h0, h0, h0};
+        const uint32_t* const hs[NR] = {L.h0, L.h0, L.h0};
         const uint32_t want[NR] = {active[0] ? rank[0] : 0u, active[1] ? rank[1] : 0u, active[2] ? rank[2] : 0u};
-        sample_pick<kBins0, NR, THREADS, true>(hs, want, L.wsum, L.res);
+        sample_pick<kBins0, NR, THREADS, true, COPIES, COPY>(hs, want, L.wsum, L.res);
     }
 #pragma unroll
     for (int z = 0; z < NR; z++) {
         prefix[z] = L.res[z][0] << 20;
         rank[z] = L.res[z][1];
     }
-    __syncthreads();
     // round 1: key[19:10] among the keys that share a rank's first digit
-    {
-        const u4a z = {0u, 0u, 0u, 0u};
-        for (int i = threadIdx.x; i < 3 * kBinsR / 4; i += THREADS) ((u4a*)h0)[i] = z;
-    }
-    __syncthreads();
     // (three comparisons per key; the few keys that share a rank's first digit take the branch)
     const uint32_t d0 = active[0] ? prefix[0] >> 20 : 0xFFFFFFFFu, d1 = active[1] ? prefix[1] >> 20 : 0xFFFFFFFFu,
                    d2 = active[2] ? prefix[2] >> 20 : 0xFFFFFFFFu;

@@ -14,14 +14,15 @@
 // one-block bucket needs no memory but its own.  Any ratio and any distribution takes this path:
 // nothing depends on how the keys are spread.
 //
-// What bounds it is latency, not bandwidth: for one bucket of 65,536 elements (1.3 MB of traffic)
-// launch 3 us, load 1.3, two rounds of 0.8 + 1.3 (barrier) + 1, list 1.3 + 1.5 (barrier), rank and
-// scan 1.5, store 0.5.  Against the six launches of the exact path: 4096 elements 7.4 us (25.5),
-// 65,537 17.4 (27.7), 262,144 19.0 (25.4 on the two-launch path), 1 M 23.5 (26.7); at a ratio of
-// 5 % 1 M elements 24.7 us (84.9) and 2 M 30.4 (144).
+// What bounds it is latency, not bandwidth.  One bucket of 1 M elements (16 MB of traffic), us from
+// the first block's start: window published 5.7, seen 6.4, first round's histogram in LDS 7.7, added up
+// and the blocks met 10.8, bin picked 11.8, listed 12.4, met 14.9, ranked 16.5, picks scanned 18.0,
+// stored 19.0.  Per call: 4096 elements 7.4 us (25.5 on the six launches of the exact path), 65,537 14.8
+// (27.7), 262,144 17.9 (25.4 on the two-launch path), 1 M 21.7 (26.7), 2 M 26.0; at a ratio of 5 % 1 M
+// elements 22.9 us (84.9) and 2 M 27.8 (144).
 //
 // The blocks of a bucket wait for one another, so they have to be resident together.  At 64
-// registers, 25 KiB of LDS and 1024 threads two blocks fit a CU, 64 an XCD; a bucket has at most 128 blocks,
+// registers, 54 KiB of LDS and 1024 threads two blocks fit a CU, 64 an XCD; a bucket has at most 128 blocks,
 // 16 per XCD.  Every XCD dispatches its share of a grid in grid order, so only the newest bucket
 // of a launch can be incompletely dispatched on it, with at most 15 blocks that wait: the four
 // hardware queues of a process can have four such launches under way and still leave a slot.
@@ -35,10 +36,10 @@ namespace {
 
 constexpr int kRThreads = 1024;
 constexpr int kRWaves = kRThreads / kWave;
-constexpr int kRBins = 2048;       // bins of one round
+constexpr int kRBits = 11;
+constexpr int kRBins = 1 << kRBits;  // bins of one round
 constexpr int kRRank = 96;          // a list longer than this is split before it is ranked
 static_assert(kRBins == 2 * kRThreads, "a thread owns two bins");
-constexpr uint32_t kRSampleMin = 1u << 18;  // buckets of this many elements start from a sampled window
 
 template <int V>
 struct ResidentLds {
@@ -99,15 +100,26 @@ __device__ __forceinline__ uint32_t pick_bin2(u2a two, uint32_t above, uint32_t 
     return total;
 }
 
-// All threads of the block; every store and atomic of the block has arrived when it is counted.
-__device__ __forceinline__ bool resident_barrier(uint32_t* counter, uint32_t parties, uint32_t* flag, uint64_t limit_ticks) {
+// All threads of block x of the bucket; every store and atomic of the block has arrived when it is
+// counted.  Atomics on one cache line are carried out one after the other, some 25 ns each: the
+// arrivals go to eight lines, and eight lanes read them at once (2 M elements, 123 blocks, one line
+// against eight: barrier after the histogram 6.3 / 5.0 us, after the list 4.0 / 3.0; a flag word per
+// block instead of counters 5.8 and 3.5).  What is left of the first is the histogram's own 64 lines,
+// to which every block adds: fewer bins take as long, copies of it give back in reading what they save.
+__device__ __forceinline__ void resident_arrive(uint32_t* counters, uint32_t x) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) {
-        __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(counters + 64 * (x % kRBarLines), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool resident_barrier(uint32_t* counters, uint32_t parties, uint32_t x, uint32_t* flag, uint64_t limit_ticks) {
+    resident_arrive(counters, x);
+    if (threadIdx.x < kWave) {
+        const uint32_t lane = threadIdx.x;
+        const bool reads = lane < kRBarLines && lane < parties;
+        const uint32_t want = (parties - lane + kRBarLines - 1) / kRBarLines;  // blocks x with x % kRBarLines == lane
         uint64_t t0 = 0;
         uint32_t ok = 1, polls = 0;
-        while (ld_agent(counter) < parties) {
+        while (__ballot(reads && ld_agent(counters + 64 * lane) < want)) {
             __builtin_amdgcn_s_sleep(1);
             if ((++polls & 255u) == 0) {
                 const uint64_t now = (uint64_t)wall_clock64();
@@ -118,7 +130,7 @@ __device__ __forceinline__ bool resident_barrier(uint32_t* counter, uint32_t par
                 }
             }
         }
-        *flag = ok;
+        if (lane == 0) *flag = ok;
     }
     __syncthreads();
     return *flag != 0;
@@ -144,19 +156,26 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
     if (blockIdx.x == 0) {
         // ---- lead block: clears what the others add into and publishes the first round's key range
         if (nblk == 1) return;
-        auto clear = [&] {
-            for (uint32_t i = threadIdx.x; i < kRZeroWords / 4; i += kRThreads) store16_agent(mem + i * 4, u4a{0u, 0u, 0u, 0u});
+        auto clear = [&](uint32_t from, uint32_t to) {
+            for (uint32_t i = from / 4 + threadIdx.x; i < to / 4; i += kRThreads) store16_agent(mem + i * 4, u4a{0u, 0u, 0u, 0u});
+        };
+        // Before the window is published: what the blocks touch before they have met once.  The rest is
+        // cleared after it, and the lead block takes part in their first barrier.
+        auto clear_first = [&] {
+            clear(0, kRRow0 + kRRow);
             if (threadIdx.x == 0) {
                 st_agent(st + S_OK, 0u);
                 st_agent(st + S_TIMEOUT, 0u);
             }
         };
         SampleWindow win = {0u, 0x7FFFFFFFu, 0u};
-        if (bn >= kRSampleMin) win = sample_window<kRThreads>(gbase, rbase, bn, k, L.s, clear);
-        else clear();
+        if (bn >= kRSampleMin) win = sample_window<kRThreads>(gbase, rbase, bn, k, L.s, clear_first);
+        else clear_first();
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (threadIdx.x == 0) store16_agent(st + S_LO_KEY, u4a{win.lo, win.hi, 0u, published});
+        clear(kRRow0 + kRRow, kRCnt);
+        resident_arrive(mem, nblk);
         return;
     }
     const uint32_t x = blockIdx.x - 1;
@@ -219,7 +238,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
     bool window = false;
     if (nblk > 1) {
         if (threadIdx.x == 0) {
-            const u4a wn = wait_window(st, epoch, limit_ticks);
+            const u4a wn = wait_window<2>(st, epoch, limit_ticks);
             L.win[0] = wn[0]; L.win[1] = wn[1]; L.win[3] = wn[3];
         }
         __syncthreads();
@@ -233,37 +252,50 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
     }
     uint32_t r = k;         // picks still to place among the keys of the range and above it
     bool first = true;      // the keys above the range are not accounted for in r yet
-    uint32_t bar = 0, sh, bin, m, row = 0;
+    uint32_t sh, bin, m, row = 0;
     for (;;) {
         sh = 32 - __clz(span - 1);
         if (span == 1) sh = 0;
-        sh = sh > 11 ? sh - 11 : 0;
+        sh = sh > (uint32_t)kRBits ? sh - kRBits : 0;
         for (int i = threadIdx.x; i < (kRBins + 4) / 4; i += kRThreads) ((u4a*)L.lh)[i] = u4a{0u, 0u, 0u, 0u};
         __syncthreads();
+        if (base == 0) {
+            // every key: zeros, which would all add to one LDS word, are counted by the wavefront
+            uint32_t zeros = 0;
 #pragma unroll
-        for (int u = 0; u < V; u++) {
-            const u4a v = vec(u);
+            for (int u = 0; u < V; u++) {
+                const u4a v = vec(u);
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const uint32_t d = (v[q] & 0x7FFFFFFFu) - base;
-                if ((int)d >= 0) atomicAdd(&L.lh[d < span ? d >> sh : (uint32_t)kRBins], 1u);
+                for (int q = 0; q < 4; q++) {
+                    const uint32_t key = v[q] & 0x7FFFFFFFu;
+                    zeros += (uint32_t)__popcll(__ballot(key == 0));
+                    if (key != 0) atomicAdd(&L.lh[key < span ? key >> sh : (uint32_t)kRBins], 1u);
+                }
+            }
+            if (lane == 0 && zeros) atomicAdd(&L.lh[0], zeros);
+        } else {
+#pragma unroll
+            for (int u = 0; u < V; u++) {
+                const u4a v = vec(u);
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const uint32_t d = (v[q] & 0x7FFFFFFFu) - base;
+                    if ((int)d >= 0) atomicAdd(&L.lh[d < span ? d >> sh : (uint32_t)kRBins], 1u);
+                }
             }
         }
         __syncthreads();
-        // two bins per thread, counted from the top: thread 0 owns the highest two
         u2a all = ((const u2a*)L.lh)[kRThreads - 1 - threadIdx.x];
         uint32_t above = first ? L.lh[kRBins] : 0u;
         if (nblk > 1) {
-            uint32_t* const gh = mem + row * kRRow;
-            for (uint32_t i = threadIdx.x; i <= (uint32_t)kRBins; i += kRThreads) {
-                const uint32_t c = L.lh[i];
-                if (c) __hip_atomic_fetch_add(gh + i, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            if (!resident_barrier(mem + kRBar + 64 * bar, nblk, &L.flag, limit_ticks)) {
+            uint32_t* const gh = mem + kRRow0 + row * kRRow;
+            const uint64_t c = ((const uint64_t*)L.lh)[threadIdx.x];
+            if (c) __hip_atomic_fetch_add((uint64_t*)gh + threadIdx.x, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // two bins
+            if (threadIdx.x == 0 && above) __hip_atomic_fetch_add(gh + kRBins, above, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (!resident_barrier(mem + kRBarWords * row, row == 0 ? nblk + 1 : nblk, x, &L.flag, limit_ticks)) {
                 give_up();
                 return;
             }
-            bar++;
             row++;
             const uint64_t two = ld_agent64((const uint64_t*)gh + (kRThreads - 1 - threadIdx.x));
             above = first ? ld_agent(gh + kRBins) : 0u;
@@ -306,7 +338,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
             if (nblk > 1) {
                 st_agent64(cnts + x, ((uint64_t)gt << 32) | eq);
                 if (!tied && eq)
-                    L.base = __hip_atomic_fetch_add(mem + kRBar + 64 * kRBars, eq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    L.base = __hip_atomic_fetch_add(mem + kRFill, eq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
         __syncthreads();
@@ -332,7 +364,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
         }
         uint32_t gt_before = 0, eq_before = 0;
         if (nblk > 1) {
-            if (!resident_barrier(mem + kRBar + 64 * bar, nblk, &L.flag, limit_ticks)) {
+            if (!resident_barrier(mem + kRBarWords * row, nblk, x, &L.flag, limit_ticks)) {
                 give_up();
                 return;
             }
@@ -352,7 +384,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
             bool in = threadIdx.x < m;
             if (m > (uint32_t)kRRank && span > 1) {  // block-uniform
                 sh = 32 - __clz(span - 1);
-                sh = sh > 11 ? sh - 11 : 0;
+                sh = sh > (uint32_t)kRBits ? sh - kRBits : 0;
                 ((u2a*)L.lh)[threadIdx.x] = u2a{0u, 0u};
                 if (threadIdx.x == 0) L.count = 0;
                 __syncthreads();
@@ -491,13 +523,17 @@ void launch(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t e
 }  // namespace
 
 // Vectors per thread for buckets of up to n elements.  The barriers cost more with more blocks, the
-// passes over a block's elements with more vectors; measured (one bucket, 1 %): 200,000 elements
-// 17.9 / 19.8 / 28.1 us with 1 / 2 / 4 vectors, 524,288 elements 22.4 / 20.6 / 21.2 us.
-int resident_vecs(uint64_t n) { return n <= 64 * 4096 ? 1 : n <= 64 * 8192 ? 2 : 4; }
+// passes over a block's elements with more vectors; measured (one bucket, 1 %): 262,144 elements
+// 17.8 / 18.0 us with 1 / 2 vectors, 400,000 19.8 / 19.5, 524,288 20.0 / 19.3 / 20.7 with 1 / 2 / 4,
+// 700,000 21.1 / 22.2 with 2 / 4, 1 M 21.7 / 22.0.  Several buckets in a launch keep to 64 blocks
+// each, so that more of them are resident at once.
+int resident_vecs(uint64_t n, uint32_t nbuckets) {
+    return n <= 64 * 4096 ? 1 : n <= (nbuckets == 1 ? 128 : 64) * 8192 ? 2 : 4;
+}
 
 void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t epoch, uint32_t published,
                      uint64_t limit_ticks, hipStream_t st) {
-    switch (resident_vecs(g.bucket_elems)) {
+    switch (resident_vecs(g.bucket_elems, g.nbuckets)) {
         case 1: launch<1>(bk, g, w, epoch, published, limit_ticks, st); break;
         case 2: launch<2>(bk, g, w, epoch, published, limit_ticks, st); break;
         default: launch<4>(bk, g, w, epoch, published, limit_ticks, st); break;

@@ -12,7 +12,8 @@ from tests._gpu_util import DEV, to_dev, to_np, bits, student_t
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [1, 3, 4095, 4096, 4097, 12_289, 262_143, 262_144, 262_145, 524_288, 524_289, 2_097_151, 2_097_152]
+SIZES = [1, 3, 4095, 4096, 4097, 12_289, 262_143, 262_144, 262_145, 524_288, 524_289, 1_048_576, 1_048_577,
+         2_097_151, 2_097_152]
 
 
 @pytest.fixture()
