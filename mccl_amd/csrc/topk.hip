@@ -1427,7 +1427,7 @@ enum Path { kPathExact, kPathStream, kPathResident };
 //     (65,536 elements: 15 against 28 exact; 1 M: 22 against 26 streaming; 8 x 262,144: 26 against
 //     29 streaming).  Beyond, its blocks wait their turn and its barriers lie open (16 x 262,144: 54
 //     against 37 streaming; 64 x 131,072: 99 against 84 exact) - except for buckets of a few blocks
-//     (1500 x 16,384: 167 against 187 exact) ...
+//     (1500 x 16,384: 166 against 187 exact) ...
 //   ... and where the streaming path's tiles run out of candidate slots (128 per 4096 elements, more
 //     than 3 % inside the sampled window: ratios above about 0.015).  Its tiles are then read again
 //     as a whole (5 %, 2 M elements: 145 us against 30 resident; 6.5 M: 448 against 144 exact; from

@@ -19,7 +19,6 @@ constexpr uint32_t kPoisonK = 0xFFFFFFFFu;    // payload header of a bucket whos
 constexpr int kRList = 1024;                  // elements of the picked bin that are ranked as a list
 constexpr uint64_t kRMaxBlocks = 128;         // blocks of one bucket
 constexpr uint64_t kRMaxBucket = kRMaxBlocks * 1024 * 4 * 4;  // 2,097,152 elements
-constexpr uint32_t kRSampleMin = 1u << 18;    // buckets of this many elements start from a sampled window
 constexpr uint32_t kRRow = 2048 + 64;         // one round's histogram: its bins, the count above them, padding
 constexpr uint32_t kRRows = 4;                // a windowed round, three on the full key range (11 + 11 + 9 bits)
 constexpr uint32_t kRBars = 6;                // barriers: at most four rounds and the list / ties
@@ -106,6 +105,7 @@ struct Buckets {
     uint8_t* lwire[kMaxListed];
     uint32_t lcount[kMaxListed];
     uint32_t lk[kMaxListed];
+    uint32_t lfirst[kMaxListed];  // resident path: the bucket's first block
 };
 // The kernels index the table by bucket number.  Indexing the by-value parameter would make
 // the compiler copy all of it to per-lane scratch memory first (2 KiB per lane, and a launch

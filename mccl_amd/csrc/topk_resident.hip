@@ -28,6 +28,7 @@
 // hardware queues of a process can have four such launches under way and still leave a slot.
 #include "topk_common.hip.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace mcclhip {
@@ -136,24 +137,50 @@ __device__ __forceinline__ bool resident_barrier(uint32_t* counters, uint32_t pa
     return *flag != 0;
 }
 
-// grid: x = 0 the bucket's lead block, then its blocks; y = bucket.
+// grid: a lead block for each of the first `nlead` buckets, then bucket by bucket its blocks.
 template <int V>
-__global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometry g, Workspace w, uint32_t epoch,
+__global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometry g, Workspace w, uint32_t nlead, uint32_t epoch,
                                                                 uint32_t published, uint64_t limit_ticks) {
     constexpr uint32_t PER = kRThreads * 4 * V;  // elements of a block
+    // Buckets of this many elements start from a sampled window.  A sample costs about 5 us and saves a
+    // round; beside buckets that need theirs anyway a second round is what ends last (24 buckets of 1001
+    // to 1.5 M elements: 31.1 us with 2^18 throughout, 29.9 with 2^16 for four vectors, 29.3 with 2^15).
+    constexpr uint32_t kSampleMin = V == 4 ? 1u << 15 : V == 2 ? 1u << 16 : 1u << 18;
     const BucketsArg bk = buckets_arg();
     __shared__ ResidentLds<V> L;
-    const uint32_t b = blockIdx.y;
+    const int lane = threadIdx.x & (kWave - 1);
+    const bool lead = blockIdx.x < nlead;
+    uint32_t b = blockIdx.x, x = 0;  // bucket, block of the bucket
+    if (!lead) {
+        const uint32_t j = blockIdx.x - nlead;
+        if (g.listed) {
+            // on the scalar unit: the block's loads wait for it
+            b = 0;
+            for (uint32_t c = 0; c < kMaxListed && bk->lfirst[c] <= j; c += 16) {
+#pragma unroll
+                for (uint32_t i = 0; i < 16; i++) {
+                    const uint32_t first = bk->lfirst[c + i];  // 0xFFFFFFFF past the list
+                    if (first <= j) {
+                        b = c + i;
+                        x = j - first;
+                    }
+                }
+            }
+        } else {
+            const uint32_t per_bucket = (uint32_t)((g.bucket_elems + PER - 1) / PER);
+            b = j / per_bucket;
+            x = j - b * per_bucket;
+        }
+    }
     const uint64_t bn = bucket_count(g, bk, b);
     const uint32_t nblk = (uint32_t)((bn + PER - 1) / PER);
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
     uint32_t* const mem = w.rmem + (uint64_t)b * kRWords;
     float* const rbase = bucket_residual(g, bk, b);
     const float* const gbase = bucket_grad(g, bk, b);
-    const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const uint32_t k = bucket_k(g, bk, b);
-    if (blockIdx.x == 0) {
+    if (lead) {
         // ---- lead block: clears what the others add into and publishes the first round's key range
         if (nblk == 1) return;
         auto clear = [&](uint32_t from, uint32_t to) {
@@ -169,7 +196,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
             }
         };
         SampleWindow win = {0u, 0x7FFFFFFFu, 0u};
-        if (bn >= kRSampleMin) win = sample_window<kRThreads>(gbase, rbase, bn, k, L.s, clear_first);
+        if (bn >= kSampleMin) win = sample_window<kRThreads>(gbase, rbase, bn, k, L.s, clear_first);
         else clear_first();
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
@@ -178,8 +205,6 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
         resident_arrive(mem, nblk);
         return;
     }
-    const uint32_t x = blockIdx.x - 1;
-    if (x >= nblk) return;
     const uint64_t b0 = (uint64_t)x * PER;                       // the block's first element
     const uint32_t e0 = (uint32_t)wave * (256 * V) + 4 * lane;   // this lane's first element, from b0; vector u is 256 u further
     const bool full = b0 + PER <= bn;
@@ -516,8 +541,35 @@ template <int V>
 void launch(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t epoch, uint32_t published,
             uint64_t limit, hipStream_t st) {
     constexpr uint64_t per = (uint64_t)kRThreads * 4 * V;
-    const uint32_t gx = (uint32_t)((g.bucket_elems + per - 1) / per) + 1;
-    k_topk_resident<V><<<dim3(gx, g.nbuckets), kRThreads, 0, st>>>(bk, g, w, epoch, published, limit);
+    const uint64_t per_bucket = (g.bucket_elems + per - 1) / per;
+    uint32_t nlead = per_bucket > 1 ? g.nbuckets : 0;
+    if (!g.listed) {
+        const uint64_t last = g.n_total - (uint64_t)(g.nbuckets - 1) * g.bucket_elems;
+        const uint32_t blocks = (uint32_t)((g.nbuckets - 1) * per_bucket + (last + per - 1) / per);
+        k_topk_resident<V><<<nlead + blocks, kRThreads, 0, st>>>(bk, g, w, nlead, epoch, published, limit);
+        return;
+    }
+    // A list goes longest bucket first: it takes longest, and its blocks start while the GPU is empty.
+    // Leads before all blocks, no block without a bucket: 24 buckets of 1001 to 1.5 M elements 28.5 us, in
+    // the caller's order with as many blocks for each bucket as for the longest 31.1.
+    uint32_t order[kMaxListed], blocks = 0;
+    for (uint32_t b = 0; b < g.nbuckets; b++) order[b] = b;
+    std::sort(order, order + g.nbuckets, [&](uint32_t p, uint32_t q) { return bk.lcount[p] != bk.lcount[q] ? bk.lcount[p] > bk.lcount[q] : p < q; });
+    Buckets sorted = bk;
+    nlead = 0;
+    for (uint32_t i = g.nbuckets; i < kMaxListed; i++) sorted.lfirst[i] = 0xFFFFFFFFu;
+    for (uint32_t i = 0; i < g.nbuckets; i++) {
+        const uint32_t b = order[i];
+        sorted.lgrad[i] = bk.lgrad[b];
+        sorted.lresidual[i] = bk.lresidual[b];
+        sorted.lwire[i] = bk.lwire[b];
+        sorted.lcount[i] = bk.lcount[b];
+        sorted.lk[i] = bk.lk[b];
+        sorted.lfirst[i] = blocks;
+        blocks += (uint32_t)((bk.lcount[b] + per - 1) / per);
+        if (bk.lcount[b] > per) nlead = i + 1;
+    }
+    k_topk_resident<V><<<nlead + blocks, kRThreads, 0, st>>>(sorted, g, w, nlead, epoch, published, limit);
 }
 
 }  // namespace

@@ -85,3 +85,18 @@ def test_resident_lists_and_uniform_buckets(ops):
         r[s:e] = sub
         assert host[b * stride: b * stride + rc].tobytes() == w.tobytes(), b
     assert np.array_equal(bits(to_np(dr, F32)), bits(r))
+
+
+def test_resident_list_longest_first(ops):
+    """A list of every length class at once - one block, several with and without a sample, 128 -
+    in an order that is not by length, up to the most buckets a call takes."""
+    rng = np.random.default_rng(11)
+    sizes = [5, 32_767, 600_001, 4097, 32_768, 16_385, 16_384, 700_003, 1, 65_537] + [1000 + 37 * i for i in range(54)]
+    grads = [student_t(rng, n) for n in sizes]
+    res = [(rng.standard_normal(n) * 1e-4).astype(np.float32) for n in sizes]
+    dres = [to_dev(r, F32) for r in res]
+    wires = ops.topk_compress_list([to_dev(x, F32) for x in grads], dres, 0.01)
+    for x, r, dr, wv in zip(grads, res, dres, wires):
+        w, rc = oracle.topk_compress(x, r, 0.01)
+        assert wv.cpu().numpy()[:rc].tobytes() == w.tobytes(), x.size
+        assert np.array_equal(bits(to_np(dr, F32)), bits(r)), x.size
