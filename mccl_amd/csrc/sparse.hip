@@ -393,7 +393,7 @@ __global__ __launch_bounds__(kAccThreads) void k_sparse_accumulate_b(float* acc,
 // 16-byte stores.  Everything that decides control flow (tile bounds, window
 // ends, counts) lives in scalar registers.
 //
-// Where a run begins: k_sparse_starts reads every 80th index (one 128-byte line
+// Where a run begins, when a block of a small call does not find it itself (block_starts): k_sparse_starts reads every 80th index (one 128-byte line
 // in five) and writes, for every run w, the window that holds the last sampled
 // index below the run's first element; every pair before that window belongs to
 // an earlier run.
@@ -404,6 +404,10 @@ constexpr int kWin = kWave;    // pairs per window
 constexpr int kStride = 80;    // pairs between two sampled indices of the position table: five 128-byte lines,
                                // so a run begins with at most 79 pairs of an earlier run in its first window
 constexpr int kRunWins = 3;    // windows of a rank a wavefront requests when its run begins
+constexpr int kOwnSamples = 16;  // samples a lane holds where a block finds its runs' starts itself: 1024 a payload
+constexpr uint64_t kOwnTotal = 2048;   // ... and over all ranks
+constexpr uint64_t kOwnBlocks = 512;   // blocks the GPU holds at once: two per CU
+constexpr uint64_t kFillWaves = 2048;  // eight wavefronts per CU
 constexpr int kXcds = 8;       // accelerator dies of an MI355X; block B runs on die B mod 8
 
 constexpr int kStartThreads = 1024;
@@ -501,9 +505,49 @@ __device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) {
 }
 
 
+// Where the block's runs begin in rank `wave`'s payload, found by that wavefront itself: it holds
+// every kStride-th index in registers, and the samples below a run's first element are counted.
+// Returns in lane q the start of run first_run + q (what k_sparse_starts would have written), and
+// whether the samples are out of order.
+__device__ __forceinline__ uint32_t block_starts(const uint8_t* wire, uint32_t kmax, uint64_t first_elem, uint64_t run_elems,
+                                                 int lane, bool* unsorted) {
+    GlobalWords wp = (GlobalWords)wire;
+    const uint32_t cap = (kmax + kStride - 1) / kStride;
+    uint32_t v[kOwnSamples];
+#pragma unroll
+    for (int i = 0; i < kOwnSamples; i++) {
+        const uint32_t j = (uint32_t)(i * kWave + lane);
+        v[i] = j < cap ? wp[1 + 2 * (uint64_t)kStride * j] : 0xFFFFFFFFu;
+    }
+    const uint32_t k = wp[0];
+    const uint32_t nsamp = k > kmax ? 0u : (k + kStride - 1) / kStride;
+    uint32_t prev = 0;
+    uint64_t bad = 0;
+#pragma unroll
+    for (int i = 0; i < kOwnSamples; i++) {
+        const uint32_t j = (uint32_t)(i * kWave + lane);
+        bad |= __ballot(j > 0 && j < nsamp && from_lane_below(v[i], prev) >= v[i]);
+        prev = lane_value(v[i], kWave - 1);
+        if (j >= nsamp) v[i] = 0xFFFFFFFFu;  // below no run's first element
+    }
+    *unsorted = bad != 0;
+    uint32_t mine = 0;
+#pragma unroll
+    for (int q = 0; q < kRunWaves; q++) {
+        const uint64_t f = first_elem + (uint64_t)q * run_elems;
+        const uint32_t first = f < 0xFFFFFFFFull ? (uint32_t)f : 0xFFFFFFFFu;
+        uint32_t n = 0;
+#pragma unroll
+        for (int i = 0; i < kOwnSamples; i++) n += (uint32_t)__popcll(__ballot(v[i] < first));
+        if (lane == q) mine = n ? (n - 1) * kStride : 0u;
+    }
+    return mine;
+}
+
 // NR: ranks the code is unrolled for (ws <= NR; the ranks past ws read rank 0's payload as if
-// its k were 0).  wire_stride holds at least one pair.
-template <int NR>
+// its k were 0).  wire_stride holds at least one pair.  OWN: no position table, the block finds
+// where its runs begin (one bucket, at most kOwnSamples * 64 samples a payload).
+template <int NR, bool OWN>
 __global__ __launch_bounds__(kRunWaves * kWave, 4) void k_sparse_accumulate_runs(
     float* acc, uint64_t n_total, uint64_t bucket_elems, WirePtrs wires, int ws, uint64_t wire_stride,
     uint32_t run_steps, uint32_t runs, uint32_t nbuckets, uint32_t blocks_per_xcd, const uint32_t* start,
@@ -518,7 +562,19 @@ __global__ __launch_bounds__(kRunWaves * kWave, 4) void k_sparse_accumulate_runs
     // that XCD's L2 and its stores move through memory in one direction.
     const uint32_t vblock = (blockIdx.x % kXcds) * blocks_per_xcd + blockIdx.x / kXcds;
     const uint64_t grun = (uint64_t)vblock * kRunWaves + (uint32_t)wave;
-    if (grun >= (uint64_t)runs * nbuckets) return;  // whole wavefront; the kernel has no block barriers
+    __shared__ uint32_t own[kRunWaves][NR];
+    if constexpr (OWN) {
+        if (wave < ws) {
+            const uint64_t run_elems = (uint64_t)run_steps * kRunL;
+            bool unsorted;
+            const uint32_t mine = block_starts(wires.w[wave], (uint32_t)((wire_stride - 4) / 8),
+                                               (uint64_t)vblock * kRunWaves * run_elems, run_elems, lane, &unsorted);
+            if (lane < kRunWaves) own[lane][wave] = mine;
+            if (unsorted && status) *status = MCCL_HIP_ERR_INDEX;
+        }
+        __syncthreads();
+    }
+    if (grun >= (uint64_t)runs * nbuckets) return;  // whole wavefront; no block barrier follows
     const uint32_t b = (uint32_t)(grun / runs), run = (uint32_t)(grun % runs);
     const uint64_t bstart = (uint64_t)b * bucket_elems;
     const uint32_t bn = (uint32_t)((n_total - bstart) < bucket_elems ? (n_total - bstart) : bucket_elems);
@@ -547,7 +603,7 @@ __global__ __launch_bounds__(kRunWaves * kWave, 4) void k_sparse_accumulate_runs
             GlobalWords wp = (GlobalWords)(wires.w[rr] + (uint64_t)b * wire_stride);
             pairs[r] = wp + 1;
             kraw[r] = wp[0];
-            craw[r] = ((GlobalWords)start)[((uint64_t)b * ws + rr) * runs + run];
+            craw[r] = OWN ? own[wave][rr] : ((GlobalWords)start)[((uint64_t)b * ws + rr) * runs + run];
         }
 #pragma unroll
         for (int r = 0; r < NR; r++) {
@@ -710,15 +766,29 @@ int accumulate(float* acc, uint64_t n_total, uint64_t bucket_elems, const void* 
         uint64_t run_steps = (uint64_t)tuning().sparse_run_steps;
         if (run_steps == 0) run_steps = per_tile ? 96 / per_tile : 8;
         if (run_steps > 8 && tuning().sparse_run_steps == 0) run_steps = 8;
+        // ... but no more than leave every CU eight wavefronts: a wavefront's tiles follow one another,
+        // 2-3 us each.  us per call, longer runs against this rule (1 %, position table): 8 ranks of
+        // 1 M elements 18.5 / 12.4 (four tiles against one), of 6.5 M 20.4 / 16.6 (four against two);
+        // one tile there 17.7
+        const uint64_t spread = (steps_bucket * nb + kFillWaves - 1) / kFillWaves;
+        if (run_steps > spread && tuning().sparse_run_steps == 0) run_steps = spread;
         if (run_steps < 1) run_steps = 1;
         if (run_steps > steps_bucket) run_steps = steps_bucket;
         const uint32_t runs = (uint32_t)((steps_bucket + run_steps - 1) / run_steps);
-        k_sparse_starts<<<(uint32_t)(nb * ws), kStartThreads, 0, st>>>(wp, ws, wire_stride,
-                                                                        (uint32_t)(run_steps * kRunL), runs, start, status);
         const uint64_t blocks = ((uint64_t)runs * nb + kRunWaves - 1) / kRunWaves;
+        // One bucket whose blocks all fit the GPU at once: a block finds its runs' starts itself, if
+        // that takes it no more than some 2048 samples over all ranks - each is a memory sector.  us per
+        // call, position table against this: 8 ranks of 1 M elements (1000 samples) 12.4 / 11.1, 4 of 2 M
+        // (1000) 10.0 / 8.2, 2 of 3 M at 2 % (1500) 10.8 / 8.4, but 8 of 6.5 M (6552) 16.6 / 19.6
+        const uint64_t samples = (kmax + kStride - 1) / kStride;
+        const bool own = nb == 1 && blocks <= kOwnBlocks && samples <= (uint64_t)kOwnSamples * kWave &&
+                         samples * (uint64_t)ws <= kOwnTotal && tuning().sparse_path != 2;
+        if (!own)
+            k_sparse_starts<<<(uint32_t)(nb * ws), kStartThreads, 0, st>>>(wp, ws, wire_stride,
+                                                                            (uint32_t)(run_steps * kRunL), runs, start, status);
         const uint32_t per_xcd = (uint32_t)((blocks + kXcds - 1) / kXcds);
 #define MCCLHIP_RUNS(NR)                                                                               \
-    k_sparse_accumulate_runs<NR><<<per_xcd * kXcds, kRunWaves * kWave, 0, st>>>(                        \
+    (own ? k_sparse_accumulate_runs<NR, true> : k_sparse_accumulate_runs<NR, false>)<<<per_xcd * kXcds, kRunWaves * kWave, 0, st>>>(                        \
         acc, n_total, bucket_elems, wp, ws, wire_stride, (uint32_t)run_steps, runs, (uint32_t)nb, per_xcd, \
         start, apply_scale, scale, status)
         if (ws == 1) MCCLHIP_RUNS(1);
