@@ -12,6 +12,7 @@
 // compiled with -ffp-contract=off); fp16/bf16 are widened, operated on in fp32
 // and narrowed once with round-to-nearest-even.
 #include "common.hip.h"
+#include "ring_cut.h"
 #include "runtime.h"
 
 #include <algorithm>
@@ -31,18 +32,7 @@ namespace {
 // moves 3 KiB, so every further instruction shows.  Measured on a bare dst += src over 402 MB
 // arrays: 178 / 181 / 187 / 190 us with 64 / 128 / 256 / 1024 threads, 185 and 193 with two and
 // four vectors per lane.
-constexpr int kFoldBlock = 64;
-// Blocks go to the XCDs in turn, and tiles start where the destination's address is a multiple of
-// 1 KiB and rows of tiles at multiples of 8 KiB (kGroupVecs vectors): an XCD always works on the same
-// eighth of every 8 KiB, and no wavefront ends inside a cache line.  Chunks that start anywhere
-// else: ring fold of 8 ranks, chunks of 819,204 elements 638 us with tiles that start with the chunk,
-// 597 with tiles on 1 KiB, 579 with rows on 8 KiB.
-constexpr int kXcds = 8;
-constexpr int kGroupVecs = kXcds * kFoldBlock;
-// Vectors per lane and rank buffer of the ring fold, in one-wavefront blocks as well: one where the
-// world size is known at compile time (all ranks' loads are in flight together; two cost 2-3 % from
-// two to eight ranks), four where the ranks come one after the other.
-constexpr int ring_unroll(int ws) { return ws == 0 ? 4 : 1; }
+static_assert(kFoldBlock == kWave, "one wavefront per block");
 
 template <bool NT>
 __device__ __forceinline__ u4a load_vec_a(const u4a* p) {
@@ -242,13 +232,6 @@ struct RingPtrs {
     const void* in[2 * MCCL_HIP_MAX_WORLD];
 };
 
-// How a call is cut: computed by the launch, so that a block starts with multiplications only.
-struct RingCut {
-    uint64_t n_total, bucket_elems;
-    uint64_t ce_full, ce_last;  // elements per chunk in a full bucket and in the last one
-    uint32_t nbuckets, chunked;
-};
-
 // blockIdx = (tile, chunk, bucket).  A row of blocks folds one chunk of one bucket, so the first
 // rank of the fold is uniform over the block.
 // Measured over 96.5 M fp32 elements per rank, 25 MiB buckets, buffers that no cache holds (TB/s, against
@@ -275,21 +258,9 @@ __global__ __launch_bounds__(kFoldBlock) void k_ring_fold(void* out, RingPtrs pt
 #pragma unroll
         for (int j = 0; j < WSC; j++) rp[j] = ptrs.in[first + j];
     }
-    const uint64_t bstart = (uint64_t)bucket * cut.bucket_elems;
-    const bool last = bucket + 1 == cut.nbuckets;
-    const uint64_t bn = last ? cut.n_total - bstart : cut.bucket_elems;
-    const uint64_t ce = last ? cut.ce_last : cut.ce_full;
-    const uint64_t cstart = (uint64_t)c * ce;
-    const uint64_t rest = cstart < bn ? bn - cstart : 0;
-    const uint64_t len = rest < ce ? rest : ce;
-    const uint64_t e0 = bstart + cstart;  // first element of the chunk in every buffer
-
-    char* o = (char*)out + e0 * ES;
-    uint64_t head = ((16 - ((uintptr_t)o & 15)) & 15) / ES;
-    if (head > len) head = len;
-    const uint64_t nvec = (len - head) / EPV;
-    // a row's tiles start at a tile group of the output's addresses: `lead` vectors lie in front of the chunk
-    const uint32_t lead = (uint32_t)(((uintptr_t)o + head * ES) >> 4) & (kGroupVecs - 1);
+    const RingRow row = ring_row(cut, (uint64_t)(uintptr_t)out, ES, bucket, c);
+    const uint64_t e0 = row.e0, len = row.len, head = row.head, nvec = row.nvec;
+    const uint32_t lead = row.lead;
     const uint64_t voff = (e0 + head) * ES - lead * 16u;  // byte offset of the first tile
 
     const uint64_t tile = (uint64_t)kFoldBlock * U;
@@ -541,22 +512,14 @@ template <int DT, int OP>
 int launch_ring_t(void* out, const RingPtrs& ptrs, int ws, uint64_t n_total, uint64_t bucket_elems,
                   int schedule, uint32_t nchunks, uint32_t nbuckets, float scale, int apply_scale,
                   int stepwise, hipStream_t st) {
-    constexpr int EPV = ElemInfo<DT>::per_vec;
-    const uint64_t bn = bucket_elems < n_total ? bucket_elems : n_total;
-    const uint64_t ce = (bn + nchunks - 1) / nchunks;
-    const uint64_t tile_vecs = (uint64_t)kFoldBlock * ring_unroll(ws >= 2 && ws <= 8 ? ws : 0);
-    const uint64_t group = 16 * kGroupVecs;
-    const bool on_groups = ((uintptr_t)out | (ce * ElemInfo<DT>::size) | (bucket_elems * ElemInfo<DT>::size)) % group == 0;
-    uint64_t tiles = (ce / EPV + (on_groups ? 0 : kGroupVecs - 1) + tile_vecs - 1) / tile_vecs;
-    if (nchunks * nbuckets > 1) tiles = (tiles + kXcds - 1) / kXcds * kXcds;  // every row starts on the same XCD
+    const RingCut cut = ring_cut(n_total, bucket_elems, nbuckets, nchunks, schedule == MCCL_HIP_RING_CHUNKED);
+    const uint64_t tiles = ring_tiles(cut, (uint64_t)(uintptr_t)out, ElemInfo<DT>::size, nchunks, ring_tile_vecs(ws));
     // One tile per block, x fastest: blocks are dispatched in address order, so
     // the set of tiles in flight is one contiguous front per rank buffer.  A
     // persistent grid looping inside each chunk row scatters the front over all
     // rows and costs about 13 % of the bandwidth on MI355X.
     if (tiles > 0xFFFFFFFFull / kFoldBlock) return MCCL_HIP_ERR_ARG;  // more than 2^32 threads in a row: a chunk of 68 GB
-    const RingCut cut = {n_total, bucket_elems, ce, (n_total - (nbuckets - 1) * bucket_elems + nchunks - 1) / nchunks,
-                         nbuckets, schedule == MCCL_HIP_RING_CHUNKED ? 1u : 0u};
-    dim3 grid((uint32_t)(tiles < 1 ? 1 : tiles), nchunks, nbuckets);
+    dim3 grid((uint32_t)tiles, nchunks, nbuckets);
 #define MCCLHIP_RING_LAUNCH(NT, WSC)                                                                  \
     k_ring_fold<DT, OP, NT, WSC><<<grid, kFoldBlock, 0, st>>>(out, ptrs, cut, ws, scale, apply_scale, stepwise)
     const bool nt = tuning().nontemporal != 0;

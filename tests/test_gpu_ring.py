@@ -146,3 +146,40 @@ def test_ring_fold_rejects_bad_arguments(ops):
         ops.ring_fold(a, [a.clone()] * 2, 5)
     with pytest.raises(MCCLHipError):
         ops.ring_fold(a, [a.clone()] * 65, OP_SUM)
+
+
+def _check_buckets(ops, ins, dt, schedule, be, n):
+    """All of `out` against the oracle, bucket by bucket; out holds a poison beforehand."""
+    ws = len(ins)
+    want = np.empty(n, ins[0].dtype)
+    for s in range(0, n, be):
+        e = min(n, s + be)
+        want[s:e] = oracle.ring_fold([x[s:e].copy() for x in ins], dt, OP_SUM, schedule, scale_by=1.0 / ws, stepwise=dt != F32)
+    out = to_dev(np.full(n, 0x7E7E, np.uint16) if dt != F32 else np.full(n, 1e30, np.float32), dt)
+    ops.ring_fold(out, [to_dev(x, dt) for x in ins], OP_SUM, schedule, bucket_elems=be, scale_by=1.0 / ws, stepwise=dt != F32)
+    got = to_np(out, dt)
+    bad = np.flatnonzero(bits(got) != bits(want))
+    assert bad.size == 0, (be, n, bad.size, bad[:4])
+
+
+# the last bucket's chunks are cut on their own: full - 1 .. full - 1000 elements, and 3/4
+@pytest.mark.parametrize("schedule", [RING_BASIC, RING_CHUNKED])
+@pytest.mark.parametrize("ws", [2, 4, 8, 12])
+@pytest.mark.parametrize("dt", [F32, F16, BF16])
+def test_last_bucket_nearly_full(ops, dt, ws, schedule):
+    rng = np.random.default_rng(ws)
+    for be in (16_384, 65_536, 262_144):
+        whole = [rand_vals(rng, 2 * be, dt, sigma=1e-3, specials=False) for _ in range(ws)]
+        for short in (1, 12, 100, 1000, be // 4):
+            n = 2 * be - short
+            _check_buckets(ops, [x[:n] for x in whole], dt, schedule, be, n)
+
+
+@pytest.mark.parametrize("dt,ws,schedule", [(F32, 8, RING_BASIC), (BF16, 8, RING_CHUNKED), (F16, 12, RING_BASIC)])
+def test_last_default_bucket_nearly_full(ops, dt, ws, schedule):
+    be = 6_553_600
+    rng = np.random.default_rng(2)
+    whole = [rand_vals(rng, 2 * be, dt, sigma=1e-3, specials=False) for _ in range(ws)]
+    for short in (1, 100, 1000, be // 4):
+        n = 2 * be - short
+        _check_buckets(ops, [x[:n] for x in whole], dt, schedule, be, n)
