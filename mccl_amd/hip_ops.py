@@ -37,7 +37,7 @@ class _Checked:
     """No extension: every call goes through the checks below."""
 
     def __getattr__(self, name):
-        return lambda *args: False
+        return lambda *args: None
 
 
 def _bind_native():
@@ -53,8 +53,8 @@ def _bind_native():
 
 
 # Well-formed calls are checked and launched in one C call (mccl_amd/csrc/ext/FastCalls.cpp), which
-# returns False, with nothing done, for everything else; that goes through the checks below and
-# through ctypes, and raises what is wrong with it.
+# returns the library's status, or None, with nothing done, for everything else; that goes through the
+# checks below and through ctypes, and raises what is wrong with it.
 _native = _Unbound()
 
 
@@ -86,8 +86,11 @@ def _dev(t: torch.Tensor, what: str, dtype: Optional[torch.dtype] = None, min_nu
 
 
 def fold2(dst: torch.Tensor, src: torch.Tensor, op: int = SUM) -> torch.Tensor:
-    if _native._fast_fold2(dst, src, op):
+    rc = _native._fast_fold2(dst, src, op)
+    if rc == 0:
         return dst
+    if rc is not None:
+        raise _lib.MCCLHipError(rc, "fold2")
     _dev(dst, "dst"); _dev(src, "src")
     if dst.shape != src.shape or dst.dtype != src.dtype:
         raise ValueError("shape / dtype mismatch")
@@ -100,8 +103,11 @@ def fold2_batch(dsts: Sequence[torch.Tensor], srcs: Sequence[torch.Tensor], op: 
     """dsts[i] (op)= srcs[i] for every i, in one launch per 128 folds.  The folds run in no
     particular order: a destination may not overlap any other fold's destination or source
     (the library refuses such a list)."""
-    if _native._fast_fold2_batch(dsts, srcs, op):
+    rc = _native._fast_fold2_batch(dsts, srcs, op)
+    if rc == 0:
         return
+    if rc is not None:
+        raise _lib.MCCLHipError(rc, "fold2_batch")
     if len(dsts) != len(srcs):
         raise ValueError("as many sources as destinations")
     if not dsts:
@@ -123,8 +129,11 @@ def scale(buf: torch.Tensor, s: float) -> torch.Tensor:
 
 
 def fold2_scale(dst: torch.Tensor, src: torch.Tensor, s: float) -> torch.Tensor:
-    if _native._fast_fold2_scale(dst, src, s):
+    rc = _native._fast_fold2_scale(dst, src, s)
+    if rc == 0:
         return dst
+    if rc is not None:
+        raise _lib.MCCLHipError(rc, "fold2_scale")
     _dev(dst, "dst"); _dev(src, "src")
     if dst.shape != src.shape or dst.dtype != src.dtype:
         raise ValueError("shape / dtype mismatch")
@@ -140,9 +149,12 @@ def _ptrs(tensors: Sequence[torch.Tensor]):
 def ring_fold(out: torch.Tensor, ins: Sequence[torch.Tensor], op: int = SUM,
               schedule: int = RING_BASIC, bucket_elems: Optional[int] = None,
               scale_by: Optional[float] = None, stepwise: bool = False) -> torch.Tensor:
-    if isinstance(out, torch.Tensor) and _native._fast_ring_fold(out, ins, op, schedule, bucket_elems or max(out.numel(), 1),
-                                                                 scale_by, int(stepwise)):
-        return out
+    if isinstance(out, torch.Tensor):
+        rc = _native._fast_ring_fold(out, ins, op, schedule, bucket_elems or max(out.numel(), 1), scale_by, int(stepwise))
+        if rc == 0:
+            return out
+        if rc is not None:
+            raise _lib.MCCLHipError(rc, "ring_fold")
     _dev(out, "out")
     for t in ins:
         _dev(t, "in")
@@ -184,9 +196,12 @@ def topk_compress(grad: torch.Tensor, residual: torch.Tensor, ratio: float,
                   status: Optional[torch.Tensor] = None):
     """Returns (wire uint8 tensor [nbuckets * stride], stride). residual is updated.
     status: int32 device tensor of one element that receives ERR_TIMEOUT (caller zeroes it)."""
-    if wire is not None and bucket_elems and _native._fast_topk_compress(grad, residual, ratio, bucket_elems, wire, workspace,
-                                                                         wire_stride, status):
-        return wire, wire_stride
+    if wire is not None and bucket_elems:
+        rc = _native._fast_topk_compress(grad, residual, ratio, bucket_elems, wire, workspace, wire_stride, status)
+        if rc == 0:
+            return wire, wire_stride
+        if rc is not None:
+            raise _lib.MCCLHipError(rc, "topk_compress")
     _dev(grad, "grad"); _dev(residual, "residual")
     if grad.dtype != torch.float32 or residual.dtype != torch.float32:
         raise _lib.MCCLHipError(-2, "TopK compression currently supports float32 only")
@@ -289,8 +304,12 @@ def sparse_accumulate(acc: torch.Tensor, wires: Sequence[torch.Tensor], wire_str
                       bucket_elems: Optional[int] = None, scale_by: Optional[float] = None,
                       status: Optional[torch.Tensor] = None, workspace="auto") -> torch.Tensor:
     """workspace: "auto" allocates the scratch, None selects the scratch-free kernel."""
-    if bucket_elems and _native._fast_sparse_accumulate(acc, wires, wire_stride, bucket_elems, scale_by, status, workspace):
-        return acc
+    if bucket_elems:
+        rc = _native._fast_sparse_accumulate(acc, wires, wire_stride, bucket_elems, scale_by, status, workspace)
+        if rc == 0:
+            return acc
+        if rc is not None:
+            raise _lib.MCCLHipError(rc, "sparse_accumulate")
     _dev(acc, "acc", torch.float32)
     n = acc.numel()
     be = bucket_elems or max(n, 1)
