@@ -1135,8 +1135,9 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
     const u2a tot = *(const u2a*)(w.bin_fill + (uint64_t)b * kCoarse + kCoarse - 2 - 2 * (threadIdx.x & (kWave - 1)));
     GroupTiles<false> G;
     G.load(g, w, b, grp, fg);
+    // a replay of a captured launch carries the same epoch: also behind a run that was given up
+    if (grp == 0 && threadIdx.x == 0) st[S_READY] = 0u;
     if (gave_up) return;  // the streaming launch gave the bucket up: its payload header says so
-    if (grp == 0 && threadIdx.x == 0) st[S_READY] = 0u;  // a replay of a captured launch carries the same epoch
     const uint32_t lo = win[0], that_key = win[2], wmul = window_mul(win[0], win[1]);
     const uint32_t k = fg.k;
     const uint64_t bn = fg.bn;

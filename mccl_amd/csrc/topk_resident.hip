@@ -537,12 +537,32 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
     }
 }
 
+// A replay of a captured launch carries the same epoch.  A run that ends well leaves S_READY zero, one
+// that a block gave up may leave it published: the blocks of the next replay would take the old window
+// and the old counters for theirs, so a capture records this kernel in front of the launch.  (One
+// bucket of 65,537 elements, replayed: 15.9 us, without it 14.3; buckets of one block wait for nobody.)
+__global__ __launch_bounds__(kBlock) void k_resident_unpublish(uint32_t* state, uint32_t nbuckets) {
+    const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
+    if (b < nbuckets) st_agent(state + (uint64_t)b * kStateWords + S_READY, 0u);
+}
+
+bool is_capturing(hipStream_t st) {
+    if (!st) return false;  // the null stream cannot be captured, and asking about it can fail while another one is
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &s) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return s != hipStreamCaptureStatusNone;
+}
+
 template <int V>
 void launch(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t epoch, uint32_t published,
             uint64_t limit, hipStream_t st) {
     constexpr uint64_t per = (uint64_t)kRThreads * 4 * V;
     const uint64_t per_bucket = (g.bucket_elems + per - 1) / per;
     uint32_t nlead = per_bucket > 1 ? g.nbuckets : 0;
+    if (nlead && is_capturing(st)) k_resident_unpublish<<<(nlead + kBlock - 1) / kBlock, kBlock, 0, st>>>(w.state, nlead);
     if (!g.listed) {
         const uint64_t last = g.n_total - (uint64_t)(g.nbuckets - 1) * g.bucket_elems;
         const uint32_t blocks = (uint32_t)((g.nbuckets - 1) * per_bucket + (last + per - 1) / per);
