@@ -308,7 +308,7 @@ int mccl_hip_fence_block_stream(uint64_t ticket, void* stream);
 int mccl_hip_sync(void* stream);
 
 /* ---- tuning knobs (benchmarks and tests; defaults need no call) ---------- */
-/* keys: "fold_blocks_per_cu", "nontemporal", "topk_path" (0 auto, 1 exact, 2 single-pass, 3 resident where it fits), "topk_barrier_ms", "topk_stall_test" (tests: 1 makes every wait
+/* keys: "fold_blocks_per_cu", "nontemporal", "topk_path" (0 auto, 1 exact, 2 single-pass, 3 resident where one launch may take the call), "topk_barrier_ms", "topk_stall_test" (tests: 1 makes every wait
  * of the single-pass top-k path run into its limit, so that the give-up path can be exercised
  * without a stuck kernel),
  * "sparse_path" (0 auto, 1 tile kernels only, 2 position table always), "sparse_run_steps" (0 auto),

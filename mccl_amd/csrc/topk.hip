@@ -10,11 +10,11 @@
 // (NaN patterns sort above infinity), so selection is an exact radix select on
 // that key.  All buckets of a gradient run in the same launches.
 //
-// RESIDENT PATH (topk_resident.hip; one launch): buckets of up to 2 M elements.
+// RESIDENT PATH (topk_resident.hip; one launch): buckets of up to 2 M elements, 2 M a call.
 // SINGLE-PASS PATH (one pass over the gradient, 12 B/element of HBM traffic, two launches):
 // larger buckets and many buckets at a time; see the section "single-pass path" below.
 // EXACT PATH (any input; six launches): large buckets with large ratios, many small buckets,
-// and topk_path = 1 (choose_path has the rule and its measurements).
+// and topk_path = 1 (topk_route.h has the rule and its measurements).
 //   [pass A]   residual <- grad + residual, histogram of key[30:20]
 //   refine x2  histograms of key[19:10], key[9:0] among prefix matches
 //   count      per 4096-element tile: #(key > T), #(key == T)
@@ -26,7 +26,6 @@
 #include "topk_common.hip.h"
 
 #include <atomic>
-#include <cmath>
 #include <vector>
 
 namespace mcclhip {
@@ -453,12 +452,10 @@ __global__ __launch_bounds__(kBlock) void k_topk_emit(float* residual, Geometry 
 
 constexpr int kFRegion = 1024;                // elements one wavefront streams
 constexpr int kFWaves = kBlock / kWave;       // 4
-constexpr int kFTile = kFRegion * kFWaves;    // elements per streaming block
+static_assert(kFTile == kFRegion * kFWaves, "elements per streaming block");
 constexpr int kFVecs = kFRegion / (kWave * 4);  // 16-byte vectors per lane and array: all issued at once
-constexpr int kTileSlots = 128;               // candidate slots per tile
 constexpr int kCoarse = 128;                  // coarse window bins; the last one holds keys >= hi
 constexpr int kBinsPerLane = kCoarse / kWave; // 2
-constexpr int kGroups = 64;                   // at most this many groups of tiles per bucket
 constexpr int kCntStride = 64;                // words between two groups' arrival counters: 256 bytes, so that the
                                               // arrivals of a bucket's tiles spread over memory channels
 constexpr int kHeld = 7;                      // tiles per wavefront whose slots a bin / select block keeps in registers
@@ -1420,40 +1417,6 @@ uint32_t next_epoch() {
     return e;
 }
 
-enum Path { kPathExact, kPathStream, kPathResident };
-
-// Which kernels a call takes (tuning key "topk_path": 1, 2, 3 fix it).  `counts`: the buckets'
-// lengths when they are listed, else null.  Measured per call, us:
-//   resident up to 512 blocks, as many as the GPU holds at once: one launch against two or six
-//     (65,536 elements: 15 against 28 exact; 1 M: 22 against 26 streaming; 8 x 262,144: 26 against
-//     29 streaming).  Beyond, its blocks wait their turn and its barriers lie open (16 x 262,144: 54
-//     against 37 streaming; 64 x 131,072: 99 against 84 exact) - except for buckets of a few blocks
-//     (1500 x 16,384: 166 against 187 exact) ...
-//   ... and where the streaming path's tiles run out of candidate slots (128 per 4096 elements, more
-//     than 3 % inside the sampled window: ratios above about 0.015).  Its tiles are then read again
-//     as a whole (5 %, 2 M elements: 145 us against 30 resident; 6.5 M: 448 against 144 exact; from
-//     eight buckets on that latency is shared: 14 x 6.5 M 826 against 905 exact).
-Path choose_path(const Geometry& g, const uint64_t* counts) {
-    const bool fits = g.bucket_elems <= kRMaxBucket;
-    const uint64_t stream_blocks = (uint64_t)g.nbuckets * ((uint64_t)g.ftiles + kGroups + 1) + kGroups;
-    const bool streams = stream_blocks < 0x7FFFFFFFull;
-    const int path = tuning().topk_path;
-    if (path == 1 && !counts) return kPathExact;
-    if (path == 2 && streams) return kPathStream;
-    if (path == 3 && fits) return kPathResident;
-    const int vecs = resident_vecs(g.bucket_elems, g.nbuckets);
-    const uint64_t per = (uint64_t)vecs * kFTile;
-    uint64_t blocks = 0;
-    if (counts) for (uint32_t b = 0; b < g.nbuckets; b++) blocks += (counts[b] + per - 1) / per;
-    else blocks = (g.n_total + per - 1) / per;
-    // expected share of a bucket inside the sampled window (see sample_window)
-    const double ks = (double)g.k_full / (double)g.bucket_elems * kFSample;
-    const bool dense = (ks + 6.0 * std::sqrt(ks) + 16.0) / kFSample > (double)kTileSlots / kFTile;
-    if (fits && (blocks <= 512 || g.bucket_elems <= 4 * per || (dense && (vecs == 4 || counts)))) return kPathResident;
-    if (counts) return streams ? kPathStream : (fits ? kPathResident : kPathExact);
-    return streams && g.bucket_elems >= kFastMinBucket && (!dense || (!fits && g.nbuckets >= 8)) ? kPathStream : kPathExact;
-}
-
 // The two launches of the single-pass path.
 void launch_single_pass(const Buckets& bk, const Geometry& g, const Workspace& w, hipStream_t st) {
     // the streaming launch: a sample block per bucket, then per bucket its tiles and 64 bin blocks
@@ -1480,13 +1443,15 @@ void launch_single_pass(const Buckets& bk, const Geometry& g, const Workspace& w
 }
 
 // False when the call has to take the exact path.
-bool launch_by_path(Path path, const Buckets& bk, const Geometry& g, const Workspace& w, hipStream_t st) {
-    if (path == kPathExact) return false;
-    if (path == kPathStream) {
+bool launch_by_path(const Buckets& bk, const Geometry& g, const Workspace& w, const uint64_t* counts, hipStream_t st) {
+    const uint64_t limit = g.bucket_elems <= kRMaxBucket ? resident_limit_on(st) : 0;
+    const Route route = choose_path({g.n_total, g.bucket_elems, g.nbuckets, counts, g.k_full}, tuning().topk_path, limit);
+    if (route.path == kPathExact) return false;
+    if (route.path == kPathStream) {
         launch_single_pass(bk, g, w, st);
     } else {
         const uint32_t epoch = next_epoch();
-        launch_resident(bk, g, w, epoch, tuning().topk_stall_test ? ~epoch : epoch,
+        launch_resident(bk, g, w, route.vecs, limit, epoch, tuning().topk_stall_test ? ~epoch : epoch,
                         (uint64_t)tuning().topk_barrier_ms * 100000ull, st);
     }
     return true;
@@ -1536,7 +1501,6 @@ int mccl_hip_topk_compress(const float* grad, float* residual, uint64_t n_total,
     void* aligned = (void*)(((uintptr_t)workspace + 15) & ~(uintptr_t)15);
     Workspace w = carve(aligned, g);
     w.status = status;
-    const Path path = choose_path(g, nullptr);
     const uint64_t cap = (uint64_t)device_info().num_cus * (uint64_t)(tuning().fold_blocks_per_cu < 256 ? tuning().fold_blocks_per_cu : 256);
     const uint64_t nvec = g.bucket_elems / 4;
     const uint64_t bx = (cap + g.nbuckets - 1) / g.nbuckets;
@@ -1548,7 +1512,7 @@ int mccl_hip_topk_compress(const float* grad, float* residual, uint64_t n_total,
     bk.residual = residual;
     bk.wire = (uint8_t*)wire;
     bk.wire_stride = wire_stride;
-    if (!launch_by_path(path, bk, g, w, st)) {
+    if (!launch_by_path(bk, g, w, nullptr, st)) {
         const uint64_t zw = zeroed_words(g);
         k_zero_words<<<clamp_u32((zw / 4 + kBlock - 1) / kBlock, 1, cap), kBlock, 0, st>>>(w.hist, zw);
         const uint64_t need_a = (nvec + kBlock * 2 - 1) / (kBlock * 2);
@@ -1603,7 +1567,7 @@ int mccl_hip_topk_compress_list(const float* const* host_grads, float* const* ho
     void* aligned = (void*)(((uintptr_t)workspace + 15) & ~(uintptr_t)15);
     Workspace w = carve(aligned, g);
     w.status = status;
-    if (!launch_by_path(choose_path(g, host_counts), bk, g, w, (hipStream_t)stream)) return MCCL_HIP_ERR_ARG;
+    if (!launch_by_path(bk, g, w, host_counts, (hipStream_t)stream)) return MCCL_HIP_ERR_ARG;
     return launch_status();
 }
 

@@ -4,6 +4,7 @@
 
 #include "common.hip.h"
 #include "runtime.h"
+#include "topk_route.h"
 
 namespace mcclhip {
 
@@ -13,12 +14,9 @@ constexpr int kBinsR = 1024;   // key[19:10], key[9:0]
 constexpr int kHistWords = kBins0 + 2 * kBinsR;
 constexpr int kStateWords = 32;
 constexpr uint32_t kDense = 0xFFFFFFFFu;  // tile count: more candidates than slots, read the residual range itself
-constexpr uint64_t kFastMinBucket = 1u << 18;
 constexpr uint32_t kPoisonK = 0xFFFFFFFFu;    // payload header of a bucket whose selection was abandoned
 // resident path (topk_resident.hip): per-bucket scratch, in words
 constexpr int kRList = 1024;                  // elements of the picked bin that are ranked as a list
-constexpr uint64_t kRMaxBlocks = 128;         // blocks of one bucket
-constexpr uint64_t kRMaxBucket = kRMaxBlocks * 1024 * 4 * 4;  // 2,097,152 elements
 constexpr uint32_t kRRow = 2048 + 64;         // one round's histogram: its bins, the count above them, padding
 constexpr uint32_t kRRows = 4;                // a windowed round, three on the full key range (11 + 11 + 9 bits)
 constexpr uint32_t kRBars = 6;                // barriers: at most four rounds and the list / ties
@@ -29,7 +27,6 @@ constexpr uint32_t kRRow0 = kRFill + 64;
 constexpr uint32_t kRCnt = kRRow0 + kRRows * kRRow;           // per block: elements above the bin, inside the bin
 constexpr uint32_t kRListAt = kRCnt + 2 * (uint32_t)kRMaxBlocks;
 constexpr uint32_t kRWords = kRListAt + 2 * kRList;
-constexpr int kFSample = 8192;                // sampled elements per bucket
 
 // per-bucket state words
 enum {
@@ -131,9 +128,12 @@ __device__ __forceinline__ uint32_t* bucket_wire(const Geometry& g, BucketsArg b
 }
 
 
-int resident_vecs(uint64_t n, uint32_t nbuckets);
-void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t epoch, uint32_t published,
-                     uint64_t limit_ticks, hipStream_t st);
+// Blocks that may wait in one resident launch on the stream (resident_limit), 0 on a stream that is
+// confined to some of the GPU's CUs.
+uint64_t resident_limit_on(hipStream_t st);
+// A list of buckets goes in as many launches as keep each under `limit`.
+void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, int vecs, uint64_t limit, uint32_t epoch,
+                     uint32_t published, uint64_t limit_ticks, hipStream_t st);
 
 // ---- what blocks of one launch use to talk to each other ----------------------------------
 __device__ __forceinline__ uint32_t ld_agent(const uint32_t* p) {

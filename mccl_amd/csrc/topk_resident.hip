@@ -21,14 +21,22 @@
 // (27.7), 262,144 17.9 (25.4 on the two-launch path), 1 M 21.7 (26.7), 2 M 26.0; at a ratio of 5 % 1 M
 // elements 22.9 us (84.9) and 2 M 27.8 (144).
 //
-// The blocks of a bucket wait for one another, so they have to be resident together.  At 64
-// registers, 54 KiB of LDS and 1024 threads two blocks fit a CU, 64 an XCD; a bucket has at most 128 blocks,
-// 16 per XCD.  Every XCD dispatches its share of a grid in grid order, so only the newest bucket
-// of a launch can be incompletely dispatched on it, with at most 15 blocks that wait: the four
-// hardware queues of a process can have four such launches under way and still leave a slot.
+// The blocks of a bucket wait for one another, so they have to be resident together, whatever else the
+// GPU runs.  At 64 registers, 54 KiB of LDS and 1024 threads two blocks fit a CU: 512 the GPU, 64 an XCD.  A
+// launch has at most resident_limit of them that wait (topk_route.h): a quarter of those slots, as
+// many launches as a process's four hardware queues can have under way.  They are consecutive in the
+// grid and dealt to the XCDs in turn, at most 16 to each.  So on every XCD, for any launches under way
+// and in any order of dispatch, the blocks that wait are at most as many as its slots, and everything
+// else that holds a slot - lead blocks, buckets of one block, other kernels - ends without waiting
+// for these.  A block that is not yet dispatched therefore finds a slot, all blocks of every bucket
+// come to be resident, and their barriers fill.  (The order of buckets within a launch does not give that: of two
+// launches of several hundred blocks one can fill XCD 0 and the other XCD 1, each with buckets that miss
+// blocks on the other.)  On a stream that is confined to some of the CUs no bucket of several blocks
+// takes this path.
 #include "topk_common.hip.h"
 
 #include <algorithm>
+#include <cstdlib>
 #include <type_traits>
 
 namespace mcclhip {
@@ -556,59 +564,99 @@ bool is_capturing(hipStream_t st) {
     return s != hipStreamCaptureStatusNone;
 }
 
+// `nlead`: buckets of more than one block, which come first.
 template <int V>
-void launch(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t epoch, uint32_t published,
-            uint64_t limit, hipStream_t st) {
-    constexpr uint64_t per = (uint64_t)kRThreads * 4 * V;
-    const uint64_t per_bucket = (g.bucket_elems + per - 1) / per;
-    uint32_t nlead = per_bucket > 1 ? g.nbuckets : 0;
+void launch_blocks(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t nlead, uint32_t blocks, uint32_t epoch,
+                   uint32_t published, uint64_t limit_ticks, hipStream_t st) {
     if (nlead && is_capturing(st)) k_resident_unpublish<<<(nlead + kBlock - 1) / kBlock, kBlock, 0, st>>>(w.state, nlead);
+    k_topk_resident<V><<<nlead + blocks, kRThreads, 0, st>>>(bk, g, w, nlead, epoch, published, limit_ticks);
+}
+
+template <int V>
+void launch(const Buckets& bk, const Geometry& g, const Workspace& w, uint64_t limit, uint32_t epoch, uint32_t published,
+            uint64_t limit_ticks, hipStream_t st) {
+    constexpr uint64_t per = kRVecElems * V;
+    static_assert(kRVecElems == kRThreads * 4, "one vector per thread");
     if (!g.listed) {
+        const uint64_t per_bucket = (g.bucket_elems + per - 1) / per;
         const uint64_t last = g.n_total - (uint64_t)(g.nbuckets - 1) * g.bucket_elems;
         const uint32_t blocks = (uint32_t)((g.nbuckets - 1) * per_bucket + (last + per - 1) / per);
-        k_topk_resident<V><<<nlead + blocks, kRThreads, 0, st>>>(bk, g, w, nlead, epoch, published, limit);
+        launch_blocks<V>(bk, g, w, per_bucket > 1 ? g.nbuckets : 0, blocks, epoch, published, limit_ticks, st);
         return;
     }
     // A list goes longest bucket first: it takes longest, and its blocks start while the GPU is empty.
     // Leads before all blocks, no block without a bucket: 24 buckets of 1001 to 1.5 M elements 28.5 us, in
-    // the caller's order with as many blocks for each bucket as for the longest 31.1.
-    uint32_t order[kMaxListed], blocks = 0;
+    // the caller's order with as many blocks for each bucket as for the longest 31.1 (both as one launch).
+    uint32_t order[kMaxListed];
     for (uint32_t b = 0; b < g.nbuckets; b++) order[b] = b;
     std::sort(order, order + g.nbuckets, [&](uint32_t p, uint32_t q) { return bk.lcount[p] != bk.lcount[q] ? bk.lcount[p] > bk.lcount[q] : p < q; });
-    Buckets sorted = bk;
-    nlead = 0;
-    for (uint32_t i = g.nbuckets; i < kMaxListed; i++) sorted.lfirst[i] = 0xFFFFFFFFu;
-    for (uint32_t i = 0; i < g.nbuckets; i++) {
-        const uint32_t b = order[i];
-        sorted.lgrad[i] = bk.lgrad[b];
-        sorted.lresidual[i] = bk.lresidual[b];
-        sorted.lwire[i] = bk.lwire[b];
-        sorted.lcount[i] = bk.lcount[b];
-        sorted.lk[i] = bk.lk[b];
-        sorted.lfirst[i] = blocks;
-        blocks += (uint32_t)((bk.lcount[b] + per - 1) / per);
-        if (bk.lcount[b] > per) nlead = i + 1;
+    for (uint32_t done = 0; done < g.nbuckets;) {
+        const uint32_t taken = next_launch(bk.lcount, order + done, g.nbuckets - done, per, limit);
+        Buckets part = bk;
+        uint32_t nlead = 0, blocks = 0;
+        for (uint32_t i = 0; i < taken; i++) {
+            const uint32_t b = order[done + i];
+            part.lgrad[i] = bk.lgrad[b];
+            part.lresidual[i] = bk.lresidual[b];
+            part.lwire[i] = bk.lwire[b];
+            part.lcount[i] = bk.lcount[b];
+            part.lk[i] = bk.lk[b];
+            part.lfirst[i] = blocks;
+            blocks += (uint32_t)((bk.lcount[b] + per - 1) / per);
+            if (bk.lcount[b] > per) nlead = i + 1;
+        }
+        for (uint32_t i = taken; i < kMaxListed; i++) part.lfirst[i] = 0xFFFFFFFFu;
+        Workspace pw = w;
+        pw.state += (uint64_t)done * kStateWords;
+        pw.rmem += (uint64_t)done * kRWords;
+        launch_blocks<V>(part, g, pw, nlead, blocks, epoch, published, limit_ticks, st);
+        done += taken;
     }
-    k_topk_resident<V><<<nlead + blocks, kRThreads, 0, st>>>(sorted, g, w, nlead, epoch, published, limit);
+}
+
+// CUs of the stream's mask; all of the device's where there is no mask to be had.
+int stream_cus(hipStream_t st) {
+    uint32_t mask[32] = {};
+    if (hipExtStreamGetCUMask(st, 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return device_info().num_cus;
+    }
+    int n = 0;
+    for (const uint32_t m : mask) n += __builtin_popcount(m);
+    return n;
 }
 
 }  // namespace
 
-// Vectors per thread for buckets of up to n elements.  The barriers cost more with more blocks, the
-// passes over a block's elements with more vectors; measured (one bucket, 1 %): 262,144 elements
-// 17.8 / 18.0 us with 1 / 2 vectors, 400,000 19.8 / 19.5, 524,288 20.0 / 19.3 / 20.7 with 1 / 2 / 4,
-// 700,000 21.1 / 22.2 with 2 / 4, 1 M 21.7 / 22.0.  Several buckets in a launch keep to 64 blocks
-// each, so that more of them are resident at once.
-int resident_vecs(uint64_t n, uint32_t nbuckets) {
-    return n <= 64 * 4096 ? 1 : n <= (nbuckets == 1 ? 128 : 64) * 8192 ? 2 : 4;
+uint64_t resident_limit_on(hipStream_t st) {
+    static const uint64_t per_cu = [] {
+        int least = 1 << 20;
+        for (const void* k : {(const void*)k_topk_resident<1>, (const void*)k_topk_resident<2>, (const void*)k_topk_resident<4>}) {
+            int n = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, kRThreads, 0) != hipSuccess) n = 0;
+            least = n < least ? n : least;
+        }
+        return (uint64_t)least;
+    }();
+    // hardware queues that the process's streams share; HIP's own default is four
+    static const uint32_t queues = [] {
+        const char* s = std::getenv("GPU_MAX_HW_QUEUES");
+        const long q = s ? std::strtol(s, nullptr, 10) : 0;
+        return (uint32_t)(q > 0 && q < 1024 ? q : 4);
+    }();
+    // (asking takes 0.2 us; the null stream's mask is the process's)
+    static const bool whole = stream_cus(nullptr) >= device_info().num_cus;
+    const int cus = device_info().num_cus;
+    if (!whole || (st && stream_cus(st) < cus)) return 0;
+    return resident_limit((uint64_t)cus * per_cu, queues);
 }
 
-void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t epoch, uint32_t published,
-                     uint64_t limit_ticks, hipStream_t st) {
-    switch (resident_vecs(g.bucket_elems, g.nbuckets)) {
-        case 1: launch<1>(bk, g, w, epoch, published, limit_ticks, st); break;
-        case 2: launch<2>(bk, g, w, epoch, published, limit_ticks, st); break;
-        default: launch<4>(bk, g, w, epoch, published, limit_ticks, st); break;
+void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, int vecs, uint64_t limit, uint32_t epoch,
+                     uint32_t published, uint64_t limit_ticks, hipStream_t st) {
+    switch (vecs) {
+        case 1: launch<1>(bk, g, w, limit, epoch, published, limit_ticks, st); break;
+        case 2: launch<2>(bk, g, w, limit, epoch, published, limit_ticks, st); break;
+        default: launch<4>(bk, g, w, limit, epoch, published, limit_ticks, st); break;
     }
 }
 

@@ -1,0 +1,110 @@
+// Which kernels a top-k compress call takes: plain arithmetic on the call's sizes and the device,
+// the same for the library and for the test that checks it on the CPU.
+#pragma once
+
+#include <cmath>
+#include <stdint.h>
+
+namespace mcclhip {
+
+enum Path { kPathExact, kPathStream, kPathResident };
+
+constexpr int kFSample = 8192;              // sampled elements per bucket
+constexpr uint64_t kFTile = 4096;           // single-pass path: elements per streaming block
+constexpr int kTileSlots = 128;             // ... candidate slots per tile
+constexpr int kGroups = 64;                 // ... at most this many groups of tiles per bucket
+constexpr uint64_t kFastMinBucket = 1u << 18;
+constexpr uint64_t kRMaxBlocks = 128;       // resident path: blocks of one bucket
+constexpr uint64_t kRVecElems = 4096;       // ... elements per block and vector of a thread
+constexpr uint64_t kRMaxBucket = kRMaxBlocks * kRVecElems * 4;  // 2,097,152 elements
+
+// The buckets of a call: consecutive ranges of bucket_elems elements, the last one shorter, or, with
+// counts, nbuckets buffers of those lengths, bucket_elems the longest.
+struct TopkCall {
+    uint64_t n_total, bucket_elems;
+    uint32_t nbuckets;
+    const uint64_t* counts;
+    uint32_t k_full;  // picks of a bucket of bucket_elems
+};
+
+// The most blocks of one resident launch that may wait for others.  Blocks of a bucket wait for each
+// other, so every launch that can be under way has to fit the GPU whole, whatever the others are: a
+// process's streams share `queues` hardware queues, each with one launch under way.  `slots` blocks
+// fit the GPU at once.  Blocks are dealt to the accelerator dies in turn, hence the multiple of eight.
+constexpr uint64_t resident_limit(uint64_t slots, uint32_t queues) { return slots / (queues ? queues : 1) / 8 * 8; }
+
+// Blocks that wait for others with `vecs` vectors per thread: those of every bucket of more than one block.
+inline uint64_t resident_waiting(const TopkCall& c, int vecs) {
+    const uint64_t per = kRVecElems * (uint64_t)vecs;
+    const auto blocks = [&](uint64_t n) { return n > per ? (n + per - 1) / per : 0; };
+    if (!c.counts) return (c.nbuckets - 1) * blocks(c.bucket_elems) + blocks(c.n_total - (c.nbuckets - 1) * c.bucket_elems);
+    uint64_t sum = 0;
+    for (uint32_t b = 0; b < c.nbuckets; b++) sum += blocks(c.counts[b]);
+    return sum;
+}
+
+// Vectors per thread of a resident launch, 0 when more than `limit` of its blocks would wait.  The barriers
+// cost more with more blocks, the passes over a block's elements with more vectors; measured (one bucket,
+// 1 %): 262,144 elements 17.8 / 18.0 us with 1 / 2 vectors, 400,000 19.8 / 19.5, 524,288 20.0 / 19.3 / 20.7
+// with 1 / 2 / 4, 700,000 21.1 / 22.2 with 2 / 4, 1 M 21.7 / 22.0.  Several buckets take as many as
+// bring the launch under the limit.
+inline int resident_vecs(const TopkCall& c, uint64_t limit) {
+    if (c.bucket_elems > kRMaxBucket) return 0;
+    int v = c.bucket_elems <= 64 * kRVecElems ? 1 : c.bucket_elems <= (c.nbuckets == 1 ? 128 : 64) * 2 * kRVecElems ? 2 : 4;
+    for (; v <= 4; v *= 2)
+        if (resident_waiting(c, v) <= limit) return v;
+    return 0;
+}
+
+// A list goes in as many launches as it takes to keep each under `limit`.  order[0 .. left): its remaining
+// buckets, longest first; brings those of the next launch to the front, in order, and returns their number.
+inline uint32_t next_launch(const uint32_t* counts, uint32_t* order, uint32_t left, uint64_t per, uint64_t limit) {
+    uint32_t taken = 0;
+    uint64_t waiting = 0;
+    for (uint32_t i = 0; i < left; i++) {
+        const uint32_t b = order[i];
+        const uint64_t blocks = counts[b] > per ? (counts[b] + per - 1) / per : 0;
+        if (waiting + blocks > limit) continue;
+        waiting += blocks;
+        for (uint32_t j = i; j > taken; j--) order[j] = order[j - 1];
+        order[taken++] = b;
+    }
+    return taken;
+}
+
+struct Route {
+    Path path;
+    int vecs;  // resident path: vectors per thread
+};
+
+// `forced`: the tuning key "topk_path" (1 exact, 2 single-pass, 3 resident where it is admitted).
+// Measured per call, us:
+//   resident where one launch may take the call: 65,536 elements 15 against 28 exact; 1 M 21 against 26
+//     streaming; 8 x 262,144 20 against 30 streaming; 16 x 65,536 18 against 31 exact; 1500 x 16,384, where a
+//     bucket is one block and nobody waits, 63 against 187 exact.
+//   Beyond, several launches are slower than the two of the streaming path (24 buckets of 1001 to 1.5 M, three
+//     launches: 68 against 52) ...
+//   ... unless the streaming path's tiles run out of candidate slots (128 per 4096 elements, more than 3 %
+//     inside the sampled window: ratios above about 0.015).  Its tiles are then read again as a whole: that
+//     list at 5 % 71 against 199, 30 buckets of 20,000 to 2 M in seven launches 169 against 240.
+//   Buckets of one buffer take the exact path instead: one of 6.5 M at 5 % 144 against 448, 16 x 262,144 57 against
+//     99, 4 x 2 M 117 against 167, 20 x 1.5 M 288 against 320; of many large ones the streaming path shares that
+//     latency: 12 x 2 M 249 exact, 230 streaming, 50 x 1.7 M 782 and 725, 14 x 6.5 M 905 and 826.
+inline Route choose_path(const TopkCall& c, int forced, uint64_t limit) {
+    const uint64_t tiles = (c.bucket_elems + kFTile - 1) / kFTile;
+    const bool streams = (uint64_t)c.nbuckets * (tiles + kGroups + 1) + kGroups < 0x7FFFFFFFull;
+    if (forced == 1 && !c.counts) return {kPathExact, 0};
+    if (forced == 2 && streams) return {kPathStream, 0};
+    // expected share of a bucket inside the sampled window (see sample_window)
+    const double ks = (double)c.k_full / (double)c.bucket_elems * kFSample;
+    const bool dense = (ks + 6.0 * std::sqrt(ks) + 16.0) / kFSample > (double)kTileSlots / kFTile;
+    int vecs = resident_vecs(c, limit);
+    // a list can go in several launches, as long as its longest bucket fits one
+    if (!vecs && c.counts && (dense || forced == 3) && c.bucket_elems <= (limit < kRMaxBlocks ? limit : kRMaxBlocks) * kRVecElems * 4) vecs = 4;
+    if (vecs) return {kPathResident, vecs};
+    if (c.counts) return {streams ? kPathStream : kPathExact, 0};
+    const bool shared = c.bucket_elems > kRMaxBucket ? c.nbuckets >= 8 : c.bucket_elems >= 400 * kFTile && c.nbuckets >= 12;
+    return {streams && c.bucket_elems >= kFastMinBucket && (!dense || shared) ? kPathStream : kPathExact, 0};
+}
+
+}  // namespace mcclhip

@@ -71,8 +71,8 @@ def test_resident_lists_and_uniform_buckets(ops):
         w, rc = oracle.topk_compress(x, r, 0.01)
         assert wv.cpu().numpy()[:rc].tobytes() == w.tobytes()
         assert np.array_equal(bits(to_np(dr, F32)), bits(r))
-    # buckets of one buffer, more blocks than are resident at once, a short last bucket
-    be, nb = 50_001, 60
+    # buckets of one buffer, as many blocks as one launch may have (128 on 256 CUs), a short last bucket
+    be, nb = 50_001, 32
     n = be * nb - 20_000
     g, r = student_t(rng, n), np.zeros(n, np.float32)
     dr = to_dev(r, F32)
@@ -100,3 +100,21 @@ def test_resident_list_longest_first(ops):
         w, rc = oracle.topk_compress(x, r, 0.01)
         assert wv.cpu().numpy()[:rc].tobytes() == w.tobytes(), x.size
         assert np.array_equal(bits(to_np(dr, F32)), bits(r)), x.size
+
+
+def test_resident_list_in_several_launches(ops):
+    """More waiting blocks than one launch may have: the longest bucket of all, whose 128 blocks fill
+    a launch, others that share one, and the short ones that go with the first."""
+    rng = np.random.default_rng(13)
+    sizes = [700_003, 4096, 2_097_152, 16_385, 1_500_001, 3, 600_001, 1_048_577, 40_000]
+    grads = [student_t(rng, n) for n in sizes]
+    res = [(rng.standard_normal(n) * 1e-4).astype(np.float32) for n in sizes]
+    dres = [to_dev(r, F32) for r in res]
+    status = torch.zeros(1, dtype=torch.int32, device=DEV)
+    for ratio in (0.01, 0.05):
+        wires = ops.topk_compress_list([to_dev(x, F32) for x in grads], dres, ratio, status=status)
+        for x, r, dr, wv in zip(grads, res, dres, wires):
+            w, rc = oracle.topk_compress(x, r, ratio)
+            assert wv.cpu().numpy()[:rc].tobytes() == w.tobytes(), (x.size, ratio)
+            assert np.array_equal(bits(to_np(dr, F32)), bits(r)), (x.size, ratio)
+    assert int(status) == 0
