@@ -150,10 +150,10 @@ template <int V>
 __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometry g, Workspace w, uint32_t nlead, uint32_t epoch,
                                                                 uint32_t published, uint64_t limit_ticks) {
     constexpr uint32_t PER = kRThreads * 4 * V;  // elements of a block
-    // Buckets of this many elements start from a sampled window.  A sample costs about 5 us and saves a
-    // round; beside buckets that need theirs anyway a second round is what ends last (24 buckets of 1001
-    // to 1.5 M elements: 31.1 us with 2^18 throughout, 29.9 with 2^16 for four vectors, 29.3 with 2^15).
-    constexpr uint32_t kSampleMin = V == 4 ? 1u << 15 : V == 2 ? 1u << 16 : 1u << 18;
+    // Buckets of this many elements start from a sampled window, which costs about 5 us and saves a round.
+    // With a sample and without, us: 8 x 70,000 elements 17.9 / 16.0, 30 x 33,000 20.7 / 18.8, 8 x 262,143 22.0 / 21.9,
+    // 3 x 300,000 18.7 / 17.4, one of 400,000 18.9 / 18.0, of 1 M 21.3 / 23.5, of 2 M 25.4 / 28.1, 2 x 1 M 22.0 / 24.0.
+    constexpr uint32_t kSampleMin = 1u << 19;
     const BucketsArg bk = buckets_arg();
     __shared__ ResidentLds<V> L;
     const int lane = threadIdx.x & (kWave - 1);
