@@ -1359,8 +1359,7 @@ uint64_t workspace_words(const Geometry& g) {
     return zeroed_words(g) + 2 * align4((uint64_t)g.nbuckets * g.tiles) + 2 * align4((uint64_t)g.nbuckets * kGroups) +
            align4((uint64_t)g.nbuckets * g.ftiles) + align4((uint64_t)g.nbuckets * g.ftiles * kTileSlots * 2) +
            align4((uint64_t)g.nbuckets * kGroups * kCntStride) + align4((uint64_t)g.nbuckets * kCoarse * kGroups) +
-           align4((uint64_t)g.nbuckets * kCoarse) + align4((uint64_t)g.nbuckets * (kCoarse - 1) * g.lcapb * 2) +
-           (g.bucket_elems <= kRMaxBucket ? (uint64_t)g.nbuckets * kRWords : 0);
+           align4((uint64_t)g.nbuckets * kCoarse) + align4((uint64_t)g.nbuckets * (kCoarse - 1) * g.lcapb * 2);
 }
 
 Workspace carve(void* base, const Geometry& g) {
@@ -1377,7 +1376,12 @@ Workspace carve(void* base, const Geometry& g) {
     w.grp_cnt = p;     p += align4((uint64_t)g.nbuckets * kGroups * kCntStride);
     w.gsuf = p;       p += align4((uint64_t)g.nbuckets * kGroups * kCoarse);
     w.bin_fill = p;    p += align4((uint64_t)g.nbuckets * kCoarse);
-    w.blist = (uint64_t*)p;  p += align4((uint64_t)g.nbuckets * (kCoarse - 1) * g.lcapb * 2);
+    w.blist = (uint64_t*)p;
+    // The resident path's scratch lies where the streaming path has its lists: a call takes one of the two.
+    // It is used for buckets of more than one block, more than kRVecElems elements; theirs hold at least 2048
+    // entries a bin.  (Words of its own would make the size fall from 2 M elements to 2 M + 1, and refuse a
+    // workspace sized for a longer bucket.)
+    static_assert((kCoarse - 1) * 2048 * 2 >= kRWords && kRVecElems >= 2048, "fits the lists");
     w.rmem = p;
     w.status = nullptr;
     return w;

@@ -48,6 +48,16 @@ def test_host_only_entry_points_agree_with_the_reference_formulas():
     assert lib.mccl_hip_set_tuning(b"no_such_key", 1) == -6
 
 
+def test_a_workspace_for_a_longer_bucket_serves_a_shorter_one():
+    from mccl_amd import _lib
+    size = _lib.load().mccl_hip_topk_workspace_bytes
+    lengths = sorted({m for e in range(1, 25) for m in (2 ** e - 1, 2 ** e, 2 ** e + 1, 2 ** e + 40_000, 3 * 2 ** e)})
+    for ratio in (0.001, 0.01, 0.05, 1.0):
+        for buckets in (1, 7):
+            sizes = [size(n * buckets, n, ratio) for n in lengths]
+            assert all(a and a <= b for a, b in zip(sizes, sizes[1:])), (ratio, buckets)
+
+
 def test_argument_errors_need_no_gpu():
     from mccl_amd import _lib
     lib = _lib.load()
