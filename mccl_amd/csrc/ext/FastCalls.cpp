@@ -35,6 +35,12 @@ const at::Tensor* gpu_tensor(PyObject* o, at::ScalarType dtype, uint64_t min_num
     return t && t->scalar_type() == dtype && static_cast<uint64_t>(t->numel()) >= min_numel ? t : nullptr;
 }
 
+// ... a byte tensor that holds `rows` rows of `stride` > 0 bytes (whatever their product).
+const at::Tensor* gpu_rows(PyObject* o, uint64_t rows, int64_t stride) {
+    const at::Tensor* t = gpu_tensor(o, at::kByte, 1);
+    return t && static_cast<uint64_t>(t->numel() / stride) >= rows ? t : nullptr;
+}
+
 bool kernel_dtype(at::ScalarType t) {
     switch (t) {
         case at::kByte: case at::kInt: case at::kLong: case at::kHalf: case at::kFloat: case at::kBool: case at::kBFloat16:
@@ -167,7 +173,7 @@ PyObject* topk_compress(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const uint64_t count = static_cast<uint64_t>(g->numel());
     const uint64_t be = std::min<uint64_t>(bucket, count), nb = (count + be - 1) / be;
     const at::Tensor* r = gpu_tensor(a[1], at::kFloat, count);
-    const at::Tensor* w = gpu_tensor(a[4], at::kByte, nb * static_cast<uint64_t>(stride));
+    const at::Tensor* w = gpu_rows(a[4], nb, stride);
     const at::Tensor* ws = gpu_tensor(a[5], at::kByte, 1);
     const at::Tensor* st = a[7] == Py_None ? nullptr : gpu_tensor(a[7], at::kInt, 1);
     if (!r || static_cast<uint64_t>(r->numel()) != count || !w || !ws || (a[7] != Py_None && !st)) Py_RETURN_NONE;
@@ -195,7 +201,7 @@ PyObject* sparse_accumulate(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const uint64_t be = std::min<uint64_t>(bucket, count), nb = (count + be - 1) / be;
     const void* wires[MCCL_HIP_MAX_WORLD];
     for (Py_ssize_t i = 0; i < nw; i++) {
-        const at::Tensor* w = gpu_tensor(wv[i], at::kByte, nb * static_cast<uint64_t>(stride));
+        const at::Tensor* w = gpu_rows(wv[i], nb, stride);
         if (!w) Py_RETURN_NONE;
         wires[i] = w->data_ptr();
     }

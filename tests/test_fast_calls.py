@@ -94,3 +94,19 @@ def test_in_place_calls_run_once_behind_an_error_left_by_another_call():
     with pytest.raises(_lib.MCCLHipError) as e:
         ops.fold2(d, b, 5)   # no such op: refused by the library, nothing launched
     assert e.value.code == -1 and (d == 5.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stride", [2 ** 62, 2 ** 62 + 4, 2 ** 63 - 4, 40])
+def test_a_payload_buffer_shorter_than_its_rows_is_refused(stride):
+    """Four rows of 2^62 bytes are 2^64, which 64 bits do not hold: nothing may be launched."""
+    dev = "cuda:0"
+    t, r = torch.ones(32, device=dev), torch.zeros(32, device=dev)
+    wire = torch.zeros(4 * 36, dtype=torch.uint8, device=dev)
+    ws = ops.topk_workspace(32, 8, 0.5, dev)
+    with pytest.raises(ValueError, match="wire holds 144 elements"):
+        ops.topk_compress(t, r, 0.5, bucket_elems=8, wire=wire, workspace=ws, wire_stride=stride)
+    with pytest.raises(ValueError, match="holds 144 elements"):
+        ops.sparse_accumulate(r, [wire], stride, bucket_elems=8, workspace=ws)
+    torch.cuda.synchronize()
+    assert (r == 0.0).all() and (wire == 0).all()
