@@ -12,7 +12,7 @@
 // compiled with -ffp-contract=off); fp16/bf16 are widened, operated on in fp32
 // and narrowed once with round-to-nearest-even.
 #include "common.hip.h"
-#include "ring_cut.h"
+#include "fold_rows.h"
 #include "runtime.h"
 
 #include <algorithm>
@@ -143,18 +143,6 @@ struct FoldInt {
 };
 
 // ---- binary fold / scale / fused ----------------------------------------------
-// Layout: [head scalars][16-byte vectors][tail scalars]; head makes the destination 16-byte aligned.
-// `lead` vectors of the first tile group lie in front of the body, and `dst`, `src` and `nvec` count
-// from the group's start.  The launch computes all of it (fold_span), so that a wavefront starts
-// with its addresses at hand.
-struct __attribute__((aligned(32))) FoldSpan {
-    char* dst;
-    const char* src;
-    uint64_t nvec;
-    uint16_t head, tail;  // elements, fewer than 16 bytes each
-    uint32_t lead;        // vectors of the first tile group that lie in front of the body
-};
-
 template <int ES, bool NT>
 __device__ __forceinline__ u4a load_src(const void* p) {
     return load_vec_u<(ES == 2 ? 2 : (ES == 1 ? 1 : 4)), NT>(p);
@@ -196,7 +184,7 @@ __global__ __launch_bounds__(kFoldBlock) void k_fold2(char* dst, const char* src
 }
 
 // ---- a list of independent binary folds in one launch ---------------------------
-// blockIdx.y = fold, blockIdx.x strides over that fold's vectors.  The table is read where
+// blockIdx.y = fold, blockIdx.x = tile of it (strided where the grid is capped).  The table is read where
 // the launch put it, in the kernel-argument segment, one 32-byte scalar load per block (indexing
 // the by-value parameter would make the compiler copy it to per-lane scratch memory first): it
 // is therefore the only parameter.
@@ -431,36 +419,29 @@ int launch_fold2_t(void* dst, const void* src, uint64_t n, float scale, hipStrea
     return launch_fold2_f<FoldFloat<DT, OP, KIND>>(dst, src, n, scale, st);
 }
 
-// One launch per kFoldBatch folds.  Every fold gets as many blocks as the longest one needs (shorter
-// folds' surplus blocks leave at once), but at most twice the average: the folds of a ring step are
-// alike, and in a ragged list a grid cut to the longest fold would consist of surplus blocks.
+// At most kFoldBatch folds a launch (fold_rows.h: how a ragged list is parted).
 template <class F>
 int launch_fold2_batch_f(void* const* dsts, const void* const* srcs, const uint64_t* counts, uint32_t nfolds,
                          hipStream_t st) {
     const uint64_t cap = (uint64_t)device_info().num_cus * (uint64_t)tuning().fold_blocks_per_cu;
     const bool nt = tuning().nontemporal != 0;
-    FoldBatch fb;
-    uint32_t m = 0;
-    uint64_t longest = 0, sum = 0;  // blocks
+    FoldSpan spans[kFoldBatch];
+    uint32_t n = 0;
     auto flush = [&]() {
-        if (m == 0) return;
-        for (uint32_t i = m; i < (uint32_t)kFoldBatch; i++) fb.f[i] = FoldSpan{};
-        const uint64_t most = 2 * ((sum + m - 1) / m) + 1;
-        uint64_t gx = longest < most ? longest : most;
-        if (m > 1) gx = (gx + kXcds - 1) / kXcds * kXcds;  // every fold starts on the same XCD
-        const dim3 grid(clamp_u32(gx, 1, cap / m > 0 ? cap / m : 1), m, 1);
-        if (nt) k_fold2_batch<F, true><<<grid, kFoldBlock, 0, st>>>(fb);
-        else k_fold2_batch<F, false><<<grid, kFoldBlock, 0, st>>>(fb);
-        m = 0;
-        longest = sum = 0;
+        if (n) fold_rows(spans, n, [&](const FoldSpan* f, uint32_t m, uint64_t gx) {
+            FoldBatch fb = {};
+            std::copy(f, f + m, fb.f);
+            if (m > 1) gx = (gx + kXcds - 1) / kXcds * kXcds;  // every fold starts on the same XCD
+            const dim3 grid(clamp_u32(gx, 1, cap / m > 0 ? cap / m : 1), m, 1);
+            if (nt) k_fold2_batch<F, true><<<grid, kFoldBlock, 0, st>>>(fb);
+            else k_fold2_batch<F, false><<<grid, kFoldBlock, 0, st>>>(fb);
+        });
+        n = 0;
     };
     for (uint32_t i = 0; i < nfolds; i++) {
         if (counts[i] == 0) continue;
-        fb.f[m] = fold_span(dsts[i], srcs[i], counts[i], F::size);
-        const uint64_t blocks = (fb.f[m].nvec + kFoldBlock - 1) / kFoldBlock;
-        longest = blocks > longest ? blocks : longest;
-        sum += blocks;
-        if (++m == (uint32_t)kFoldBatch) flush();
+        spans[n] = fold_span(dsts[i], srcs[i], counts[i], F::size);
+        if (++n == (uint32_t)kFoldBatch) flush();
     }
     flush();
     return launch_status();
