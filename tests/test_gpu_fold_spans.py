@@ -46,7 +46,7 @@ def test_edges_single_and_list(dt):
 
 
 def test_list_longer_than_one_launch_and_strided_grid():
-    from mccl_amd import hip_ops as ops
+    from mccl_amd import _lib, hip_ops as ops
     n = 2_000_000
     d = torch.arange(n, device=DEV, dtype=torch.float32)
     s = torch.ones(n, device=DEV)
@@ -55,10 +55,12 @@ def test_list_longer_than_one_launch_and_strided_grid():
     ops.fold2_batch(dl, [s[a:b] for a, b in zip(cuts, cuts[1:])], ops.SUM)
     want = torch.arange(n, device=DEV, dtype=torch.float32) + 1
     assert torch.equal(d, want)
+    shipped = _lib.load().mccl_hip_get_tuning(b"fold_blocks_per_cu")
+    assert shipped == 4096                             # the folds above ran on the grid that is shipped
     try:
         ops.set_tuning("fold_blocks_per_cu", 1)        # the grid cap: blocks stride over the vectors
         ops.fold2(d, s, ops.SUM)
         ops.fold2_batch(dl, [s[a:b] for a, b in zip(cuts, cuts[1:])], ops.SUM)
     finally:
-        ops.set_tuning("fold_blocks_per_cu", 4096)
+        ops.set_tuning("fold_blocks_per_cu", shipped)
     assert torch.equal(d, want + 2)
