@@ -225,7 +225,8 @@ def test_compressor_errors_and_decompress(k):
         comp.decompress(wire, idx_max)
 
 
-def test_compressor_reports_a_give_up_of_the_compress_launch(k):
+@pytest.mark.parametrize("path", [2, 3])  # single-pass, resident
+def test_compressor_reports_a_give_up_of_the_compress_launch(k, path):
     """compress() is asynchronous; a launch that gives up (every wait forced into its limit from
     the host, all kernels exit normally) is reported by the calls that wait for the stream:
     check_compress_status() and decompress() raise, and the payload is rejected."""
@@ -236,6 +237,7 @@ def test_compressor_reports_a_give_up_of_the_compress_launch(k):
     good = comp.compress(g, stable_id=1)
     comp.check_compress_status()
     try:
+        ops.set_tuning("topk_path", path)
         ops.set_tuning("topk_stall_test", 1)
         ops.set_tuning("topk_barrier_ms", 1)
         bad = comp.compress(g, stable_id=1)
@@ -243,6 +245,7 @@ def test_compressor_reports_a_give_up_of_the_compress_launch(k):
     finally:
         ops.set_tuning("topk_stall_test", 0)
         ops.set_tuning("topk_barrier_ms", 2000)
+        ops.set_tuning("topk_path", 0)
     with pytest.raises(RuntimeError, match="Timeout"):
         comp.check_compress_status()
     comp.check_compress_status()   # reported once

@@ -32,7 +32,9 @@ def oracle_buckets(g, r, ratio, be):
     return wires, res
 
 
-PATHS = {"exact": 1, "single-pass": 2}  # both must give the oracle's bytes on every input
+# All must give the oracle's bytes on every input.  (A call the resident path does not admit takes one of the
+# others under its name.)
+PATHS = {"exact": 1, "single-pass": 2, "resident": 3}
 
 
 def check_compress(ops, g, r, ratio, be=None, pad=0):
@@ -203,14 +205,14 @@ def _with_bits(x, positions, patterns):
     return x
 
 
-def test_compress_orders_nan_and_inf_by_bit_pattern(ops):
+@pytest.mark.parametrize("n", [400_000, 600_000])  # the resident path without a sampled window and with one
+def test_compress_orders_nan_and_inf_by_bit_pattern(ops, n):
     """Selection orders magnitudes by `bits & 0x7FFFFFFF`: infinities above every finite value,
     NaN patterns above infinity (by payload), ties to the lower index.  A gradient that carries
-    NaN or inf therefore gives a defined payload, the same on both paths as in the oracle: NaNs
+    NaN or inf therefore gives a defined payload, the same on every path as in the oracle: NaNs
     spread over the bucket, a NaN inside a cluster of large values (a tile with more candidates
     than slots), and a threshold that falls among equal NaN patterns (tie-break by index)."""
     rng = np.random.default_rng(606)
-    n = 400_000
     qnan, qnan2, neg_qnan, top = 0x7FC00000, 0x7FC00123, 0xFFC00001, 0x7FFFFFFF
     pinf, ninf = 0x7F800000, 0xFF800000
     # (a) a few specials spread over the bucket
@@ -224,7 +226,7 @@ def test_compress_orders_nan_and_inf_by_bit_pattern(ops):
     g[200_000:203_000] = student_t(rng, 3_000, ties=0.0) * np.float32(50.0)
     g = _with_bits(g, [200_500, 201_000, 201_001, 202_999], [qnan, pinf, neg_qnan, top])
     check_compress(ops, g.copy(), np.zeros(n, np.float32), 0.01)
-    # (c) the threshold falls among equal NaN patterns: k = 4000, 6000 identical NaNs, 1000 larger patterns
+    # (c) the threshold falls among equal NaN patterns: k = n / 100, 6000 identical NaNs, 1000 larger patterns
     g = student_t(rng, n, ties=0.0)
     same = rng.choice(n, 6_000, replace=False)
     g = _with_bits(g, same, np.full(6_000, qnan, np.uint32))
@@ -262,9 +264,10 @@ def test_timeout_word_is_reported(ops):
         ops.topk_path_report(ws, n, be, 0.01)
 
 
-def test_give_up_path_poisons_the_payload_and_sets_the_status(ops):
-    """Every wait of the single-pass path runs into its limit (the sample blocks are told to
-    publish a number nobody waits for; every kernel still exits normally): the status word
+@pytest.mark.parametrize("path", [2, 3])
+def test_give_up_path_poisons_the_payload_and_sets_the_status(ops, path):
+    """Every wait of the single-pass or the resident path runs into its limit (the sample blocks
+    are told to publish a number nobody waits for; every kernel still exits normally): the status word
     receives the timeout, the path report raises, every payload header holds 0xFFFFFFFF, and
     decompress / sparse accumulate reject such a payload.  The next ordinary call on the same
     workspace is exact again."""
@@ -276,6 +279,7 @@ def test_give_up_path_poisons_the_payload_and_sets_the_status(ops):
     ws = ops.topk_workspace(n, be, 0.01, DEV)
     status = torch.zeros(1, dtype=torch.int32, device=DEV)
     try:
+        ops.set_tuning("topk_path", path)
         ops.set_tuning("topk_stall_test", 1)
         ops.set_tuning("topk_barrier_ms", 1)
         wire, stride = ops.topk_compress(to_dev(g, F32), torch.zeros(n, device=DEV), 0.01, bucket_elems=be,
@@ -284,6 +288,7 @@ def test_give_up_path_poisons_the_payload_and_sets_the_status(ops):
     finally:
         ops.set_tuning("topk_stall_test", 0)
         ops.set_tuning("topk_barrier_ms", 2000)
+        ops.set_tuning("topk_path", 0)
     assert int(status) == -9   # MCCL_HIP_ERR_TIMEOUT
     with pytest.raises(MCCLHipError, match="timed out"):
         ops.topk_path_report(ws, n, be, 0.01)
