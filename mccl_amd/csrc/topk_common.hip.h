@@ -128,8 +128,7 @@ __device__ __forceinline__ uint32_t* bucket_wire(const Geometry& g, BucketsArg b
 }
 
 
-// Blocks that may wait in one resident launch on the stream (resident_limit), 0 on a stream that is
-// confined to some of the GPU's CUs.
+// Blocks that may wait in one resident launch on the stream (stream_limit).
 uint64_t resident_limit_on(hipStream_t st);
 // A list of buckets goes in as many launches as keep each under `limit`.
 void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, int vecs, uint64_t limit, uint32_t epoch,

@@ -31,8 +31,8 @@
 // for these.  A block that is not yet dispatched therefore finds a slot, all blocks of every bucket
 // come to be resident, and their barriers fill.  (The order of buckets within a launch does not give that: of two
 // launches of several hundred blocks one can fill XCD 0 and the other XCD 1, each with buckets that miss
-// blocks on the other.)  On a stream that is confined to some of the CUs no bucket of several blocks
-// takes this path.
+// blocks on the other.)  On a stream that is confined to some of the CUs or has a priority no bucket of several
+// blocks takes this path (stream_limit).
 #include "topk_common.hip.h"
 
 #include <algorithm>
@@ -645,10 +645,16 @@ uint64_t resident_limit_on(hipStream_t st) {
         return (uint32_t)(q > 0 && q < 1024 ? q : 4);
     }();
     // (asking takes 0.2 us; the null stream's mask is the process's)
-    static const bool whole = stream_cus(nullptr) >= device_info().num_cus;
-    const int cus = device_info().num_cus;
-    if (!whole || (st && stream_cus(st) < cus)) return 0;
-    return resident_limit((uint64_t)cus * per_cu, queues);
+    static const int process_cus = stream_cus(nullptr);
+    StreamShare share = {process_cus, 0};
+    if (st) {
+        share.cus = std::min(process_cus, stream_cus(st));
+        if (hipStreamGetPriority(st, &share.priority) != hipSuccess) {
+            (void)hipGetLastError();
+            share.priority = 0;
+        }
+    }
+    return stream_limit(share, device_info().num_cus, per_cu, queues);
 }
 
 void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, int vecs, uint64_t limit, uint32_t epoch,

@@ -33,6 +33,16 @@ struct TopkCall {
 // fit the GPU at once.  Blocks are dealt to the accelerator dies in turn, hence the multiple of eight.
 constexpr uint64_t resident_limit(uint64_t slots, uint32_t queues) { return slots / (queues ? queues : 1) / 8 * 8; }
 
+// ... on a stream.  One that is confined to some of the GPU's CUs finds fewer slots, and the runtime gives
+// streams of each priority `queues` hardware queues of their own, so that twice or three times as many
+// launches could be under way: on neither do blocks wait for others.
+struct StreamShare {
+    int cus, priority;  // 0: the default
+};
+constexpr uint64_t stream_limit(const StreamShare& s, int cus, uint64_t per_cu, uint32_t queues) {
+    return s.cus < cus || s.priority != 0 ? 0 : resident_limit((uint64_t)cus * per_cu, queues);
+}
+
 // Blocks that wait for others with `vecs` vectors per thread: those of every bucket of more than one block.
 inline uint64_t resident_waiting(const TopkCall& c, int vecs) {
     const uint64_t per = kRVecElems * (uint64_t)vecs;

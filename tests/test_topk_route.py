@@ -113,6 +113,9 @@ int main() {
     // two blocks per CU, four queues
     REQUIRE(resident_limit(512, 4) == 128 && resident_limit(128, 4) == 32 && resident_limit(64, 4) == 16);
     REQUIRE(resident_limit(512, 32) == 16 && resident_limit(0, 4) == 0);
+    // a stream that has part of the GPU, or a priority and with it queues beside the four
+    REQUIRE(stream_limit({256, 0}, 256, 2, 4) == 128 && stream_limit({32, 0}, 32, 2, 4) == 16);
+    REQUIRE(stream_limit({255, 0}, 256, 2, 4) == 0 && stream_limit({256, -1}, 256, 2, 4) == 0 && stream_limit({256, 1}, 256, 2, 4) == 0);
     const double r1 = 0.01, r5 = 0.05;
     const auto path = [](const TopkCall& c, uint64_t limit) { return choose_path(c, 0, limit).path; };
     const auto vecs = [](const TopkCall& c, uint64_t limit) { return choose_path(c, 0, limit).vecs; };
