@@ -233,6 +233,13 @@ int mccl_hip_topk_decompress(const void* wire, uint64_t wire_bytes, float* dense
 int mccl_hip_topk_decompress_sorted(const void* wire, uint64_t wire_bytes, float* dense, uint64_t count,
                                     int* status, void* stream);
 
+/* ... that also copies *flag, a device word which earlier work on the stream may
+ * have written (a compress call's status), to *flag_out (device memory or pinned
+ * host memory), so that a caller who waits for this call reads both without a
+ * copy of its own.  flag and flag_out are both given or both NULL. */
+int mccl_hip_topk_decompress_sorted_flag(const void* wire, uint64_t wire_bytes, float* dense, uint64_t count,
+                                         int* status, const int* flag, int* flag_out, void* stream);
+
 /* Decompress + accumulate of `ws` ranks' payloads into one dense buffer, the
  * sparse equivalent of decompressing every peer's payload and folding the
  * dense buffers in ascending rank order, then the AVG multiply

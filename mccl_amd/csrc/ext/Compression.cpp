@@ -94,13 +94,6 @@ at::Tensor& TopKCompressor::residual_for(uint64_t stable_id, size_t count) {
 }
 
 namespace {
-// One int in pinned host memory: kernels write it where it lies, the host reads it after a stream
-// wait with no copy of its own (a device word costs a copy kernel and a second wait per read).
-at::Tensor pinned_word() {
-    return at::zeros({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-}
-int read_word(const at::Tensor& t) { return *static_cast<const volatile int*>(t.data_ptr<int>()); }
-
 void wait_for_current_stream() {
     throw_on_status(mccl_hip_sync(c10::hip::getCurrentHIPStream().stream()), "TopK stream wait");
 }
@@ -108,18 +101,19 @@ void wait_for_current_stream() {
 
 // The word the compress launches report a give-up through (a block of a launch that waited too
 // long for another block of it).  The launches are asynchronous, so the word is looked at by the
-// calls that wait for the stream anyway: decompress() and check_compress_status().  Caller holds mu_.
+// calls that wait for the stream anyway: decompress() and check_compress_status().  It is device
+// memory, which goes back to its allocator in stream order: launches may still be under way when the
+// compressor goes (a pinned word would be another tensor's by then).  Caller holds mu_.
 int* TopKCompressor::compress_status() {
-    if (!compress_status_.defined()) compress_status_ = pinned_word();
+    if (!compress_status_.defined())
+        compress_status_ = at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(at::kCUDA));
     return compress_status_.data_ptr<int>();
 }
 
-// The current stream has been waited for.
-void TopKCompressor::throw_if_compress_failed() {
-    if (!compress_status_.defined()) return;
-    const int st = read_word(compress_status_);
+// `st`: what the word held when the current stream had been waited for.
+void TopKCompressor::throw_if_compress_failed(int st) {
     if (st == 0) return;
-    *compress_status_.data_ptr<int>() = 0;
+    compress_status_.zero_();
     if (st == MCCL_HIP_ERR_TIMEOUT)
         throw TimeoutError("TopK compress: a block gave up waiting for another block of its launch; "
                            "the payloads of that call are invalid");
@@ -129,8 +123,7 @@ void TopKCompressor::throw_if_compress_failed() {
 void TopKCompressor::check_compress_status() {
     std::lock_guard<std::mutex> lock(mu_);
     if (!compress_status_.defined()) return;
-    wait_for_current_stream();
-    throw_if_compress_failed();
+    throw_if_compress_failed(compress_status_.item<int>());
 }
 
 // One bucket on `stream`: csrc/compression/TopKCompression.cpp:38-120.  Caller holds mu_.
@@ -230,9 +223,10 @@ std::vector<at::Tensor> TopKCompressor::compress_many(const std::vector<at::Tens
 }
 
 // csrc/compression/TopKCompression.cpp:122-152.  The reference validates while
-// it scatters and throws; here the kernel reports through a word in host memory
-// that is read once the stream has drained (the call is synchronous, as the
-// reference's is).  A payload that does not ascend, or that breaks a rule, is
+// it scatters and throws; here the kernel reports through a word in pinned host
+// memory, and brings the compress status to a second one; both are read once the
+// stream has drained, with no copy and no second wait (the call is synchronous, as
+// the reference's is).  A payload that does not ascend, or that breaks a rule, is
 // expanded (again) by the kernels that take pairs in any order.
 void TopKCompressor::decompress(const void* src, size_t compressed_size, void* dst, size_t nbytes,
                                 at::ScalarType dtype) {
@@ -240,20 +234,30 @@ void TopKCompressor::decompress(const void* src, size_t compressed_size, void* d
     const size_t count = nbytes / sizeof(float);
     std::lock_guard<std::mutex> lock(mu_);
     metal_kernels_init();
-    if (!status_.defined()) status_ = pinned_word();
+    if (!status_.defined()) status_ = at::zeros({2}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
     int* const word = status_.data_ptr<int>();
     void* const stream = c10::hip::getCurrentHIPStream().stream();
-    auto expand = [&](auto fn) {
-        *word = 0;
-        const int rc = fn(src, compressed_size, static_cast<float*>(dst), count, word, stream);
+    float* const dense = static_cast<float*>(dst);
+    const int* const flag = compress_status_.defined() ? compress_status_.data_ptr<int>() : nullptr;
+    auto expand = [&](auto launch) {
+        word[0] = word[1] = 0;
+        const int rc = launch();
         if (rc == MCCL_HIP_ERR_SIZE) throw MCCLError("TopK decompress: size mismatch");
         throw_on_status(rc, "TopK decompress");
         wait_for_current_stream();
-        return read_word(status_);
+        return *static_cast<const volatile int*>(word);
     };
-    int st = count ? expand(mccl_hip_topk_decompress_sorted) : MCCL_HIP_ERR_ORDER;
-    if (st != 0) st = expand(mccl_hip_topk_decompress);
-    throw_if_compress_failed();
+    int st = MCCL_HIP_ERR_ORDER;
+    if (count)
+        st = expand([&] {
+            return mccl_hip_topk_decompress_sorted_flag(src, compressed_size, dense, count, word, flag, flag ? word + 1 : nullptr, stream);
+        });
+    if (st == 0) {
+        throw_if_compress_failed(*static_cast<const volatile int*>(word + 1));
+        return;
+    }
+    st = expand([&] { return mccl_hip_topk_decompress(src, compressed_size, dense, count, word, stream); });
+    if (flag) throw_if_compress_failed(compress_status_.item<int>());
     if (st == MCCL_HIP_ERR_SIZE) throw MCCLError("TopK decompress: size mismatch");
     if (st == MCCL_HIP_ERR_INDEX) throw MCCLError("TopK decompress: index out of bounds");
 }

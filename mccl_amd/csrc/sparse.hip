@@ -77,7 +77,7 @@ constexpr int kDecSamples = kBlock;      // one per thread
 constexpr uint32_t kDecMaxStride = 4096;  // beyond (over a million pairs) fill and scatter are as fast
 
 __global__ __launch_bounds__(kBlock) void k_decompress_sorted(const uint32_t* wire, uint32_t k, uint32_t stride, float* dense,
-                                                              uint64_t count, int* status) {
+                                                              uint64_t count, int* status, const int* flag, int* flag_out) {
     __shared__ __attribute__((aligned(16))) float tile[kDecTile];
     __shared__ uint32_t samp[kDecSamples + 1];
     __shared__ uint32_t below[2];
@@ -87,6 +87,8 @@ __global__ __launch_bounds__(kBlock) void k_decompress_sorted(const uint32_t* wi
     const uint64_t mypos = (uint64_t)threadIdx.x * stride;
     const uint32_t have_k = wire[0];
     const uint32_t mine = mypos < k ? pairs[2 * mypos] : 0xFFFFFFFFu;
+    const bool brings = flag && blockIdx.x == 0 && threadIdx.x == 0;
+    const int brought = brings ? *flag : 0;
 #pragma unroll
     for (int i = 0; i < kDecTile / (4 * kBlock); i++) ((u4a*)tile)[i * kBlock + threadIdx.x] = u4a{0u, 0u, 0u, 0u};
     if (threadIdx.x < 2) below[threadIdx.x] = 0;
@@ -94,8 +96,10 @@ __global__ __launch_bounds__(kBlock) void k_decompress_sorted(const uint32_t* wi
     samp[threadIdx.x] = mine;
     if (have_k != k) {  // the same in every lane of the grid
         if (blockIdx.x == 0 && threadIdx.x == 0) *status = MCCL_HIP_ERR_SIZE;
+        if (brings) *flag_out = brought;
         return;
     }
+    if (brings) *flag_out = brought;  // (its load went with the samples)
     __syncthreads();
     int bad = 0;
     if (mypos + stride < k && mine >= samp[threadIdx.x + 1]) bad = MCCL_HIP_ERR_ORDER;
@@ -130,6 +134,8 @@ __global__ __launch_bounds__(kBlock) void k_decompress_sorted(const uint32_t* wi
         for (uint32_t i = threadIdx.x; i < len; i += kBlock) out[i] = tile[i];
     }
 }
+
+__global__ void k_copy_word(const int* from, int* to) { *to = *from; }
 
 struct WirePtrs {
     const uint8_t* w[MCCL_HIP_MAX_WORLD];
@@ -847,7 +853,12 @@ int mccl_hip_topk_decompress(const void* wire, uint64_t wire_bytes, float* dense
 
 int mccl_hip_topk_decompress_sorted(const void* wire, uint64_t wire_bytes, float* dense, uint64_t count,
                                     int* status, void* stream) {
-    if (!wire || !dense || !status || ((uintptr_t)wire & 3)) return MCCL_HIP_ERR_ARG;
+    return mccl_hip_topk_decompress_sorted_flag(wire, wire_bytes, dense, count, status, nullptr, nullptr, stream);
+}
+
+int mccl_hip_topk_decompress_sorted_flag(const void* wire, uint64_t wire_bytes, float* dense, uint64_t count,
+                                         int* status, const int* flag, int* flag_out, void* stream) {
+    if (!wire || !dense || !status || ((uintptr_t)wire & 3) || !flag != !flag_out) return MCCL_HIP_ERR_ARG;
     if (count == 0 || count > 0xFFFFFFFFull) return MCCL_HIP_ERR_ARG;
     if (wire_bytes < 4 || ((wire_bytes - 4) & 7)) return MCCL_HIP_ERR_SIZE;
     const uint64_t k = (wire_bytes - 4) / 8;
@@ -855,10 +866,12 @@ int mccl_hip_topk_decompress_sorted(const void* wire, uint64_t wire_bytes, float
     int rc = mccl_hip_init();
     if (rc) return rc;
     const uint64_t stride = k ? (k + kDecSamples - 1) / kDecSamples : 1;
-    if (stride > kDecMaxStride)
+    if (stride > kDecMaxStride) {
+        if (flag) k_copy_word<<<1, 1, 0, (hipStream_t)stream>>>(flag, flag_out);
         return mccl_hip_topk_decompress(wire, wire_bytes, dense, count, status, stream);
+    }
     k_decompress_sorted<<<(uint32_t)((count + kDecTile - 1) / kDecTile), kBlock, 0, (hipStream_t)stream>>>(
-        (const uint32_t*)wire, (uint32_t)k, (uint32_t)stride, dense, count, status);
+        (const uint32_t*)wire, (uint32_t)k, (uint32_t)stride, dense, count, status, flag, flag_out);
     return launch_status();
 }
 

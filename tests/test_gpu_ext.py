@@ -254,6 +254,29 @@ def test_compressor_reports_a_give_up_of_the_compress_launch(k, path):
     comp.decompress(good, 400_000)
 
 
+def test_a_give_up_behind_the_compressor_writes_nobodys_memory(k):
+    """The compressor may go while a compress launch of its own is under way, and that launch may
+    still report a give-up: not into pinned memory that by then is another tensor's."""
+    from mccl_amd import hip_ops as ops
+    C = k["C"]
+    g = torch.from_numpy(student_t(np.random.default_rng(4), 400_000)).to(DEV)
+    comp = C.TopKCompressor(0.01)
+    comp.decompress(comp.compress(g, stable_id=1), 400_000)
+    try:
+        ops.set_tuning("topk_stall_test", 1)
+        ops.set_tuning("topk_barrier_ms", 100)
+        bad = comp.compress(g, stable_id=1)
+        under_way = not torch.cuda.current_stream().query()
+        del comp
+        words = [torch.full((m,), 7, dtype=torch.int32, pin_memory=True) for m in (1, 1, 2, 2, 1, 2)]
+        torch.cuda.synchronize()
+    finally:
+        ops.set_tuning("topk_stall_test", 0)
+        ops.set_tuning("topk_barrier_ms", 2000)
+    assert under_way and bad.cpu().numpy()[:4].tobytes() == b"\xff" * 4
+    assert all((w == 7).all() for w in words)
+
+
 def test_two_bucket_residual_isolation(k):
     # tests/test_compression_e2e.py:33-75: alternate two buckets of very different scale
     # through one compressor; each bucket's residual must only ever see its own gradients.
