@@ -104,8 +104,8 @@ int mccl_hip_pointer_check(const void* ptr, uint64_t nbytes, void** device_ptr);
 int mccl_hip_fold2(void* dst, const void* src, uint64_t n, int dtype, int op, void* stream);
 
 /* host_dsts[i] = host_dsts[i] (op) host_srcs[i] over host_counts[i] elements, for
- * i < nfolds: the binary fold above on a list of chunk views, one launch per 128
- * folds, every fold's result bit-identical to mccl_hip_fold2 on the same pair.
+ * i < nfolds: the binary fold above on a list of chunk views, one launch per 120
+ * folds (more where their lengths differ widely), every fold's result bit-identical to mccl_hip_fold2 on the same pair.
  * For a caller that holds several folds which do not depend on one another -
  * the folds of one ring step over all gradient buckets, which the reference
  * issues one by one (csrc/backend/ProcessGroupMCCL.cpp:492-512, reduce_op ->

@@ -189,7 +189,7 @@ std::vector<at::Tensor> TopKCompressor::compress_many(const std::vector<at::Tens
                    "compress_many: more distinct stable ids than the compressor holds residuals for");
         residuals.push_back(&it->second);
     }
-    // the list goes to the library in chunks of MCCL_HIP_TOPK_LIST_MAX buckets: two launches per chunk
+    // the list goes to the library in chunks of MCCL_HIP_TOPK_LIST_MAX buckets: one launch per chunk or a few (topk_route.h)
     const int device = buckets[0].get_device();
     void* stream = c10::hip::getCurrentHIPStream(device).stream();
     std::vector<size_t> used(buckets.size());

@@ -25,7 +25,7 @@ uint64_t metal_reduce_op_fenced(const at::Tensor& dst, const at::Tensor& src,
                                 c10d::ReduceOp::RedOpType op);
 
 /// metal_reduce_op on a list of (dst, src) pairs that do not depend on one another, in one
-/// launch per 128 pairs; every pair's result is bit-identical to metal_reduce_op on it.  No
+/// launch per 120 pairs (more where their lengths differ widely); every pair's result is bit-identical to metal_reduce_op on it.  No
 /// counterpart in the reference's header: its ring loop issues the folds of one ring step
 /// one by one (csrc/backend/ProcessGroupMCCL.cpp:492-512).  All tensors share dtype and device;
 /// a destination that overlaps another pair's destination or source throws.

@@ -100,8 +100,8 @@ def fold2(dst: torch.Tensor, src: torch.Tensor, op: int = SUM) -> torch.Tensor:
 
 
 def fold2_batch(dsts: Sequence[torch.Tensor], srcs: Sequence[torch.Tensor], op: int = SUM) -> None:
-    """dsts[i] (op)= srcs[i] for every i, in one launch per 128 folds.  The folds run in no
-    particular order: a destination may not overlap any other fold's destination or source
+    """dsts[i] (op)= srcs[i] for every i, in one launch per 120 folds, or more where the
+    list is ragged.  The folds run in no particular order: a destination may not overlap any other fold's destination or source
     (the library refuses such a list)."""
     rc = _native._fast_fold2_batch(dsts, srcs, op)
     if rc == 0:
