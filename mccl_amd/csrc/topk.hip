@@ -405,22 +405,22 @@ __global__ __launch_bounds__(kBlock) void k_topk_emit(float* residual, Geometry 
 //                   residual <- grad + residual (0.0f at or above the predicted threshold)
 //                   and stages its candidates (key >= lo) in LDS in index order; the block
 //                   writes them to the tile's slots and counts itself into its group of
-//                   tiles (at most 64 groups per bucket).
-//   bin blocks      64 per bucket.  Block g waits until group g's tiles are finished (when it
+//                   tiles (topk_groups of them per bucket).
+//   bin blocks      one per group.  Block g waits until group g's tiles are finished (when it
 //                   is dispatched - one bucket later - they are, except in the last bucket),
 //                   counts the group's candidates per coarse window bin (128 bins), publishes
 //                   the counts and copies the candidates, binned, to the bucket's per-bin
 //                   lists.  It waits for nothing else.
-// k_topk_select - 64 blocks per bucket; nothing crosses blocks any more: every block
+// k_topk_select - one block per group; nothing crosses blocks any more: every block
 //                   redundantly finds the bin that holds the k-th largest key (from the
 //                   groups' counts), the exact threshold and the tie rule (from that bin's
 //                   list) and the number of picks in the groups before its own, then writes
 //                   its group's picks, in index order, at that offset of the payload and
 //                   repairs the residual where the predicted threshold and the true one
 //                   disagree.  A failed selection (threshold outside the window, a bin list
-//                   overflow) hands the bucket to the exact selection, run by the bucket's 64
-//                   blocks together through counter barriers; the launch covers at most 16
-//                   buckets, so that all its blocks are resident at the same time.
+//                   overflow) hands the bucket to the exact selection, run by the bucket's
+//                   blocks together through counter barriers; a launch covers at most 1024
+//                   blocks, so that all of them are resident at the same time.
 //
 // Progress in k_topk_stream.  The hardware deals the blocks of a grid to the XCDs round-robin
 // and every XCD dispatches its share in grid order.  A streaming block waits only for its
@@ -459,7 +459,7 @@ constexpr int kBinsPerLane = kCoarse / kWave; // 2
 constexpr int kCntStride = 64;                // words between two groups' arrival counters: 256 bytes, so that the
                                               // arrivals of a bucket's tiles spread over memory channels
 constexpr int kHeld = 7;                      // tiles per wavefront whose slots a bin / select block keeps in registers
-constexpr int kSelBuckets = 16;               // buckets per k_topk_select launch: 1024 blocks, all resident
+constexpr uint32_t kSelBlocks = 1024;         // blocks of a k_topk_select launch: all resident
 constexpr uint32_t kGaveUp = 0xFFFFFFFEu;     // a wavefront's count: its wait for the sample timed out
 static_assert(kFVecs == 4, "the streaming role is written for four vectors per lane");
 
@@ -487,7 +487,7 @@ __device__ __forceinline__ FusedGeo fused_geo(const Geometry& g, BucketsArg bk, 
     f.bn = bucket_count(g, bk, b);
     f.k = bucket_k(g, bk, b);
     f.ntiles = (uint32_t)((f.bn + kFTile - 1) / kFTile);
-    f.tpg = (f.ntiles + kGroups - 1) / kGroups;
+    f.tpg = (f.ntiles + (1u << g.gshift) - 1) >> g.gshift;
     f.ng = (f.ntiles + f.tpg - 1) / f.tpg;
     return f;
 }
@@ -551,7 +551,7 @@ __device__ __forceinline__ void fused_sample(BucketsArg bk, const Geometry& g, c
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
     const SampleWindow win = sample_window<kBlock>(bucket_grad(g, bk, b), bucket_residual(g, bk, b), fg.bn, fg.k, L.s, [&] {
         // (the acknowledgements are back long before the window is published)
-        if (threadIdx.x < kGroups) st_agent(w.grp_cnt + ((uint64_t)b * kGroups + threadIdx.x) * kCntStride, 0u);
+        if (threadIdx.x >> g.gshift == 0) st_agent(w.grp_cnt + (((uint64_t)b << g.gshift) + threadIdx.x) * kCntStride, 0u);
         if (threadIdx.x < kCoarse) st_agent(w.bin_fill + (uint64_t)b * kCoarse + threadIdx.x, 0u);
         if (threadIdx.x == 0) {
             st_agent(st + S_OK, 0u);
@@ -684,7 +684,7 @@ __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, cons
         // the counter is only meaningful once the sample block has cleared it
         if (threadIdx.x == 0) {
             u4a wn = wait_window(st, epoch, limit_ticks);
-            if (wn[3] && !wait_word(w.grp_cnt + ((uint64_t)b * kGroups + grp) * kCntStride, in_group, limit_ticks)) wn[3] = 0u;
+            if (wn[3] && !wait_word(w.grp_cnt + (((uint64_t)b << g.gshift) + grp) * kCntStride, in_group, limit_ticks)) wn[3] = 0u;
             L.e.win[0] = wn[0]; L.e.win[1] = wn[1]; L.e.win[2] = wn[2]; L.e.win[3] = wn[3];
         }
         __syncthreads();
@@ -729,9 +729,9 @@ __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, cons
         // this group's candidates above each bin: lane l takes bins 127 - 2 l and 126 - 2 l
         const uint32_t c_hi = L.e.cnt[kCoarse - 1 - 2 * lane], c_lo = L.e.cnt[kCoarse - 2 - 2 * lane];
         const uint32_t inc = wave_inclusive_scan(c_hi + c_lo);
-        uint32_t* col = w.gsuf + (uint64_t)b * kCoarse * kGroups + grp;
-        col[(uint64_t)(kCoarse - 1 - 2 * lane) * kGroups] = inc - c_hi - c_lo;
-        col[(uint64_t)(kCoarse - 2 - 2 * lane) * kGroups] = inc - c_lo;
+        uint32_t* col = w.gsuf + (((uint64_t)b * kCoarse) << g.gshift) + grp;
+        col[(uint64_t)(kCoarse - 1 - 2 * lane) << g.gshift] = inc - c_hi - c_lo;
+        col[(uint64_t)(kCoarse - 2 - 2 * lane) << g.gshift] = inc - c_lo;
     }
     __syncthreads();
     // binned copies (read by the next launch: plain stores)
@@ -768,7 +768,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_topk_stream(Buckets, Geometry g, 
     // segment s of the grid: the tiles of bucket s, then the bin blocks of bucket s - 1 (whose
     // tiles are finished or about to be by then: a bin block that is dispatched early only
     // polls); after the last segment the bin blocks of the last bucket
-    const uint32_t per = g.ftiles + kGroups;
+    const uint32_t per = g.ftiles + (1u << g.gshift);
     const uint32_t j = blockIdx.x - g.nbuckets;
     uint32_t b = j / per, t = j - b * per;
     bool emit = false;
@@ -946,7 +946,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_topk_stream(Buckets, Geometry g, 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0)
-        __hip_atomic_fetch_add(w.grp_cnt + ((uint64_t)b * kGroups + t / fg.tpg) * kCntStride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_add(w.grp_cnt + (((uint64_t)b << g.gshift) + t / fg.tpg) * kCntStride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The need-th smallest index among the list's entries with key == T: radix select over
@@ -1071,14 +1071,14 @@ __device__ __forceinline__ bool select_exact_group(BucketsArg bk, const Geometry
         eq_blk += wsum[NW + i];
     }
     if (threadIdx.x == 0) {
-        st_agent(&w.blk_above[(uint64_t)b * kGroups + grp], gt_blk);
-        st_agent(&w.blk_eq[(uint64_t)b * kGroups + grp], eq_blk);
+        st_agent(&w.blk_above[((uint64_t)b << g.gshift) + grp], gt_blk);
+        st_agent(&w.blk_eq[((uint64_t)b << g.gshift) + grp], eq_blk);
     }
     if (!bucket_barrier(st + S_BARF + 3, fg.ng, &L.flag, limit_ticks)) return false;
     {
-        static_assert(kGroups <= kBlock, "one thread per group of the bucket");
-        const uint32_t vg = threadIdx.x < grp ? ld_agent(&w.blk_above[(uint64_t)b * kGroups + threadIdx.x]) : 0u;
-        const uint32_t ve = threadIdx.x < grp ? ld_agent(&w.blk_eq[(uint64_t)b * kGroups + threadIdx.x]) : 0u;
+        static_assert(kMaxGroups <= kBlock, "one thread per group of the bucket");
+        const uint32_t vg = threadIdx.x < grp ? ld_agent(&w.blk_above[((uint64_t)b << g.gshift) + threadIdx.x]) : 0u;
+        const uint32_t ve = threadIdx.x < grp ? ld_agent(&w.blk_eq[((uint64_t)b << g.gshift) + threadIdx.x]) : 0u;
         uint32_t gt_before, eq_before;
         block_exclusive_scan(vg, L.scratch, &gt_before);
         block_exclusive_scan(ve, L.scratch, &eq_before);
@@ -1166,7 +1166,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
     const uint32_t need = k - above_total;                              // picks inside the bin, 1..n2
     // certain picks (bins above the threshold bin) in the groups before this one: requested now,
     // summed when the bin's list has been requested as well
-    const uint32_t ab = threadIdx.x < grp ? w.gsuf[((uint64_t)b * kCoarse + jstar) * kGroups + threadIdx.x] : 0u;
+    const uint32_t ab = threadIdx.x < grp ? w.gsuf[(((uint64_t)b * kCoarse + jstar) << g.gshift) + threadIdx.x] : 0u;
     if (n2 > g.lcapb) {  // more keys in the threshold bin than its list holds (heavy ties, clustered values)
         failed = true;
         break;
@@ -1356,9 +1356,9 @@ uint64_t zeroed_words(const Geometry& g) {
 }
 
 uint64_t workspace_words(const Geometry& g) {
-    return zeroed_words(g) + 2 * align4((uint64_t)g.nbuckets * g.tiles) + 2 * align4((uint64_t)g.nbuckets * kGroups) +
+    return zeroed_words(g) + 2 * align4((uint64_t)g.nbuckets * g.tiles) + 2 * align4((uint64_t)g.nbuckets << g.gshift) +
            align4((uint64_t)g.nbuckets * g.ftiles) + align4((uint64_t)g.nbuckets * g.ftiles * kTileSlots * 2) +
-           align4((uint64_t)g.nbuckets * kGroups * kCntStride) + align4((uint64_t)g.nbuckets * kCoarse * kGroups) +
+           align4(((uint64_t)g.nbuckets << g.gshift) * kCntStride) + align4(((uint64_t)g.nbuckets << g.gshift) * kCoarse) +
            align4((uint64_t)g.nbuckets * kCoarse) + align4((uint64_t)g.nbuckets * (kCoarse - 1) * g.lcapb * 2);
 }
 
@@ -1369,12 +1369,12 @@ Workspace carve(void* base, const Geometry& g) {
     w.state = p;       p += align4((uint64_t)g.nbuckets * kStateWords);
     w.tile_gt = p;     p += align4((uint64_t)g.nbuckets * g.tiles);
     w.tile_eq = p;     p += align4((uint64_t)g.nbuckets * g.tiles);
-    w.blk_above = p;   p += align4((uint64_t)g.nbuckets * kGroups);
-    w.blk_eq = p;      p += align4((uint64_t)g.nbuckets * kGroups);
+    w.blk_above = p;   p += align4((uint64_t)g.nbuckets << g.gshift);
+    w.blk_eq = p;      p += align4((uint64_t)g.nbuckets << g.gshift);
     w.tile_cnt = p;    p += align4((uint64_t)g.nbuckets * g.ftiles);
     w.slots = (uint64_t*)p;  p += align4((uint64_t)g.nbuckets * g.ftiles * kTileSlots * 2);
-    w.grp_cnt = p;     p += align4((uint64_t)g.nbuckets * kGroups * kCntStride);
-    w.gsuf = p;       p += align4((uint64_t)g.nbuckets * kGroups * kCoarse);
+    w.grp_cnt = p;     p += align4(((uint64_t)g.nbuckets << g.gshift) * kCntStride);
+    w.gsuf = p;       p += align4(((uint64_t)g.nbuckets << g.gshift) * kCoarse);
     w.bin_fill = p;    p += align4((uint64_t)g.nbuckets * kCoarse);
     w.blist = (uint64_t*)p;
     // The resident path's scratch lies where the streaming path has its lists: a call takes one of the two.
@@ -1401,6 +1401,7 @@ bool make_geometry(uint64_t n_total, uint64_t bucket_elems, double ratio, Geomet
     g->k_last = mccl_hip_topk_k(n_total - (nb - 1) * bucket_elems, ratio);
     g->listed = 0;
     g->ftiles = (uint32_t)((bucket_elems + kFTile - 1) / kFTile);
+    g->gshift = topk_group_shift(g->ftiles);
     // a coarse bin holds about k / 80 candidates when the window is as wide as a sample of 8192
     // leaves it, the bins at the window's lower end three times that; k / 10 + 2048 entries
     // leave room for more uneven ones
@@ -1423,8 +1424,8 @@ uint32_t next_epoch() {
 
 // The two launches of the single-pass path.
 void launch_single_pass(const Buckets& bk, const Geometry& g, const Workspace& w, hipStream_t st) {
-    // the streaming launch: a sample block per bucket, then per bucket its tiles and 64 bin blocks
-    const uint64_t blocks = (uint64_t)g.nbuckets * ((uint64_t)g.ftiles + kGroups + 1) + kGroups;
+    // the streaming launch: a sample block per bucket, then per bucket its tiles and bin blocks
+    const uint64_t blocks = (uint64_t)g.nbuckets * ((uint64_t)g.ftiles + (1u << g.gshift) + 1) + (1u << g.gshift);
     const uint32_t epoch = next_epoch();
     // 100 MHz ticks a block may wait before it gives up
     const uint64_t lim = (uint64_t)tuning().topk_barrier_ms * 100000ull;
@@ -1438,11 +1439,12 @@ void launch_single_pass(const Buckets& bk, const Geometry& g, const Workspace& w
     // (tests of the give-up path: the sample blocks publish a number nobody waits for)
     const uint32_t published = tuning().topk_stall_test ? ~epoch : epoch;
     k_topk_stream<<<(uint32_t)blocks, kBlock, 0, st>>>(bk, g, w, epoch, published, first_wave, lim);
-    // the select launch, at most kSelBuckets buckets at a time: all its blocks are resident
+    // the select launch, at most kSelBlocks blocks at a time: all of them are resident
     // together, whatever the order in which the hardware dispatches them
-    for (uint32_t b0 = 0; b0 < g.nbuckets; b0 += kSelBuckets) {
-        const uint32_t nb = g.nbuckets - b0 < (uint32_t)kSelBuckets ? g.nbuckets - b0 : (uint32_t)kSelBuckets;
-        k_topk_select<<<dim3(kGroups, nb), kBlock, 0, st>>>(bk, g, w, b0, lim);
+    const uint32_t at_once = kSelBlocks >> g.gshift;
+    for (uint32_t b0 = 0; b0 < g.nbuckets; b0 += at_once) {
+        const uint32_t nb = g.nbuckets - b0 < at_once ? g.nbuckets - b0 : at_once;
+        k_topk_select<<<dim3(1u << g.gshift, nb), kBlock, 0, st>>>(bk, g, w, b0, lim);
     }
 }
 

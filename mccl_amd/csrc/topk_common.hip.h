@@ -54,6 +54,7 @@ struct Geometry {
     uint32_t k_last;   // k of the last bucket
     uint32_t listed;   // single-pass path: 1 when the buckets are separate buffers (see Buckets)
     uint32_t ftiles;   // single-pass path: streaming tiles allotted per bucket
+    uint32_t gshift;   // single-pass path: at most 1 << gshift groups of tiles per bucket
     uint32_t lcapb;    // single-pass path: capacity of one coarse bin's list (entries)
 };
 
@@ -64,13 +65,13 @@ struct Workspace {
     // scratch, written before read
     uint32_t* tile_gt;      // [nbuckets][tiles]
     uint32_t* tile_eq;      // [nbuckets][tiles]
-    uint32_t* blk_above;    // [nbuckets][64] exact selection inside the select launch: keys above the threshold per group
-    uint32_t* blk_eq;       // [nbuckets][64] ... keys equal to the threshold per group
+    uint32_t* blk_above;    // [nbuckets][groups] exact selection inside the select launch: keys above the threshold per group
+    uint32_t* blk_eq;       // [nbuckets][groups] ... keys equal to the threshold per group
     // single-pass path
     uint32_t* tile_cnt;     // [nbuckets][ftiles] candidates in the tile's slots, or kDense
     uint64_t* slots;        // [nbuckets][ftiles][128] (bits << 32) | index, index order
-    uint32_t* grp_cnt;      // [nbuckets][64][kCntStride] finished tiles per group (first word of each 256 bytes)
-    uint32_t* gsuf;         // [nbuckets][128 bins][64 groups] a group's candidates in the bins above bin j
+    uint32_t* grp_cnt;      // [nbuckets][groups][kCntStride] finished tiles per group (first word of each 256 bytes)
+    uint32_t* gsuf;         // [nbuckets][128 bins][groups] a group's candidates in the bins above bin j
     uint32_t* bin_fill;     // [nbuckets][128] the bucket's candidates per coarse window bin (= entries of the bin's list)
     uint64_t* blist;        // [nbuckets][63][lcapb] the window's candidates by coarse bin, any order
     uint32_t* rmem;         // [nbuckets][kRWords] resident path

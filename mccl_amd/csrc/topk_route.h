@@ -12,11 +12,17 @@ enum Path { kPathExact, kPathStream, kPathResident };
 constexpr int kFSample = 8192;              // sampled elements per bucket
 constexpr uint64_t kFTile = 4096;           // single-pass path: elements per streaming block
 constexpr int kTileSlots = 128;             // ... candidate slots per tile
-constexpr int kGroups = 64;                 // ... at most this many groups of tiles per bucket
+constexpr uint32_t kMaxGroups = 1u << 8;    // ... at most this many groups of tiles per bucket
 constexpr uint64_t kFastMinBucket = 1u << 18;
 constexpr uint64_t kRMaxBlocks = 128;       // resident path: blocks of one bucket
 constexpr uint64_t kRVecElems = 4096;       // ... elements per block and vector of a thread
 constexpr uint64_t kRMaxBucket = kRMaxBlocks * kRVecElems * 4;  // 2,097,152 elements
+
+// Groups of tiles per bucket, the power of two: 64 groups, more for buckets that would have more than 28
+// tiles in each: so many a bin or select block keeps in registers, the others it reads again on every
+// pass.  us per call at 1 %, 64 groups against this rule: one bucket of 10 M elements 58 / 47, of 13.1 M 72 / 54, of
+// 26.2 M 136 / 89.
+constexpr uint32_t topk_group_shift(uint64_t tiles) { return tiles <= 64 * 28 ? 6 : tiles <= 128 * 28 ? 7 : 8; }
 
 // The buckets of a call: consecutive ranges of bucket_elems elements, the last one shorter, or, with
 // counts, nbuckets buffers of those lengths, bucket_elems the longest.
@@ -102,7 +108,7 @@ struct Route {
 //     latency: 12 x 2 M 249 exact, 230 streaming, 50 x 1.7 M 782 and 725, 14 x 6.5 M 905 and 826.
 inline Route choose_path(const TopkCall& c, int forced, uint64_t limit) {
     const uint64_t tiles = (c.bucket_elems + kFTile - 1) / kFTile;
-    const bool streams = (uint64_t)c.nbuckets * (tiles + kGroups + 1) + kGroups < 0x7FFFFFFFull;
+    const bool streams = (uint64_t)c.nbuckets * (tiles + kMaxGroups + 1) + kMaxGroups < 0x7FFFFFFFull;
     if (forced == 1 && !c.counts) return {kPathExact, 0};
     if (forced == 2 && streams) return {kPathStream, 0};
     // expected share of a bucket inside the sampled window (see sample_window)
