@@ -451,14 +451,22 @@ __global__ __launch_bounds__(kBlock) void k_topk_emit(float* residual, Geometry 
 // its stores' acknowledgements before it signals.
 
 constexpr int kFRegion = 1024;                // elements one wavefront streams
-constexpr int kFWaves = kBlock / kWave;       // 4
-static_assert(kFTile == kFRegion * kFWaves, "elements per streaming block");
+constexpr int kFWaves = 4;                    // wavefronts of a tile
+static_assert(kFTile == kFRegion * kFWaves, "elements per streaming tile");
+// The streaming launch's blocks have 256 threads or 512 (THREADS), a streaming block a tile for every 256.
+template <int THREADS>
+struct StreamShape {
+    static constexpr int kWaves = THREADS / kWave;
+    static constexpr uint32_t kTiles = kWaves / kFWaves;       // of a streaming block
+    static constexpr int kHeld = kTiles == 1 ? 7 : 4;          // tiles per wavefront whose slots a bin block keeps in registers
+    static constexpr int kPerSimd = kTiles == 1 ? 6 : 8;       // wavefronts that the registers are to leave room for
+};
 constexpr int kFVecs = kFRegion / (kWave * 4);  // 16-byte vectors per lane and array: all issued at once
 constexpr int kCoarse = 128;                  // coarse window bins; the last one holds keys >= hi
 constexpr int kBinsPerLane = kCoarse / kWave; // 2
 constexpr int kCntStride = 64;                // words between two groups' arrival counters: 256 bytes, so that the
                                               // arrivals of a bucket's tiles spread over memory channels
-constexpr int kHeld = 7;                      // tiles per wavefront whose slots a bin / select block keeps in registers
+constexpr int kHeld = 7;                      // tiles per wavefront whose slots a select block keeps in registers
 constexpr uint32_t kSelBlocks = 1024;         // blocks of a k_topk_select launch: all resident
 constexpr uint32_t kGaveUp = 0xFFFFFFFEu;     // a wavefront's count: its wait for the sample timed out
 static_assert(kFVecs == 4, "the streaming role is written for four vectors per lane");
@@ -516,16 +524,18 @@ __device__ __forceinline__ bool wait_word(const uint32_t* p, uint32_t want, uint
     return true;
 }
 
+template <int THREADS>
 struct StreamLds {
+    static constexpr int kWaves = StreamShape<THREADS>::kWaves;
     union {
-        SampleLds<kBlock> s;  // sample block
+        SampleLds<THREADS> s;  // sample block
         struct {  // streaming block
-            uint64_t stage[kFWaves][kWave];  // a wavefront's candidates, (bits << 32) | index, in index order
-            uint32_t wcnt[kFWaves];
+            uint64_t stage[kWaves][kWave];  // a wavefront's candidates, (bits << 32) | index, in index order
+            uint32_t wcnt[kWaves];
             uint32_t win[4];                 // the bucket's window as wavefront 0 read it: lo, hi, predicted threshold, ready
         } a;
         struct {  // bin block
-            uint32_t dbuf[kFWaves][16 * kWave];  // dense_tile_walk's staging area, one per wavefront
+            uint32_t dbuf[kWaves][16 * kWave];  // dense_tile_walk's staging area, one per wavefront
             uint32_t cnt[kCoarse];
             uint32_t base[kCoarse];
             uint32_t win[4];
@@ -545,11 +555,12 @@ struct SelectLds {
 
 // The bucket's candidate window; clears what the launches accumulate into, then publishes the
 // window and the epoch with one store.
+template <int THREADS>
 __device__ __forceinline__ void fused_sample(BucketsArg bk, const Geometry& g, const Workspace& w, uint32_t b,
-                                             uint32_t epoch, StreamLds& L) {
+                                             uint32_t epoch, StreamLds<THREADS>& L) {
     const FusedGeo fg = fused_geo(g, bk, b);
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
-    const SampleWindow win = sample_window<kBlock>(bucket_grad(g, bk, b), bucket_residual(g, bk, b), fg.bn, fg.k, L.s, [&] {
+    const SampleWindow win = sample_window<THREADS>(bucket_grad(g, bk, b), bucket_residual(g, bk, b), fg.bn, fg.k, L.s, [&] {
         // (the acknowledgements are back long before the window is published)
         if (threadIdx.x >> g.gshift == 0) st_agent(w.grp_cnt + (((uint64_t)b << g.gshift) + threadIdx.x) * kCntStride, 0u);
         if (threadIdx.x < kCoarse) st_agent(w.bin_fill + (uint64_t)b * kCoarse + threadIdx.x, 0u);
@@ -565,7 +576,7 @@ __device__ __forceinline__ void fused_sample(BucketsArg bk, const Geometry& g, c
         store16_agent(st + S_LO_KEY, u4a{win.lo, win.hi, win.that, epoch});
     }
     // off the critical path: the histograms of the exact selection, should the select launch need it
-    for (int i = threadIdx.x; i < kHistWords; i += kBlock) w.hist[(uint64_t)b * kHistWords + i] = 0u;
+    for (int i = threadIdx.x; i < kHistWords; i += THREADS) w.hist[(uint64_t)b * kHistWords + i] = 0u;
 }
 
 // ---- a dense tile's elements ---------------------------------------------------------
@@ -599,11 +610,12 @@ __device__ __forceinline__ void dense_tile_walk(const float* rp, uint64_t bn, ui
 }
 
 // ---- a group's tiles as a bin block / select block sees them ------------------------------
-// The slots of up to kHeld tiles per wavefront stay in registers, the rest (buckets of more
-// than 64 * 4 * kHeld tiles) are re-read from memory on every sweep.  AGENT: the slots were
+// The slots of up to HELD tiles per wavefront stay in registers, the rest (buckets of more
+// than 64 * NW * HELD tiles) are re-read from memory on every sweep.  AGENT: the slots were
 // written by other blocks of the same launch (agent-scope loads), else by an earlier launch.
-template <bool AGENT>
+template <bool AGENT, int NW, int HELD>
 struct GroupTiles {
+    static constexpr int kHeld = HELD;
     const uint32_t* tcnt;
     const uint64_t* slots;
     uint32_t t0;        // the group's first tile
@@ -624,7 +636,6 @@ struct GroupTiles {
     // every load issued at once
     __device__ __forceinline__ void load(const Geometry& g, const Workspace& w, uint32_t b, uint32_t grp,
                                          const FusedGeo& fg) {
-        constexpr int NW = kBlock / kWave;
         lane = threadIdx.x & (kWave - 1);
         const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
         tcnt = w.tile_cnt + (uint64_t)b * g.ftiles;
@@ -673,9 +684,10 @@ struct GroupTiles {
 __device__ __forceinline__ uint32_t key64(uint64_t e) { return (uint32_t)(e >> 32) & 0x7FFFFFFFu; }
 
 // ---- bin block -----------------------------------------------------------------------------
+template <int THREADS>
 __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, const Workspace& w, uint32_t b,
                                           uint32_t grp, const FusedGeo& fg, uint32_t epoch, uint64_t limit_ticks,
-                                          StreamLds& L) {
+                                          StreamLds<THREADS>& L) {
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
     // the group's tiles are finished: all its streaming blocks have arrived
     {
@@ -698,11 +710,11 @@ __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, cons
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const float* rp = bucket_residual(g, bk, b);
-    GroupTiles<true> G;
+    GroupTiles<true, StreamShape<THREADS>::kWaves, StreamShape<THREADS>::kHeld> G;
     G.load(g, w, b, grp, fg);
     // candidates per coarse bin
     if (threadIdx.x < kCoarse) L.e.cnt[threadIdx.x] = 0;
-    static_assert(kCoarse <= kBlock, "one thread per coarse bin");
+    static_assert(kCoarse <= THREADS, "one thread per coarse bin");
     __syncthreads();
     G.sweep([&](uint32_t, uint32_t, uint32_t cnt, uint64_t a0, uint64_t a1) {
                 if ((uint32_t)lane < cnt) atomicAdd(&L.e.cnt[coarse_bin(key64(a0), lo, hi, wmul)], 1u);
@@ -756,19 +768,22 @@ __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, cons
 }
 
 // ---- the streaming launch ------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock, 6) void k_topk_stream(Buckets, Geometry g, Workspace w, uint32_t epoch,
+template <int THREADS>
+__global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_topk_stream(Buckets, Geometry g, Workspace w, uint32_t epoch,
                                                         uint32_t published, uint32_t first_wave,
                                                         uint64_t limit_ticks) {
     const BucketsArg bk = buckets_arg();
-    __shared__ StreamLds L;
+    constexpr uint32_t kTiles = StreamShape<THREADS>::kTiles;
+    __shared__ StreamLds<THREADS> L;
     if (blockIdx.x < g.nbuckets) {
-        fused_sample(bk, g, w, blockIdx.x, published, L);
+        fused_sample<THREADS>(bk, g, w, blockIdx.x, published, L);
         return;
     }
     // segment s of the grid: the tiles of bucket s, then the bin blocks of bucket s - 1 (whose
     // tiles are finished or about to be by then: a bin block that is dispatched early only
     // polls); after the last segment the bin blocks of the last bucket
-    const uint32_t per = g.ftiles + (1u << g.gshift);
+    const uint32_t sblocks = (g.ftiles + kTiles - 1) / kTiles;
+    const uint32_t per = sblocks + (1u << g.gshift);
     const uint32_t j = blockIdx.x - g.nbuckets;
     uint32_t b = j / per, t = j - b * per;
     bool emit = false;
@@ -776,18 +791,18 @@ __global__ __launch_bounds__(kBlock, 6) void k_topk_stream(Buckets, Geometry g, 
         t = j - g.nbuckets * per;
         b = g.nbuckets - 1;
         emit = true;
-    } else if (t >= g.ftiles) {
+    } else if (t >= sblocks) {
         if (b == 0) return;
-        t -= g.ftiles;
+        t -= sblocks;
         b -= 1;
         emit = true;
     }
     const FusedGeo fg = fused_geo(g, bk, b);
     if (emit) {
-        if (t < fg.ng) fused_bin(bk, g, w, b, t, fg, epoch, limit_ticks, L);
+        if (t < fg.ng) fused_bin<THREADS>(bk, g, w, b, t, fg, epoch, limit_ticks, L);
         return;
     }
-    if (t >= fg.ntiles) return;
+    if (t * kTiles >= fg.ntiles) return;
     // The blocks that start together with the sample blocks would bury the samples' few loads under
     // 40 MB of their own and then wait for the samples all the same: they hold back for two
     // microseconds, and the memory system is busy with their loads while the samples are evaluated.
@@ -795,7 +810,9 @@ __global__ __launch_bounds__(kBlock, 6) void k_topk_stream(Buckets, Geometry g, 
     const uint64_t bn = fg.bn;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-    const uint64_t w0 = (uint64_t)t * kFTile + (uint64_t)wave * kFRegion;  // first element of this wave's region
+    const int first_wave_of_tile = wave / kFWaves * kFWaves;
+    t = t * kTiles + (uint32_t)(wave / kFWaves);  // the wavefront's tile
+    const uint64_t w0 = (uint64_t)t * kFTile + (uint64_t)(wave - first_wave_of_tile) * kFRegion;  // first element of this wave's region
     const bool live = w0 < bn;                                             // wave-uniform
     float* const rbase = bucket_residual(g, bk, b);
     const float* gp = bucket_grad(g, bk, b) + w0;
@@ -925,10 +942,10 @@ __global__ __launch_bounds__(kBlock, 6) void k_topk_stream(Buckets, Geometry g, 
     bool tile_dense = false, gave_up = false;
 #pragma unroll
     for (int i = 0; i < kFWaves; i++) {
-        const uint32_t c = L.a.wcnt[i];
+        const uint32_t c = L.a.wcnt[first_wave_of_tile + i];
         gave_up |= c == kGaveUp;
         tile_dense |= c == kDense;
-        if (i < wave) before += c;
+        if (first_wave_of_tile + i < wave) before += c;
         total += c;
     }
     if (gave_up) {  // a wavefront never saw the sample arrive: the bucket's result is invalid
@@ -941,11 +958,12 @@ __global__ __launch_bounds__(kBlock, 6) void k_topk_stream(Buckets, Geometry g, 
     } else if ((uint32_t)lane < staged) {
         st_agent64(w.slots + ((uint64_t)b * g.ftiles + t) * kTileSlots + before + lane, slots[lane]);
     }
-    if (threadIdx.x == 0) st_agent(w.tile_cnt + (uint64_t)b * g.ftiles + t, tile_dense ? kDense : total);
+    const bool counts = wave == first_wave_of_tile && lane == 0 && t < fg.ntiles;
+    if (counts) st_agent(w.tile_cnt + (uint64_t)b * g.ftiles + t, tile_dense ? kDense : total);
     // ---- the block counts itself into its group once all its stores have arrived ----------
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0)
+    if (counts)
         __hip_atomic_fetch_add(w.grp_cnt + (((uint64_t)b << g.gshift) + t / fg.tpg) * kCntStride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -983,7 +1001,7 @@ __device__ __forceinline__ uint32_t resolve_ties64(ForList&& for_list, uint32_t 
 // element range; four barriers.  Returns false when a barrier wait timed out.
 __device__ __forceinline__ bool select_exact_group(BucketsArg bk, const Geometry& g, const Workspace& w, uint32_t b,
                                                    uint32_t grp, const FusedGeo& fg, uint32_t that_key,
-                                                   const GroupTiles<false>& G, SelectLds& L, uint64_t limit_ticks) {
+                                                   const GroupTiles<false, kFWaves, kHeld>& G, SelectLds& L, uint64_t limit_ticks) {
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
     const uint64_t bn = fg.bn;
     float* rp = bucket_residual(g, bk, b);
@@ -1130,7 +1148,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
     static_assert(kBinsPerLane == 2, "a lane owns two neighbouring bins");
     // scanned from the top bin downwards: lane l looks at bins 127 - 2 l (tot[1]) and 126 - 2 l (tot[0])
     const u2a tot = *(const u2a*)(w.bin_fill + (uint64_t)b * kCoarse + kCoarse - 2 - 2 * (threadIdx.x & (kWave - 1)));
-    GroupTiles<false> G;
+    GroupTiles<false, kFWaves, kHeld> G;
     G.load(g, w, b, grp, fg);
     // a replay of a captured launch carries the same epoch: also behind a run that was given up
     if (grp == 0 && threadIdx.x == 0) st[S_READY] = 0u;
@@ -1423,22 +1441,30 @@ uint32_t next_epoch() {
 }
 
 // The two launches of the single-pass path.
-void launch_single_pass(const Buckets& bk, const Geometry& g, const Workspace& w, hipStream_t st) {
-    // the streaming launch: a sample block per bucket, then per bucket its tiles and bin blocks
-    const uint64_t blocks = (uint64_t)g.nbuckets * ((uint64_t)g.ftiles + (1u << g.gshift) + 1) + (1u << g.gshift);
+template <int THREADS>
+void launch_stream(const Buckets& bk, const Geometry& g, const Workspace& w, uint64_t limit_ticks, hipStream_t st) {
+    // a sample block per bucket, then per bucket its tiles and its bin blocks
+    constexpr uint32_t per = StreamShape<THREADS>::kTiles;
+    const uint64_t blocks = (uint64_t)g.nbuckets * ((g.ftiles + per - 1) / per + (1u << g.gshift) + 1) + (1u << g.gshift);
     const uint32_t epoch = next_epoch();
-    // 100 MHz ticks a block may wait before it gives up
-    const uint64_t lim = (uint64_t)tuning().topk_barrier_ms * 100000ull;
     // blocks that are resident from the start of the launch: they wait for the sample blocks
     static const int per_cu = [] {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_topk_stream, kBlock, 0) != hipSuccess || n < 1) n = 6;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_topk_stream<THREADS>, THREADS, 0) != hipSuccess || n < 1)
+            n = StreamShape<THREADS>::kPerSimd * 4 * kWave / THREADS;
         return n;
     }();
     const uint32_t first_wave = g.nbuckets + (uint32_t)device_info().num_cus * (uint32_t)per_cu;
     // (tests of the give-up path: the sample blocks publish a number nobody waits for)
     const uint32_t published = tuning().topk_stall_test ? ~epoch : epoch;
-    k_topk_stream<<<(uint32_t)blocks, kBlock, 0, st>>>(bk, g, w, epoch, published, first_wave, lim);
+    k_topk_stream<THREADS><<<(uint32_t)blocks, THREADS, 0, st>>>(bk, g, w, epoch, published, first_wave, limit_ticks);
+}
+
+void launch_single_pass(const Buckets& bk, const Geometry& g, const Workspace& w, hipStream_t st) {
+    // 100 MHz ticks a block may wait before it gives up
+    const uint64_t lim = (uint64_t)tuning().topk_barrier_ms * 100000ull;
+    if (stream_wide((uint64_t)g.nbuckets * g.ftiles)) launch_stream<512>(bk, g, w, lim, st);
+    else launch_stream<256>(bk, g, w, lim, st);
     // the select launch, at most kSelBlocks blocks at a time: all of them are resident
     // together, whatever the order in which the hardware dispatches them
     const uint32_t at_once = kSelBlocks >> g.gshift;

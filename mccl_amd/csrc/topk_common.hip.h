@@ -241,7 +241,7 @@ __device__ __forceinline__ u4a wait_window(const uint32_t* st, uint32_t epoch, u
 // exponents, and lanes that add to one LDS word take turns (8192 keys: 1.6 to 2.4 us with one copy).
 template <int THREADS>
 struct SampleLds {
-    static constexpr int kCopies = THREADS >= 1024 ? 4 : 1;
+    static constexpr int kCopies = THREADS >= 1024 ? 4 : THREADS >= 512 ? 2 : 1;
     static constexpr int kCopy = kBins0 + 8;  // words
     uint32_t h0[kCopies * kCopy] __attribute__((aligned(16)));
     uint32_t lh[3][kBinsR] __attribute__((aligned(16)));

@@ -12,6 +12,7 @@ enum Path { kPathExact, kPathStream, kPathResident };
 constexpr int kFSample = 8192;              // sampled elements per bucket
 constexpr uint64_t kFTile = 4096;           // single-pass path: elements per streaming block
 constexpr int kTileSlots = 128;             // ... candidate slots per tile
+constexpr uint64_t kWideTiles = 6144;       // ... a launch of at most this many has blocks of 512 threads
 constexpr uint32_t kMaxGroups = 1u << 8;    // ... at most this many groups of tiles per bucket
 constexpr uint64_t kFastMinBucket = 1u << 18;
 constexpr uint64_t kRMaxBlocks = 128;       // resident path: blocks of one bucket
@@ -23,6 +24,14 @@ constexpr uint64_t kRMaxBucket = kRMaxBlocks * kRVecElems * 4;  // 2,097,152 ele
 // pass.  us per call at 1 %, 64 groups against this rule: one bucket of 10 M elements 58 / 47, of 13.1 M 72 / 54, of
 // 26.2 M 136 / 89.
 constexpr uint32_t topk_group_shift(uint64_t tiles) { return tiles <= 64 * 28 ? 6 : tiles <= 128 * 28 ? 7 : 8; }
+
+// Whether the blocks of a streaming launch over that many tiles have 512 threads instead of 256.  Their sample
+// is evaluated sooner, and 2048 tiles are resident instead of 1536 (a bucket of 6,553,600 elements has 1600: a
+// second round of 64 tiles took as long as half the first); where many rounds follow each other, slots that are
+// given back 256 threads at a time are filled sooner.  us per call at 1 %, 256 threads against 512: one bucket of 2.5 M
+// elements 30.1 / 28.8, of 6,553,600 38.6 / 36.2, of 10 M 48.0 / 47.3, two of 6,553,600 52.4 / 52.5, four 80.2 / 79.7,
+// 24 of 1.7 M 119.1 / 120.4, four of 13.1 M 133 / 138, 15 of 6,553,600 216.6 / 221.3.
+constexpr bool stream_wide(uint64_t tiles) { return tiles <= kWideTiles; }
 
 // The buckets of a call: consecutive ranges of bucket_elems elements, the last one shorter, or, with
 // counts, nbuckets buffers of those lengths, bucket_elems the longest.

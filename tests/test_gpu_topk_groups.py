@@ -45,3 +45,26 @@ def test_fallback_with_more_than_64_groups():
     assert ops.topk_path_report(ws, n, n, 0.01) == (0, 1)
     assert wire.cpu().numpy()[:size].tobytes() == want.tobytes()
     assert np.array_equal(bits(to_np(dres, F32)), bits(res))
+
+
+@pytest.mark.parametrize("n, bucket", [(3 * TILE, 3 * TILE), (TILE + 1, TILE + 1), (2_000_003, 500_001),
+                                       (24_576_000 - 4096, 6_144_000), (24_576_001, 6_144_000)])
+def test_blocks_of_one_or_two_tiles(n, bucket):
+    """Odd numbers of tiles, and both sides of the number (6144) up to which a streaming block has two."""
+    from mccl_amd import hip_ops as ops
+    rng = np.random.default_rng(n)
+    grad = student_t(rng, n, ties=0.01)
+    res = (rng.standard_normal(n) * 1e-4).astype(np.float32)
+    dres = to_dev(res, F32)
+    try:
+        ops.set_tuning("topk_path", 2)
+        wire, stride = ops.topk_compress(to_dev(grad, F32), dres, 0.01, bucket_elems=bucket)
+    finally:
+        ops.set_tuning("topk_path", 0)
+    w = wire.cpu().numpy()
+    for b, lo in enumerate(range(0, n, bucket)):
+        part = res[lo:lo + bucket].copy()
+        want, size = oracle.topk_compress(grad[lo:lo + bucket], part, 0.01)
+        res[lo:lo + bucket] = part
+        assert w[b * stride: b * stride + size].tobytes() == want.tobytes(), b
+    assert np.array_equal(bits(to_np(dres, F32)), bits(res))
