@@ -400,6 +400,9 @@ __global__ __launch_bounds__(kBlock) void k_topk_emit(float* residual, Geometry 
 //                   publishes the call's epoch number in S_READY.
 //   then, segment by segment (segment s = the tiles of bucket s, then the bin blocks of
 //   bucket s - 1; the bin blocks of the last bucket close the grid):
+//   (The buckets of a list go longest first, each with the blocks it has.  24 buckets of 1001 to 1.5 M elements,
+//   5.5 M together, 1 %: as many blocks for each as for the longest, streaming blocks and select launches chosen by
+//   that number, 50.5 us; so, 37.6.)
 //   streaming blocks one per 4096-element tile, in address order.  A wavefront loads its
 //                   1024 elements, waits until the bucket's S_READY shows the epoch, stores
 //                   residual <- grad + residual (0.0f at or above the predicted threshold)
@@ -495,7 +498,7 @@ __device__ __forceinline__ FusedGeo fused_geo(const Geometry& g, BucketsArg bk, 
     f.bn = bucket_count(g, bk, b);
     f.k = bucket_k(g, bk, b);
     f.ntiles = (uint32_t)((f.bn + kFTile - 1) / kFTile);
-    f.tpg = (f.ntiles + (1u << g.gshift) - 1) >> g.gshift;
+    f.tpg = topk_group_tiles(f.ntiles, g.gshift);
     f.ng = (f.ntiles + f.tpg - 1) / f.tpg;
     return f;
 }
@@ -768,10 +771,13 @@ __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, cons
 }
 
 // ---- the streaming launch ------------------------------------------------------------------
-template <int THREADS>
+// LISTED: the call's buckets are a list (g.listed), known to the compiler: a block finds its work before it can
+// load, and one kernel for both layouts kept 13 more scalar registers in vector lanes (the 96.5 M gradient 2.5 us).
+template <int THREADS, bool LISTED>
 __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_topk_stream(Buckets, Geometry g, Workspace w, uint32_t epoch,
                                                         uint32_t published, uint32_t first_wave,
                                                         uint64_t limit_ticks) {
+    g.listed = LISTED;
     const BucketsArg bk = buckets_arg();
     constexpr uint32_t kTiles = StreamShape<THREADS>::kTiles;
     __shared__ StreamLds<THREADS> L;
@@ -782,20 +788,36 @@ __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_top
     // segment s of the grid: the tiles of bucket s, then the bin blocks of bucket s - 1 (whose
     // tiles are finished or about to be by then: a bin block that is dispatched early only
     // polls); after the last segment the bin blocks of the last bucket
-    const uint32_t sblocks = (g.ftiles + kTiles - 1) / kTiles;
-    const uint32_t per = sblocks + (1u << g.gshift);
     const uint32_t j = blockIdx.x - g.nbuckets;
-    uint32_t b = j / per, t = j - b * per;
+    uint32_t b, t;
     bool emit = false;
-    if (b >= g.nbuckets) {
-        t = j - g.nbuckets * per;
-        b = g.nbuckets - 1;
-        emit = true;
-    } else if (t >= sblocks) {
-        if (b == 0) return;
-        t -= sblocks;
-        b -= 1;
-        emit = true;
+    if constexpr (LISTED) {
+        b = listed_bucket(bk, j, &t);
+        const uint32_t sblocks = (topk_tiles(bk->lcount[b]) + kTiles - 1) / kTiles;
+        if (t >= sblocks) {
+            t -= sblocks;
+            emit = true;
+            if (b) {
+                const uint32_t before = topk_groups(topk_tiles(bk->lcount[b - 1]), g.gshift);
+                if (t < before) b -= 1;
+                else t -= before;
+            }
+        }
+    } else {
+        const uint32_t sblocks = (g.ftiles + kTiles - 1) / kTiles;
+        const uint32_t per = sblocks + g.ngroups;
+        b = j / per;
+        t = j - b * per;
+        if (b >= g.nbuckets) {
+            t = j - g.nbuckets * per;
+            b = g.nbuckets - 1;
+            emit = true;
+        } else if (t >= sblocks) {
+            if (b == 0) return;
+            t -= sblocks;
+            b -= 1;
+            emit = true;
+        }
     }
     const FusedGeo fg = fused_geo(g, bk, b);
     if (emit) {
@@ -1129,13 +1151,17 @@ __device__ __forceinline__ bool select_exact_group(BucketsArg bk, const Geometry
 
 
 // ---- the select launch ----------------------------------------------------------------------
-// blockIdx.x = group, blockIdx.y = bucket - first_bucket.  Everything the streaming launch
+// blockIdx.x = group, blockIdx.y = bucket - first_bucket; of a list, blocks of all its buckets in a row
+// (Buckets::lfirst).  Everything the streaming launch
 // left behind is read with plain loads; only the exact fallback talks across blocks.
+template <bool LISTED>
 __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, Workspace w, uint32_t first_bucket,
                                                            uint64_t limit_ticks) {
+    g.listed = LISTED;
     const BucketsArg bk = buckets_arg();
     __shared__ SelectLds L;
-    const uint32_t b = first_bucket + blockIdx.y, grp = blockIdx.x;
+    uint32_t b = first_bucket + blockIdx.y, grp = blockIdx.x;
+    if (g.listed) b = listed_bucket(bk, blockIdx.x, &grp);
     const FusedGeo fg = fused_geo(g, bk, b);
     if (grp >= fg.ng) return;
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
@@ -1420,6 +1446,7 @@ bool make_geometry(uint64_t n_total, uint64_t bucket_elems, double ratio, Geomet
     g->listed = 0;
     g->ftiles = (uint32_t)((bucket_elems + kFTile - 1) / kFTile);
     g->gshift = topk_group_shift(g->ftiles);
+    g->ngroups = topk_groups(g->ftiles, g->gshift);
     // a coarse bin holds about k / 80 candidates when the window is as wide as a sample of 8192
     // leaves it, the bins at the window's lower end three times that; k / 10 + 2048 entries
     // leave room for more uneven ones
@@ -1441,36 +1468,82 @@ uint32_t next_epoch() {
 }
 
 // The two launches of the single-pass path.
-template <int THREADS>
-void launch_stream(const Buckets& bk, const Geometry& g, const Workspace& w, uint64_t limit_ticks, hipStream_t st) {
+template <int THREADS, bool LISTED>
+void launch_stream(Buckets& bk, const Geometry& g, const Workspace& w, uint64_t limit_ticks, hipStream_t st) {
     // a sample block per bucket, then per bucket its tiles and its bin blocks
     constexpr uint32_t per = StreamShape<THREADS>::kTiles;
-    const uint64_t blocks = (uint64_t)g.nbuckets * ((g.ftiles + per - 1) / per + (1u << g.gshift) + 1) + (1u << g.gshift);
+    uint64_t blocks = (uint64_t)g.nbuckets * ((g.ftiles + per - 1) / per + g.ngroups + 1) + g.ngroups;
+    if constexpr (LISTED) {
+        // segment b: the tiles of bucket b, then the bin blocks of bucket b - 1
+        uint32_t at = 0, before = 0;
+        for (uint32_t b = 0; b < g.nbuckets; b++) {
+            const uint32_t tiles = topk_tiles(bk.lcount[b]);
+            bk.lfirst[b] = at;
+            at += (tiles + per - 1) / per + before;
+            before = topk_groups(tiles, g.gshift);
+        }
+        blocks = g.nbuckets + at + before;
+    }
     const uint32_t epoch = next_epoch();
     // blocks that are resident from the start of the launch: they wait for the sample blocks
     static const int per_cu = [] {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_topk_stream<THREADS>, THREADS, 0) != hipSuccess || n < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_topk_stream<THREADS, LISTED>, THREADS, 0) != hipSuccess || n < 1)
             n = StreamShape<THREADS>::kPerSimd * 4 * kWave / THREADS;
         return n;
     }();
     const uint32_t first_wave = g.nbuckets + (uint32_t)device_info().num_cus * (uint32_t)per_cu;
     // (tests of the give-up path: the sample blocks publish a number nobody waits for)
     const uint32_t published = tuning().topk_stall_test ? ~epoch : epoch;
-    k_topk_stream<THREADS><<<(uint32_t)blocks, THREADS, 0, st>>>(bk, g, w, epoch, published, first_wave, limit_ticks);
+    k_topk_stream<THREADS, LISTED><<<(uint32_t)blocks, THREADS, 0, st>>>(bk, g, w, epoch, published, first_wave, limit_ticks);
 }
 
-void launch_single_pass(const Buckets& bk, const Geometry& g, const Workspace& w, hipStream_t st) {
+void launch_single_pass(const Buckets& call, const Geometry& g, const Workspace& w, hipStream_t st) {
     // 100 MHz ticks a block may wait before it gives up
     const uint64_t lim = (uint64_t)tuning().topk_barrier_ms * 100000ull;
-    if (stream_wide((uint64_t)g.nbuckets * g.ftiles)) launch_stream<512>(bk, g, w, lim, st);
-    else launch_stream<256>(bk, g, w, lim, st);
+    // A list's blocks are those that its buckets have, longest bucket first: the bin blocks that nothing is
+    // streamed beside are those of the shortest.
+    Buckets bk = call;
+    uint64_t tiles = (uint64_t)g.nbuckets * g.ftiles;
+    if (g.listed) {
+        uint32_t order[kMaxListed];
+        longest_first(call, g.nbuckets, order);
+        tiles = 0;
+        for (uint32_t b = 0; b < g.nbuckets; b++) {
+            place_bucket(&bk, b, call, order[b], 0);
+            tiles += topk_tiles(bk.lcount[b]);
+        }
+        for (uint32_t b = g.nbuckets; b < kMaxListed; b++) bk.lfirst[b] = 0xFFFFFFFFu;
+    }
+    if (g.listed) {
+        if (stream_wide(tiles)) launch_stream<512, true>(bk, g, w, lim, st);
+        else launch_stream<256, true>(bk, g, w, lim, st);
+    } else {
+        if (stream_wide(tiles)) launch_stream<512, false>(bk, g, w, lim, st);
+        else launch_stream<256, false>(bk, g, w, lim, st);
+    }
     // the select launch, at most kSelBlocks blocks at a time: all of them are resident
     // together, whatever the order in which the hardware dispatches them
-    const uint32_t at_once = kSelBlocks >> g.gshift;
-    for (uint32_t b0 = 0; b0 < g.nbuckets; b0 += at_once) {
-        const uint32_t nb = g.nbuckets - b0 < at_once ? g.nbuckets - b0 : at_once;
-        k_topk_select<<<dim3(1u << g.gshift, nb), kBlock, 0, st>>>(bk, g, w, b0, lim);
+    if (!g.listed) {
+        const uint32_t at_once = kSelBlocks / g.ngroups;
+        for (uint32_t b0 = 0; b0 < g.nbuckets; b0 += at_once) {
+            const uint32_t nb = g.nbuckets - b0 < at_once ? g.nbuckets - b0 : at_once;
+            k_topk_select<false><<<dim3(g.ngroups, nb), kBlock, 0, st>>>(bk, g, w, b0, lim);
+        }
+        return;
+    }
+    for (uint32_t b0 = 0; b0 < g.nbuckets;) {
+        uint32_t blocks = 0, b = b0;
+        for (uint32_t i = 0; i < b0; i++) bk.lfirst[i] = 0;  // before b0, which starts there and is the last that does
+        for (; b < g.nbuckets; b++) {
+            const uint32_t groups = topk_groups(topk_tiles(bk.lcount[b]), g.gshift);
+            if (blocks + groups > kSelBlocks) break;
+            bk.lfirst[b] = blocks;
+            blocks += groups;
+        }
+        for (uint32_t i = b; i < g.nbuckets; i++) bk.lfirst[i] = 0xFFFFFFFFu;
+        k_topk_select<true><<<blocks, kBlock, 0, st>>>(bk, g, w, b0, lim);
+        b0 = b;
     }
 }
 

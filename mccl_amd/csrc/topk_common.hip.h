@@ -55,6 +55,7 @@ struct Geometry {
     uint32_t listed;   // single-pass path: 1 when the buckets are separate buffers (see Buckets)
     uint32_t ftiles;   // single-pass path: streaming tiles allotted per bucket
     uint32_t gshift;   // single-pass path: at most 1 << gshift groups of tiles per bucket
+    uint32_t ngroups;  // single-pass path: groups of a (full) bucket
     uint32_t lcapb;    // single-pass path: capacity of one coarse bin's list (entries)
 };
 
@@ -103,7 +104,7 @@ struct Buckets {
     uint8_t* lwire[kMaxListed];
     uint32_t lcount[kMaxListed];
     uint32_t lk[kMaxListed];
-    uint32_t lfirst[kMaxListed];  // resident path: the bucket's first block
+    uint32_t lfirst[kMaxListed];  // the bucket's first block in the launch; 0xFFFFFFFF past the list
 };
 // The kernels index the table by bucket number.  Indexing the by-value parameter would make
 // the compiler copy all of it to per-lane scratch memory first (2 KiB per lane, and a launch
@@ -127,7 +128,36 @@ __device__ __forceinline__ float* bucket_residual(const Geometry& g, BucketsArg 
 __device__ __forceinline__ uint32_t* bucket_wire(const Geometry& g, BucketsArg bk, uint32_t b) {
     return (uint32_t*)(g.listed ? bk->lwire[b] : bk->wire + (uint64_t)b * bk->wire_stride);
 }
+// Bucket of block j of a list's launch, and which of the bucket's blocks it is.  On the scalar unit: the
+// block's loads wait for it.
+__device__ __forceinline__ uint32_t listed_bucket(BucketsArg bk, uint32_t j, uint32_t* x) {
+    uint32_t b = 0;
+    *x = j;
+    for (uint32_t c = 0; c < kMaxListed && bk->lfirst[c] <= j; c += 16) {
+#pragma unroll
+        for (uint32_t i = 0; i < 16; i++) {
+            const uint32_t first = bk->lfirst[c + i];
+            if (first <= j) {
+                b = c + i;
+                *x = j - first;
+            }
+        }
+    }
+    return b;
+}
 
+
+// The list's buckets by length, longest first.
+void longest_first(const Buckets& bk, uint32_t nbuckets, uint32_t* order);
+// Entry i of the table `to` is entry b of `from`; its blocks start at `first`.
+inline void place_bucket(Buckets* to, uint32_t i, const Buckets& from, uint32_t b, uint32_t first) {
+    to->lgrad[i] = from.lgrad[b];
+    to->lresidual[i] = from.lresidual[b];
+    to->lwire[i] = from.lwire[b];
+    to->lcount[i] = from.lcount[b];
+    to->lk[i] = from.lk[b];
+    to->lfirst[i] = first;
+}
 
 // Blocks that may wait in one resident launch on the stream (stream_limit).
 uint64_t resident_limit_on(hipStream_t st);

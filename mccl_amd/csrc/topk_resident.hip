@@ -162,18 +162,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
     if (!lead) {
         const uint32_t j = blockIdx.x - nlead;
         if (g.listed) {
-            // on the scalar unit: the block's loads wait for it
-            b = 0;
-            for (uint32_t c = 0; c < kMaxListed && bk->lfirst[c] <= j; c += 16) {
-#pragma unroll
-                for (uint32_t i = 0; i < 16; i++) {
-                    const uint32_t first = bk->lfirst[c + i];  // 0xFFFFFFFF past the list
-                    if (first <= j) {
-                        b = c + i;
-                        x = j - first;
-                    }
-                }
-            }
+            b = listed_bucket(bk, j, &x);
         } else {
             const uint32_t per_bucket = (uint32_t)((g.bucket_elems + PER - 1) / PER);
             b = j / per_bucket;
@@ -588,20 +577,14 @@ void launch(const Buckets& bk, const Geometry& g, const Workspace& w, uint64_t l
     // Leads before all blocks, no block without a bucket: 24 buckets of 1001 to 1.5 M elements 28.5 us, in
     // the caller's order with as many blocks for each bucket as for the longest 31.1 (both as one launch).
     uint32_t order[kMaxListed];
-    for (uint32_t b = 0; b < g.nbuckets; b++) order[b] = b;
-    std::sort(order, order + g.nbuckets, [&](uint32_t p, uint32_t q) { return bk.lcount[p] != bk.lcount[q] ? bk.lcount[p] > bk.lcount[q] : p < q; });
+    longest_first(bk, g.nbuckets, order);
     for (uint32_t done = 0; done < g.nbuckets;) {
         const uint32_t taken = next_launch(bk.lcount, order + done, g.nbuckets - done, per, limit);
         Buckets part = bk;
         uint32_t nlead = 0, blocks = 0;
         for (uint32_t i = 0; i < taken; i++) {
             const uint32_t b = order[done + i];
-            part.lgrad[i] = bk.lgrad[b];
-            part.lresidual[i] = bk.lresidual[b];
-            part.lwire[i] = bk.lwire[b];
-            part.lcount[i] = bk.lcount[b];
-            part.lk[i] = bk.lk[b];
-            part.lfirst[i] = blocks;
+            place_bucket(&part, i, bk, b, blocks);
             blocks += (uint32_t)((bk.lcount[b] + per - 1) / per);
             if (bk.lcount[b] > per) nlead = i + 1;
         }
@@ -627,6 +610,11 @@ int stream_cus(hipStream_t st) {
 }
 
 }  // namespace
+
+void longest_first(const Buckets& bk, uint32_t nbuckets, uint32_t* order) {
+    for (uint32_t b = 0; b < nbuckets; b++) order[b] = b;
+    std::sort(order, order + nbuckets, [&](uint32_t p, uint32_t q) { return bk.lcount[p] != bk.lcount[q] ? bk.lcount[p] > bk.lcount[q] : p < q; });
+}
 
 uint64_t resident_limit_on(hipStream_t st) {
     static const uint64_t per_cu = [] {

@@ -25,6 +25,16 @@ constexpr uint64_t kRMaxBucket = kRMaxBlocks * kRVecElems * 4;  // 2,097,152 ele
 // 26.2 M 136 / 89.
 constexpr uint32_t topk_group_shift(uint64_t tiles) { return tiles <= 64 * 28 ? 6 : tiles <= 128 * 28 ? 7 : 8; }
 
+constexpr uint32_t topk_tiles(uint64_t elems) { return (uint32_t)((elems + kFTile - 1) / kFTile); }
+// Tiles of a group and groups of a bucket.  A group has a tile at least for each of a block's four wavefronts.
+constexpr uint32_t topk_group_tiles(uint32_t tiles, uint32_t shift) {
+    const uint32_t per = (tiles + (1u << shift) - 1) >> shift;
+    return per < 4 ? 4 : per;
+}
+constexpr uint32_t topk_groups(uint32_t tiles, uint32_t shift) {
+    return (tiles + topk_group_tiles(tiles, shift) - 1) / topk_group_tiles(tiles, shift);
+}
+
 // Whether the blocks of a streaming launch over that many tiles have 512 threads instead of 256.  Their sample
 // is evaluated sooner, and 2048 tiles are resident instead of 1536 (a bucket of 6,553,600 elements has 1600: a
 // second round of 64 tiles took as long as half the first); where many rounds follow each other, slots that are
@@ -108,7 +118,7 @@ struct Route {
 //     streaming; 8 x 262,144 20 against 30 streaming; 16 x 65,536 18 against 31 exact; 1500 x 16,384, where a
 //     bucket is one block and nobody waits, 63 against 187 exact.
 //   Beyond, several launches are slower than the two of the streaming path (24 buckets of 1001 to 1.5 M, three
-//     launches: 68 against 52) ...
+//     launches: 68 against 38) ...
 //   ... unless the streaming path's tiles run out of candidate slots (128 per 4096 elements, more than 3 %
 //     inside the sampled window: ratios above about 0.015).  Its tiles are then read again as a whole: that
 //     list at 5 % 71 against 199, 30 buckets of 20,000 to 2 M in seven launches 169 against 240.

@@ -68,3 +68,27 @@ def test_blocks_of_one_or_two_tiles(n, bucket):
         res[lo:lo + bucket] = part
         assert w[b * stride: b * stride + size].tobytes() == want.tobytes(), b
     assert np.array_equal(bits(to_np(dres, F32)), bits(res))
+
+
+@pytest.mark.parametrize("lengths", [
+    [TILE + 1, 5, 3 * TILE + 7, 1_000_003, 4 * TILE, 16 * TILE + 1, 2_200_001, 257 * TILE, 256 * TILE],  # odd tiles, groups of four to nine
+    [1_100_001 - 7 * i for i in range(20)] + [9],                         # 1341 groups: two select launches
+    [100 + i for i in range(63)] + [2 * TILE],                            # as many buckets as a list holds
+    [2_500_003] * 11 + [999],                                             # streaming blocks of one tile
+])
+def test_list_of_ragged_buckets(lengths):
+    """Single-pass top-k of a list: its launches hold the blocks that its buckets have."""
+    from mccl_amd import hip_ops as ops
+    rng = np.random.default_rng(len(lengths))
+    grads = [student_t(rng, n, ties=0.01) for n in lengths]
+    residuals = [(rng.standard_normal(n) * 1e-4).astype(np.float32) for n in lengths]
+    dres = [to_dev(r, F32) for r in residuals]
+    try:
+        ops.set_tuning("topk_path", 2)
+        wires = ops.topk_compress_list([to_dev(g, F32) for g in grads], dres, 0.01)
+    finally:
+        ops.set_tuning("topk_path", 0)
+    for g, r, d, w in zip(grads, residuals, dres, wires):
+        want, size = oracle.topk_compress(g, r, 0.01)
+        assert w.cpu().numpy()[:size].tobytes() == want.tobytes(), g.size
+        assert np.array_equal(bits(to_np(d, F32)), bits(r)), g.size
