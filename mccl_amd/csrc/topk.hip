@@ -13,7 +13,7 @@
 // RESIDENT PATH (topk_resident.hip; one launch): buckets of up to 2 M elements, 2 M a call.
 // SINGLE-PASS PATH (one pass over the gradient, 12 B/element of HBM traffic, two launches):
 // larger buckets and many buckets at a time; see the section "single-pass path" below.
-// EXACT PATH (any input; six launches): large buckets with large ratios, many small buckets,
+// EXACT PATH (any input; six launches): ratios above 12 %, many small buckets,
 // and topk_path = 1 (topk_route.h has the rule and its measurements).
 //   [pass A]   residual <- grad + residual, histogram of key[30:20]
 //   refine x2  histograms of key[19:10], key[9:0] among prefix matches
@@ -26,6 +26,7 @@
 #include "topk_common.hip.h"
 
 #include <atomic>
+#include <type_traits>
 #include <vector>
 
 namespace mcclhip {
@@ -464,6 +465,16 @@ struct StreamShape {
     static constexpr int kHeld = kTiles == 1 ? 7 : 4;          // tiles per wavefront whose slots a bin block keeps in registers
     static constexpr int kPerSimd = kTiles == 1 ? 6 : 8;       // wavefronts that the registers are to leave room for
 };
+// What a tile keeps of its candidates.  MANY: calls whose ratio makes more of them than kTileSlots take (topk_many); a
+// quarter of a wavefront's elements, which a ratio of 12 % leaves half empty.  15 buckets of 6,553,600 elements, us: at 2 % 669 on
+// the path with 128 slots (most tiles dense), 230 so; at 5 % 852 / 252; one bucket at 5 % 140 on the exact path, 38.5 so.  What
+// bounds it is the same stream as at 1 % (186 us of it) and, at 5 %, the candidates' 16 bytes written, read twice and listed.
+template <bool MANY>
+struct TileShape {
+    static constexpr int kStage = MANY ? 256 : 64;                        // candidates a wavefront stages
+    static constexpr int kSlots = MANY ? kManySlots : kTileSlots;         // of a tile
+};
+static_assert(kManySlots >= kFWaves * 256, "what a tile's wavefronts stage fits its slots");
 constexpr int kFVecs = kFRegion / (kWave * 4);  // 16-byte vectors per lane and array: all issued at once
 constexpr int kCoarse = 128;                  // coarse window bins; the last one holds keys >= hi
 constexpr int kBinsPerLane = kCoarse / kWave; // 2
@@ -527,13 +538,13 @@ __device__ __forceinline__ bool wait_word(const uint32_t* p, uint32_t want, uint
     return true;
 }
 
-template <int THREADS>
+template <int THREADS, bool MANY>
 struct StreamLds {
     static constexpr int kWaves = StreamShape<THREADS>::kWaves;
     union {
         SampleLds<THREADS> s;  // sample block
         struct {  // streaming block
-            uint64_t stage[kWaves][kWave];  // a wavefront's candidates, (bits << 32) | index, in index order
+            uint64_t stage[kWaves][TileShape<MANY>::kStage];  // a wavefront's candidates, (bits << 32) | index, in index order
             uint32_t wcnt[kWaves];
             uint32_t win[4];                 // the bucket's window as wavefront 0 read it: lo, hi, predicted threshold, ready
         } a;
@@ -558,9 +569,9 @@ struct SelectLds {
 
 // The bucket's candidate window; clears what the launches accumulate into, then publishes the
 // window and the epoch with one store.
-template <int THREADS>
+template <int THREADS, class Lds>
 __device__ __forceinline__ void fused_sample(BucketsArg bk, const Geometry& g, const Workspace& w, uint32_t b,
-                                             uint32_t epoch, StreamLds<THREADS>& L) {
+                                             uint32_t epoch, Lds& L) {
     const FusedGeo fg = fused_geo(g, bk, b);
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
     const SampleWindow win = sample_window<THREADS>(bucket_grad(g, bk, b), bucket_residual(g, bk, b), fg.bn, fg.k, L.s, [&] {
@@ -684,13 +695,90 @@ struct GroupTiles {
         }
     }
 };
+// The same for tiles with slots for many candidates: nothing is kept, every sweep reads the slots again, in
+// index order, a tile's (up to 384 candidates, what a ratio of 7 % makes) while the tile before it is looked at.
+// One round trip of 0.7 us a sweep is exposed; registers for 384 entries of each tile would halve
+// the blocks that fit a CU.
+template <bool AGENT, int NW>
+struct ManyTiles {
+    static constexpr int kPairs = 3;  // of 128 entries, read ahead
+    static constexpr int kSlots = TileShape<true>::kSlots;
+    const uint32_t* tcnt;
+    const uint64_t* slots;
+    uint32_t t0, wt0, wt1;  // as GroupTiles'
+    int lane;
+
+    static __device__ __forceinline__ uint64_t ld64(const uint64_t* p) {
+        if constexpr (AGENT) return ld_agent64(p);
+        else return *p;
+    }
+    __device__ __forceinline__ void load(const Geometry& g, const Workspace& w, uint32_t b, uint32_t grp, const FusedGeo& fg) {
+        lane = threadIdx.x & (kWave - 1);
+        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+        tcnt = w.tile_cnt + (uint64_t)b * g.ftiles;
+        slots = w.slots + (uint64_t)b * g.ftiles * kSlots;
+        t0 = grp * fg.tpg;
+        const uint32_t t1 = t0 + fg.tpg < fg.ntiles ? t0 + fg.tpg : fg.ntiles;
+        const uint32_t pw = (t1 - t0 + NW - 1) / NW;
+        wt0 = t0 + wave * pw < t1 ? t0 + wave * pw : t1;
+        wt1 = wt0 + pw < t1 ? wt0 + pw : t1;
+    }
+    // nd(~0u, t, cnt, e0, e1) for every 128 candidates of an ordinary tile (cnt: how many of them there are),
+    // dn(~0u, t) for a dense one, all in index order.
+    template <class ND, class DN>
+    __device__ __forceinline__ void sweep(ND&& nd, DN&& dn) const {
+#pragma unroll 1
+        for (uint32_t c0 = wt0; c0 < wt1; c0 += kWave) {
+            const uint32_t n = wt1 - c0 < (uint32_t)kWave ? wt1 - c0 : (uint32_t)kWave;
+            uint32_t cnts = 0;
+            if ((uint32_t)lane < n) {
+                if constexpr (AGENT) cnts = ld_agent(tcnt + c0 + lane);
+                else cnts = tcnt[c0 + lane];
+            }
+            uint64_t e[2 * kPairs], next[2 * kPairs];
+            // (lanes past the count read entry 0: no branches between the loads, no lines touched for nothing)
+            auto fetch = [&](uint32_t i, uint64_t (&to)[2 * kPairs]) {
+                const uint32_t cnt = (uint32_t)__builtin_amdgcn_readlane((int)cnts, (int)i);
+                const uint64_t* p = slots + (uint64_t)(c0 + i) * kSlots;
+#pragma unroll
+                for (int r = 0; r < 2 * kPairs; r++) {
+                    const uint32_t at = (uint32_t)(r * kWave + lane);
+                    to[r] = ld64(p + (at < cnt ? at : 0u));
+                }
+            };
+            fetch(0, e);
+#pragma unroll 1
+            for (uint32_t i = 0; i < n; i++) {
+                fetch(i + 1 < n ? i + 1 : i, next);
+                const uint32_t t = c0 + i, cnt = (uint32_t)__builtin_amdgcn_readlane((int)cnts, (int)i);
+                if (cnt == kDense) {
+                    dn(~0u, t);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < kPairs; v++)
+                        if (cnt > (uint32_t)(v * 2 * kWave)) nd(~0u, t, cnt - v * 2 * kWave, e[2 * v], e[2 * v + 1]);
+#pragma unroll 1
+                    for (uint32_t from = kPairs * 2 * kWave; from < cnt; from += 2 * kWave) {
+                        const uint64_t* p = slots + (uint64_t)t * kSlots + from;
+                        const uint32_t left = cnt - from;
+                        const uint64_t a0 = ld64(p + ((uint32_t)lane < left ? lane : 0));
+                        const uint64_t a1 = ld64(p + ((uint32_t)(kWave + lane) < left ? kWave + lane : 0));
+                        nd(~0u, t, left, a0, a1);
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 2 * kPairs; r++) e[r] = next[r];
+            }
+        }
+    }
+};
 __device__ __forceinline__ uint32_t key64(uint64_t e) { return (uint32_t)(e >> 32) & 0x7FFFFFFFu; }
 
 // ---- bin block -----------------------------------------------------------------------------
-template <int THREADS>
+template <int THREADS, bool MANY>
 __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, const Workspace& w, uint32_t b,
                                           uint32_t grp, const FusedGeo& fg, uint32_t epoch, uint64_t limit_ticks,
-                                          StreamLds<THREADS>& L) {
+                                          StreamLds<THREADS, MANY>& L) {
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
     // the group's tiles are finished: all its streaming blocks have arrived
     {
@@ -713,7 +801,8 @@ __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, cons
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
     const float* rp = bucket_residual(g, bk, b);
-    GroupTiles<true, StreamShape<THREADS>::kWaves, StreamShape<THREADS>::kHeld> G;
+    typedef StreamShape<THREADS> Shape;
+    std::conditional_t<MANY, ManyTiles<true, Shape::kWaves>, GroupTiles<true, Shape::kWaves, Shape::kHeld>> G;
     G.load(g, w, b, grp, fg);
     // candidates per coarse bin
     if (threadIdx.x < kCoarse) L.e.cnt[threadIdx.x] = 0;
@@ -773,14 +862,15 @@ __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, cons
 // ---- the streaming launch ------------------------------------------------------------------
 // LISTED: the call's buckets are a list (g.listed), known to the compiler: a block finds its work before it can
 // load, and one kernel for both layouts kept 13 more scalar registers in vector lanes (the 96.5 M gradient 2.5 us).
-template <int THREADS, bool LISTED>
+template <int THREADS, bool LISTED, bool MANY>
 __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_topk_stream(Buckets, Geometry g, Workspace w, uint32_t epoch,
                                                         uint32_t published, uint32_t first_wave,
                                                         uint64_t limit_ticks) {
     g.listed = LISTED;
     const BucketsArg bk = buckets_arg();
     constexpr uint32_t kTiles = StreamShape<THREADS>::kTiles;
-    __shared__ StreamLds<THREADS> L;
+    constexpr int kStage = TileShape<MANY>::kStage, kSlots = TileShape<MANY>::kSlots;
+    __shared__ StreamLds<THREADS, MANY> L;
     if (blockIdx.x < g.nbuckets) {
         fused_sample<THREADS>(bk, g, w, blockIdx.x, published, L);
         return;
@@ -821,7 +911,7 @@ __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_top
     }
     const FusedGeo fg = fused_geo(g, bk, b);
     if (emit) {
-        if (t < fg.ng) fused_bin<THREADS>(bk, g, w, b, t, fg, epoch, limit_ticks, L);
+        if (t < fg.ng) fused_bin<THREADS, MANY>(bk, g, w, b, t, fg, epoch, limit_ticks, L);
         return;
     }
     if (t * kTiles >= fg.ntiles) return;
@@ -875,9 +965,12 @@ __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_top
     };
     // Puts back the region's staged candidates that were stored as zeros.
     auto restore_staged = [&]() {
-        if ((uint32_t)lane < staged) {
-            const uint64_t e = slots[lane];
-            if (((uint32_t)(e >> 32) & 0x7FFFFFFFu) >= that_key) st_agent((uint32_t*)rbase + (uint32_t)e, (uint32_t)(e >> 32));
+#pragma unroll
+        for (int i = 0; i < kStage; i += kWave) {
+            if ((uint32_t)(i + lane) < staged) {
+                const uint64_t e = slots[i + lane];
+                if (((uint32_t)(e >> 32) & 0x7FFFFFFFu) >= that_key) st_agent((uint32_t*)rbase + (uint32_t)e, (uint32_t)(e >> 32));
+            }
         }
     };
     // Appends the lanes' candidates (mask4: which of a lane's four elements) in index
@@ -901,7 +994,7 @@ __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_top
         }
         if (dense) return;
         total = (uint32_t)__builtin_amdgcn_readfirstlane((int)total);
-        if (staged + total > (uint32_t)kWave) {
+        if (staged + total > (uint32_t)kStage) {
             // the region goes dense: its earlier candidates were stored as zeros where
             // they reached the predicted threshold; put those values back
             dense = 1u;
@@ -974,11 +1067,14 @@ __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_top
         fused_give_up(w, st, out);
         return;     // without counting the tile: the bucket's bin blocks give up as well
     }
-    tile_dense |= total > (uint32_t)kTileSlots;
+    tile_dense |= total > (uint32_t)kSlots;
     if (tile_dense) {
         if (!dense) restore_staged();  // a tile is dense as a whole: its residual holds plain sums
-    } else if ((uint32_t)lane < staged) {
-        st_agent64(w.slots + ((uint64_t)b * g.ftiles + t) * kTileSlots + before + lane, slots[lane]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < kStage; i += kWave)
+            if ((uint32_t)(i + lane) < staged)
+                st_agent64(w.slots + ((uint64_t)b * g.ftiles + t) * kSlots + before + i + lane, slots[i + lane]);
     }
     const bool counts = wave == first_wave_of_tile && lane == 0 && t < fg.ntiles;
     if (counts) st_agent(w.tile_cnt + (uint64_t)b * g.ftiles + t, tile_dense ? kDense : total);
@@ -1021,9 +1117,10 @@ __device__ __forceinline__ uint32_t resolve_ties64(ForList&& for_list, uint32_t 
 // The exact selection of one bucket by its select blocks together (same algorithm as the exact
 // path: three radix rounds over the key, then an ordered emit), each on its own group's
 // element range; four barriers.  Returns false when a barrier wait timed out.
+template <class Tiles>
 __device__ __forceinline__ bool select_exact_group(BucketsArg bk, const Geometry& g, const Workspace& w, uint32_t b,
                                                    uint32_t grp, const FusedGeo& fg, uint32_t that_key,
-                                                   const GroupTiles<false, kFWaves, kHeld>& G, SelectLds& L, uint64_t limit_ticks) {
+                                                   const Tiles& G, SelectLds& L, uint64_t limit_ticks) {
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
     const uint64_t bn = fg.bn;
     float* rp = bucket_residual(g, bk, b);
@@ -1154,7 +1251,7 @@ __device__ __forceinline__ bool select_exact_group(BucketsArg bk, const Geometry
 // blockIdx.x = group, blockIdx.y = bucket - first_bucket; of a list, blocks of all its buckets in a row
 // (Buckets::lfirst).  Everything the streaming launch
 // left behind is read with plain loads; only the exact fallback talks across blocks.
-template <bool LISTED>
+template <bool LISTED, bool MANY>
 __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, Workspace w, uint32_t first_bucket,
                                                            uint64_t limit_ticks) {
     g.listed = LISTED;
@@ -1174,7 +1271,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
     static_assert(kBinsPerLane == 2, "a lane owns two neighbouring bins");
     // scanned from the top bin downwards: lane l looks at bins 127 - 2 l (tot[1]) and 126 - 2 l (tot[0])
     const u2a tot = *(const u2a*)(w.bin_fill + (uint64_t)b * kCoarse + kCoarse - 2 - 2 * (threadIdx.x & (kWave - 1)));
-    GroupTiles<false, kFWaves, kHeld> G;
+    std::conditional_t<MANY, ManyTiles<false, kFWaves>, GroupTiles<false, kFWaves, kHeld>> G;
     G.load(g, w, b, grp, fg);
     // a replay of a captured launch carries the same epoch: also behind a run that was given up
     if (grp == 0 && threadIdx.x == 0) st[S_READY] = 0u;
@@ -1343,7 +1440,14 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
         });
         return pos;
     };
-    {
+    if constexpr (MANY) {
+        uint32_t pos = wave_off;
+        G.sweep([&](uint32_t, uint32_t, uint32_t cnt, uint64_t a0, uint64_t a1) {
+                    pos = emit_half((uint32_t)lane < cnt, a0, pos);
+                    pos = emit_half((uint32_t)(kWave + lane) < cnt, a1, pos);
+                },
+                [&](uint32_t, uint32_t t) { pos = emit_dense(t, pos); });
+    } else {
         uint32_t pos = wave_off;
 #pragma unroll
         for (int h = 0; h < kHeld; h++) {
@@ -1356,21 +1460,21 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
                 }
             }
         }
-    }
-    if (G.more) {
-        uint32_t pos = wave_off;
+        if (G.more) {
+            pos = wave_off;
 #pragma unroll 1
-        for (uint32_t t = G.wt0; t < G.wt1; t++) {
-            const uint32_t cnt = (uint32_t)__builtin_amdgcn_readfirstlane((int)G.tcnt[t]);
-            if (cnt == kDense) {
-                pos = emit_dense(t, pos);
-            } else if (t - G.wt0 < (uint32_t)kHeld) {
-                pos += L.rcnt[wave][t - G.wt0];
-            } else {
-                const uint64_t a0 = G.slots[(uint64_t)t * kTileSlots + lane];
-                const uint64_t a1 = G.slots[(uint64_t)t * kTileSlots + kWave + lane];
-                pos = emit_half((uint32_t)lane < cnt, a0, pos);
-                pos = emit_half((uint32_t)(kWave + lane) < cnt, a1, pos);
+            for (uint32_t t = G.wt0; t < G.wt1; t++) {
+                const uint32_t cnt = (uint32_t)__builtin_amdgcn_readfirstlane((int)G.tcnt[t]);
+                if (cnt == kDense) {
+                    pos = emit_dense(t, pos);
+                } else if (t - G.wt0 < (uint32_t)kHeld) {
+                    pos += L.rcnt[wave][t - G.wt0];
+                } else {
+                    const uint64_t a0 = G.slots[(uint64_t)t * kTileSlots + lane];
+                    const uint64_t a1 = G.slots[(uint64_t)t * kTileSlots + kWave + lane];
+                    pos = emit_half((uint32_t)lane < cnt, a0, pos);
+                    pos = emit_half((uint32_t)(kWave + lane) < cnt, a1, pos);
+                }
             }
         }
     }
@@ -1399,10 +1503,15 @@ uint64_t zeroed_words(const Geometry& g) {
     return align4((uint64_t)g.nbuckets * kHistWords) + align4((uint64_t)g.nbuckets * kStateWords);
 }
 
+// Groups that the workspace has room for.  (Calls with slots for many candidates cut fewer buckets into more of
+// them; their workspace does not shrink where a bucket more makes them cut into fewer.)
+uint64_t all_groups(const Geometry& g) { return (uint64_t)g.nbuckets * (g.many ? kMaxGroups : 1u << g.gshift); }
+
 uint64_t workspace_words(const Geometry& g) {
-    return zeroed_words(g) + 2 * align4((uint64_t)g.nbuckets * g.tiles) + 2 * align4((uint64_t)g.nbuckets << g.gshift) +
-           align4((uint64_t)g.nbuckets * g.ftiles) + align4((uint64_t)g.nbuckets * g.ftiles * kTileSlots * 2) +
-           align4(((uint64_t)g.nbuckets << g.gshift) * kCntStride) + align4(((uint64_t)g.nbuckets << g.gshift) * kCoarse) +
+    const uint64_t groups = all_groups(g);
+    return zeroed_words(g) + 2 * align4((uint64_t)g.nbuckets * g.tiles) + 2 * align4(groups) +
+           align4((uint64_t)g.nbuckets * g.ftiles) + align4((uint64_t)g.nbuckets * g.ftiles * g.slots * 2) +
+           align4(groups * kCntStride) + align4(groups * kCoarse) +
            align4((uint64_t)g.nbuckets * kCoarse) + align4((uint64_t)g.nbuckets * (kCoarse - 1) * g.lcapb * 2);
 }
 
@@ -1413,12 +1522,12 @@ Workspace carve(void* base, const Geometry& g) {
     w.state = p;       p += align4((uint64_t)g.nbuckets * kStateWords);
     w.tile_gt = p;     p += align4((uint64_t)g.nbuckets * g.tiles);
     w.tile_eq = p;     p += align4((uint64_t)g.nbuckets * g.tiles);
-    w.blk_above = p;   p += align4((uint64_t)g.nbuckets << g.gshift);
-    w.blk_eq = p;      p += align4((uint64_t)g.nbuckets << g.gshift);
+    w.blk_above = p;   p += align4(all_groups(g));
+    w.blk_eq = p;      p += align4(all_groups(g));
     w.tile_cnt = p;    p += align4((uint64_t)g.nbuckets * g.ftiles);
-    w.slots = (uint64_t*)p;  p += align4((uint64_t)g.nbuckets * g.ftiles * kTileSlots * 2);
-    w.grp_cnt = p;     p += align4(((uint64_t)g.nbuckets << g.gshift) * kCntStride);
-    w.gsuf = p;       p += align4(((uint64_t)g.nbuckets << g.gshift) * kCoarse);
+    w.slots = (uint64_t*)p;  p += align4((uint64_t)g.nbuckets * g.ftiles * g.slots * 2);
+    w.grp_cnt = p;     p += align4(all_groups(g) * kCntStride);
+    w.gsuf = p;        p += align4(all_groups(g) * kCoarse);
     w.bin_fill = p;    p += align4((uint64_t)g.nbuckets * kCoarse);
     w.blist = (uint64_t*)p;
     // The resident path's scratch lies where the streaming path has its lists: a call takes one of the two.
@@ -1429,6 +1538,11 @@ Workspace carve(void* base, const Geometry& g) {
     w.rmem = p;
     w.status = nullptr;
     return w;
+}
+
+void set_groups(Geometry* g, uint32_t shift) {
+    g->gshift = shift;
+    g->ngroups = topk_groups(g->ftiles, shift);
 }
 
 bool make_geometry(uint64_t n_total, uint64_t bucket_elems, double ratio, Geometry* g) {
@@ -1445,8 +1559,9 @@ bool make_geometry(uint64_t n_total, uint64_t bucket_elems, double ratio, Geomet
     g->k_last = mccl_hip_topk_k(n_total - (nb - 1) * bucket_elems, ratio);
     g->listed = 0;
     g->ftiles = (uint32_t)((bucket_elems + kFTile - 1) / kFTile);
-    g->gshift = topk_group_shift(g->ftiles);
-    g->ngroups = topk_groups(g->ftiles, g->gshift);
+    g->many = topk_many(bucket_elems, ratio) ? 1 : 0;
+    g->slots = g->many ? kManySlots : kTileSlots;
+    set_groups(g, g->many ? topk_group_shift_many(g->ftiles, (uint64_t)nb * topk_groups(g->ftiles, 8)) : topk_group_shift(g->ftiles));
     // a coarse bin holds about k / 80 candidates when the window is as wide as a sample of 8192
     // leaves it, the bins at the window's lower end three times that; k / 10 + 2048 entries
     // leave room for more uneven ones
@@ -1468,7 +1583,7 @@ uint32_t next_epoch() {
 }
 
 // The two launches of the single-pass path.
-template <int THREADS, bool LISTED>
+template <int THREADS, bool LISTED, bool MANY>
 void launch_stream(Buckets& bk, const Geometry& g, const Workspace& w, uint64_t limit_ticks, hipStream_t st) {
     // a sample block per bucket, then per bucket its tiles and its bin blocks
     constexpr uint32_t per = StreamShape<THREADS>::kTiles;
@@ -1488,72 +1603,72 @@ void launch_stream(Buckets& bk, const Geometry& g, const Workspace& w, uint64_t 
     // blocks that are resident from the start of the launch: they wait for the sample blocks
     static const int per_cu = [] {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_topk_stream<THREADS, LISTED>, THREADS, 0) != hipSuccess || n < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_topk_stream<THREADS, LISTED, MANY>, THREADS, 0) != hipSuccess || n < 1)
             n = StreamShape<THREADS>::kPerSimd * 4 * kWave / THREADS;
         return n;
     }();
     const uint32_t first_wave = g.nbuckets + (uint32_t)device_info().num_cus * (uint32_t)per_cu;
     // (tests of the give-up path: the sample blocks publish a number nobody waits for)
     const uint32_t published = tuning().topk_stall_test ? ~epoch : epoch;
-    k_topk_stream<THREADS, LISTED><<<(uint32_t)blocks, THREADS, 0, st>>>(bk, g, w, epoch, published, first_wave, limit_ticks);
+    k_topk_stream<THREADS, LISTED, MANY><<<(uint32_t)blocks, THREADS, 0, st>>>(bk, g, w, epoch, published, first_wave, limit_ticks);
 }
 
-void launch_single_pass(const Buckets& call, const Geometry& g, const Workspace& w, hipStream_t st) {
+template <bool LISTED, bool MANY>
+void launch_single_pass(const Buckets& call, const Geometry& geometry, const Workspace& w, hipStream_t st) {
     // 100 MHz ticks a block may wait before it gives up
     const uint64_t lim = (uint64_t)tuning().topk_barrier_ms * 100000ull;
     // A list's blocks are those that its buckets have, longest bucket first: the bin blocks that nothing is
     // streamed beside are those of the shortest.
     Buckets bk = call;
+    Geometry g = geometry;
     uint64_t tiles = (uint64_t)g.nbuckets * g.ftiles;
-    if (g.listed) {
+    if constexpr (LISTED) {
         uint32_t order[kMaxListed];
         longest_first(call, g.nbuckets, order);
+        uint64_t groups = 0;
         tiles = 0;
         for (uint32_t b = 0; b < g.nbuckets; b++) {
             place_bucket(&bk, b, call, order[b], 0);
             tiles += topk_tiles(bk.lcount[b]);
+            groups += topk_groups(topk_tiles(bk.lcount[b]), 8);
         }
         for (uint32_t b = g.nbuckets; b < kMaxListed; b++) bk.lfirst[b] = 0xFFFFFFFFu;
+        if constexpr (MANY) set_groups(&g, topk_group_shift_many(g.ftiles, groups));
     }
-    if (g.listed) {
-        if (stream_wide(tiles)) launch_stream<512, true>(bk, g, w, lim, st);
-        else launch_stream<256, true>(bk, g, w, lim, st);
-    } else {
-        if (stream_wide(tiles)) launch_stream<512, false>(bk, g, w, lim, st);
-        else launch_stream<256, false>(bk, g, w, lim, st);
-    }
+    if (stream_wide(tiles)) launch_stream<512, LISTED, MANY>(bk, g, w, lim, st);
+    else launch_stream<256, LISTED, MANY>(bk, g, w, lim, st);
     // the select launch, at most kSelBlocks blocks at a time: all of them are resident
     // together, whatever the order in which the hardware dispatches them
-    if (!g.listed) {
-        const uint32_t at_once = kSelBlocks / g.ngroups;
-        for (uint32_t b0 = 0; b0 < g.nbuckets; b0 += at_once) {
-            const uint32_t nb = g.nbuckets - b0 < at_once ? g.nbuckets - b0 : at_once;
-            k_topk_select<false><<<dim3(g.ngroups, nb), kBlock, 0, st>>>(bk, g, w, b0, lim);
-        }
-        return;
-    }
     for (uint32_t b0 = 0; b0 < g.nbuckets;) {
-        uint32_t blocks = 0, b = b0;
-        for (uint32_t i = 0; i < b0; i++) bk.lfirst[i] = 0;  // before b0, which starts there and is the last that does
-        for (; b < g.nbuckets; b++) {
-            const uint32_t groups = topk_groups(topk_tiles(bk.lcount[b]), g.gshift);
-            if (blocks + groups > kSelBlocks) break;
-            bk.lfirst[b] = blocks;
-            blocks += groups;
+        if constexpr (LISTED) {
+            uint32_t blocks = 0, b = b0;
+            for (uint32_t i = 0; i < b0; i++) bk.lfirst[i] = 0;  // before b0, which starts there and is the last that does
+            for (; b < g.nbuckets; b++) {
+                const uint32_t groups = topk_groups(topk_tiles(bk.lcount[b]), g.gshift);
+                if (blocks + groups > kSelBlocks) break;
+                bk.lfirst[b] = blocks;
+                blocks += groups;
+            }
+            for (uint32_t i = b; i < g.nbuckets; i++) bk.lfirst[i] = 0xFFFFFFFFu;
+            k_topk_select<true, MANY><<<blocks, kBlock, 0, st>>>(bk, g, w, b0, lim);
+            b0 = b;
+        } else {
+            const uint32_t at_once = kSelBlocks / g.ngroups;
+            const uint32_t nb = g.nbuckets - b0 < at_once ? g.nbuckets - b0 : at_once;
+            k_topk_select<false, MANY><<<dim3(g.ngroups, nb), kBlock, 0, st>>>(bk, g, w, b0, lim);
+            b0 += nb;
         }
-        for (uint32_t i = b; i < g.nbuckets; i++) bk.lfirst[i] = 0xFFFFFFFFu;
-        k_topk_select<true><<<blocks, kBlock, 0, st>>>(bk, g, w, b0, lim);
-        b0 = b;
     }
 }
 
 // False when the call has to take the exact path.
 bool launch_by_path(const Buckets& bk, const Geometry& g, const Workspace& w, const uint64_t* counts, hipStream_t st) {
     const uint64_t limit = g.bucket_elems <= kRMaxBucket ? resident_limit_on(st) : 0;
-    const Route route = choose_path({g.n_total, g.bucket_elems, g.nbuckets, counts, g.k_full}, tuning().topk_path, limit);
+    const Route route = choose_path({g.n_total, g.bucket_elems, g.nbuckets, counts, g.k_full, g.many != 0}, tuning().topk_path, limit);
     if (route.path == kPathExact) return false;
     if (route.path == kPathStream) {
-        launch_single_pass(bk, g, w, st);
+        if (g.listed) (g.many ? launch_single_pass<true, true> : launch_single_pass<true, false>)(bk, g, w, st);
+        else (g.many ? launch_single_pass<false, true> : launch_single_pass<false, false>)(bk, g, w, st);
     } else {
         const uint32_t epoch = next_epoch();
         launch_resident(bk, g, w, route.vecs, limit, epoch, tuning().topk_stall_test ? ~epoch : epoch,

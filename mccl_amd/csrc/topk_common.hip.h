@@ -56,6 +56,8 @@ struct Geometry {
     uint32_t ftiles;   // single-pass path: streaming tiles allotted per bucket
     uint32_t gshift;   // single-pass path: at most 1 << gshift groups of tiles per bucket
     uint32_t ngroups;  // single-pass path: groups of a (full) bucket
+    uint32_t many;     // single-pass path: 1 when tiles have slots for many candidates (topk_many)
+    uint32_t slots;    // single-pass path: candidate slots of a tile
     uint32_t lcapb;    // single-pass path: capacity of one coarse bin's list (entries)
 };
 
@@ -70,7 +72,7 @@ struct Workspace {
     uint32_t* blk_eq;       // [nbuckets][groups] ... keys equal to the threshold per group
     // single-pass path
     uint32_t* tile_cnt;     // [nbuckets][ftiles] candidates in the tile's slots, or kDense
-    uint64_t* slots;        // [nbuckets][ftiles][128] (bits << 32) | index, index order
+    uint64_t* slots;        // [nbuckets][ftiles][slots] (bits << 32) | index, index order
     uint32_t* grp_cnt;      // [nbuckets][groups][kCntStride] finished tiles per group (first word of each 256 bytes)
     uint32_t* gsuf;         // [nbuckets][128 bins][groups] a group's candidates in the bins above bin j
     uint32_t* bin_fill;     // [nbuckets][128] the bucket's candidates per coarse window bin (= entries of the bin's list)

@@ -12,6 +12,7 @@ enum Path { kPathExact, kPathStream, kPathResident };
 constexpr int kFSample = 8192;              // sampled elements per bucket
 constexpr uint64_t kFTile = 4096;           // single-pass path: elements per streaming block
 constexpr int kTileSlots = 128;             // ... candidate slots per tile
+constexpr int kManySlots = 1024;            // ... of calls with large ratios
 constexpr uint64_t kWideTiles = 6144;       // ... a launch of at most this many has blocks of 512 threads
 constexpr uint32_t kMaxGroups = 1u << 8;    // ... at most this many groups of tiles per bucket
 constexpr uint64_t kFastMinBucket = 1u << 18;
@@ -35,6 +36,29 @@ constexpr uint32_t topk_groups(uint32_t tiles, uint32_t shift) {
     return (tiles + topk_group_tiles(tiles, shift) - 1) / topk_group_tiles(tiles, shift);
 }
 
+// Expected share of a bucket inside the sampled window (see sample_window).
+inline double window_share(double ratio) {
+    const double ks = ratio * kFSample;
+    return (ks + 6.0 * std::sqrt(ks) + 16.0) / kFSample;
+}
+
+// Whether a call's tiles have slots for many candidates (kManySlots): where the ratio fills 65 % of kTileSlots,
+// about 1.13 %, tiles begin to run out of them, and one that does is read again as a whole by every later pass.  us
+// per call, 128 slots against 1024: one bucket of 2.5 M elements at 1.1 % 28.8 / 30.1, of 6,553,600 at 1.1 % 36.5 / 35.7, at
+// 1.2 % 41.9 / 35.0, at 1.6 % 164 / 35.5, 15 of them at 1.1 % 226 / 223, at 1.2 % 244 / 223, at 1.6 % 430 / 226.
+// By the ratio and the bucket's length alone, as the workspace is sized by it, and not for buckets so
+// short that their workspace would no longer serve ratios below the line.
+constexpr uint64_t kManyMinBucket = 1u << 16;
+inline bool topk_many(uint64_t bucket_elems, double ratio) {
+    return bucket_elems >= kManyMinBucket && window_share(ratio) > 0.65 * kTileSlots / kFTile;
+}
+// ... their groups of tiles per bucket, the power of two.  Their blocks read slots again on every pass, a tile
+// after the other: as many groups as keep the call's select launch in one (`groups`: with 256 for every bucket).
+constexpr uint32_t topk_group_shift_many(uint64_t tiles, uint64_t groups) {
+    const uint32_t s = groups <= 1024 ? 8 : groups <= 2048 ? 7 : 6;
+    return s > topk_group_shift(tiles) ? s : topk_group_shift(tiles);
+}
+
 // Whether the blocks of a streaming launch over that many tiles have 512 threads instead of 256.  Their sample
 // is evaluated sooner, and 2048 tiles are resident instead of 1536 (a bucket of 6,553,600 elements has 1600: a
 // second round of 64 tiles took as long as half the first); where many rounds follow each other, slots that are
@@ -50,6 +74,7 @@ struct TopkCall {
     uint32_t nbuckets;
     const uint64_t* counts;
     uint32_t k_full;  // picks of a bucket of bucket_elems
+    bool many = false;  // topk_many of the call
 };
 
 // The most blocks of one resident launch that may wait for others.  Blocks of a bucket wait for each
@@ -119,12 +144,16 @@ struct Route {
 //     bucket is one block and nobody waits, 63 against 187 exact.
 //   Beyond, several launches are slower than the two of the streaming path (24 buckets of 1001 to 1.5 M, three
 //     launches: 68 against 38) ...
-//   ... unless the streaming path's tiles run out of candidate slots (128 per 4096 elements, more than 3 %
-//     inside the sampled window: ratios above about 0.015).  Its tiles are then read again as a whole: that
-//     list at 5 % 71 against 199, 30 buckets of 20,000 to 2 M in seven launches 169 against 240.
-//   Buckets of one buffer take the exact path instead: one of 6.5 M at 5 % 144 against 448, 16 x 262,144 57 against
-//     99, 4 x 2 M 117 against 167, 20 x 1.5 M 288 against 320; of many large ones the streaming path shares that
-//     latency: 12 x 2 M 249 exact, 230 streaming, 50 x 1.7 M 782 and 725, 14 x 6.5 M 905 and 826.
+//   ... unless the streaming path's tiles run out of candidate slots (share of a bucket inside the sampled window
+//     times 4096; of 1024 slots 60 % are counted on: ratios up to 0.12).  With slots for many candidates,
+//     at 5 %, several resident launches or the exact path against the streaming path: that list 73 / 43, 30 buckets of
+//     20,000 to 2 M 172 / 65, one bucket of 2.2 M 65 / 31, of 6.5 M 140 / 38, 4 x 2 M 115 / 43, 20 x 300,000 74 / 39,
+//     20 x 1.5 M 291 / 107; one of 6.5 M at 12 % 144 / 51.  Tiles that run out are read again as a whole: with 128 slots
+//     that list at 5 % 71 against 199, 30 buckets of 20,000 to 2 M in seven launches 169 against 240.
+//   Buckets of one buffer take the exact path then: with 128 slots, at 5 %, one of 6.5 M 144 against 448, 16 x 262,144 57
+//     against 99, 4 x 2 M 117 against 167, 20 x 1.5 M 288 against 320; of many large ones the streaming path shares that
+//     latency: 12 x 2 M 249 exact, 230 streaming, 50 x 1.7 M 782 and 725, 14 x 6.5 M 905 and 826, 15 x 6.5 M at 20 % with
+//     1024 slots 889 and 730.
 inline Route choose_path(const TopkCall& c, int forced, uint64_t limit) {
     const uint64_t tiles = (c.bucket_elems + kFTile - 1) / kFTile;
     const bool streams = (uint64_t)c.nbuckets * (tiles + kMaxGroups + 1) + kMaxGroups < 0x7FFFFFFFull;
@@ -132,7 +161,7 @@ inline Route choose_path(const TopkCall& c, int forced, uint64_t limit) {
     if (forced == 2 && streams) return {kPathStream, 0};
     // expected share of a bucket inside the sampled window (see sample_window)
     const double ks = (double)c.k_full / (double)c.bucket_elems * kFSample;
-    const bool dense = (ks + 6.0 * std::sqrt(ks) + 16.0) / kFSample > (double)kTileSlots / kFTile;
+    const bool dense = (ks + 6.0 * std::sqrt(ks) + 16.0) / kFSample > (c.many ? 0.6 * kManySlots : (double)kTileSlots) / kFTile;
     int vecs = resident_vecs(c, limit);
     // a list can go in several launches, as long as its longest bucket fits one
     if (!vecs && c.counts && (dense || forced == 3) && c.bucket_elems <= (limit < kRMaxBlocks ? limit : kRMaxBlocks) * kRVecElems * 4) vecs = 4;

@@ -60,6 +60,18 @@ def test_a_workspace_for_a_longer_bucket_serves_a_shorter_one():
             assert all(a and a <= b for a, b in zip(sizes, sizes[1:])), (ratio, buckets)
 
 
+def test_a_workspace_for_a_larger_ratio_or_more_buckets_serves_less():
+    from mccl_amd import _lib
+    size = _lib.load().mccl_hip_topk_workspace_bytes
+    ratios = [0.001, 0.005, 0.01, 0.011, 0.0115, 0.02, 0.05, 0.1, 0.3, 1.0]
+    for n in (1000, 65_535, 65_536, 300_000, 6_553_600, 30_000_000):
+        sizes = [size(n, n, r) for r in ratios]
+        assert all(a and a <= b for a, b in zip(sizes, sizes[1:])), n
+        for ratio in (0.01, 0.05):
+            sizes = [size(n * b, n, ratio) for b in (1, 3, 4, 5, 8, 9, 16, 17, 40)]
+            assert all(a and a <= b for a, b in zip(sizes, sizes[1:])), (n, ratio)
+
+
 def test_argument_errors_need_no_gpu():
     from mccl_amd import _lib
     lib = _lib.load()

@@ -92,3 +92,73 @@ def test_list_of_ragged_buckets(lengths):
         want, size = oracle.topk_compress(g, r, 0.01)
         assert w.cpu().numpy()[:size].tobytes() == want.tobytes(), g.size
         assert np.array_equal(bits(to_np(d, F32)), bits(r)), g.size
+
+
+def _check(ops, grad, res, ratio, bucket):
+    dres = to_dev(res, F32)
+    n = grad.size
+    ws = ops.topk_workspace(n, bucket, ratio, DEV)
+    try:
+        ops.set_tuning("topk_path", 2)
+        wire, stride = ops.topk_compress(to_dev(grad, F32), dres, ratio, bucket_elems=bucket, workspace=ws)
+    finally:
+        ops.set_tuning("topk_path", 0)
+    w = wire.cpu().numpy()
+    for b, lo in enumerate(range(0, n, bucket)):
+        part = res[lo:lo + bucket].copy()
+        want, size = oracle.topk_compress(grad[lo:lo + bucket], part, ratio)
+        res[lo:lo + bucket] = part
+        assert w[b * stride: b * stride + size].tobytes() == want.tobytes(), b
+    assert np.array_equal(bits(to_np(dres, F32)), bits(res))
+    return ops.topk_path_report(ws, n, bucket, ratio)
+
+
+@pytest.mark.parametrize("n, bucket, ratio", [
+    (65_536, 65_536, 0.0115), (65_541, 65_541, 0.05),          # the shortest buckets with 1024 slots a tile
+    (3_000_001, 3_000_001, 0.05), (13_107_203, 6_553_600, 0.02),
+    (3_000_000, 3_000_000, 0.1),                               # about 500 candidates a tile: more than are read ahead
+    (40_000_000, 8_000_000, 0.05),                             # 128 groups a bucket, several tiles a wavefront
+    (17 * 1_048_576 - 3, 1_048_576, 0.05),                     # 64 groups a bucket, two select launches
+])
+def test_many_candidates(n, bucket, ratio):
+    from mccl_amd import hip_ops as ops
+    rng = np.random.default_rng(n)
+    buckets = -(-n // bucket)
+    done = _check(ops, student_t(rng, n, ties=0.01), (rng.standard_normal(n) * 1e-4).astype(np.float32), ratio, bucket)
+    assert done == (buckets, buckets)   # no fallback
+
+
+def test_many_candidates_in_one_place():
+    """A wavefront that runs out of its 256 staged candidates: dense tiles between ordinary ones, their zeros put back."""
+    from mccl_amd import hip_ops as ops
+    n = 2_500_000
+    rng = np.random.default_rng(11)
+    grad = student_t(rng, n, ties=0.0) * np.float32(1e-3)
+    for lo in range(0, n, 50_000):
+        grad[lo:lo + 2_000] = student_t(rng, 2_000, ties=0.0)
+    _check(ops, grad, np.zeros(n, np.float32), 0.03, n)
+    grad[::3] = 2.0                          # more equal keys than are picked
+    _check(ops, grad, np.zeros(n, np.float32), 0.05, n)
+    stride = n // 4 // 256 * 4               # the sample misleads: the exact selection, zeros put back first
+    grad = student_t(rng, n, ties=0.0) * np.float32(1e-6)
+    for i in range(0, 256, 2):
+        grad[i * stride: i * stride + 32] = 5.0
+    assert _check(ops, grad, np.zeros(n, np.float32), 0.05, n) == (0, 1)
+
+
+@pytest.mark.parametrize("lengths", [[1_500_001, 65_537, 4097, 5, 3_000_003, 300_007], [1_300_001 - i for i in range(16)] + [3]])
+def test_list_with_many_candidates(lengths):
+    from mccl_amd import hip_ops as ops
+    rng = np.random.default_rng(len(lengths))
+    grads = [student_t(rng, n, ties=0.01) for n in lengths]
+    residuals = [(rng.standard_normal(n) * 1e-4).astype(np.float32) for n in lengths]
+    dres = [to_dev(r, F32) for r in residuals]
+    try:
+        ops.set_tuning("topk_path", 2)
+        wires = ops.topk_compress_list([to_dev(g, F32) for g in grads], dres, 0.05)
+    finally:
+        ops.set_tuning("topk_path", 0)
+    for g, r, d, w in zip(grads, residuals, dres, wires):
+        want, size = oracle.topk_compress(g, r, 0.05)
+        assert w.cpu().numpy()[:size].tobytes() == want.tobytes(), g.size
+        assert np.array_equal(bits(to_np(d, F32)), bits(r)), g.size
