@@ -1503,9 +1503,16 @@ uint64_t zeroed_words(const Geometry& g) {
     return align4((uint64_t)g.nbuckets * kHistWords) + align4((uint64_t)g.nbuckets * kStateWords);
 }
 
-// Groups that the workspace has room for.  (Calls with slots for many candidates cut fewer buckets into more of
-// them; their workspace does not shrink where a bucket more makes them cut into fewer.)
-uint64_t all_groups(const Geometry& g) { return (uint64_t)g.nbuckets * (g.many ? kMaxGroups : 1u << g.gshift); }
+// Groups that the workspace has room for: the most that a call with such tiles cuts its buckets into, so that it does
+// not shrink where a bucket more makes them fewer.
+uint32_t most_groups_shift(const Geometry& g) { return g.many ? 8 : topk_group_shift_few(g.ftiles); }
+uint64_t all_groups(const Geometry& g) { return (uint64_t)g.nbuckets << most_groups_shift(g); }
+
+// `groups`: those of the whole call with as many as that.
+void set_groups(Geometry* g, uint64_t groups) {
+    g->gshift = g->many ? topk_group_shift_many(g->ftiles, groups) : topk_group_shift(g->ftiles, groups);
+    g->ngroups = topk_groups(g->ftiles, g->gshift);
+}
 
 uint64_t workspace_words(const Geometry& g) {
     const uint64_t groups = all_groups(g);
@@ -1540,11 +1547,6 @@ Workspace carve(void* base, const Geometry& g) {
     return w;
 }
 
-void set_groups(Geometry* g, uint32_t shift) {
-    g->gshift = shift;
-    g->ngroups = topk_groups(g->ftiles, shift);
-}
-
 bool make_geometry(uint64_t n_total, uint64_t bucket_elems, double ratio, Geometry* g) {
     if (n_total == 0 || bucket_elems == 0 || n_total > MCCL_HIP_MAX_ELEMS) return false;
     if (bucket_elems > n_total) bucket_elems = n_total;
@@ -1561,7 +1563,7 @@ bool make_geometry(uint64_t n_total, uint64_t bucket_elems, double ratio, Geomet
     g->ftiles = (uint32_t)((bucket_elems + kFTile - 1) / kFTile);
     g->many = topk_many(bucket_elems, ratio) ? 1 : 0;
     g->slots = g->many ? kManySlots : kTileSlots;
-    set_groups(g, g->many ? topk_group_shift_many(g->ftiles, (uint64_t)nb * topk_groups(g->ftiles, 8)) : topk_group_shift(g->ftiles));
+    set_groups(g, nb * topk_groups(g->ftiles, most_groups_shift(*g)));
     // a coarse bin holds about k / 80 candidates when the window is as wide as a sample of 8192
     // leaves it, the bins at the window's lower end three times that; k / 10 + 2048 entries
     // leave room for more uneven ones
@@ -1630,10 +1632,10 @@ void launch_single_pass(const Buckets& call, const Geometry& geometry, const Wor
         for (uint32_t b = 0; b < g.nbuckets; b++) {
             place_bucket(&bk, b, call, order[b], 0);
             tiles += topk_tiles(bk.lcount[b]);
-            groups += topk_groups(topk_tiles(bk.lcount[b]), 8);
+            groups += topk_groups(topk_tiles(bk.lcount[b]), most_groups_shift(g));
         }
         for (uint32_t b = g.nbuckets; b < kMaxListed; b++) bk.lfirst[b] = 0xFFFFFFFFu;
-        if constexpr (MANY) set_groups(&g, topk_group_shift_many(g.ftiles, groups));
+        set_groups(&g, groups);
     }
     if (stream_wide(tiles)) launch_stream<512, LISTED, MANY>(bk, g, w, lim, st);
     else launch_stream<256, LISTED, MANY>(bk, g, w, lim, st);

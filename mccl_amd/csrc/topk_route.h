@@ -20,11 +20,18 @@ constexpr uint64_t kRMaxBlocks = 128;       // resident path: blocks of one buck
 constexpr uint64_t kRVecElems = 4096;       // ... elements per block and vector of a thread
 constexpr uint64_t kRMaxBucket = kRMaxBlocks * kRVecElems * 4;  // 2,097,152 elements
 
-// Groups of tiles per bucket, the power of two: 64 groups, more for buckets that would have more than 28
-// tiles in each: so many a bin or select block keeps in registers, the others it reads again on every
-// pass.  us per call at 1 %, 64 groups against this rule: one bucket of 10 M elements 58 / 47, of 13.1 M 72 / 54, of
-// 26.2 M 136 / 89.
-constexpr uint32_t topk_group_shift(uint64_t tiles) { return tiles <= 64 * 28 ? 6 : tiles <= 128 * 28 ? 7 : 8; }
+// Groups of tiles per bucket, the power of two.  A group is a bin block and a select block, whose wavefronts go
+// through its tiles one after the other, at the end of the call with nothing beside them: the fewer tiles the sooner, as
+// long as the call's select blocks go in one launch of 1024 (`groups`: with topk_group_shift_few for every bucket).
+// us per call at 1 %, 64 groups against 128: one bucket of 2.5 M elements 27.5 / 28.3, of 6,553,600 34.6 / 32.8, five of
+// them 90.7 / 89.6, 15, whose select blocks then go in two launches, 212 / 225; 128 against 256: one of 6,553,600
+// 32.8 / 33.9, of 13 M through compress and decompress 77.4 / 75.4.
+constexpr uint32_t topk_group_shift_few(uint64_t tiles) { return tiles <= 64 * 14 ? 6 : tiles <= 128 * 16 ? 7 : 8; }
+// Otherwise more than 64 only past 28 tiles in each: so many a block keeps in registers, the others it reads again on
+// every pass.  64 groups against more: one bucket of 10 M elements 58 / 47, of 13.1 M 72 / 54, of 26.2 M 136 / 89.
+constexpr uint32_t topk_group_shift(uint64_t tiles, uint64_t groups) {
+    return groups <= 1024 ? topk_group_shift_few(tiles) : tiles <= 64 * 28 ? 6 : tiles <= 128 * 28 ? 7 : 8;
+}
 
 constexpr uint32_t topk_tiles(uint64_t elems) { return (uint32_t)((elems + kFTile - 1) / kFTile); }
 // Tiles of a group and groups of a bucket.  A group has a tile at least for each of a block's four wavefronts.
@@ -56,7 +63,7 @@ inline bool topk_many(uint64_t bucket_elems, double ratio) {
 // after the other: as many groups as keep the call's select launch in one (`groups`: with 256 for every bucket).
 constexpr uint32_t topk_group_shift_many(uint64_t tiles, uint64_t groups) {
     const uint32_t s = groups <= 1024 ? 8 : groups <= 2048 ? 7 : 6;
-    return s > topk_group_shift(tiles) ? s : topk_group_shift(tiles);
+    return s > topk_group_shift(tiles, groups) ? s : topk_group_shift(tiles, groups);
 }
 
 // Whether the blocks of a streaming launch over that many tiles have 512 threads instead of 256.  Their sample

@@ -162,3 +162,15 @@ def test_list_with_many_candidates(lengths):
         want, size = oracle.topk_compress(g, r, 0.05)
         assert w.cpu().numpy()[:size].tobytes() == want.tobytes(), g.size
         assert np.array_equal(bits(to_np(d, F32)), bits(r)), g.size
+
+
+@pytest.mark.parametrize("n, bucket", [
+    (64 * 14 * TILE, 64 * 14 * TILE), (64 * 14 * TILE + 1, 64 * 14 * TILE + 1), (128 * 16 * TILE, 128 * 16 * TILE),
+    (128 * 16 * TILE + 3, 128 * 16 * TILE + 3),
+    (9 * 900 * TILE, 900 * TILE), (8 * 900 * TILE, 900 * TILE)])   # 128 groups each would be more than 1024, and are not
+def test_groups_of_few_buckets(n, bucket):
+    from mccl_amd import hip_ops as ops
+    rng = np.random.default_rng(n)
+    buckets = n // bucket
+    done = _check(ops, student_t(rng, n, ties=0.01), np.zeros(n, np.float32), 0.01, bucket)
+    assert done == (buckets, buckets)
