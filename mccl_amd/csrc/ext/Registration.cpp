@@ -54,6 +54,10 @@ void check_payload(const at::Tensor& wire, const py::object& size, int64_t numel
                    "decompress: compressed_size exceeds the payload tensor");
 }
 
+at::Tensor first_bytes(const at::Tensor& t, size_t n) {
+    return static_cast<size_t>(t.numel()) == n ? t : t.narrow(0, 0, static_cast<int64_t>(n));
+}
+
 uint64_t stable_id_of(const at::Tensor& t) {
     // storage address + offset, stable across steps for DDP buckets
     // (csrc/backend/ProcessGroupMCCL.cpp:1080-1083)
@@ -234,12 +238,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def("compress", [](mccl::TopKCompressor& c, const at::Tensor& t, py::object stable_id, py::object capacity) {
             mccl::check_single_tensor(t);
             const size_t nbytes = mccl::tensor_nbytes(t);
-            const size_t cap = capacity.is_none() ? c.max_compressed_size(nbytes) : capacity.cast<size_t>();
+            const size_t cap = capacity.is_none() ? c.compressed_size(nbytes / sizeof(float)) : capacity.cast<size_t>();
             at::Tensor out = at::empty({static_cast<int64_t>(cap)},
                                        at::TensorOptions().dtype(at::kByte).device(t.device()));
             const uint64_t id = stable_id.is_none() ? stable_id_of(t) : stable_id.cast<uint64_t>();
             const size_t used = c.compress(t.data_ptr(), nbytes, out.data_ptr(), cap, t.scalar_type(), id);
-            return out.narrow(0, 0, static_cast<int64_t>(used));
+            return first_bytes(out, used);
         }, py::arg("tensor"), py::arg("stable_id") = py::none(), py::arg("capacity") = py::none(),
            "Top-k payload of a gradient bucket as a uint8 device tensor; error feedback is kept per stable_id")
         .def("decompress", [](mccl::TopKCompressor& c, const at::Tensor& wire, int64_t numel, py::object size) {
@@ -276,7 +280,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
             at::Tensor out = at::empty({static_cast<int64_t>(cap)},
                                        at::TensorOptions().dtype(at::kByte).device(t.device()));
             const size_t used = c.compress(t.data_ptr(), nbytes, out.data_ptr(), cap, t.scalar_type());
-            return out.narrow(0, 0, static_cast<int64_t>(used));
+            return first_bytes(out, used);
         }, py::arg("tensor"), py::arg("capacity") = py::none(),
            "Half-precision payload of a float32 bucket (a float16 bucket is copied) as a uint8 device tensor")
         .def("decompress", [](mccl::FP16Compressor& c, const at::Tensor& wire, int64_t numel, py::object size,
