@@ -240,6 +240,20 @@ int mccl_hip_topk_decompress_sorted(const void* wire, uint64_t wire_bytes, float
 int mccl_hip_topk_decompress_sorted_flag(const void* wire, uint64_t wire_bytes, float* dense, uint64_t count,
                                          int* status, const int* flag, int* flag_out, void* stream);
 
+/* ... for a caller who waits for the result: the launch writes *host_word (8-byte
+ * aligned, pinned host memory) when everything it stores to dense has arrived,
+ * before the launch itself ends.  The word's upper half is then `ticket`; its lower
+ * half is the value of *flag (0 without one), or MCCL_HIP_ERR_ORDER when the payload
+ * breaks any of mccl_hip_topk_decompress' rules or does not ascend.  `counters`:
+ * MCCL_HIP_DONE_BYTES of device memory, 8-byte aligned, zeroed once and then left to
+ * these calls, which take turns with it (the next is made when the word of the last
+ * has been seen, or on the same stream).  MCCL_HIP_ERR_CAPACITY, and no launch, for
+ * payloads of more than 2^20 pairs: they go through the calls above. */
+#define MCCL_HIP_DONE_BYTES 8448
+int mccl_hip_topk_decompress_sorted_done(const void* wire, uint64_t wire_bytes, float* dense, uint64_t count,
+                                         const int* flag, void* counters, uint64_t* host_word, uint32_t ticket,
+                                         void* stream);
+
 /* Decompress + accumulate of `ws` ranks' payloads into one dense buffer, the
  * sparse equivalent of decompressing every peer's payload and folding the
  * dense buffers in ascending rank order, then the AVG multiply

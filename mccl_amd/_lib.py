@@ -35,6 +35,7 @@ SIGNATURES = {
     "mccl_hip_topk_decompress": (_i32, [_vp, _u64, _vp, _u64, _vp, _vp]),
     "mccl_hip_topk_decompress_sorted": (_i32, [_vp, _u64, _vp, _u64, _vp, _vp]),
     "mccl_hip_topk_decompress_sorted_flag": (_i32, [_vp, _u64, _vp, _u64, _vp, _vp, _vp, _vp]),
+    "mccl_hip_topk_decompress_sorted_done": (_i32, [_vp, _u64, _vp, _u64, _vp, _vp, _vp, _u32, _vp]),
     "mccl_hip_sparse_accumulate": (_i32, [_vp, _u64, _u64, C.POINTER(_vp), _i32, _u64, _i32, _f32, _vp, _vp, _u64, _vp]),
     "mccl_hip_sparse_accumulate_workspace_bytes": (_u64, [_u64, _u64, _i32]),
     "mccl_hip_sparse_accumulate_static": (_i32, [_vp, _u64, _u64, C.POINTER(_vp), _i32, _u64, _i32, _f32, _vp, _vp]),

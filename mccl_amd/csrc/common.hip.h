@@ -36,6 +36,10 @@ __device__ __forceinline__ void store8_agent(void* p, u2a v) {
     asm volatile("global_store_dwordx2 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
 }
 
+__device__ __forceinline__ void store4_agent(float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 enum { kAdd = 0, kMul = 1, kMin = 2, kMax = 3 };
 
 // Maps a c10d reduce-op code to the kernel op set; -1 when unsupported.

@@ -3,6 +3,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
+#include <chrono>
 
 #include "../../../include/mccl_hip.h"
 #include <hip/hip_runtime_api.h>
@@ -104,16 +105,45 @@ void wait_for_current_stream() {
 // calls that wait for the stream anyway: decompress() and check_compress_status().  It is device
 // memory, which goes back to its allocator in stream order: launches may still be under way when the
 // compressor goes (a pinned word would be another tensor's by then).  Caller holds mu_.
+namespace {
+constexpr int64_t kCountersAt = 64;  // words
+
+bool capturing(void* stream) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    if (!stream) return false;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+}  // namespace
+
+// The decompress launches' counters lie behind the word, so that a compressor's first call clears both at once.
+at::Tensor TopKCompressor::zeroed_words() {
+    void* const stream = c10::hip::getCurrentHIPStream().stream();
+    counters_ = at::zeros({kCountersAt + MCCL_HIP_DONE_BYTES / 4}, at::TensorOptions().dtype(at::kInt).device(at::kCUDA));
+    counters_stream_ = stream;
+    counters_usable_ = !capturing(stream);  // else nothing has been cleared
+    counters_seen_ = false;
+    return counters_;
+}
+
 int* TopKCompressor::compress_status() {
-    if (!compress_status_.defined())
-        compress_status_ = at::zeros({1}, at::TensorOptions().dtype(at::kInt).device(at::kCUDA));
-    return compress_status_.data_ptr<int>();
+    if (!words_.defined()) words_ = zeroed_words();
+    compressed_ = true;
+    return words_.data_ptr<int>();
+}
+
+// Counters for a decompress launch on `stream`; null when they belong to another GPU.  Until a launch has reported
+// through them they are known to be zero only in the order of the stream that cleared them.
+void* TopKCompressor::decompress_counters(void* stream) {
+    if (!counters_.defined() || !counters_usable_ || (!counters_seen_ && stream != counters_stream_)) zeroed_words();
+    return counters_.get_device() == c10::hip::current_device() ? counters_.data_ptr<int>() + kCountersAt : nullptr;
 }
 
 // `st`: what the word held when the current stream had been waited for.
 void TopKCompressor::throw_if_compress_failed(int st) {
     if (st == 0) return;
-    compress_status_.zero_();
+    words_.narrow(0, 0, 1).zero_();
     if (st == MCCL_HIP_ERR_TIMEOUT)
         throw TimeoutError("TopK compress: a block gave up waiting for another block of its launch; "
                            "the payloads of that call are invalid");
@@ -122,8 +152,8 @@ void TopKCompressor::throw_if_compress_failed(int st) {
 
 void TopKCompressor::check_compress_status() {
     std::lock_guard<std::mutex> lock(mu_);
-    if (!compress_status_.defined()) return;
-    throw_if_compress_failed(compress_status_.item<int>());
+    if (!compressed_) return;
+    throw_if_compress_failed(words_.select(0, 0).item<int>());
 }
 
 // One bucket on `stream`: csrc/compression/TopKCompression.cpp:38-120.  Caller holds mu_.
@@ -223,42 +253,82 @@ std::vector<at::Tensor> TopKCompressor::compress_many(const std::vector<at::Tens
     return payloads;
 }
 
+// Waits until the decompress launch `ticket` has reported in status_, and returns what it reported: that
+// precedes the end of the launch.  A report that takes longer than half a millisecond - earlier work on the stream -
+// is waited for through the stream, like any other launch.
+int TopKCompressor::wait_for_ticket(uint32_t ticket) {
+    const uint64_t* const word = reinterpret_cast<const uint64_t*>(status_.data_ptr<int>() + 2);
+    uint64_t seen = 0;
+    const auto reported = [&] { return (seen = __atomic_load_n(word, __ATOMIC_ACQUIRE)) >> 32 == ticket; };
+    const auto start = std::chrono::steady_clock::now();
+    for (uint32_t polls = 0; !reported(); polls++) {
+        __builtin_ia32_pause();
+        if ((polls & 63) == 63 && std::chrono::steady_clock::now() - start > std::chrono::microseconds(500)) {
+            counters_usable_ = false;  // should the launch not have ended well
+            wait_for_current_stream();
+            MCCL_CHECK(reported(), "TopK decompress: the launch ended without a result");
+            counters_usable_ = true;
+            break;
+        }
+    }
+    counters_seen_ = true;
+    return static_cast<int>(static_cast<uint32_t>(seen));
+}
+
 // csrc/compression/TopKCompression.cpp:122-152.  The reference validates while
-// it scatters and throws; here the kernel reports through a word in pinned host
-// memory, and brings the compress status to a second one; both are read once the
-// stream has drained, with no copy and no second wait (the call is synchronous, as
-// the reference's is).  A payload that does not ascend, or that breaks a rule, is
-// expanded (again) by the kernels that take pairs in any order.
+// it scatters and throws; here the launch reports in pinned host memory as soon as its
+// stores have arrived, and brings the compress status along: no copy, and no wait for the
+// end of the launch (the call is synchronous, as the reference's is).  A payload that does
+// not ascend, or that breaks a rule, is expanded (again) by the kernels that take pairs in
+// any order.
 void TopKCompressor::decompress(const void* src, size_t compressed_size, void* dst, size_t nbytes,
                                 at::ScalarType dtype) {
     MCCL_CHECK(dtype == at::kFloat, "TopK decompression currently supports float32 only");
     const size_t count = nbytes / sizeof(float);
     std::lock_guard<std::mutex> lock(mu_);
     metal_kernels_init();
-    if (!status_.defined()) status_ = at::zeros({2}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    // int32 0: of the kernels that report a status, 1: the compress status as they bring it; 2, 3: wait_for_ticket's word
+    if (!status_.defined()) status_ = at::zeros({4}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
     int* const word = status_.data_ptr<int>();
     void* const stream = c10::hip::getCurrentHIPStream().stream();
     float* const dense = static_cast<float*>(dst);
-    const int* const flag = compress_status_.defined() ? compress_status_.data_ptr<int>() : nullptr;
-    auto expand = [&](auto launch) {
-        word[0] = word[1] = 0;
-        const int rc = launch();
+    const int* const flag = compressed_ ? words_.data_ptr<int>() : nullptr;
+    const auto launched = [&](int rc) {
         if (rc == MCCL_HIP_ERR_SIZE) throw MCCLError("TopK decompress: size mismatch");
         throw_on_status(rc, "TopK decompress");
+    };
+    auto expand = [&](auto launch) {
+        word[0] = word[1] = 0;
+        launched(launch());
         wait_for_current_stream();
         return *static_cast<const volatile int*>(word);
     };
     int st = MCCL_HIP_ERR_ORDER;
-    if (count)
-        st = expand([&] {
-            return mccl_hip_topk_decompress_sorted_flag(src, compressed_size, dense, count, word, flag, flag ? word + 1 : nullptr, stream);
-        });
-    if (st == 0) {
-        throw_if_compress_failed(*static_cast<const volatile int*>(word + 1));
-        return;
+    if (count) {
+        // (a stream that is being captured refuses the wait, as it always has; the counters serve one GPU)
+        int rc = MCCL_HIP_ERR_CAPACITY;
+        void* const counters = capturing(stream) ? nullptr : decompress_counters(stream);
+        if (counters) {
+            if (++ticket_ == 0) ++ticket_;
+            rc = mccl_hip_topk_decompress_sorted_done(src, compressed_size, dense, count, flag, counters,
+                                                      reinterpret_cast<uint64_t*>(word + 2), ticket_, stream);
+        }
+        if (rc != MCCL_HIP_ERR_CAPACITY) {
+            launched(rc);
+            st = wait_for_ticket(ticket_);
+        } else {
+            st = expand([&] {
+                return mccl_hip_topk_decompress_sorted_flag(src, compressed_size, dense, count, word, flag, flag ? word + 1 : nullptr, stream);
+            });
+            if (st == 0) st = *static_cast<const volatile int*>(word + 1);
+        }
+        if (st != MCCL_HIP_ERR_ORDER && st != MCCL_HIP_ERR_SIZE && st != MCCL_HIP_ERR_INDEX) {
+            throw_if_compress_failed(st);
+            return;
+        }
     }
     st = expand([&] { return mccl_hip_topk_decompress(src, compressed_size, dense, count, word, stream); });
-    if (flag) throw_if_compress_failed(compress_status_.item<int>());
+    if (flag) throw_if_compress_failed(words_.select(0, 0).item<int>());
     if (st == MCCL_HIP_ERR_SIZE) throw MCCLError("TopK decompress: size mismatch");
     if (st == MCCL_HIP_ERR_INDEX) throw MCCLError("TopK decompress: index out of bounds");
 }

@@ -77,3 +77,66 @@ def test_unordered_payloads_take_the_other_kernels(k):
         comp.decompress(w, int(idx[-1]))
     w[:4] = 0
     assert _status(w, n)[1] == oracle.ERR_SIZE
+
+
+@pytest.mark.parametrize("n", [8192, 64 * 8192, 64 * 8192 + 1, 97 * 8192 + 5])  # one block, and both ways of arriving
+def test_calls_that_report_before_their_launch_ends(n):
+    """Good payloads between ones that break a rule, on two streams in turn and behind earlier work: every call sees its
+    own report, and the counters are left as they were found."""
+    from mccl_amd import _C
+    rng = np.random.default_rng(n)
+    k = n // 50
+    comp = _C.TopKCompressor(0.02)
+    other = torch.cuda.Stream()
+    idx = np.sort(rng.choice(n - 1, k, replace=False)).astype(np.uint32)
+    sw = idx.copy()
+    sw[k // 2], sw[k // 2 + 1] = idx[k // 2 + 1], idx[k // 2]
+    past = idx.copy()
+    past[-1] = n
+    for i in range(6):
+        with torch.cuda.stream(other if i % 2 else torch.cuda.default_stream()):
+            for ids in (idx, sw, past):
+                w = _payload(ids, rng.standard_normal(k).astype(np.float32))
+                dw = torch.from_numpy(w).to(DEV)
+                if i >= 4:
+                    torch.cuda._sleep(5_000_000)   # a few milliseconds
+                if ids is past:
+                    with pytest.raises(RuntimeError, match="index out of bounds"):
+                        comp.decompress(dw, n)
+                else:
+                    want, _ = oracle.topk_decompress(w, n)
+                    assert np.array_equal(bits(to_np(comp.decompress(dw, n), F32)), bits(want))
+
+
+def test_reports_of_the_entry_point():
+    from mccl_amd import _lib
+    lib = _lib.load()
+    n, k = 700_001, 7000
+    rng = np.random.default_rng(5)
+    counters = torch.zeros(8448 // 8, dtype=torch.int64, device=DEV)
+    word = torch.zeros(1, dtype=torch.int64).pin_memory()
+    flag = torch.zeros(1, dtype=torch.int32, device=DEV)
+    idx = np.sort(rng.choice(n, k, replace=False)).astype(np.uint32)
+    rep = idx.copy()
+    rep[1] = rep[0]
+    dense = torch.empty(n, device=DEV)
+    for ticket, (ids, count, f, want) in enumerate([(idx, k, 0, 0), (idx, k, -10, -10), (rep, k, 0, -11), (idx, k - 1, 0, -11),
+                                                    (idx, k, 0, 0)], 1):
+        w = _payload(ids, np.ones(k, np.float32))
+        w.view(np.uint32)[0] = count
+        dw = torch.from_numpy(w).to(DEV)
+        flag.fill_(f)
+        dense.fill_(3.0)
+        assert lib.mccl_hip_topk_decompress_sorted_done(
+            ct.c_void_p(dw.data_ptr()), dw.numel(), ct.c_void_p(dense.data_ptr()), n, ct.c_void_p(flag.data_ptr()),
+            ct.c_void_p(counters.data_ptr()), ct.c_void_p(word.data_ptr()), ticket, None) == 0
+        torch.cuda.synchronize()
+        v = int(word) & (2 ** 64 - 1)
+        assert (v >> 32, v & 0xFFFFFFFF) == (ticket, want & 0xFFFFFFFF)
+        assert not counters.any()
+        if want != -11:
+            assert int(dense.sum()) == k and int((dense == 0).sum()) == n - k
+    many = torch.empty(4 + 8 * (2 ** 20 + 1), dtype=torch.uint8, device=DEV)   # more than 2^20 pairs: not launched
+    assert lib.mccl_hip_topk_decompress_sorted_done(
+        ct.c_void_p(many.data_ptr()), many.numel(), ct.c_void_p(dense.data_ptr()), n, None, ct.c_void_p(counters.data_ptr()),
+        ct.c_void_p(word.data_ptr()), 99, None) == -3
