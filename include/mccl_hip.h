@@ -332,7 +332,7 @@ int mccl_hip_sync(void* stream);
 /* keys: "fold_blocks_per_cu", "nontemporal", "topk_path" (0 auto, 1 exact, 2 single-pass, 3 resident where one launch may take the call), "topk_barrier_ms", "topk_stall_test" (tests: 1 makes every wait
  * of the single-pass top-k path run into its limit, so that the give-up path can be exercised
  * without a stuck kernel),
- * "sparse_path" (0 auto, 1 tile kernels only, 2 position table always), "sparse_run_steps" (0 auto),
+ * "sparse_path" (0 auto, 1 tile kernels only, 2 runs with a position table, 3 runs wherever they can), "sparse_run_steps" (0 auto),
  * "fp16_portable" (1: the casts follow the reference's portable branch, FP16Compression.cpp:38-73,:96-111) */
 int mccl_hip_set_tuning(const char* key, int value);
 int mccl_hip_get_tuning(const char* key);

@@ -25,7 +25,7 @@ struct Tuning {
     int topk_stall_test = 0;     // tests only: 1 = the sample blocks publish a wrong epoch, so that every wait of the single-pass path runs into its limit
     int topk_barrier_ms = 2000;  // single-pass path: longest wait of a block for another block of its launch
     int fp16_portable = 0;       // FP16 casts: 1 = the reference's portable branch (half subnormals flushed, NaN bits passed through)
-    int sparse_path = 0;         // sparse accumulate with a workspace: 0 auto (runs of tiles up to 8 ranks), 1 tile kernels only, 2 runs with a position table
+    int sparse_path = 0;         // sparse accumulate with a workspace: 0 auto, 1 tile kernels only, 2 runs with a position table, 3 runs wherever they can
     int sparse_run_steps = 0;    // runs of tiles: 2048-element tiles per wavefront, 0 = from the input's size
 };
 Tuning& tuning();

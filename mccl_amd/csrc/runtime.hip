@@ -166,7 +166,7 @@ int mccl_hip_set_tuning(const char* key, int value) {
     } else if (!std::strcmp(key, "fp16_portable")) {
         t.fp16_portable = value ? 1 : 0;
     } else if (!std::strcmp(key, "sparse_path")) {
-        if (value < 0 || value > 2) return MCCL_HIP_ERR_ARG;
+        if (value < 0 || value > 3) return MCCL_HIP_ERR_ARG;
         t.sparse_path = value;
     } else if (!std::strcmp(key, "sparse_run_steps")) {
         if (value < 0 || value > (1 << 20)) return MCCL_HIP_ERR_ARG;

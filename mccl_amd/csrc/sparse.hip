@@ -459,7 +459,7 @@ __global__ __launch_bounds__(kAccThreads) void k_sparse_accumulate_b(float* acc,
 // an earlier run.
 constexpr int kRunL = 2048;    // elements per tile of a wavefront (1024 and 4096 measured 4-5 % slower)
 constexpr int kRunWaves = 8;   // wavefronts (= runs) per block: 64 KiB of LDS, two blocks per CU (4 measured 3 % slower, 2 slower still)
-constexpr int kRunRanks = 8;   // ranks a wavefront holds windows for; larger worlds use the tile kernels
+constexpr int kRunRanks = 12;  // ranks a wavefront holds windows for (12: 122 registers of 128); larger worlds use the tile kernels
 constexpr int kWin = kWave;    // pairs per window
 constexpr int kStride = 80;    // pairs between two sampled indices of the position table: five 128-byte lines,
                                // so a run begins with at most 79 pairs of an earlier run in its first window
@@ -604,7 +604,8 @@ __device__ __forceinline__ uint32_t block_starts(const uint8_t* wire, uint32_t k
     return mine;
 }
 
-// NR: ranks the code is unrolled for (ws <= NR; the ranks past ws read rank 0's payload as if
+// NR: ranks the code is unrolled for (six ranks as eight, at 2 %: 94.6 us for 90 M elements, as six 85.8; 9 to 12 ranks,
+// 50 M at 1 %: tile kernels 70 to 80 us, so 57 to 66) (ws <= NR; the ranks past ws read rank 0's payload as if
 // its k were 0).  wire_stride holds at least one pair.  OWN: no position table, the block finds
 // where its runs begin (one bucket, at most kOwnSamples * 64 samples a payload).
 template <int NR, bool OWN>
@@ -624,6 +625,7 @@ __global__ __launch_bounds__(kRunWaves * kWave, 4) void k_sparse_accumulate_runs
     const uint64_t grun = (uint64_t)vblock * kRunWaves + (uint32_t)wave;
     __shared__ uint32_t own[kRunWaves][NR];
     if constexpr (OWN) {
+        static_assert(NR <= kRunWaves, "a rank per wavefront");
         if (wave < ws) {
             const uint64_t run_elems = (uint64_t)run_steps * kRunL;
             bool unsorted;
@@ -786,9 +788,9 @@ __global__ __launch_bounds__(kRunWaves * kWave, 4) void k_sparse_accumulate_runs
 }
 
 // Validates the arguments and enqueues the kernels; `workspace` (may be null:
-// scratch-free kernel) is known to be large enough.
+// scratch-free kernel) is known to be large enough.  `shared_table`: it is not the caller's own.
 int accumulate(float* acc, uint64_t n_total, uint64_t bucket_elems, const void* const* host_wires, int ws,
-               uint64_t wire_stride, int apply_scale, float scale, int* status, void* workspace,
+               uint64_t wire_stride, int apply_scale, float scale, int* status, void* workspace, bool shared_table,
                void* stream) {
     if (!acc || !host_wires || ws < 1 || ws > MCCL_HIP_MAX_WORLD) return MCCL_HIP_ERR_ARG;
     if (n_total == 0 || n_total > MCCL_HIP_MAX_ELEMS || bucket_elems == 0) return MCCL_HIP_ERR_ARG;
@@ -818,12 +820,17 @@ int accumulate(float* acc, uint64_t n_total, uint64_t bucket_elems, const void* 
     // pairs of one rank in a 2048-element tile when the payload is full
     const uint64_t steps_bucket = (bucket_elems + kRunL - 1) / kRunL;
     const uint64_t per_tile = (kmax + steps_bucket - 1) / steps_bucket;
-    if (ws <= kRunRanks && tuning().sparse_path != 1 && per_tile <= 96 && kmax >= 1 &&
-        (kmax + kStride - 1) / kStride <= kStartSamples) {
+    const int path = tuning().sparse_path;
+    const uint64_t samples = (kmax + kStride - 1) / kStride;
+    bool runs_take = ws <= kRunRanks && path != 1 && per_tile <= 96 && kmax >= 1 && samples <= kStartSamples;
+    uint64_t run_steps = 1, blocks = 0;
+    uint32_t runs = 0;
+    bool own = false;
+    if (runs_take) {
         // a run is as many tiles as bring about 96 pairs of a rank: with up to 79 pairs of the run
         // before it in the first window, the three windows requested at its start (192 pairs) hold a
         // run of the usual density whole, and it never loads again
-        uint64_t run_steps = (uint64_t)tuning().sparse_run_steps;
+        run_steps = (uint64_t)tuning().sparse_run_steps;
         if (run_steps == 0) run_steps = per_tile ? 96 / per_tile : 8;
         if (run_steps > 8 && tuning().sparse_run_steps == 0) run_steps = 8;
         // ... but no more than leave every CU eight wavefronts: a wavefront's tiles follow one another,
@@ -834,27 +841,42 @@ int accumulate(float* acc, uint64_t n_total, uint64_t bucket_elems, const void* 
         if (run_steps > spread && tuning().sparse_run_steps == 0) run_steps = spread;
         if (run_steps < 1) run_steps = 1;
         if (run_steps > steps_bucket) run_steps = steps_bucket;
-        const uint32_t runs = (uint32_t)((steps_bucket + run_steps - 1) / run_steps);
-        const uint64_t blocks = ((uint64_t)runs * nb + kRunWaves - 1) / kRunWaves;
+        runs = (uint32_t)((steps_bucket + run_steps - 1) / run_steps);
+        blocks = ((uint64_t)runs * nb + kRunWaves - 1) / kRunWaves;
         // One bucket whose blocks all fit the GPU at once: a block finds its runs' starts itself, if
         // that takes it no more than some 2048 samples over all ranks - each is a memory sector.  us per
         // call, position table against this: 8 ranks of 1 M elements (1000 samples) 12.4 / 11.1, 4 of 2 M
         // (1000) 10.0 / 8.2, 2 of 3 M at 2 % (1500) 10.8 / 8.4, but 8 of 6.5 M (6552) 16.6 / 19.6
-        const uint64_t samples = (kmax + kStride - 1) / kStride;
-        const bool own = nb == 1 && blocks <= kOwnBlocks && samples <= (uint64_t)kOwnSamples * kWave &&
-                         samples * (uint64_t)ws <= kOwnTotal && tuning().sparse_path != 2;
+        own = nb == 1 && ws <= kRunWaves && blocks <= kOwnBlocks && samples <= (uint64_t)kOwnSamples * kWave &&
+              samples * (uint64_t)ws <= kOwnTotal && path != 2;
+        // Where the tile kernels take less time all the same: a wavefront's ranks follow one another, a block of theirs
+        // has eight wavefronts for a tile.  That tells while the call leaves CUs idle or is dense, and for more ranks
+        // than eight.  us per call, runs against tiles: at 1 % 8 ranks of 250,000 elements 11.1 / 9.5, of 6 M 15.6 / 12.5, of
+        // 13 M 19.8 / 20.2, 5 ranks of 6 M 13.7 / 11.2, of 13 M 17.5 / 17.9, 3 of 3 M (which find their starts) 8.7 / 9.4, of 6 M
+        // 11.6 / 10.5, 12 of 13 M 26.4 / 24.6, of 26 M 39.3 / 46.4; at 2 % 8 of 26 M 45.8 / 40.2, of 60 M 82 / 95, 3 of 26 M
+        // 29.0 / 26.7, of 60 M 51.8 / 68.1, 9 of 96.5 M 134 / 127, 12 164 / 148; at 0.1 % 9 of 13 M 19.6 / 20.2.
+        const uint64_t few = per_tile > 32 ? 32u << 20 : ws > kRunWaves && per_tile > 8 ? 16u << 20 : 8u << 20;
+        const bool tiles_faster = ws > kRunWaves && per_tile > 32 ? true : n_total <= few && (ws >= 5 || (ws >= 2 && !own));
+        // (calls that share a table keep to the runs, which notice a table that is not theirs, and to eight ranks)
+        if (path == 0 && tuning().sparse_run_steps == 0) runs_take = shared_table ? ws <= kRunWaves : !tiles_faster;
+    }
+    if (runs_take) {
         if (!own)
             k_sparse_starts<<<(uint32_t)(nb * ws), kStartThreads, 0, st>>>(wp, ws, wire_stride,
                                                                             (uint32_t)(run_steps * kRunL), runs, start, status);
         const uint32_t per_xcd = (uint32_t)((blocks + kXcds - 1) / kXcds);
 #define MCCLHIP_RUNS(NR)                                                                               \
-    (own ? k_sparse_accumulate_runs<NR, true> : k_sparse_accumulate_runs<NR, false>)<<<per_xcd * kXcds, kRunWaves * kWave, 0, st>>>(                        \
+    (own ? k_sparse_accumulate_runs<(NR <= kRunWaves ? NR : 1), true> : k_sparse_accumulate_runs<NR, false>)<<<per_xcd * kXcds, kRunWaves * kWave, 0, st>>>(                        \
         acc, n_total, bucket_elems, wp, ws, wire_stride, (uint32_t)run_steps, runs, (uint32_t)nb, per_xcd, \
         start, apply_scale, scale, status)
         if (ws == 1) MCCLHIP_RUNS(1);
         else if (ws == 2) MCCLHIP_RUNS(2);
-        else if (ws <= 4) MCCLHIP_RUNS(4);
-        else MCCLHIP_RUNS(8);
+        else if (ws == 3) MCCLHIP_RUNS(3);
+        else if (ws == 4) MCCLHIP_RUNS(4);
+        else if (ws <= 6) MCCLHIP_RUNS(6);
+        else if (ws <= 8) MCCLHIP_RUNS(8);
+        else if (ws <= 10) MCCLHIP_RUNS(10);
+        else MCCLHIP_RUNS(12);
 #undef MCCLHIP_RUNS
         return launch_status();
     }
@@ -963,7 +985,7 @@ int mccl_hip_sparse_accumulate(float* acc, uint64_t n_total, uint64_t bucket_ele
     if (workspace && workspace_bytes < mccl_hip_sparse_accumulate_workspace_bytes(n_total, bucket_elems, ws))
         return MCCL_HIP_ERR_WORKSPACE;
     return accumulate(acc, n_total, bucket_elems, host_wires, ws, wire_stride, apply_scale, scale, status,
-                      workspace, stream);
+                      workspace, false, stream);
 }
 
 int mccl_hip_sparse_accumulate_static(float* acc, uint64_t n_total, uint64_t bucket_elems,
@@ -977,7 +999,7 @@ int mccl_hip_sparse_accumulate_static(float* acc, uint64_t n_total, uint64_t buc
     const int dev = device_info().device;
     if (dev < 0 || dev >= kMaxDevices || !g_static_ptr[dev]) return MCCL_HIP_ERR_RUNTIME;
     return accumulate(acc, n_total, bucket_elems, host_wires, ws, wire_stride, apply_scale, scale, status,
-                      g_static_ptr[dev], stream);
+                      g_static_ptr[dev], true, stream);
 }
 
 }  // extern "C"

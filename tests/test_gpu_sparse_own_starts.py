@@ -61,3 +61,49 @@ def test_payloads_out_of_order_are_flagged(at):
         finally:
             hip_ops.set_tuning("sparse_path", 0)
         assert int(status) == oracle.ERR_INDEX, path
+
+
+@pytest.mark.parametrize("ws,n,be,k", [
+    (5, 2049, 2049, 81), (6, 16385, 16385, 161), (8, 1_000_001, 1_000_001, 10_000),   # a block finds its runs' starts
+    (9, 2049, 2049, 20), (10, 300_001, 100_000, 1000), (11, 65_537, 65_537, 700), (12, 1_000_003, 400_000, 4000),
+    (12, 30_000, 30_000, 1400),                                                       # more pairs than the windows hold
+    (3, 40_000_000, 6_553_600, 60_000), (10, 9_000_001, 6_553_600, 65_536)])          # on either side of the rule's lines
+def test_runs_and_tiles(ws, n, be, k):
+    """The runs for up to twelve ranks, forced and where the sizes choose them, and the tile kernels."""
+    rng = np.random.default_rng(n + ws)
+    buckets = [min(be, n - lo) for lo in range(0, n, be)]
+    per_rank = []
+    for r in range(ws):
+        row = []
+        for m in buckets:
+            kr = max(1, min(m, k) - r)
+            idx = np.unique(rng.integers(0, m, kr)) if m > 1_000_000 else np.sort(rng.choice(m, kr, replace=False))
+            row.append((idx, rng.standard_normal(idx.size).astype(np.float32)))
+        per_rank.append(row)
+    run_case(hip_ops, per_rank, n, be, 1.0 / ws, paths=("auto", "tiles"))
+    hip_ops.set_tuning("sparse_run_steps", 2)   # (the runs, whatever the size)
+    try:
+        run_case(hip_ops, per_rank, n, be, 1.0 / ws, paths=("auto",))
+    finally:
+        hip_ops.set_tuning("sparse_run_steps", 0)
+
+
+@pytest.mark.parametrize("ws", [6, 9, 12])
+@pytest.mark.parametrize("at", [0, 63, 79, 80, 3000])
+def test_many_ranks_flag_payloads_out_of_order(ws, at):
+    n, k = 300_000, 3003
+    rng = np.random.default_rng(at)
+    wires = []
+    for r in range(ws):
+        idx = np.sort(rng.choice(n, k, replace=False))
+        if r == ws - 1:
+            idx[[at, at + 1]] = idx[[at + 1, at]]
+        wires.append(torch.from_numpy(payload(idx, np.ones(k, np.float32), k)).to(DEV))
+    for path in (0, 1, 2, 3):
+        status = torch.zeros(1, dtype=torch.int32, device=DEV)
+        hip_ops.set_tuning("sparse_path", path)
+        try:
+            hip_ops.sparse_accumulate(torch.empty(n, device=DEV), wires, 4 + 8 * k, bucket_elems=n, status=status)
+        finally:
+            hip_ops.set_tuning("sparse_path", 0)
+        assert int(status) == oracle.ERR_INDEX, path
