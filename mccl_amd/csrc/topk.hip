@@ -1511,7 +1511,7 @@ uint64_t all_groups(const Geometry& g) { return (uint64_t)g.nbuckets << most_gro
 // `groups`: those of the whole call with as many as that.
 void set_groups(Geometry* g, uint64_t groups) {
     g->gshift = g->many ? topk_group_shift_many(g->ftiles, groups) : topk_group_shift(g->ftiles, groups);
-    g->ngroups = topk_groups(g->ftiles, g->gshift);
+    g->ngroups = topk_launched_groups(g->ftiles, topk_tiles(g->n_total - (uint64_t)(g->nbuckets - 1) * g->bucket_elems), g->gshift);
 }
 
 uint64_t workspace_words(const Geometry& g) {

@@ -55,7 +55,7 @@ struct Geometry {
     uint32_t listed;   // single-pass path: 1 when the buckets are separate buffers (see Buckets)
     uint32_t ftiles;   // single-pass path: streaming tiles allotted per bucket
     uint32_t gshift;   // single-pass path: at most 1 << gshift groups of tiles per bucket
-    uint32_t ngroups;  // single-pass path: groups of a (full) bucket
+    uint32_t ngroups;  // single-pass path: groups of the bucket with the most of them (topk_launched_groups)
     uint32_t many;     // single-pass path: 1 when tiles have slots for many candidates (topk_many)
     uint32_t slots;    // single-pass path: candidate slots of a tile
     uint32_t lcapb;    // single-pass path: capacity of one coarse bin's list (entries)

@@ -42,6 +42,11 @@ constexpr uint32_t topk_group_tiles(uint32_t tiles, uint32_t shift) {
 constexpr uint32_t topk_groups(uint32_t tiles, uint32_t shift) {
     return (tiles + topk_group_tiles(tiles, shift) - 1) / topk_group_tiles(tiles, shift);
 }
+// Groups that the launches of a buffer's buckets have blocks for, for each bucket: a shorter last bucket can have more of
+// them than the others (of at most 128, 1600 tiles make 124 of 13, 1536 make 128 of 12).
+constexpr uint32_t topk_launched_groups(uint32_t tiles, uint32_t last_tiles, uint32_t shift) {
+    return topk_groups(tiles, shift) > topk_groups(last_tiles, shift) ? topk_groups(tiles, shift) : topk_groups(last_tiles, shift);
+}
 
 // Expected share of a bucket inside the sampled window (see sample_window).
 inline double window_share(double ratio) {

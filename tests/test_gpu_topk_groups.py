@@ -174,3 +174,25 @@ def test_groups_of_few_buckets(n, bucket):
     buckets = n // bucket
     done = _check(ops, student_t(rng, n, ties=0.01), np.zeros(n, np.float32), 0.01, bucket)
     assert done == (buckets, buckets)
+
+
+@pytest.mark.parametrize("tiles, last, ratio", [(520, 512, 0.01),     # 58 groups, the last bucket 64
+                                                (1600, 1536, 0.01),   # 124 and 128
+                                                (1600, 1536, 0.05)])  # 229 and 256, slots for many candidates
+def test_last_bucket_with_more_groups(tiles, last, ratio):
+    from mccl_amd import hip_ops as ops
+    bucket, n = tiles * TILE, (tiles + last) * TILE
+    rng = np.random.default_rng(tiles + last)
+    grad = student_t(rng, n, ties=0.01)
+    res = (rng.standard_normal(n) * 1e-4).astype(np.float32)
+    dres = to_dev(res, F32)
+    ws = ops.topk_workspace(n, bucket, ratio, DEV)
+    wire, stride = ops.topk_compress(to_dev(grad, F32), dres, ratio, bucket_elems=bucket, workspace=ws)
+    w = wire.cpu().numpy()
+    assert ops.topk_path_report(ws, n, bucket, ratio) == (2, 2)
+    for b, lo in enumerate(range(0, n, bucket)):
+        part = res[lo:lo + bucket].copy()
+        want, size = oracle.topk_compress(grad[lo:lo + bucket], part, ratio)
+        res[lo:lo + bucket] = part
+        assert w[b * stride: b * stride + size].tobytes() == want.tobytes(), b
+    assert np.array_equal(bits(to_np(dres, F32)), bits(res))

@@ -189,3 +189,33 @@ def test_admitted_launches_always_end(tmp_path):
                     str(exe)], check=True)
     p = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True, timeout=100)
     assert p.returncode == 0, p.stdout[:2000]
+
+
+GROUPS = r"""
+#include "topk_route.h"
+#include <cstdio>
+using namespace mcclhip;
+int main() {
+    int more = 0;
+    for (uint32_t shift = 6; shift <= 8; shift++)
+        for (uint32_t tiles = 1; tiles <= 4000; tiles += tiles < 700 ? 1 : 13)
+            for (uint32_t last = 1; last <= tiles; last++) {
+                const uint32_t launched = topk_launched_groups(tiles, last, shift);
+                more += topk_groups(last, shift) > topk_groups(tiles, shift);
+                if (launched < topk_groups(tiles, shift) || launched < topk_groups(last, shift) || launched > 1u << shift) {
+                    std::printf("%u tiles, the last bucket %u, shift %u: %u\n", tiles, last, shift, launched);
+                    return 1;
+                }
+            }
+    return more > 1000 ? 0 : 2;
+}
+"""
+
+
+def test_a_shorter_last_bucket_has_all_its_groups(tmp_path):
+    src, exe = tmp_path / "groups.cpp", tmp_path / "groups"
+    src.write_text(GROUPS)
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", "-I", os.path.join(ROOT, "mccl_amd", "csrc"), str(src), "-o",
+                    str(exe)], check=True)
+    p = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True, timeout=100)
+    assert p.returncode == 0, p.stdout[:2000]
