@@ -45,7 +45,11 @@ def per_kernel(path: str, counter: str) -> dict:
             if "k_ring_fold" in name and "k_ring_fold<6, 0, true, 8>" not in name:
                 continue                                  # only the fp32 SUM fold of 8 ranks (config 2)
             # config 5 (8 ranks, with a workspace) runs k_sparse_starts + k_sparse_accumulate_runs; the
-            # bench's other sparse lines run other kernels, which are left out here
+            # bench's other sparse lines (twelve ranks, no workspace) are left out here
+            if "k_sparse_accumulate_runs" in name and "k_sparse_accumulate_runs<8," not in name:
+                continue
+            if "k_sparse_starts" in name and int(row["Grid_Size"]) != 15 * 8 * 1024:  # a block per bucket and rank
+                continue
             for key in ("k_ring_fold", "k_topk_stream", "k_topk_select", "k_sparse_starts",
                         "k_sparse_accumulate_runs", "copyBuffer"):
                 if key in name:
