@@ -75,7 +75,9 @@ TopKCompressor::TopKCompressor(double k_ratio) : k_ratio_(k_ratio) {
     MCCL_CHECK(k_ratio > 0 && k_ratio <= 1.0, "k_ratio must be in (0, 1], got " + std::to_string(k_ratio));
 }
 
-TopKCompressor::~TopKCompressor() = default;
+TopKCompressor::~TopKCompressor() {
+    if (end_) (void)hipEventDestroy(static_cast<hipEvent_t>(end_));
+}
 
 // The residual map keeps the reference's rules (csrc/compression/TopKCompression.cpp:57-67):
 // a new id while 1024 ids are live clears the map; an id whose element count changed starts
@@ -253,6 +255,24 @@ std::vector<at::Tensor> TopKCompressor::compress_many(const std::vector<at::Tens
     return payloads;
 }
 
+// Marks the end of the launch on its stream, which the host does while it would only poll.  A program that waits for the
+// stream or the GPU right behind the call has such a marker put there, and waits for that one, unless one is there
+// already.  Compress and decompress at 1 % with a wait for the GPU behind them, us, waiting for the stream / reporting /
+// reporting with the marker: 2000 elements 24.8 / 29.0 / 23.0, 65,537 32.6 / 36.4 / 30.5, 6,553,600 56.8 / 61.7 / 55.7.
+void TopKCompressor::mark_end(void* stream) {
+    if (end_ && end_device_ != counters_.get_device()) {
+        (void)hipEventDestroy(static_cast<hipEvent_t>(end_));
+        end_ = nullptr;
+    }
+    if (!end_) {
+        hipEvent_t event = nullptr;
+        if (hipEventCreateWithFlags(&event, hipEventDisableTiming) == hipSuccess) end_ = event;
+        end_device_ = counters_.get_device();
+    }
+    // (nothing but time depends on it)
+    if (!end_ || hipEventRecord(static_cast<hipEvent_t>(end_), static_cast<hipStream_t>(stream)) != hipSuccess) (void)hipGetLastError();
+}
+
 // Waits until the decompress launch `ticket` has reported in status_, and returns what it reported: that
 // precedes the end of the launch.  A report that takes longer than half a millisecond - earlier work on the stream -
 // is waited for through the stream, like any other launch.
@@ -315,6 +335,7 @@ void TopKCompressor::decompress(const void* src, size_t compressed_size, void* d
         }
         if (rc != MCCL_HIP_ERR_CAPACITY) {
             launched(rc);
+            mark_end(stream);
             st = wait_for_ticket(ticket_);
         } else {
             st = expand([&] {

@@ -81,9 +81,9 @@ constexpr uint32_t kDecMaxStride = 4096;  // beyond (over a million pairs) fill 
 
 // DONE: the launch tells the host when its stores have arrived, in one word of pinned host memory; the end of the
 // launch itself reaches a host that waits for the stream 5.4 us after such a word does (a launch of one block: 11.6
-// against 6.1 us).  Compress and decompress at 1 %, us until the call returns: 2000 elements 22.4 / 18.3, 65,537 29.5 / 24.9, 6,553,600
-// 58.0 / 49.5 (3 of that by the launches' other changes); a program that waits for the whole GPU right behind the call meets the launch's end there (65,537
-// elements with that wait 32.5 / 36.4, 6,553,600 60.3 / 60.4).  A block arrives when its stores - written past the L2 - have been acknowledged; the block
+// against 6.1 us).  Compress and decompress at 1 %, us, waiting for the stream / the word, until the call returns and with a fold
+// of the result behind it: 2000 elements 22.5 / 18.1 and 25.6 / 22.0, 65,537 29.7 / 25.3 and 33.0 / 28.5, 6,553,600
+// 53.5 / 50.9 and 67.6 / 64.4.  A block arrives when its stores - written past the L2 - have been acknowledged; the block
 // that arrives last has seen the others arrive, and nobody waits.  Arrivals at one word take turns, some 25 ns
 // each, so that larger grids arrive at 32 words and those at one.
 constexpr uint32_t kDoneLines = 32;

@@ -2,6 +2,7 @@
 against the oracle at the edges of its tiles (8192 elements) and of its 256 samples, for spread,
 clustered, unordered and repeated indices, and for indices past the end."""
 import ctypes as ct
+import time
 
 import numpy as np
 import pytest
@@ -140,3 +141,32 @@ def test_reports_of_the_entry_point():
     assert lib.mccl_hip_topk_decompress_sorted_done(
         ct.c_void_p(many.data_ptr()), many.numel(), ct.c_void_p(dense.data_ptr()), n, None, ct.c_void_p(counters.data_ptr()),
         ct.c_void_p(word.data_ptr()), 99, None) == -3
+
+
+@pytest.mark.parametrize("n", [2000, 65_537, 6_553_600])
+def test_waiting_right_behind_a_call(n):
+    """A program that waits for the GPU behind the call finds the marker of the launch's end on the stream: it waits for
+    less than a launch and its marker take (measured 0.4 of that; 0.8 where the wait has to put a marker there)."""
+    from mccl_amd import _C, hip_ops
+    comp = _C.TopKCompressor(0.01)
+    wire = comp.compress(torch.randn(n, device=DEV), stable_id=1)
+    x = torch.zeros(64, device=DEV)
+
+    def best(call, wait):
+        times = []
+        for _ in range(300):
+            start = time.perf_counter()
+            call()
+            if wait:
+                torch.cuda.synchronize()
+            times.append(time.perf_counter() - start)
+            torch.cuda.synchronize()
+        return min(times)
+
+    def back():
+        return comp.decompress(wire, n)
+
+    launch = best(lambda: hip_ops.fold2(x, x, hip_ops.SUM), True)
+    returns, idle = best(back, False), best(back, True)
+    print(f"{n}: launch {launch * 1e6:.1f} returns {returns * 1e6:.1f} idle {idle * 1e6:.1f}")
+    assert idle - returns < 0.6 * launch, (launch, returns, idle)
