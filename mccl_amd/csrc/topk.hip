@@ -1508,9 +1508,9 @@ uint64_t zeroed_words(const Geometry& g) {
 uint32_t most_groups_shift(const Geometry& g) { return g.many ? 8 : topk_group_shift_few(g.ftiles); }
 uint64_t all_groups(const Geometry& g) { return (uint64_t)g.nbuckets << most_groups_shift(g); }
 
-// `groups`: those of the whole call with as many as that.
-void set_groups(Geometry* g, uint64_t groups) {
-    g->gshift = g->many ? topk_group_shift_many(g->ftiles, groups) : topk_group_shift(g->ftiles, groups);
+// `groups`: those of the whole call with as many as that; `fits`: see topk_group_shift_fits.
+void set_groups(Geometry* g, uint64_t groups, uint64_t fits) {
+    g->gshift = topk_shift(g->ftiles, groups, g->many != 0, fits);
     g->ngroups = topk_launched_groups(g->ftiles, topk_tiles(g->n_total - (uint64_t)(g->nbuckets - 1) * g->bucket_elems), g->gshift);
 }
 
@@ -1563,7 +1563,7 @@ bool make_geometry(uint64_t n_total, uint64_t bucket_elems, double ratio, Geomet
     g->ftiles = (uint32_t)((bucket_elems + kFTile - 1) / kFTile);
     g->many = topk_many(bucket_elems, ratio) ? 1 : 0;
     g->slots = g->many ? kManySlots : kTileSlots;
-    set_groups(g, nb * topk_groups(g->ftiles, most_groups_shift(*g)));
+    g->gshift = g->ngroups = 0;  // launch_single_pass' part
     // a coarse bin holds about k / 80 candidates when the window is as wide as a sample of 8192
     // leaves it, the bins at the window's lower end three times that; k / 10 + 2048 entries
     // leave room for more uneven ones
@@ -1616,7 +1616,7 @@ void launch_stream(Buckets& bk, const Geometry& g, const Workspace& w, uint64_t 
 }
 
 template <bool LISTED, bool MANY>
-void launch_single_pass(const Buckets& call, const Geometry& geometry, const Workspace& w, hipStream_t st) {
+void launch_single_pass(const Buckets& call, const Geometry& geometry, const Workspace& w, uint64_t fits, hipStream_t st) {
     // 100 MHz ticks a block may wait before it gives up
     const uint64_t lim = (uint64_t)tuning().topk_barrier_ms * 100000ull;
     // A list's blocks are those that its buckets have, longest bucket first: the bin blocks that nothing is
@@ -1624,6 +1624,7 @@ void launch_single_pass(const Buckets& call, const Geometry& geometry, const Wor
     Buckets bk = call;
     Geometry g = geometry;
     uint64_t tiles = (uint64_t)g.nbuckets * g.ftiles;
+    if constexpr (!LISTED) set_groups(&g, g.nbuckets * (uint64_t)topk_groups(g.ftiles, most_groups_shift(g)), fits);
     if constexpr (LISTED) {
         uint32_t order[kMaxListed];
         longest_first(call, g.nbuckets, order);
@@ -1635,7 +1636,7 @@ void launch_single_pass(const Buckets& call, const Geometry& geometry, const Wor
             groups += topk_groups(topk_tiles(bk.lcount[b]), most_groups_shift(g));
         }
         for (uint32_t b = g.nbuckets; b < kMaxListed; b++) bk.lfirst[b] = 0xFFFFFFFFu;
-        set_groups(&g, groups);
+        set_groups(&g, groups, fits);
     }
     if (stream_wide(tiles)) launch_stream<512, LISTED, MANY>(bk, g, w, lim, st);
     else launch_stream<256, LISTED, MANY>(bk, g, w, lim, st);
@@ -1663,14 +1664,30 @@ void launch_single_pass(const Buckets& call, const Geometry& geometry, const Wor
     }
 }
 
+// Blocks of a select launch that may wait for others: those of a bucket whose selection falls back.
+uint64_t select_limit_on(const StreamShare& share) {
+    static const uint64_t per_cu = [] {
+        int least = 1 << 20;
+        for (const void* k : {(const void*)k_topk_select<false, false>, (const void*)k_topk_select<false, true>,
+                              (const void*)k_topk_select<true, false>, (const void*)k_topk_select<true, true>}) {
+            int n = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, kBlock, 0) != hipSuccess) n = 0;
+            least = n < least ? n : least;
+        }
+        return (uint64_t)least;
+    }();
+    return waiting_limit(share, per_cu);
+}
+
 // False when the call has to take the exact path.
 bool launch_by_path(const Buckets& bk, const Geometry& g, const Workspace& w, const uint64_t* counts, hipStream_t st) {
-    const uint64_t limit = g.bucket_elems <= kRMaxBucket ? resident_limit_on(st) : 0;
-    const Route route = choose_path({g.n_total, g.bucket_elems, g.nbuckets, counts, g.k_full, g.many != 0}, tuning().topk_path, limit);
+    const StreamShare share = stream_share(st);
+    const uint64_t limit = g.bucket_elems <= kRMaxBucket ? resident_limit_on(share) : 0, fits = select_limit_on(share);
+    const Route route = choose_path({g.n_total, g.bucket_elems, g.nbuckets, counts, g.k_full, g.many != 0}, tuning().topk_path, limit, fits);
     if (route.path == kPathExact) return false;
     if (route.path == kPathStream) {
-        if (g.listed) (g.many ? launch_single_pass<true, true> : launch_single_pass<true, false>)(bk, g, w, st);
-        else (g.many ? launch_single_pass<false, true> : launch_single_pass<false, false>)(bk, g, w, st);
+        if (g.listed) (g.many ? launch_single_pass<true, true> : launch_single_pass<true, false>)(bk, g, w, fits, st);
+        else (g.many ? launch_single_pass<false, true> : launch_single_pass<false, false>)(bk, g, w, fits, st);
     } else {
         const uint32_t epoch = next_epoch();
         launch_resident(bk, g, w, route.vecs, limit, epoch, tuning().topk_stall_test ? ~epoch : epoch,

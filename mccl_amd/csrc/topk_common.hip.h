@@ -161,8 +161,12 @@ inline void place_bucket(Buckets* to, uint32_t i, const Buckets& from, uint32_t 
     to->lfirst[i] = first;
 }
 
-// Blocks that may wait in one resident launch on the stream (stream_limit).
-uint64_t resident_limit_on(hipStream_t st);
+// The stream's share of the device, and how many blocks of a launch on it, of which `per_cu` fit a CU, may wait for
+// others (stream_limit).
+StreamShare stream_share(hipStream_t st);
+uint64_t waiting_limit(const StreamShare& share, uint64_t per_cu);
+// ... of a resident launch.
+uint64_t resident_limit_on(const StreamShare& share);
 // A list of buckets goes in as many launches as keep each under `limit`.
 void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, int vecs, uint64_t limit, uint32_t epoch,
                      uint32_t published, uint64_t limit_ticks, hipStream_t st);

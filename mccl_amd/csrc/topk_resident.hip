@@ -616,22 +616,7 @@ void longest_first(const Buckets& bk, uint32_t nbuckets, uint32_t* order) {
     std::sort(order, order + nbuckets, [&](uint32_t p, uint32_t q) { return bk.lcount[p] != bk.lcount[q] ? bk.lcount[p] > bk.lcount[q] : p < q; });
 }
 
-uint64_t resident_limit_on(hipStream_t st) {
-    static const uint64_t per_cu = [] {
-        int least = 1 << 20;
-        for (const void* k : {(const void*)k_topk_resident<1>, (const void*)k_topk_resident<2>, (const void*)k_topk_resident<4>}) {
-            int n = 0;
-            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, kRThreads, 0) != hipSuccess) n = 0;
-            least = n < least ? n : least;
-        }
-        return (uint64_t)least;
-    }();
-    // hardware queues that the process's streams share; HIP's own default is four
-    static const uint32_t queues = [] {
-        const char* s = std::getenv("GPU_MAX_HW_QUEUES");
-        const long q = s ? std::strtol(s, nullptr, 10) : 0;
-        return (uint32_t)(q > 0 && q < 1024 ? q : 4);
-    }();
+StreamShare stream_share(hipStream_t st) {
     // (asking takes 0.2 us; the null stream's mask is the process's)
     static const int process_cus = stream_cus(nullptr);
     StreamShare share = {process_cus, 0};
@@ -642,7 +627,30 @@ uint64_t resident_limit_on(hipStream_t st) {
             share.priority = 0;
         }
     }
+    return share;
+}
+
+uint64_t waiting_limit(const StreamShare& share, uint64_t per_cu) {
+    // hardware queues that the process's streams share; HIP's own default is four
+    static const uint32_t queues = [] {
+        const char* s = std::getenv("GPU_MAX_HW_QUEUES");
+        const long q = s ? std::strtol(s, nullptr, 10) : 0;
+        return (uint32_t)(q > 0 && q < 1024 ? q : 4);
+    }();
     return stream_limit(share, device_info().num_cus, per_cu, queues);
+}
+
+uint64_t resident_limit_on(const StreamShare& share) {
+    static const uint64_t per_cu = [] {
+        int least = 1 << 20;
+        for (const void* k : {(const void*)k_topk_resident<1>, (const void*)k_topk_resident<2>, (const void*)k_topk_resident<4>}) {
+            int n = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, kRThreads, 0) != hipSuccess) n = 0;
+            least = n < least ? n : least;
+        }
+        return (uint64_t)least;
+    }();
+    return waiting_limit(share, per_cu);
 }
 
 void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, int vecs, uint64_t limit, uint32_t epoch,

@@ -115,6 +115,18 @@ inline uint64_t resident_waiting(const TopkCall& c, int vecs) {
     return sum;
 }
 
+// Groups per bucket, the power of two, where `fits` blocks of a select launch may wait (stream_limit): a bucket whose
+// selection falls back to the exact one has its groups' blocks wait for each other.  64 of them are resident together on
+// 16 CUs; more only where they are whatever else runs.  A wait that runs out instead costs the bucket its payload.
+constexpr uint32_t topk_group_shift_fits(uint32_t shift, uint64_t fits) {
+    const uint32_t most = fits >= 256 ? 8 : fits >= 128 ? 7 : 6;
+    return shift < most ? shift : most;
+}
+constexpr uint32_t topk_shift(uint64_t tiles, uint64_t groups, bool many, uint64_t fits) {
+    return topk_group_shift_fits(many ? topk_group_shift_many(tiles, groups) : topk_group_shift(tiles, groups), fits);
+}
+constexpr uint64_t kFewestFits = 64;  // blocks of the fewest groups that a long bucket has
+
 // Vectors per thread of a resident launch, 0 when more than `limit` of its blocks would wait.  The barriers
 // cost more with more blocks, the passes over a block's elements with more vectors; measured (one bucket,
 // 1 %): 262,144 elements 17.8 / 18.0 us with 1 / 2 vectors, 400,000 19.8 / 19.5, 524,288 20.0 / 19.3 / 20.7
@@ -166,14 +178,16 @@ struct Route {
 //     against 99, 4 x 2 M 117 against 167, 20 x 1.5 M 288 against 320; of many large ones the streaming path shares that
 //     latency: 12 x 2 M 249 exact, 230 streaming, 50 x 1.7 M 782 and 725, 14 x 6.5 M 905 and 826, 15 x 6.5 M at 20 % with
 //     1024 slots 889 and 730.
-inline Route choose_path(const TopkCall& c, int forced, uint64_t limit) {
+// `fits`: blocks of a select launch that may wait.  Where not even 64 do, large ratios go by what 128 slots hold: one
+// bucket takes the exact path, in which nothing waits.
+inline Route choose_path(const TopkCall& c, int forced, uint64_t limit, uint64_t fits = kMaxGroups) {
     const uint64_t tiles = (c.bucket_elems + kFTile - 1) / kFTile;
     const bool streams = (uint64_t)c.nbuckets * (tiles + kMaxGroups + 1) + kMaxGroups < 0x7FFFFFFFull;
     if (forced == 1 && !c.counts) return {kPathExact, 0};
     if (forced == 2 && streams) return {kPathStream, 0};
     // expected share of a bucket inside the sampled window (see sample_window)
     const double ks = (double)c.k_full / (double)c.bucket_elems * kFSample;
-    const bool dense = (ks + 6.0 * std::sqrt(ks) + 16.0) / kFSample > (c.many ? 0.6 * kManySlots : (double)kTileSlots) / kFTile;
+    const bool dense = (ks + 6.0 * std::sqrt(ks) + 16.0) / kFSample > (c.many && fits >= kFewestFits ? 0.6 * kManySlots : (double)kTileSlots) / kFTile;
     int vecs = resident_vecs(c, limit);
     // a list can go in several launches, as long as its longest bucket fits one
     if (!vecs && c.counts && (dense || forced == 3) && c.bucket_elems <= (limit < kRMaxBlocks ? limit : kRMaxBlocks) * kRVecElems * 4) vecs = 4;

@@ -219,3 +219,66 @@ def test_a_shorter_last_bucket_has_all_its_groups(tmp_path):
                     str(exe)], check=True)
     p = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True, timeout=100)
     assert p.returncode == 0, p.stdout[:2000]
+
+
+FALLBACK = SOURCE[:SOURCE.index("int main()")] + r"""
+// Groups of the longest bucket of a call, as the library launches them.
+static uint32_t groups_of(const TopkCall& c, uint64_t fits) {
+    const uint32_t tiles = topk_tiles(c.bucket_elems), most = c.many ? 8 : topk_group_shift_few(tiles);
+    return topk_groups(tiles, topk_shift(tiles, c.nbuckets * (uint64_t)topk_groups(tiles, most), c.many, fits));
+}
+static TopkCall call(uint64_t n, uint64_t be, double ratio) {
+    TopkCall c = uniform(n, be, ratio);
+    c.many = topk_many(be, ratio);
+    return c;
+}
+
+int main() {
+    // four blocks of the select launch per CU, four queues: the whole GPU, a half, a quarter, an eighth of it
+    const auto fits = [](int cus, uint32_t queues) { return stream_limit({cus, 0}, cus, 4, queues); };
+    REQUIRE(fits(256, 4) == 256 && fits(128, 4) == 128 && fits(64, 4) == 64 && fits(32, 4) == 32);
+    const TopkCall one = call(10000000, 10000000, 0.01);
+    REQUIRE(groups_of(one, fits(256, 4)) == 245 && groups_of(one, fits(128, 4)) <= 128 && groups_of(one, fits(64, 4)) <= 64);
+    REQUIRE(groups_of(one, fits(32, 4)) <= 64 && groups_of(one, fits(256, 8)) <= 128 && groups_of(one, fits(256, 16)) <= 64);
+    // a stream that has part of the GPU, or queues beside the four
+    REQUIRE(groups_of(one, stream_limit({60, 0}, 256, 4, 4)) <= 64 && groups_of(one, stream_limit({256, 1}, 256, 4, 4)) <= 64);
+    // large ratios: the exact path, which waits for nobody, where the fewest groups might not be resident together
+    for (double r : {0.02, 0.05, 0.12})
+        for (uint64_t n : {2200000ull, 6553600ull, 30000000ull}) {
+            const TopkCall c = call(n, n, r);
+            REQUIRE(choose_path(c, 0, 0, fits(256, 4)).path == kPathStream && choose_path(c, 0, 0, fits(64, 4)).path == kPathStream);
+            REQUIRE(choose_path(c, 0, 0, fits(32, 4)).path == kPathExact);
+            REQUIRE(choose_path(c, 0, 0, 0).path == kPathExact);
+        }
+    REQUIRE(choose_path(one, 0, 0, 0).path == kPathStream);
+    // buckets that fall back in every queue at once, one each, with whatever groups they have
+    std::mt19937 rng(2);
+    for (int i = 0; i < 2000; i++) {
+        const int cus[] = {64, 128, 256}, c = cus[rng() % 3];
+        const uint32_t queues = 1 + rng() % 8;
+        const uint64_t f = fits(c, queues);
+        std::vector<Blocks> under_way;
+        for (uint32_t q = 0; q < queues; q++) {
+            const uint64_t be = 300000 + rng() % 40000000;
+            under_way.push_back({groups_of(call(be * (1 + rng() % 3), be, rng() % 2 ? 0.01 : 0.05), f)});
+            if (f >= kFewestFits) REQUIRE(under_way.back()[0] <= f);
+        }
+        if (f >= kFewestFits) REQUIRE(all_end(under_way, c / 32, 128, rng));
+    }
+    // the model does find one bucket of 245 groups on an eighth of the GPU, three of them on a half, stuck
+    REQUIRE(!all_end({{245}}, 1, 128, rng));
+    int stuck = 0;
+    for (int i = 0; i < 200; i++) stuck += !all_end({{245}, {245}, {245}}, 4, 128, rng);
+    REQUIRE(stuck > 0);
+    return 0;
+}
+"""
+
+
+def test_a_bucket_that_falls_back_has_its_blocks_resident(tmp_path):
+    src, exe = tmp_path / "fallback.cpp", tmp_path / "fallback"
+    src.write_text(FALLBACK)
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wno-unused-function", "-Werror", "-I", os.path.join(ROOT, "mccl_amd", "csrc"), str(src),
+                    "-o", str(exe)], check=True)
+    p = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True, timeout=100)
+    assert p.returncode == 0, p.stdout[:2000]
