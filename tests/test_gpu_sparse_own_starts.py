@@ -1,5 +1,6 @@
 """Sparse accumulate of one bucket, where a block finds the starts of its runs itself: at the edges
-of the run, the block and the sample count, against the oracle and against the position table."""
+of the run, the block and the sample count, against the oracle and against the position table.  The path "runs" takes
+the runs at every size; which sizes take them by themselves is another rule's matter."""
 import numpy as np
 import pytest
 import torch
@@ -7,7 +8,7 @@ import torch
 import oracle
 from mccl_amd import hip_ops
 from tests._gpu_util import DEV
-from tests.test_gpu_sparse_runs import payload, run_case
+from tests.test_gpu_sparse_runs import RUNS, payload, run_case
 
 pytestmark = pytest.mark.gpu
 
@@ -31,7 +32,7 @@ def ranks(rng, ws, n, k):
 ])
 def test_one_bucket(ws, n, k):
     rng = np.random.default_rng(n + k)
-    run_case(hip_ops, ranks(rng, ws, n, k), n, n, 1.0 / ws, paths=("auto",))
+    run_case(hip_ops, ranks(rng, ws, n, k), n, n, 1.0 / ws, paths=("runs", "table", "auto"))
 
 
 @pytest.mark.parametrize("steps,ws,n,k", [
@@ -53,7 +54,7 @@ def test_payloads_out_of_order_are_flagged(at):
     idx = np.sort(np.random.default_rng(at).choice(n, k, replace=False))
     idx[[at, at + 1]] = idx[[at + 1, at]]
     wires = [torch.from_numpy(payload(idx, np.ones(k, np.float32), k)).to(DEV)]
-    for path in (0, 2):
+    for path in (0, 1, 2, 3):
         status = torch.zeros(1, dtype=torch.int32, device=DEV)
         hip_ops.set_tuning("sparse_path", path)
         try:
@@ -67,7 +68,8 @@ def test_payloads_out_of_order_are_flagged(at):
     (5, 2049, 2049, 81), (6, 16385, 16385, 161), (8, 1_000_001, 1_000_001, 10_000),   # a block finds its runs' starts
     (9, 2049, 2049, 20), (10, 300_001, 100_000, 1000), (11, 65_537, 65_537, 700), (12, 1_000_003, 400_000, 4000),
     (12, 30_000, 30_000, 1400),                                                       # more pairs than the windows hold
-    (3, 40_000_000, 6_553_600, 60_000), (10, 9_000_001, 6_553_600, 65_536)])          # on either side of the rule's lines
+    (3, 40_000_000, 6_553_600, 60_000), (6, 8_388_608, 8_388_608, 80_000),            # more than 8 M elements, not more
+    (10, 16_777_217, 6_553_600, 65_536), (12, 16_777_216, 6_553_600, 65_536)])        # more than 16 M, not more
 def test_runs_and_tiles(ws, n, be, k):
     """The runs for up to twelve ranks, forced and where the sizes choose them, and the tile kernels."""
     rng = np.random.default_rng(n + ws)
@@ -80,7 +82,7 @@ def test_runs_and_tiles(ws, n, be, k):
             idx = np.unique(rng.integers(0, m, kr)) if m > 1_000_000 else np.sort(rng.choice(m, kr, replace=False))
             row.append((idx, rng.standard_normal(idx.size).astype(np.float32)))
         per_rank.append(row)
-    run_case(hip_ops, per_rank, n, be, 1.0 / ws, paths=("auto", "tiles"))
+    run_case(hip_ops, per_rank, n, be, 1.0 / ws, paths=RUNS)
     hip_ops.set_tuning("sparse_run_steps", 2)   # (the runs, whatever the size)
     try:
         run_case(hip_ops, per_rank, n, be, 1.0 / ws, paths=("auto",))

@@ -1,13 +1,15 @@
 """Sparse accumulate on hand-built payloads (csrc/backend/ProcessGroupMCCL.cpp:1692-1709,
 :2272-2296: decompress every rank, fold the dense buffers in rank order): the cases
-that decide whether the GPU walk over the payloads is exact.
+that decide whether the GPU walk over the payloads is exact, on each of its kernels: the runs of tiles
+(a block finds its runs' starts, or a table holds them), the tile kernels, the one without a
+workspace, and whichever the sizes choose.
 
     values    subnormals, both zeros, infinities, NaN, sums that overflow, many
               ranks on one element: the adds happen in rank order, in IEEE single
               precision with subnormals kept
     density   from a handful of pairs per bucket to 4.5 % (a rank's pairs of one
               tile no longer fit the registers requested up front), clustered
-              payloads, one to eight ranks, short last bucket, misaligned output
+              payloads, one to twelve ranks, short last bucket, misaligned output
     order     a payload out of order (or with a repeated index) at any position,
               lane 15/16, 31/32 and 63/64 included, is flagged; sorted payloads
               whose first index is 0 or whose k is a multiple of 64 are not
@@ -39,7 +41,11 @@ def payload(idx, val, kcap):
     return np.concatenate([np.array([k], "<u4").view(np.uint8), body.reshape(-1).view(np.uint8)])
 
 
-def run_case(ops, per_rank, n, be, scale, expect_status=0, pad_front=0, paths=("auto", "tiles", None)):
+TUNING = {"auto": 0, "tiles": 1, "table": 2, "runs": 3, None: 0}   # None: no workspace
+RUNS = ("auto", "runs", "table", "tiles")
+
+
+def run_case(ops, per_rank, n, be, scale, expect_status=0, pad_front=0, paths=RUNS + (None,)):
     """per_rank[r][b] = (idx, val) of rank r's bucket-b payload.  Returns the GPU result."""
     ws = len(per_rank)
     nb = (n + be - 1) // be
@@ -63,8 +69,7 @@ def run_case(ops, per_rank, n, be, scale, expect_status=0, pad_front=0, paths=("
         big = torch.full((n + pad_front + 8,), 3.0, device=DEV)
         acc = big[pad_front:pad_front + n]
         status.zero_()
-        if path == "tiles":
-            ops.set_tuning("sparse_path", 1)
+        ops.set_tuning("sparse_path", TUNING[path])
         try:
             ops.sparse_accumulate(acc, wires, stride, bucket_elems=be, scale_by=scale, status=status,
                                   workspace=None if path is None else "auto")
@@ -87,7 +92,7 @@ SPECIALS = np.array([0.0, -0.0, 1e-40, -1e-40, 1e-45, -1e-45, 5.877e-39, -5.877e
                     dtype=np.float32)
 
 
-@pytest.mark.parametrize("ws", [2, 3, 8])
+@pytest.mark.parametrize("ws", [2, 3, 6, 8, 9, 12])
 def test_special_values_add_in_rank_order(ops, ws):
     rng = np.random.default_rng(100 + ws)
     n, be = 40_000, 16_384
@@ -123,7 +128,8 @@ def test_three_way_sums_need_rank_order(ops):
 
 @pytest.mark.parametrize("ws,n,be,density", [
     (1, 10_000, 10_000, 0.01), (2, 70_001, 32_768, 0.001), (5, 200_000, 65_536, 0.03),
-    (8, 150_000, 65_536, 0.045), (3, 2048 * 5 + 1, 2048 * 5 + 1, 0.02), (4, 9, 4, 0.5), (8, 300_000, 100_000, 0.0001)])
+    (8, 150_000, 65_536, 0.045), (3, 2048 * 5 + 1, 2048 * 5 + 1, 0.02), (4, 9, 4, 0.5), (8, 300_000, 100_000, 0.0001),
+    (10, 200_000, 65_536, 0.03), (12, 150_000, 65_536, 0.045)])
 def test_densities_worlds_and_geometries(ops, ws, n, be, density):
     rng = np.random.default_rng(ws * 1000 + n)
     nb = (n + be - 1) // be
@@ -137,7 +143,7 @@ def test_densities_worlds_and_geometries(ops, ws, n, be, density):
             ranks.append((idx, rng.standard_normal(k).astype(np.float32)))
         per_rank.append(ranks)
     run_case(ops, per_rank, n, be, 1.0 / ws)
-    run_case(ops, per_rank, n, be, None, pad_front=1, paths=("auto",))       # output not 16-byte aligned
+    run_case(ops, per_rank, n, be, None, pad_front=1, paths=RUNS)       # output not 16-byte aligned
 
 
 def test_clustered_payloads(ops):
@@ -171,11 +177,11 @@ def test_sorted_payloads_are_not_flagged(ops, k):
     n = 100_000
     for first_zero in (True, False):
         per_rank = [[sorted_payload(rng, n, k, first_zero)] for _ in range(3)]
-        run_case(ops, per_rank, n, n, None, paths=("auto",))
+        run_case(ops, per_rank, n, n, None, paths=RUNS)
     # the largest index the bucket allows
     idx, val = sorted_payload(rng, n, k, False)
     idx[-1] = n - 1
-    run_case(ops, [[(idx, val)]], n, n, None, paths=("auto",))
+    run_case(ops, [[(idx, val)]], n, n, None, paths=RUNS)
 
 
 @pytest.mark.parametrize("pos", [0, 14, 15, 16, 31, 32, 47, 48, 62, 63, 64, 65, 127, 128, 191, 192, 193, 255, 256, 300, 998])
@@ -189,11 +195,11 @@ def test_order_violation_at_any_position_is_flagged(ops, pos):
             idx[pos], idx[pos + 1] = idx[pos + 1], idx[pos]
         else:
             idx[pos + 1] = idx[pos]
-        run_case(ops, [good[0], [(idx, val)]], n, n, None, expect_status=oracle.ERR_INDEX, paths=("auto",))
+        run_case(ops, [good[0], [(idx, val)]], n, n, None, expect_status=oracle.ERR_INDEX, paths=RUNS)
     # an index equal to the bucket's size, in the middle of the payload's last window
     idx, val = good[1][0][0].copy(), good[1][0][1]
     idx[k - 1] = n
-    run_case(ops, [good[0], [(idx, val)]], n, n, None, expect_status=oracle.ERR_INDEX, paths=("auto",))
+    run_case(ops, [good[0], [(idx, val)]], n, n, None, expect_status=oracle.ERR_INDEX, paths=RUNS)
 
 
 def test_buckets_that_start_off_a_16_byte_boundary(ops):
@@ -214,11 +220,12 @@ def test_buckets_that_start_off_a_16_byte_boundary(ops):
     run_case(ops, per_rank, n, be, 1.0 / 3.0)
 
 
-def test_random_shapes_and_payload_shapes(ops):
+@pytest.mark.parametrize("fewest,most,seed,cases", [(1, 8, 20260, 40), (9, 12, 20261, 20)])
+def test_random_shapes_and_payload_shapes(ops, fewest, most, seed, cases):
     # seeded sweep: world size, bucket length (aligned or not), last bucket, density and clustering all vary
-    rng = np.random.default_rng(20260)
-    for case in range(40):
-        ws = int(rng.integers(1, 9))
+    rng = np.random.default_rng(seed)
+    for case in range(cases):
+        ws = int(rng.integers(fewest, most + 1))
         be = int(rng.choice([1, 3, 64, 2047, 2048, 2049, 4096, 10_000, 33_333, 70_000]))
         nb = int(rng.integers(1, 5))
         n = max(1, be * (nb - 1) + int(rng.integers(1, be + 1)))
@@ -238,4 +245,4 @@ def test_random_shapes_and_payload_shapes(ops):
                 ranks.append((idx, (rng.standard_normal(k) * 10.0 ** rng.integers(-20, 20)).astype(np.float32)))
             per_rank.append(ranks)
         scale = [None, 1.0 / ws, 0.3][case % 3]
-        run_case(ops, per_rank, n, be, scale, paths=("auto", None))
+        run_case(ops, per_rank, n, be, scale)
