@@ -316,7 +316,7 @@ def test_give_up_path_poisons_the_payload_and_sets_the_status(ops, path):
 def test_more_buckets_than_the_gpu_holds_blocks_for(ops):
     """48 buckets of 300,000 elements in one call, and a list of 64 buckets: far more bin and
     select blocks than are resident at once.  Nothing in the streaming launch waits for a later
-    block, and the select launch goes out in groups of 16 buckets: exact bytes, no give-up."""
+    block, and a select launch covers 1024 blocks at most, whole buckets: exact bytes, no give-up."""
     rng = np.random.default_rng(48)
     be, nb = 300_000, 48
     n = be * nb - 12_345

@@ -1,5 +1,7 @@
-"""Single-pass top-k of buckets around the sizes where the number of tile groups changes: 64 groups of up to
-28 tiles (4096 elements each), then more groups, then, past 256 groups, more tiles in each."""
+"""Single-pass top-k of buckets around the sizes where the number of tile groups (of 4096 elements a tile) changes.
+A call whose select blocks fit one launch has up to 64 groups a bucket, 128 past 64 * 14 tiles, 256 past 128 * 16; another
+more than 64 only past 64 * 28 tiles, more than 128 past 128 * 28.  tests/test_topk_route.py holds the groups and
+launches of the sizes used here against the rule."""
 import numpy as np
 import pytest
 import torch
@@ -12,7 +14,8 @@ pytestmark = pytest.mark.gpu
 TILE = 4096
 
 
-@pytest.mark.parametrize("n", [64 * 28 * TILE, 64 * 28 * TILE + 1, 65 * 28 * TILE + 5, 256 * 28 * TILE + 4097])
+@pytest.mark.parametrize("n", [64 * 28 * TILE, 64 * 28 * TILE + 1, 65 * 28 * TILE + 5,   # 128 groups of 14 or 15 tiles
+                               256 * 28 * TILE + 4097])                            # 248 of 29: more than a block keeps
 def test_groups_of_tiles(n):
     from mccl_amd import hip_ops as ops
     rng = np.random.default_rng(n)
@@ -92,6 +95,16 @@ def test_list_of_ragged_buckets(lengths):
         want, size = oracle.topk_compress(g, r, 0.01)
         assert w.cpu().numpy()[:size].tobytes() == want.tobytes(), g.size
         assert np.array_equal(bits(to_np(d, F32)), bits(r)), g.size
+
+
+def _misled(rng, n):
+    """Values whose sample misleads (every sampled run that meets one of the 5.0 blocks is all 5.0), so that the selection
+    falls back to the exact one."""
+    grad = student_t(rng, n, ties=0.0) * np.float32(1e-6)
+    stride = n // 4 // 256 * 4   # elements between two sampled runs of 32
+    for i in range(0, 256, 2):
+        grad[i * stride: i * stride + 32] = 5.0
+    return grad
 
 
 def _check(ops, grad, res, ratio, bucket):
@@ -196,3 +209,76 @@ def test_last_bucket_with_more_groups(tiles, last, ratio):
         res[lo:lo + bucket] = part
         assert w[b * stride: b * stride + size].tobytes() == want.tobytes(), b
     assert np.array_equal(bits(to_np(dres, F32)), bits(res))
+
+
+@pytest.mark.parametrize("tiles, last, ratio", [(1600, 1536, 0.01), (1600, 1536, 0.05)])   # 124 and 128 groups, 229 and 256
+@pytest.mark.parametrize("which", [(0,), (1,), (0, 1)])
+def test_last_bucket_with_more_groups_falls_back(tiles, last, ratio, which):
+    from mccl_amd import hip_ops as ops
+    rng = np.random.default_rng(tiles + last)
+    parts = [(_misled if b in which else student_t)(rng, n * TILE) for b, n in enumerate((tiles, last))]
+    n = (tiles + last) * TILE
+    done = _check(ops, np.concatenate(parts), (rng.standard_normal(n) * 1e-9).astype(np.float32), ratio, tiles * TILE)
+    assert done == (2 - len(which), 2)
+
+
+@pytest.mark.parametrize("ratio", [0.01, 0.05])
+@pytest.mark.parametrize("lengths", [
+    [1_500_001, 65_537, 4097, 2_200_001, 300_007, 1_000_003],
+    [1_100_001 - 7 * i for i in range(20)] + [9]])         # two select launches, the second from the middle of the table
+def test_list_whose_buckets_fall_back(lengths, ratio):
+    """Every second bucket by length falls back, the others beside it don't."""
+    from mccl_amd import hip_ops as ops
+    rng = np.random.default_rng(len(lengths))
+    by_length = sorted(range(len(lengths)), key=lambda i: -lengths[i])
+    misled = {i for at, i in enumerate(by_length) if at % 2 == 0 and lengths[i] > 500_000}
+    grads = [(_misled if i in misled else student_t)(rng, n) for i, n in enumerate(lengths)]
+    _check_list(ops, grads, ratio, len(lengths) - len(misled))
+
+
+def test_list_with_dense_tiles():
+    """Lists with slots for many candidates: tiles that run out of them between others, many equal keys, a fallback."""
+    from mccl_amd import hip_ops as ops
+    rng = np.random.default_rng(17)
+    lengths = [2_500_000, 300_007, 1_200_001, 65_541, 4099]
+    grads = [student_t(rng, n, ties=0.0) * np.float32(1e-3) for n in lengths]
+    for g in grads:
+        for lo in range(0, g.size - 2_000, 50_000):
+            g[lo:lo + 2_000] = student_t(rng, 2_000, ties=0.0)
+    _check_list(ops, [g.copy() for g in grads], 0.03)
+    grads[2][::3] = 2.0                                    # more equal keys than are picked
+    grads[1] = _misled(rng, lengths[1])
+    _check_list(ops, grads, 0.05)
+
+
+def _check_list(ops, grads, ratio, single_pass=None):
+    longest, count = max(g.size for g in grads), len(grads)
+    residuals = [np.zeros(g.size, np.float32) for g in grads]
+    dres = [to_dev(r, F32) for r in residuals]
+    status = torch.zeros(1, dtype=torch.int32, device=DEV)
+    ws = ops.topk_workspace(longest * count, longest, ratio, DEV)
+    try:
+        ops.set_tuning("topk_path", 2)
+        wires = ops.topk_compress_list([to_dev(g, F32) for g in grads], dres, ratio, workspace=ws, status=status)
+    finally:
+        ops.set_tuning("topk_path", 0)
+    assert int(status) == 0
+    if single_pass is not None:
+        assert ops.topk_path_report(ws, longest * count, longest, ratio) == (single_pass, count)
+    for g, r, d, w in zip(grads, residuals, dres, wires):
+        want, size = oracle.topk_compress(g, r, ratio)
+        assert w.cpu().numpy()[:size].tobytes() == want.tobytes(), g.size
+        assert np.array_equal(bits(to_np(d, F32)), bits(r)), g.size
+
+
+@pytest.mark.parametrize("tiles, count, short", [(1850, 9, 0), (1850, 9, 3_000_001)])   # 128 groups at most, 124 in each
+def test_many_large_buckets(tiles, count, short):
+    """More select blocks than one launch holds, and more than 64 groups a bucket all the same; the second launch starts
+    at bucket 8, the last of them, whole or shorter."""
+    from mccl_amd import hip_ops as ops
+    bucket = tiles * TILE
+    rng = np.random.default_rng(tiles)
+    base = student_t(rng, bucket, ties=0.01)
+    grad = np.concatenate([np.roll(base, 1000 * b) * np.float32(1 + b) for b in range(count)])[:bucket * count - short]
+    done = _check(ops, grad, np.zeros(grad.size, np.float32), 0.01, bucket)
+    assert done == (count, count)

@@ -251,6 +251,24 @@ int main() {
             REQUIRE(choose_path(c, 0, 0, 0).path == kPathExact);
         }
     REQUIRE(choose_path(one, 0, 0, 0).path == kPathStream);
+    // the sizes of test_gpu_topk_groups.py: elements, bucket, ratio, groups of a bucket, select launches
+    const uint64_t tile = kFTile;
+    const struct { uint64_t n, be; double ratio; uint32_t groups, launches; } sizes[] = {
+        {64 * 14 * tile, 64 * 14 * tile, 0.01, 64, 1}, {64 * 14 * tile + 1, 64 * 14 * tile + 1, 0.01, 113, 1},
+        {64 * 28 * tile, 64 * 28 * tile, 0.01, 128, 1}, {64 * 28 * tile + 1, 64 * 28 * tile + 1, 0.01, 120, 1},
+        {128 * 16 * tile, 128 * 16 * tile, 0.01, 128, 1}, {128 * 16 * tile + 3, 128 * 16 * tile + 3, 0.01, 228, 1},
+        {256 * 28 * tile + 4097, 256 * 28 * tile + 4097, 0.01, 248, 1},
+        {8 * 900 * tile, 900 * tile, 0.01, 113, 1}, {9 * 900 * tile, 900 * tile, 0.01, 113, 1}, {10 * 900 * tile, 900 * tile, 0.01, 60, 1},
+        {9 * 1850 * tile, 1850 * tile, 0.01, 124, 2}, {9 * 1850 * tile - 3000001, 1850 * tile, 0.01, 124, 2},
+        {1600 * tile, 1600 * tile, 0.05, 229, 1}, {40000000, 8000000, 0.05, 123, 1}, {17 * 1048576 - 3, 1048576, 0.05, 64, 2}};
+    for (const auto& s : sizes) {
+        const TopkCall c = call(s.n, s.be, s.ratio);
+        const uint32_t g = groups_of(c, fits(256, 4)), at_once = 1024 / g;
+        if (g != s.groups || (c.nbuckets + at_once - 1) / at_once != s.launches) {
+            std::printf("%llu / %llu at %g: %u groups\n", (unsigned long long)s.n, (unsigned long long)s.be, s.ratio, g);
+            return 1;
+        }
+    }
     // buckets that fall back in every queue at once, one each, with whatever groups they have
     std::mt19937 rng(2);
     for (int i = 0; i < 2000; i++) {
