@@ -287,8 +287,11 @@ __global__ __launch_bounds__(kBlock) void k_sparse_accumulate(float* acc, uint64
 // blocks write into one 32-byte sector and made this kernel 40 % slower.  One
 // thread per pair: pair p writes the
 // entry of every tile that begins between pair p-1 and pair p (usually none), so
-// each entry is written exactly once for a sorted payload.  A thread takes eight
-// consecutive pairs.  The pair loads do not wait for k: they stay inside the
+// each entry is written exactly once for a sorted payload; the entries of a gap of
+// more than four tiles are shared by the wavefront: one thread that wrote them took 25 ns
+// for each, after all others.  us per call, one thread / so: two ranks of 6 M elements at 1 % whose pairs lie at the
+// bucket's front 33.8 / 13.5, eight of 8 M in two buckets, the last a fifth as long, 32.7 / 14.3 (where entries past the
+// last bucket's own tiles were written as well).  A thread takes eight consecutive pairs.  The pair loads do not wait for k: they stay inside the
 // payload's stride and are masked afterwards.
 __global__ __launch_bounds__(kBlock) void k_sparse_bounds(WirePtrs wires, int ws, uint64_t wire_stride,
                                                           uint64_t n_total, uint64_t bucket_elems, uint32_t tiles,
@@ -325,26 +328,45 @@ __global__ __launch_bounds__(kBlock) void k_sparse_bounds(WirePtrs wires, int ws
         for (uint32_t t = blockIdx.x * kBlock + threadIdx.x; t <= tiles; t += gridDim.x * kBlock) st[t] = 0;
         return;
     }
+    // entries past the bucket's own tiles are read by nobody
+    const uint32_t own_tiles = (uint32_t)((bn + kAccTile - 1) / kAccTile);
+    const int lane = threadIdx.x & (kWave - 1);
+    // st[from .. to] = p, for the lane's own; a long gap - between clustered pairs, in front of the first, behind the
+    // last - is written by the whole wavefront
+    auto fill = [&](uint32_t from, uint32_t to, uint32_t p) {
+        const uint32_t n = from <= to ? to - from + 1 : 0u;
+        constexpr uint32_t kAlone = 4;
+        if (n && n <= kAlone)
+            for (uint32_t t = from; t <= to; t++) st[t] = p;
+        for (uint64_t far = __ballot(n > kAlone); far; far &= far - 1) {
+            const int l = __ffsll((long long)far) - 1;
+            const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)from, l), c = (uint32_t)__builtin_amdgcn_readlane((int)n, l);
+            const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)p, l);
+            for (uint32_t i = (uint32_t)lane; i < c; i += kWave) st[f + i] = v;
+        }
+    };
     uint32_t prev = before;
+    uint32_t behind = own_tiles + 1;  // of the lane that holds the last pair: the first entry that is k
 #pragma unroll
     for (int j = 0; j < PP; j++) {
         const uint32_t p = p0 + (uint32_t)j;
         const uint32_t idx = v[j / 2][(j & 1) * 2];
+        uint32_t from = 1, to = 0;
         if (p < k) {
             if (idx >= bn && status) *status = MCCL_HIP_ERR_INDEX;
-            uint32_t t_hi = idx / kAccTile;  // tiles (t_prev, t_hi] begin at pair p
-            if (t_hi > tiles) t_hi = tiles;
-            int64_t t_prev = -1;
+            to = idx / kAccTile;  // tiles [from, to] begin at pair p
+            if (to > own_tiles) to = own_tiles;
+            from = 0;
             if (p > 0) {
                 if (prev >= idx && status) *status = MCCL_HIP_ERR_INDEX;  // not ascending
-                t_prev = prev / kAccTile;
+                from = prev / kAccTile + 1;
             }
-            for (int64_t t = t_prev + 1; t <= (int64_t)t_hi; t++) st[t] = p;
-            if (p == k - 1)
-                for (uint32_t t = t_hi + 1; t <= tiles; t++) st[t] = k;
+            if (p == k - 1) behind = to + 1;
         }
+        fill(from, to, p);
         prev = idx;
     }
+    fill(behind, own_tiles, k);
 }
 
 // Accumulate with precomputed bounds: every block reads its 2 * ws bounds with one
@@ -865,9 +887,11 @@ int accumulate(float* acc, uint64_t n_total, uint64_t bucket_elems, const void* 
             k_sparse_starts<<<(uint32_t)(nb * ws), kStartThreads, 0, st>>>(wp, ws, wire_stride,
                                                                             (uint32_t)(run_steps * kRunL), runs, start, status);
         const uint32_t per_xcd = (uint32_t)((blocks + kXcds - 1) / kXcds);
-#define MCCLHIP_RUNS(NR)                                                                               \
-    (own ? k_sparse_accumulate_runs<(NR <= kRunWaves ? NR : 1), true> : k_sparse_accumulate_runs<NR, false>)<<<per_xcd * kXcds, kRunWaves * kWave, 0, st>>>(                        \
-        acc, n_total, bucket_elems, wp, ws, wire_stride, (uint32_t)run_steps, runs, (uint32_t)nb, per_xcd, \
+        // (more ranks than a block has wavefronts never find their starts: no kernel for those)
+#define MCCLHIP_RUNS(NR)                                                                                     \
+    (own ? k_sparse_accumulate_runs<(NR <= kRunWaves ? NR : 1), true>                                        \
+         : k_sparse_accumulate_runs<NR, false>)<<<per_xcd * kXcds, kRunWaves * kWave, 0, st>>>(              \
+        acc, n_total, bucket_elems, wp, ws, wire_stride, (uint32_t)run_steps, runs, (uint32_t)nb, per_xcd,   \
         start, apply_scale, scale, status)
         if (ws == 1) MCCLHIP_RUNS(1);
         else if (ws == 2) MCCLHIP_RUNS(2);

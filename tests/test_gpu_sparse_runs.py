@@ -246,3 +246,66 @@ def test_random_shapes_and_payload_shapes(ops, fewest, most, seed, cases):
             per_rank.append(ranks)
         scale = [None, 1.0 / ws, 0.3][case % 3]
         run_case(ops, per_rank, n, be, scale)
+
+
+TILE = 8192   # of the tile kernels
+
+
+@pytest.mark.parametrize("ws", [2, 9])
+def test_gaps_between_pairs(ops, ws):
+    """Tiles without pairs, none to more than a wavefront's number of them: in front of a payload's first pair, between
+    two, behind the last, in a bucket shorter than the others."""
+    rng = np.random.default_rng(ws)
+    be, last = 140 * TILE + 5, 3 * TILE + 1
+    tiles = [0, 3, 4, 5, 9, 10, 14, 78, 139, 140]
+    ids = [[t * TILE for t in tiles], [t * TILE + TILE - 1 for t in tiles[:-1]], [0], [be - 1], [70 * TILE], [], [2 * TILE, 2 * TILE + 1],
+           [5, 139 * TILE], [136 * TILE]]
+    short = [[0], [last - 1], [], [2 * TILE], [0, 3 * TILE], [TILE - 1, TILE], [5], [0, 1, 2], [3 * TILE]]
+    per_rank = [[(np.array(i, np.uint32), rng.standard_normal(len(i)).astype(np.float32)) for i in (ids[r], short[r])]
+                for r in range(ws)]
+    run_case(ops, per_rank, be + last, be, 0.5)
+
+
+def _us(ops, wires, n, be, ws):
+    acc = torch.empty(n, device=DEV)
+    table = ops.sparse_workspace(n, be, ws, DEV)
+    status = torch.zeros(1, dtype=torch.int32, device=DEV)
+    times = []
+    for _ in range(7):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(40):
+            ops.sparse_accumulate(acc, wires, wires[0].numel() // -(-n // be), bucket_elems=be, status=status, workspace=table)
+        end.record()
+        end.synchronize()
+        times.append(start.elapsed_time(end) * 1e3 / 40)
+    assert int(status) == 0
+    return sorted(times)[3]
+
+
+def test_tile_kernels_do_not_wait_for_one_thread(ops):
+    """Tiles without pairs cost the tile kernels no more than a round trip: a bucket a fifth as long as the one before it,
+    and pairs that all lie at the front, against the same number of pairs spread evenly (1.0 and 1.3 measured; 2.4 and 3.3 when
+    one thread wrote the starts of them all)."""
+    n, k = 8_000_000, 80_000
+    rng = np.random.default_rng(3)
+
+    def wires(be, front):
+        out = []
+        for _ in range(2):
+            rows = []
+            for lo in range(0, n, be):
+                m = min(be, n - lo)
+                kk = k * m // n
+                idx = np.arange(kk) * 2 if front else np.arange(kk, dtype=np.uint64) * m // kk
+                rows.append(payload(idx, rng.standard_normal(kk).astype(np.float32), k * be // n + 1))
+            out.append(torch.from_numpy(np.concatenate(rows)).to(DEV))
+        return out
+
+    ops.set_tuning("sparse_path", 1)
+    try:
+        one, two, front = (_us(ops, wires(be, f), n, be, 2) for be, f in ((n, False), (6_553_600, False), (n, True)))
+    finally:
+        ops.set_tuning("sparse_path", 0)
+    print(f"one bucket {one:.1f} us, two {two:.1f}, pairs at the front {front:.1f}")
+    assert two < 1.6 * one and front < 2 * one, (one, two, front)
