@@ -873,12 +873,14 @@ int accumulate(float* acc, uint64_t n_total, uint64_t bucket_elems, const void* 
               samples * (uint64_t)ws <= kOwnTotal && path != 2;
         // Where the tile kernels take less time all the same: a wavefront's ranks follow one another, a block of theirs
         // has eight wavefronts for a tile.  That tells while the call leaves CUs idle or is dense, and for more ranks
-        // than eight.  us per call, runs against tiles: at 1 % 8 ranks of 250,000 elements 11.1 / 9.5, of 6 M 15.6 / 12.5, of
-        // 13 M 19.8 / 20.2, 5 ranks of 6 M 13.7 / 11.2, of 13 M 17.5 / 17.9, 3 of 3 M (which find their starts) 8.7 / 9.4, of 6 M
-        // 11.6 / 10.5, 12 of 13 M 26.4 / 24.6, of 26 M 39.3 / 46.4; at 2 % 8 of 26 M 45.8 / 40.2, of 60 M 82 / 95, 3 of 26 M
-        // 29.0 / 26.7, of 60 M 51.8 / 68.1, 9 of 96.5 M 134 / 127, 12 164 / 148; at 0.1 % 9 of 13 M 19.6 / 20.2.
-        const uint64_t few = per_tile > 32 ? 32u << 20 : ws > kRunWaves && per_tile > 8 ? 16u << 20 : 8u << 20;
-        const bool tiles_faster = ws > kRunWaves && per_tile > 32 ? true : n_total <= few && (ws >= 5 || (ws >= 2 && !own));
+        // than eight.  us per call, runs against tiles: at 1 % 8 ranks of 200,000 elements 10.9 / 9.9, of 4 M 13.2 / 11.3, of
+        // 13 M 19.9 / 20.4, 5 ranks of 4 M 11.7 / 10.5, of 13 M 18.1 / 17.9, 3 of 2 M (which find their starts) 7.5 / 8.8, of 8 M
+        // 14.1 / 12.3, 12 of 13 M 26.6 / 24.7, of 26 M 39.0 / 46.3; at 2 % 8 of 34 M 56.1 / 49.6, of 60 M 82.4 / 76.7, of 96.5 M
+        // 117 / 113, 5 of 60 M 61.2 / 60.1, of 96.5 M 84.5 / 88.8, 9 of 96.5 M 135 / 121, 12 165 / 143; at 0.1 % 9 of 13 M 20.0 / 20.2,
+        // and where a block finds its starts 5 of 2 M 9.6 / 10.9, 6 of 4 M 10.4 / 12.0, 8 of 2 M 11.1 / 11.6.
+        const uint64_t few = per_tile > 32 ? 64u << 20 : ws > kRunWaves && per_tile > 8 ? 16u << 20 : 8u << 20;
+        const bool alone = own && (ws < 5 || per_tile <= 8);  // finds its starts, and its ranks are few or short
+        const bool tiles_faster = ws > kRunWaves && per_tile > 32 ? true : n_total <= few && ws >= 2 && !alone;
         // (calls that share a table keep to the runs, which notice a table that is not theirs, and to eight ranks)
         if (path == 0 && tuning().sparse_run_steps == 0) runs_take = shared_table ? ws <= kRunWaves : !tiles_faster;
     }
