@@ -288,8 +288,8 @@ __global__ __launch_bounds__(kBlock) void k_sparse_accumulate(float* acc, uint64
 // thread per pair: pair p writes the
 // entry of every tile that begins between pair p-1 and pair p (usually none), so
 // each entry is written exactly once for a sorted payload; the entries of a gap of
-// more than four tiles are shared by the wavefront: one thread that wrote them took 25 ns
-// for each, after all others.  us per call, one thread / so: two ranks of 6 M elements at 1 % whose pairs lie at the
+// more than four tiles are shared by the wavefront, once a thread of it has found one (asked for behind every pair, nine
+// ranks of 4 M elements at 1 % took 11.9 us instead of 11.7): one thread that wrote them took 25 ns for each, after all others.  us per call, one thread / so: two ranks of 6 M elements at 1 % whose pairs lie at the
 // bucket's front 33.8 / 13.5, eight of 8 M in two buckets, the last a fifth as long, 32.7 / 14.3 (where entries past the
 // last bucket's own tiles were written as well).  A thread takes eight consecutive pairs.  The pair loads do not wait for k: they stay inside the
 // payload's stride and are masked afterwards.
@@ -331,42 +331,51 @@ __global__ __launch_bounds__(kBlock) void k_sparse_bounds(WirePtrs wires, int ws
     // entries past the bucket's own tiles are read by nobody
     const uint32_t own_tiles = (uint32_t)((bn + kAccTile - 1) / kAccTile);
     const int lane = threadIdx.x & (kWave - 1);
-    // st[from .. to] = p, for the lane's own; a long gap - between clustered pairs, in front of the first, behind the
-    // last - is written by the whole wavefront
-    auto fill = [&](uint32_t from, uint32_t to, uint32_t p) {
-        const uint32_t n = from <= to ? to - from + 1 : 0u;
-        constexpr uint32_t kAlone = 4;
-        if (n && n <= kAlone)
-            for (uint32_t t = from; t <= to; t++) st[t] = p;
-        for (uint64_t far = __ballot(n > kAlone); far; far &= far - 1) {
-            const int l = __ffsll((long long)far) - 1;
-            const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)from, l), c = (uint32_t)__builtin_amdgcn_readlane((int)n, l);
-            const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)p, l);
-            for (uint32_t i = (uint32_t)lane; i < c; i += kWave) st[f + i] = v;
-        }
-    };
-    uint32_t prev = before;
-    uint32_t behind = own_tiles + 1;  // of the lane that holds the last pair: the first entry that is k
+    // The n entries from `from` on are `value`: those of pair p0 + j or, j = PP, the ones behind the bucket's last pair, if
+    // the thread has that.
+    struct Gap { uint32_t from, n, value; };
+    auto index = [&](int j) { return v[j / 2][(j & 1) * 2]; };
+    auto gap = [&](int j) {
+        const bool behind = j == PP;
+        const uint32_t p = behind ? k - 1 : p0 + (uint32_t)j;
+        if (behind ? k - 1 - p0 >= (uint32_t)PP : p >= k) return Gap{0u, 0u, 0u};
+        uint32_t at = behind ? 0u : index(j < PP ? j : 0);
+        if (behind) {
 #pragma unroll
-    for (int j = 0; j < PP; j++) {
-        const uint32_t p = p0 + (uint32_t)j;
-        const uint32_t idx = v[j / 2][(j & 1) * 2];
-        uint32_t from = 1, to = 0;
-        if (p < k) {
-            if (idx >= bn && status) *status = MCCL_HIP_ERR_INDEX;
-            to = idx / kAccTile;  // tiles [from, to] begin at pair p
-            if (to > own_tiles) to = own_tiles;
-            from = 0;
-            if (p > 0) {
-                if (prev >= idx && status) *status = MCCL_HIP_ERR_INDEX;  // not ascending
-                from = prev / kAccTile + 1;
-            }
-            if (p == k - 1) behind = to + 1;
+            for (int i = 0; i < PP; i++)
+                if (p0 + (uint32_t)i == p) at = index(i);
         }
-        fill(from, to, p);
-        prev = idx;
+        uint32_t to = at / kAccTile;  // the tile in which the pair lies
+        if (to > own_tiles) to = own_tiles;
+        if (behind) return Gap{to + 1, own_tiles - to, k};
+        const uint32_t from = p == 0 ? 0u : (j ? index(j ? j - 1 : 0) : before) / kAccTile + 1;
+        return Gap{from, from <= to ? to - from + 1 : 0u, p};
+    };
+    // a long gap - between clustered pairs, in front of the first, behind the last - is written by the whole wavefront
+    constexpr uint32_t kAlone = 4;
+    bool far = false;
+#pragma unroll
+    for (int j = 0; j <= PP; j++) {
+        const Gap g = gap(j);
+        if (g.n > kAlone) far = true;
+        else
+            for (uint32_t t = 0; t < g.n; t++) st[g.from + t] = g.value;
+        if (j < PP && p0 + (uint32_t)j < k && status) {
+            if (index(j) >= bn) *status = MCCL_HIP_ERR_INDEX;
+            if (p0 + (uint32_t)j > 0 && (j ? index(j - 1) : before) >= index(j)) *status = MCCL_HIP_ERR_INDEX;  // not ascending
+        }
     }
-    fill(behind, own_tiles, k);
+    if (!__ballot(far)) return;
+#pragma unroll
+    for (int j = 0; j <= PP; j++) {
+        const Gap g = gap(j);
+        for (uint64_t of = __ballot(g.n > kAlone); of; of &= of - 1) {
+            const int l = __ffsll((long long)of) - 1;
+            const uint32_t f = (uint32_t)__builtin_amdgcn_readlane((int)g.from, l), c = (uint32_t)__builtin_amdgcn_readlane((int)g.n, l);
+            const uint32_t value = (uint32_t)__builtin_amdgcn_readlane((int)g.value, l);
+            for (uint32_t i = (uint32_t)lane; i < c; i += kWave) st[f + i] = value;
+        }
+    }
 }
 
 // Accumulate with precomputed bounds: every block reads its 2 * ws bounds with one
