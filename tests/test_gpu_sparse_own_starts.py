@@ -67,6 +67,7 @@ def test_payloads_out_of_order_are_flagged(at):
 @pytest.mark.parametrize("ws,n,be,k", [
     (5, 2049, 2049, 81), (6, 16385, 16385, 161), (8, 1_000_001, 1_000_001, 10_000),   # a block finds its runs' starts
     (9, 2049, 2049, 20), (10, 300_001, 100_000, 1000), (11, 65_537, 65_537, 700), (12, 1_000_003, 400_000, 4000),
+    (3, 16_900_001, 6_553_600, 131_072),                                              # runs of two dense tiles
     (12, 30_000, 30_000, 1400),                                                       # more pairs than the windows hold
     (3, 40_000_000, 6_553_600, 60_000), (6, 8_388_608, 8_388_608, 80_000),            # more than 8 M elements, not more
     (10, 16_777_217, 6_553_600, 65_536), (12, 16_777_216, 6_553_600, 65_536)])        # more than 16 M, not more
