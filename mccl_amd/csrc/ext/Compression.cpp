@@ -282,7 +282,9 @@ int TopKCompressor::wait_for_ticket(uint32_t ticket) {
     const auto reported = [&] { return (seen = __atomic_load_n(word, __ATOMIC_ACQUIRE)) >> 32 == ticket; };
     const auto start = std::chrono::steady_clock::now();
     for (uint32_t polls = 0; !reported(); polls++) {
+#if defined(__x86_64__)
         __builtin_ia32_pause();
+#endif
         if ((polls & 63) == 63 && std::chrono::steady_clock::now() - start > std::chrono::microseconds(500)) {
             counters_usable_ = false;  // should the launch not have ended well
             wait_for_current_stream();

@@ -466,7 +466,7 @@ struct StreamShape {
     static constexpr int kPerSimd = kTiles == 1 ? 6 : 8;       // wavefronts that the registers are to leave room for
 };
 // What a tile keeps of its candidates.  MANY: calls whose ratio makes more of them than kTileSlots take (topk_many); a
-// quarter of a wavefront's elements, which a ratio of 12 % leaves half empty.  15 buckets of 6,553,600 elements, us: at 2 % 669 on
+// quarter of a wavefront's elements is staged, of which a ratio of 12 % takes 58 % (window_share: 148 of 256).  15 buckets of 6,553,600 elements, us: at 2 % 669 on
 // the path with 128 slots (most tiles dense), 230 so; at 5 % 852 / 252; one bucket at 5 % 140 on the exact path, 38.5 so.  What
 // bounds it is the same stream as at 1 % (186 us of it) and, at 5 %, the candidates' 16 bytes written, read twice and listed.
 template <bool MANY>
@@ -624,8 +624,8 @@ __device__ __forceinline__ void dense_tile_walk(const float* rp, uint64_t bn, ui
 }
 
 // ---- a group's tiles as a bin block / select block sees them ------------------------------
-// The slots of up to HELD tiles per wavefront stay in registers, the rest (buckets of more
-// than 64 * NW * HELD tiles) are re-read from memory on every sweep.  AGENT: the slots were
+// The slots of up to HELD tiles per wavefront stay in registers, the rest (groups of more
+// than NW * HELD tiles) are re-read from memory on every sweep.  AGENT: the slots were
 // written by other blocks of the same launch (agent-scope loads), else by an earlier launch.
 template <bool AGENT, int NW, int HELD>
 struct GroupTiles {
@@ -633,7 +633,7 @@ struct GroupTiles {
     const uint32_t* tcnt;
     const uint64_t* slots;
     uint32_t t0;        // the group's first tile
-    uint32_t wt0, wt1;  // this wavefront's tiles: a contiguous quarter of the group's
+    uint32_t wt0, wt1;  // this wavefront's tiles: a contiguous share of the group's, one of NW
     int lane;
     bool more;          // wave-uniform: dense tiles, or tiles past the register window
     uint32_t cnt[kHeld];            // candidates in the tile's slots, or kDense (wave-uniform)
