@@ -259,6 +259,7 @@ std::vector<at::Tensor> TopKCompressor::compress_many(const std::vector<at::Tens
 // stream or the GPU right behind the call has such a marker put there, and waits for that one, unless one is there
 // already.  Compress and decompress at 1 % with a wait for the GPU behind them, us, waiting for the stream / reporting /
 // reporting with the marker: 2000 elements 24.8 / 29.0 / 23.0, 65,537 32.6 / 36.4 / 30.5, 6,553,600 56.8 / 61.7 / 55.7.
+// Pass after pass, without a wait, 1000 elements 21.1 / 18.0 / 17 to 20 from process to process, 65,537 29.1 / 25.8 / 25.2 to 26.6.
 void TopKCompressor::mark_end(void* stream) {
     if (end_ && end_device_ != counters_.get_device()) {
         (void)hipEventDestroy(static_cast<hipEvent_t>(end_));

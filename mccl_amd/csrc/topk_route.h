@@ -26,6 +26,9 @@ constexpr uint64_t kRMaxBucket = kRMaxBlocks * kRVecElems * 4;  // 2,097,152 ele
 // us per call at 1 %, 64 groups against 128: one bucket of 2.5 M elements 27.5 / 28.3, of 6,553,600 34.6 / 32.8, five of
 // them 90.7 / 89.6, 15, whose select blocks then go in two launches, 212 / 225; 128 against 256: one of 6,553,600
 // 32.8 / 33.9, of 13 M through compress and decompress 77.4 / 75.4.
+// At the lines, 64 / 128 / 256 groups: one bucket of 3.6 M 29.0 / 29.1 / 30.5, of 4 M 29.5 / 30.3 / 33.1, of 5 M 31.3 / 32.1 / 34.3, of 7.3 M 37.3 /
+// 35.5 / 37.4, of 8.4 M 41.7 / 37.4 / 38.6, of 8.5 M 46.0 / 39.9 / 42.0, of 9.5 M 50.6 / 42.7 / 42.9, of 13.1 M 66.9 / 52.4 / 51.8; two buckets of 4 M
+// 37.0 / 35.8 / 41.3, eight 91.4 / 92.0 / 115; 24 listed ones of 1001 to 4 M 53.0 / 54.8 / 58.7.
 constexpr uint32_t topk_group_shift_few(uint64_t tiles) { return tiles <= 64 * 14 ? 6 : tiles <= 128 * 16 ? 7 : 8; }
 // Otherwise more than 64 only past 28 tiles in each: so many a block keeps in registers, the others it reads again on
 // every pass.  64 groups against more: one bucket of 10 M elements 58 / 47, of 13.1 M 72 / 54, of 26.2 M 136 / 89.
