@@ -16,7 +16,7 @@ constexpr int kStateWords = 32;
 constexpr uint32_t kDense = 0xFFFFFFFFu;  // tile count: more candidates than slots, read the residual range itself
 constexpr uint32_t kPoisonK = 0xFFFFFFFFu;    // payload header of a bucket whose selection was abandoned
 // resident path (topk_resident.hip): per-bucket scratch, in words
-constexpr int kRList = 1024;                  // elements of the picked bin that are ranked as a list
+constexpr int kRList = 2048;                  // elements of the picked bin that are selected from as a list
 constexpr uint32_t kRRow = 2048 + 64;         // one round's histogram: its bins, the count above them, padding
 constexpr uint32_t kRRows = 4;                // a windowed round, three on the full key range (11 + 11 + 9 bits)
 constexpr uint32_t kRBars = 6;                // barriers: at most four rounds and the list / ties

@@ -7,19 +7,21 @@
 // and payload once.  The threshold is found by radix selection over the key's bits: a round
 // histograms the keys inside the current key range into 2048 bins in LDS, the blocks add theirs into
 // the bucket's histogram in memory, meet at a counter barrier and all pick the same bin.  When the
-// picked bin holds at most kRList elements they are gathered into one list, which every block ranks
-// by itself; otherwise the next round splits the bin, down to a single key whose ties are taken in
+// picked bin holds at most kRList elements they are gathered into one list, in which every block finds the
+// threshold by itself; otherwise the next round splits the bin, down to a single key whose ties are taken in
 // index order.  The first round covers a window around the threshold taken from a sample (large
 // buckets; the rounds restart on the full key range if it misleads) or every key (small ones); a
 // one-block bucket needs no memory but its own.  Any ratio and any distribution takes this path:
 // nothing depends on how the keys are spread.
 //
-// What bounds it is latency, not bandwidth.  One bucket of 1 M elements (16 MB of traffic), us from
-// the first block's start: window published 5.7, seen 6.4, first round's histogram in LDS 7.7, added up
-// and the blocks met 10.8, bin picked 11.8, listed 12.4, met 14.9, ranked 16.5, picks scanned 18.0,
-// stored 19.0.  Per call: 4096 elements 7.4 us (25.5 on the six launches of the exact path), 65,537 14.8
-// (27.7), 262,144 17.9 (25.4 on the two-launch path), 1 M 21.7 (26.7), 2 M 26.0; at a ratio of 5 % 1 M
-// elements 22.9 us (84.9) and 2 M 27.8 (144).
+// What bounds it is latency, not bandwidth: round trips of 0.6 us to memory that the XCDs share, and sixteen wavefronts
+// on four SIMDs, in which 150 instructions take a microsecond.  One bucket of 65,537 elements, us from the first block's
+// start: sums loaded 1.1, first round's histogram in LDS 2.3, added up and the blocks met 4.0, bin picked 5.0, listed 5.9,
+// met 7.7, threshold 9.5, picks counted 10.0, stored 10.4; of 1 M elements, whose window is published at 6.0, 17.9.
+// Per call, with lists of 1024 that were ranked as a whole up to 96, a wait for the lead block in front of the first
+// histogram, and picks counted through bits in LDS / so: 1000 elements 6.9 / 6.1 us, 4096 7.3 / 6.9, 8192 (then in two blocks)
+// 12.0 / 8.7, 16,384 12.2 / 10.7, 65,537 14.1 / 12.7, 262,144 16.8 / 15.8, 1 M 21.1 / 20.8, 2 M 25.0 / 24.5; at a ratio of
+// 5 % 65,537 14.5 / 13.2.  Blocks of 512 threads with twice the vectors are no faster (65,537 12.9, 1 M 21.8), of 256 slower.
 //
 // The blocks of a bucket wait for one another, so they have to be resident together, whatever else the
 // GPU runs.  At 64 registers, 54 KiB of LDS and 1024 threads two blocks fit a CU: 512 the GPU, 64 an XCD.  A
@@ -47,19 +49,18 @@ constexpr int kRThreads = 1024;
 constexpr int kRWaves = kRThreads / kWave;
 constexpr int kRBits = 11;
 constexpr int kRBins = 1 << kRBits;  // bins of one round
-constexpr int kRRank = 96;          // a list longer than this is split before it is ranked
+constexpr int kRRank = 64;           // a list longer than this is split before it is ranked
 static_assert(kRBins == 2 * kRThreads, "a thread owns two bins");
+static_assert(kRList == 2 * kRThreads, "a thread has two entries");
 
-template <int V>
 struct ResidentLds {
-    // a round's histogram, [kRBins] = keys above the range; later the block's picks, one bit per element
-    uint32_t lh[kRBins + 4] __attribute__((aligned(16)));
+    uint32_t lh[kRBins + 4] __attribute__((aligned(16)));  // a round's histogram, [kRBins] = keys above the range
     union {
         struct {
             uint64_t list[kRList];             // the picked bin's elements
-            uint64_t sub[kRList];              // ... those of one bin of the list
+            uint64_t sub[kRRank];              // ... those that are ranked
+            uint32_t rank[kRRank];
         };
-        uint32_t pre[kRThreads * 4 * V / 32];   // picks before each 32 elements
         SampleLds<kRThreads> s;
     };
     uint32_t scratch[kRWaves];
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
     // 3 x 300,000 18.7 / 17.4, one of 400,000 18.9 / 18.0, of 1 M 21.3 / 23.5, of 2 M 25.4 / 28.1, 2 x 1 M 22.0 / 24.0.
     constexpr uint32_t kSampleMin = 1u << 19;
     const BucketsArg bk = buckets_arg();
-    __shared__ ResidentLds<V> L;
+    __shared__ ResidentLds L;
     const int lane = threadIdx.x & (kWave - 1);
     const bool lead = blockIdx.x < nlead;
     uint32_t b = blockIdx.x, x = 0;  // bucket, block of the bucket
@@ -207,6 +208,11 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
     const bool full = b0 + PER <= bn;
     uint32_t* out = bucket_wire(g, bk, b);
 
+    const auto clear_histogram = [&] {
+        for (int i = threadIdx.x; i < (kRBins + 4) / 4; i += kRThreads) ((u4a*)L.lh)[i] = u4a{0u, 0u, 0u, 0u};
+    };
+    clear_histogram();
+    if (threadIdx.x == 0) L.count = 0;
     // ---- load: grad + residual, once ----------------------------------------------------------
     u4a a[V];
     {
@@ -258,11 +264,17 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
     // ---- rounds -----------------------------------------------------------------------------------
     uint32_t base = 0, span = 0x80000000u;  // keys base .. base + span - 1
     bool window = false;
-    if (nblk > 1) {
+    // Thread 0 waits for the lead block, the others for it at the next barrier: where there is a window to be had before
+    // the first histogram, else only before it is added to the bucket's, which the lead block has cleared by then.
+    const bool sampled = nblk > 1 && bn >= kSampleMin;
+    const auto wait_for_lead = [&] {
         if (threadIdx.x == 0) {
             const u4a wn = wait_window<2>(st, epoch, limit_ticks);
             L.win[0] = wn[0]; L.win[1] = wn[1]; L.win[3] = wn[3];
         }
+    };
+    if (sampled) {
+        wait_for_lead();
         __syncthreads();
         if (!L.win[3]) {
             give_up();
@@ -279,7 +291,6 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
         sh = 32 - __clz(span - 1);
         if (span == 1) sh = 0;
         sh = sh > (uint32_t)kRBits ? sh - kRBits : 0;
-        for (int i = threadIdx.x; i < (kRBins + 4) / 4; i += kRThreads) ((u4a*)L.lh)[i] = u4a{0u, 0u, 0u, 0u};
         __syncthreads();
         if (base == 0) {
             // every key: zeros, which would all add to one LDS word, are counted by the wavefront
@@ -306,10 +317,15 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
                 }
             }
         }
+        if (nblk > 1 && !sampled && row == 0) wait_for_lead();
         __syncthreads();
         u2a all = ((const u2a*)L.lh)[kRThreads - 1 - threadIdx.x];
         uint32_t above = first ? L.lh[kRBins] : 0u;
         if (nblk > 1) {
+            if (row == 0 && !L.win[3]) {
+                give_up();
+                return;
+            }
             uint32_t* const gh = mem + kRRow0 + row * kRRow;
             const uint64_t c = ((const uint64_t*)L.lh)[threadIdx.x];
             if (c) __hip_atomic_fetch_add((uint64_t*)gh + threadIdx.x, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // two bins
@@ -328,6 +344,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
             base = 0;
             span = 0x80000000u;
             window = false;
+            clear_histogram();
             continue;
         }
         bin = L.pick[0];
@@ -338,32 +355,20 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
         const uint32_t left = span - (bin << sh);
         span = left < (1u << sh) ? left : 1u << sh;
         if (m <= (uint32_t)kRList || span == 1) break;
-        __syncthreads();
+        clear_histogram();  // (what it held is in registers, and the pick lies behind two barriers)
     }
 
     // ---- the picked bin -----------------------------------------------------------------------------
+    static_assert(PER / 32 <= kRThreads, "a thread for each 32 elements");
     const bool tied = m > (uint32_t)kRList;  // one key, more often than the list holds: ties by index
     const uint32_t eq = L.lh[bin];           // this block's elements in the bin
-    uint32_t gt;                             // ... and above it
-    {
-        const u2a own = ((const u2a*)L.lh)[threadIdx.x];
-        uint32_t s = threadIdx.x == 0 ? L.lh[kRBins] : 0u;
-#pragma unroll
-        for (int q = 0; q < 2; q++) s += 2 * threadIdx.x + q > bin ? own[q] : 0u;
-        gt = block_sum(s, L.scratch);
-    }
     uint32_t T, istar, before;  // picks: key > T, or key == T and index <= istar; picks of earlier blocks
     {
         uint64_t* const cnts = (uint64_t*)(mem + kRCnt);
-        if (threadIdx.x == 0) {
-            L.count = 0;
-            if (nblk > 1) {
-                st_agent64(cnts + x, ((uint64_t)gt << 32) | eq);
-                if (!tied && eq)
-                    L.base = __hip_atomic_fetch_add(mem + kRFill, eq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        __syncthreads();
+        // where the block's elements go in the list (asked for first: the answer takes as long as what follows)
+        uint32_t list_at = 0;
+        if (nblk > 1 && threadIdx.x == 0 && !tied && eq)
+            list_at = __hip_atomic_fetch_add(mem + kRFill, eq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (!tied && eq) {  // block-uniform
 #pragma unroll
             for (int u = 0; u < V; u++) {
@@ -378,63 +383,103 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
                     }
                 }
             }
-            __syncthreads();
-            if (nblk > 1) {
+        }
+        uint64_t c = 0;  // of an earlier block: elements above the bin, inside the bin
+        if (nblk > 1) {
+            const u2a own = ((const u2a*)L.lh)[threadIdx.x];
+            uint32_t s = threadIdx.x == 0 ? L.lh[kRBins] : 0u;
+#pragma unroll
+            for (int q = 0; q < 2; q++) s += 2 * threadIdx.x + q > bin ? own[q] : 0u;
+            if (threadIdx.x == 0) L.base = list_at;
+            const uint32_t gt = block_sum(s, L.scratch);
+            if (threadIdx.x == 0) st_agent64(cnts + x, ((uint64_t)gt << 32) | eq);
+            if (!tied) {
                 uint64_t* gl = (uint64_t*)(mem + kRListAt) + L.base;
                 for (uint32_t i = threadIdx.x; i < eq && L.base + i < (uint32_t)kRList; i += kRThreads) st_agent64(gl + i, L.list[i]);
             }
-        }
-        uint32_t gt_before = 0, eq_before = 0;
-        if (nblk > 1) {
             if (!resident_barrier(mem + kRBarWords * row, nblk, x, &L.flag, limit_ticks)) {
                 give_up();
                 return;
             }
-            const uint64_t c = threadIdx.x < x ? ld_agent64(cnts + threadIdx.x) : 0ull;
-            static_assert(kRList <= kRThreads, "one entry per thread");
-            if (!tied && threadIdx.x < m) L.list[threadIdx.x] = ld_agent64((const uint64_t*)(mem + kRListAt) + threadIdx.x);
-            gt_before = block_sum((uint32_t)(c >> 32), L.scratch);
-            if (tied) eq_before = block_sum((uint32_t)c, L.scratch);
+            if (threadIdx.x < x) c = ld_agent64(cnts + threadIdx.x);
+        } else {
+            __syncthreads();
         }
         if (!tied) {
-            // The r-th largest entry.  A long list is split once more first: 2048 bins over its key range,
-            // and only the bin that holds the entry is ranked, by counting for each of its entries the larger
-            // ones (1024 entries ranked that way take 10 us, a few dozen less than one).
-            const uint64_t me = threadIdx.x < m ? L.list[threadIdx.x] : 0ull;
-            const uint64_t* ranked = L.list;
+            // The r-th largest entry: by radix rounds over key and index (entries differ in their index), until few enough
+            // share a prefix to rank them, by counting for each of them the larger ones.
+            uint64_t me[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const uint32_t i = (uint32_t)j * kRThreads + threadIdx.x;
+                me[j] = i >= m ? 0ull : nblk > 1 ? ld_agent64((const uint64_t*)(mem + kRListAt) + i) : L.list[i];
+            }
+            if (threadIdx.x == 0) L.count = 0;
+            if (threadIdx.x < (uint32_t)kRRank) L.rank[threadIdx.x] = 0;
+            const uint64_t low = (uint64_t)base << 32;
             uint32_t rm = m, rr = r;
-            bool in = threadIdx.x < m;
-            if (m > (uint32_t)kRRank && span > 1) {  // block-uniform
-                sh = 32 - __clz(span - 1);
-                sh = sh > (uint32_t)kRBits ? sh - kRBits : 0;
+            int bits = 32 + (span > 1 ? 32 - __clz((int)(span - 1)) : 0);  // of the entries, less the smallest key's, still open
+            uint64_t prefix = 0;
+            const auto shares = [&](int j) {
+                return (uint32_t)j * kRThreads + threadIdx.x < m && (me[j] - low) >> bits == prefix >> bits;
+            };
+#pragma unroll 1
+            while (rm > (uint32_t)kRRank) {  // block-uniform
+                const int at = bits > kRBits ? bits - kRBits : 0;
+                __syncthreads();
                 ((u2a*)L.lh)[threadIdx.x] = u2a{0u, 0u};
-                if (threadIdx.x == 0) L.count = 0;
                 __syncthreads();
-                const uint32_t mybin = ((uint32_t)(me >> 32) - base) >> sh;
-                if (in) atomicAdd(&L.lh[mybin], 1u);
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    if (shares(j)) atomicAdd(&L.lh[(uint32_t)((me[j] - low ^ prefix) >> at)], 1u);
                 __syncthreads();
-                pick_bin2(((const u2a*)L.lh)[kRThreads - 1 - threadIdx.x], 0u, r, L.scratch, L.pick);
-                in = in && mybin == L.pick[0];
-                if (in) L.sub[atomicAdd(&L.count, 1u)] = me;
+                pick_bin2(((const u2a*)L.lh)[kRThreads - 1 - threadIdx.x], 0u, rr, L.scratch, L.pick);
+                prefix |= (uint64_t)L.pick[0] << at;
                 rr = L.pick[1];
                 rm = L.pick[2];
-                ranked = L.sub;
-                __syncthreads();
-            }
-            if (in) {
-                uint32_t rank = 0;
-#pragma unroll 4
-                for (uint32_t j = 0; j < rm; j++) rank += ranked[j] > me ? 1u : 0u;
-                if (rank == rr - 1) L.cut = me;
+                bits = at;
             }
             __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                if (shares(j)) {
+                    const uint32_t i = atomicAdd(&L.count, 1u);
+                    if (i < (uint32_t)kRRank) L.sub[i] = me[j];
+                }
+            __syncthreads();
+            {
+                // an entry a lane, and for each wavefront a part of the entries to compare it with
+                static_assert(kRRank == kWave, "a lane for each entry");
+                const uint32_t per = (rm + kRWaves - 1) / kRWaves, from = per * wave, to = from + per < rm ? from + per : rm;
+                if (from < to) {
+                    const uint64_t mine = L.sub[lane];
+                    uint32_t rank = 0;
+#pragma unroll 4
+                    for (uint32_t j = from; j < to; j++) rank += L.sub[j] > mine ? 1u : 0u;
+                    if ((uint32_t)lane < rm && rank) atomicAdd(&L.rank[lane], rank);
+                }
+                __syncthreads();
+                if (threadIdx.x < rm && L.rank[threadIdx.x] == rr - 1) L.cut = L.sub[threadIdx.x];
+                __syncthreads();
+            }
             const uint64_t cut = L.cut;
             T = (uint32_t)(cut >> 32);
             istar = ~(uint32_t)cut;
-            const uint32_t mine = threadIdx.x < m && me >= cut && ~(uint32_t)me < (uint32_t)b0 ? 1u : 0u;
-            before = gt_before + block_sum(mine, L.scratch);
+            before = 0;
+            if (nblk > 1) {
+                uint32_t mine = (uint32_t)(c >> 32);
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    mine += (uint32_t)j * kRThreads + threadIdx.x < m && me[j] >= cut && ~(uint32_t)me[j] < (uint32_t)b0 ? 1u : 0u;
+                before = block_sum(mine, L.scratch);
+            }
         } else {
             T = base;
+            uint32_t gt_before = 0, eq_before = 0;
+            if (nblk > 1) {
+                gt_before = block_sum((uint32_t)(c >> 32), L.scratch);
+                eq_before = block_sum((uint32_t)c, L.scratch);
+            }
             const uint32_t quota = r > eq_before ? (r - eq_before < eq ? r - eq_before : eq) : 0u;
             before = gt_before + (eq_before < r ? eq_before : r);
             istar = 0xFFFFFFFFu;
@@ -468,13 +513,12 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
         }
     }
 
-    // ---- picks: a bit per element, prefix sums over words of 32, then residual and payload ------
-    constexpr uint32_t WORDS = PER / 32;
-    static_assert(WORDS <= kRThreads && WORDS <= kRBins, "one word per thread");
-    __syncthreads();
-    if (threadIdx.x < WORDS) L.lh[threadIdx.x] = 0;
-    __syncthreads();
-    uint32_t nibs = 0;
+    // ---- picks, counted over the wavefront's vectors (256 consecutive elements each) and the block's wavefronts, then
+    // residual and payload
+    uint32_t nibs = 0;  // a bit per element, four of each vector
+    uint32_t inc[(V + 1) / 2];  // picks of vectors 2 i and 2 i + 1 in the lanes up to this one, 16 bits each
+#pragma unroll
+    for (int i = 0; i < (V + 1) / 2; i++) inc[i] = 0;
 #pragma unroll
     for (int u = 0; u < V; u++) {
         const u4a v = vec(u);
@@ -486,15 +530,22 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
             nib |= (key >= T + ((uint32_t)b0 + e + q > istar ? 1u : 0u) ? 1u : 0u) << q;
         }
         nibs |= nib << (4 * u);
-        if (nib) atomicOr(&L.lh[e >> 5], nib << (e & 31));
+        inc[u / 2] += (uint32_t)__popc(nib) << (16 * (u & 1));
     }
+    uint32_t total = 0;  // of the wavefront
+#pragma unroll
+    for (int i = 0; i < (V + 1) / 2; i++) {
+        inc[i] = wave_inclusive_scan(inc[i]);
+        const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)inc[i], kWave - 1);
+        total += (all & 0xFFFFu) + (all >> 16);
+    }
+    if (lane == 0) L.scratch[wave] = total;
     __syncthreads();
+    uint32_t pos0 = before;  // the position of the wavefront's first pick, then of each vector's
     {
-        uint32_t total;
-        const uint32_t run = block_scan(threadIdx.x < WORDS ? __popc(L.lh[threadIdx.x]) : 0u, L.scratch, &total);
-        if (threadIdx.x < WORDS) L.pre[threadIdx.x] = before + run;
+        const uint32_t t = lane < kRWaves ? L.scratch[lane] : 0u;
+        pos0 += (uint32_t)__builtin_amdgcn_readlane((int)(wave_inclusive_scan(t) - t), wave);
     }
-    __syncthreads();
     float* const rp = rbase + b0 + (uint32_t)wave * (256 * V);
     const uint32_t l4 = 4 * lane;
     const uint32_t left = full ? PER : (uint32_t)(bn - b0);
@@ -512,8 +563,9 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
             for (int q = 0; q < 3; q++)
                 if (e + q < left) rp[256 * u + l4 + q] = u2f(z[q]);
         }
+        const uint32_t up_to = inc[u / 2] >> (16 * (u & 1)) & 0xFFFFu;
         if (nib) {
-            uint32_t pos = L.pre[e >> 5] + __popc(L.lh[e >> 5] & ((1u << (e & 31)) - 1u));
+            uint32_t pos = pos0 + up_to - (uint32_t)__popc(nib);
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 if ((nib >> q & 1u) && pos < k) {  // (pos < k whatever the scratch memory held)
@@ -523,6 +575,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
                 }
             }
         }
+        pos0 += (uint32_t)__builtin_amdgcn_readlane((int)up_to, kWave - 1);
     }
     if (x == 0 && threadIdx.x == 0) {
         st[S_T] = T;

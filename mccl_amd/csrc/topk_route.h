@@ -131,13 +131,14 @@ constexpr uint32_t topk_shift(uint64_t tiles, uint64_t groups, bool many, uint64
 constexpr uint64_t kFewestFits = 64;  // blocks of the fewest groups that a long bucket has
 
 // Vectors per thread of a resident launch, 0 when more than `limit` of its blocks would wait.  The barriers
-// cost more with more blocks, the passes over a block's elements with more vectors; measured (one bucket,
-// 1 %): 262,144 elements 17.8 / 18.0 us with 1 / 2 vectors, 400,000 19.8 / 19.5, 524,288 20.0 / 19.3 / 20.7
+// cost more with more blocks, the passes over a block's elements with more vectors, and a bucket of one block has none of
+// the former; measured (one bucket, 1 %): 4097 elements 10.6 / 8.1 us with 1 / 2 vectors, 8192 10.9 / 8.6, but 12,000
+// 11.4 / 11.9 with 1 / 4, 16,384 12.2 / 12.1; 262,144 elements 17.8 / 18.0 us with 1 / 2 vectors, 400,000 19.8 / 19.5, 524,288 20.0 / 19.3 / 20.7
 // with 1 / 2 / 4, 700,000 21.1 / 22.2 with 2 / 4, 1 M 21.7 / 22.0.  Several buckets take as many as
 // bring the launch under the limit.
 inline int resident_vecs(const TopkCall& c, uint64_t limit) {
     if (c.bucket_elems > kRMaxBucket) return 0;
-    int v = c.bucket_elems <= 64 * kRVecElems ? 1 : c.bucket_elems <= (c.nbuckets == 1 ? 128 : 64) * 2 * kRVecElems ? 2 : 4;
+    int v = c.bucket_elems > kRVecElems && c.bucket_elems <= 2 * kRVecElems ? 2 : c.bucket_elems <= 64 * kRVecElems ? 1 : c.bucket_elems <= (c.nbuckets == 1 ? 128 : 64) * 2 * kRVecElems ? 2 : 4;
     for (; v <= 4; v *= 2)
         if (resident_waiting(c, v) <= limit) return v;
     return 0;
