@@ -559,7 +559,7 @@ struct StreamLds {
 struct SelectLds {
     uint32_t lh[kBins0] __attribute__((aligned(16)));  // radix rounds, tie-break, exact fallback
     uint32_t dbuf[kFWaves][16 * kWave];  // dense_tile_walk's staging area, one per wavefront
-    uint32_t wsum[1][kBlock / kWave];
+    uint32_t wsum[kBlock / kWave];
     uint32_t res[1][2];
     uint32_t rcnt[kFWaves][kHeld];
     uint32_t wtot[kFWaves];
@@ -864,7 +864,7 @@ __device__ __forceinline__ void fused_bin(BucketsArg bk, const Geometry& g, cons
 // load, and one kernel for both layouts kept 13 more scalar registers in vector lanes (the 96.5 M gradient 2.5 us).
 template <int THREADS, bool LISTED, bool MANY>
 __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_topk_stream(Buckets, Geometry g, Workspace w, uint32_t epoch,
-                                                        uint32_t published, uint32_t first_wave,
+                                                        uint32_t published, uint32_t first_wave, uint32_t hold,
                                                         uint64_t limit_ticks) {
     g.listed = LISTED;
     const BucketsArg bk = buckets_arg();
@@ -915,10 +915,9 @@ __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_top
         return;
     }
     if (t * kTiles >= fg.ntiles) return;
-    // The blocks that start together with the sample blocks would bury the samples' few loads under
-    // 40 MB of their own and then wait for the samples all the same: they hold back for two
-    // microseconds, and the memory system is busy with their loads while the samples are evaluated.
-    if (blockIdx.x < first_wave) __builtin_amdgcn_s_sleep(80);
+    // The blocks that start together with the sample blocks hold back (stream_hold).
+    if (blockIdx.x < first_wave)
+        for (uint32_t i = 0; i < hold; i++) __builtin_amdgcn_s_sleep(8);
     const uint64_t bn = fg.bn;
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
@@ -1353,9 +1352,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
         });
         __syncthreads();
         {
-            const uint32_t* const hists[1] = {lh};
             const uint32_t wants[1] = {want};
-            sample_pick<kBinsR, 1, kBlock>(hists, wants, L.wsum, L.res);
+            sample_pick<kBinsR, 1, kBlock>(lh, wants, L.wsum, L.res);
         }
         const uint32_t bin = L.res[0][0], left = L.res[0][1];
         __syncthreads();  // res is rewritten by the next round
@@ -1586,7 +1584,7 @@ uint32_t next_epoch() {
 
 // The two launches of the single-pass path.
 template <int THREADS, bool LISTED, bool MANY>
-void launch_stream(Buckets& bk, const Geometry& g, const Workspace& w, uint64_t limit_ticks, hipStream_t st) {
+void launch_stream(Buckets& bk, const Geometry& g, const Workspace& w, uint64_t tiles, uint64_t limit_ticks, hipStream_t st) {
     // a sample block per bucket, then per bucket its tiles and its bin blocks
     constexpr uint32_t per = StreamShape<THREADS>::kTiles;
     uint64_t blocks = (uint64_t)g.nbuckets * ((g.ftiles + per - 1) / per + g.ngroups + 1) + g.ngroups;
@@ -1612,7 +1610,8 @@ void launch_stream(Buckets& bk, const Geometry& g, const Workspace& w, uint64_t 
     const uint32_t first_wave = g.nbuckets + (uint32_t)device_info().num_cus * (uint32_t)per_cu;
     // (tests of the give-up path: the sample blocks publish a number nobody waits for)
     const uint32_t published = tuning().topk_stall_test ? ~epoch : epoch;
-    k_topk_stream<THREADS, LISTED, MANY><<<(uint32_t)blocks, THREADS, 0, st>>>(bk, g, w, epoch, published, first_wave, limit_ticks);
+    k_topk_stream<THREADS, LISTED, MANY><<<(uint32_t)blocks, THREADS, 0, st>>>(bk, g, w, epoch, published, first_wave,
+                                                                                          stream_hold(tiles, g.nbuckets), limit_ticks);
 }
 
 template <bool LISTED, bool MANY>
@@ -1638,8 +1637,8 @@ void launch_single_pass(const Buckets& call, const Geometry& geometry, const Wor
         for (uint32_t b = g.nbuckets; b < kMaxListed; b++) bk.lfirst[b] = 0xFFFFFFFFu;
         set_groups(&g, groups, fits);
     }
-    if (stream_wide(tiles)) launch_stream<512, LISTED, MANY>(bk, g, w, lim, st);
-    else launch_stream<256, LISTED, MANY>(bk, g, w, lim, st);
+    if (stream_wide(tiles)) launch_stream<512, LISTED, MANY>(bk, g, w, tiles, lim, st);
+    else launch_stream<256, LISTED, MANY>(bk, g, w, tiles, lim, st);
     // the select launch, at most kSelBlocks blocks at a time: all of them are resident
     // together, whatever the order in which the hardware dispatches them
     for (uint32_t b0 = 0; b0 < g.nbuckets;) {

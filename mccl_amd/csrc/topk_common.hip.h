@@ -280,73 +280,61 @@ struct SampleLds {
     static constexpr int kCopies = THREADS >= 1024 ? 4 : THREADS >= 512 ? 2 : 1;
     static constexpr int kCopy = kBins0 + 8;  // words
     uint32_t h0[kCopies * kCopy] __attribute__((aligned(16)));
-    uint32_t lh[3][kBinsR] __attribute__((aligned(16)));
-    uint32_t wsum[3][THREADS / kWave];
+    uint32_t h1[kBins0] __attribute__((aligned(16)));
+    uint32_t wsum[THREADS / kWave];
     uint32_t res[3][2];
 };
 
-// For NR ranks at once: the bin in which a top-down scan of histogram h[z] reaches rank[z],
+// For NR ranks at once: the bin in which a top-down scan of the histogram reaches rank[z],
 // and how many of the rank's elements fall inside that bin.  Thread t owns the PER bins below
 // BINS - PER t (vector LDS reads).  res[z] = {bin, left}; bin = BINS when the histogram holds
-// fewer than rank[z] elements or rank[z] == 0.  SHARED: all ranks are read off h[0].  Called
-// by all threads of the block.  COPIES: every histogram is the sum of that many, STRIDE words apart.
-template <int BINS, int NR, int THREADS, bool SHARED = false, int COPIES = 1, int STRIDE = 0>
-__device__ __forceinline__ void sample_pick(const uint32_t* const (&h)[NR], const uint32_t (&rank)[NR],
-                                            uint32_t (*wsum)[THREADS / kWave], uint32_t (*res)[2]) {
+// fewer than rank[z] elements or rank[z] == 0.  Called by all threads of the block.  COPIES: the
+// histogram is the sum of that many, STRIDE words apart.
+template <int BINS, int NR, int THREADS, int COPIES = 1, int STRIDE = 0>
+__device__ __forceinline__ void sample_pick(const uint32_t* h, const uint32_t (&rank)[NR], uint32_t* wsum, uint32_t (*res)[2]) {
     constexpr int PER = BINS / THREADS;
     constexpr int RW = PER % 4 == 0 ? 4 : PER;  // bins per LDS read
-    constexpr int NH = SHARED ? 1 : NR;       // histograms actually scanned
     static_assert(PER % RW == 0, "whole vectors");
     typedef uint32_t Row __attribute__((ext_vector_type(RW)));
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-    uint32_t c[NH][PER], sum[NH], inc[NH];  // c[z][j]: bin BINS - 1 - PER t - j
+    uint32_t c[PER], sum = 0;  // c[j]: bin BINS - 1 - PER t - j
+    const Row* row = (const Row*)&h[BINS - PER * (threadIdx.x + 1)];
 #pragma unroll
-    for (int z = 0; z < NH; z++) {
-        const Row* row = (const Row*)&h[z][BINS - PER * (threadIdx.x + 1)];
-        sum[z] = 0;
+    for (int v = 0; v < PER / RW; v++) {
+        Row x = row[PER / RW - 1 - v];
 #pragma unroll
-        for (int v = 0; v < PER / RW; v++) {
-            Row x = row[PER / RW - 1 - v];
+        for (int d = 1; d < COPIES; d++) x += row[PER / RW - 1 - v + d * (STRIDE / RW)];
 #pragma unroll
-            for (int d = 1; d < COPIES; d++) x += row[PER / RW - 1 - v + d * (STRIDE / RW)];
-#pragma unroll
-            for (int q = 0; q < RW; q++) {
-                c[z][v * RW + q] = x[RW - 1 - q];
-                sum[z] += x[RW - 1 - q];
-            }
+        for (int q = 0; q < RW; q++) {
+            c[v * RW + q] = x[RW - 1 - q];
+            sum += x[RW - 1 - q];
         }
-        inc[z] = wave_inclusive_scan(sum[z]);
-        if (lane == kWave - 1) wsum[z][wave] = inc[z];
     }
+    const uint32_t inc = wave_inclusive_scan(sum);
+    if (lane == kWave - 1) wsum[wave] = inc;
     if (threadIdx.x < NR) { res[threadIdx.x][0] = BINS; res[threadIdx.x][1] = 0; }
     __syncthreads();
-    uint32_t above0[NH];
+    const uint32_t s = lane < THREADS / kWave ? wsum[lane] : 0u;
+    uint32_t above = inc - sum + (uint32_t)__builtin_amdgcn_readlane((int)(wave_inclusive_scan(s) - s), wave);
 #pragma unroll
-    for (int z = 0; z < NH; z++) {
-        const uint32_t s = lane < THREADS / kWave ? wsum[z][lane] : 0u;
-        above0[z] = inc[z] - sum[z] + (uint32_t)__builtin_amdgcn_readlane((int)(wave_inclusive_scan(s) - s), wave);
-    }
+    for (int j = 0; j < PER; j++) {
 #pragma unroll
-    for (int z = 0; z < NR; z++) {
-        const int zh = SHARED ? 0 : z;
-        uint32_t above = above0[zh];
-#pragma unroll
-        for (int j = 0; j < PER; j++) {
-            if (above < rank[z] && rank[z] <= above + c[zh][j]) {
+        for (int z = 0; z < NR; z++) {
+            if (above < rank[z] && rank[z] <= above + c[j]) {
                 res[z][0] = (uint32_t)(BINS - 1 - PER * (int)threadIdx.x - j);
                 res[z][1] = rank[z] - above;
             }
-            above += c[zh][j];
         }
+        above += c[j];
     }
     __syncthreads();
 }
 
 // Candidate window of a bucket from 8192 evenly spread elements of grad + residual, whose keys stay
-// in registers: radix select (11 + 10 key bits) of three ranks - upper and lower end of the window,
-// 6 sigma of the sampling noise away from the expected rank of the k-th largest key, and the
-// predicted threshold.  Called by all THREADS threads of a block; the result is valid in thread 0.
+// in registers: select of three ranks - upper and lower end of the window, 6 sigma of the sampling
+// noise away from the expected rank of the k-th largest key, and the predicted threshold - by 11 key
+// bits and then, in one histogram for all three, by 2048 bins over the digits that they lie in.  Called by all THREADS threads of a block; the result is valid in thread 0.
 // `under_way()` runs while the sample's loads are under way.
 struct SampleWindow {
     uint32_t lo, hi, that;
@@ -373,8 +361,8 @@ __device__ __forceinline__ SampleWindow sample_window(const float* gp, const flo
     constexpr int COPIES = SampleLds<THREADS>::kCopies, COPY = SampleLds<THREADS>::kCopy;
     {
         const u4a z = {0u, 0u, 0u, 0u};
-        static_assert(offsetof(SampleLds<THREADS>, lh) == sizeof(L.h0), "cleared as one");
-        for (int i = threadIdx.x; i < (COPIES * COPY + 3 * kBinsR) / 4; i += THREADS) ((u4a*)L.h0)[i] = z;
+        static_assert(offsetof(SampleLds<THREADS>, h1) == sizeof(L.h0), "cleared as one");
+        for (int i = threadIdx.x; i < (COPIES * COPY + kBins0) / 4; i += THREADS) ((u4a*)L.h0)[i] = z;
     }
     uint32_t* const h0 = L.h0 + (threadIdx.x % COPIES) * COPY;
     uint32_t key[PV][4];
@@ -398,9 +386,8 @@ __device__ __forceinline__ SampleWindow sample_window(const float* gp, const flo
     rank[1] = (uint32_t)(ks + margin) + 1u;                       // > S: no lower end
     rank[2] = ks >= 1.0f ? (uint32_t)ks : 1u;
     const bool active[NR] = {rank[0] >= 1u && rank[0] <= S, rank[1] <= S, rank[2] <= S};
-    uint32_t prefix[NR];
     __syncthreads();
-    // round 0: key[30:20], one histogram for all ranks
+    // round 0: key[30:20]
 #pragma unroll
     for (int j = 0; j < PV; j++)
 #pragma unroll
@@ -408,47 +395,48 @@ __device__ __forceinline__ SampleWindow sample_window(const float* gp, const flo
             if (key[j][q] != 0xFFFFFFFFu) atomicAdd(&h0[key[j][q] >> 20], 1u);
     __syncthreads();
     {
-        const uint32_t* const hs[NR] = {L.h0, L.h0, L.h0};
         const uint32_t want[NR] = {active[0] ? rank[0] : 0u, active[1] ? rank[1] : 0u, active[2] ? rank[2] : 0u};
-        sample_pick<kBins0, NR, THREADS, true, COPIES, COPY>(hs, want, L.wsum, L.res);
+        sample_pick<kBins0, NR, THREADS, COPIES, COPY>(L.h0, want, L.wsum, L.res);
     }
+    // round 1: the digits that the ranks lie in and those between, few of the keys, in one histogram.  (Compared with each
+    // rank's digit and counted in a histogram of its own, the keys take 40 instructions each instead of six: 1.6 us of a
+    // block of 512 threads, 1.9 with the three scans.)
+    uint32_t first = kBins0, last = 0, above = 0;  // of those digits; the keys above them
 #pragma unroll
     for (int z = 0; z < NR; z++) {
-        prefix[z] = L.res[z][0] << 20;
-        rank[z] = L.res[z][1];
+        const uint32_t d = L.res[z][0];
+        if (active[z] && d < first) first = d;
+        if (active[z] && d >= last) {
+            last = d;
+            above = rank[z] - L.res[z][1];
+        }
     }
-    // round 1: key[19:10] among the keys that share a rank's first digit
-    // (three comparisons per key; the few keys that share a rank's first digit take the branch)
-    const uint32_t d0 = active[0] ? prefix[0] >> 20 : 0xFFFFFFFFu, d1 = active[1] ? prefix[1] >> 20 : 0xFFFFFFFFu,
-                   d2 = active[2] ? prefix[2] >> 20 : 0xFFFFFFFFu;
+    const uint32_t base = first << 20, span = (last - first + 1) << 20;
+    const int open = 32 - __clz((int)(span - 1)), sh = open > 11 ? open - 11 : 0;
 #pragma unroll
     for (int j = 0; j < PV; j++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const uint32_t kq = key[j][q], d = kq >> 20;
-            if (d == d0 || d == d1 || d == d2) {
-                const uint32_t bin = (kq >> 10) & (kBinsR - 1);
-                if (d == d0) atomicAdd(&L.lh[0][bin], 1u);
-                if (d == d1) atomicAdd(&L.lh[1][bin], 1u);
-                if (d == d2) atomicAdd(&L.lh[2][bin], 1u);
-            }
+            const uint32_t d = key[j][q] - base;
+            if (d < span) atomicAdd(&L.h1[d >> sh], 1u);
         }
+    // (what under_way stored has long arrived; every wavefront makes sure of its part before thread 0 publishes)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     {
-        const uint32_t* const hs[NR] = {L.lh[0], L.lh[1], L.lh[2]};
-        const uint32_t want[NR] = {active[0] ? rank[0] : 0u, active[1] ? rank[1] : 0u, active[2] ? rank[2] : 0u};
-        sample_pick<kBinsR, NR, THREADS>(hs, want, L.wsum, L.res);
+        const uint32_t want[NR] = {active[0] ? rank[0] - above : 0u, active[1] ? rank[1] - above : 0u, active[2] ? rank[2] - above : 0u};
+        sample_pick<kBins0, NR, THREADS>(L.h1, want, L.wsum, L.res);
     }
     SampleWindow win = {0u, 0x7FFFFFFFu, 0x7FFFFFFFu};
     if (threadIdx.x == 0) {
-#pragma unroll
-        for (int z = 0; z < NR; z++) prefix[z] |= (L.res[z][0] & (uint32_t)(kBinsR - 1)) << 10;
-        win.lo = active[1] ? prefix[1] : 0u;
-        win.hi = active[0] ? (prefix[0] | 0x3FFu) : 0x7FFFFFFFu;  // upper end of the window: rounded up
+        const auto cell = [&](int z) { return base + (L.res[z][0] << sh); };
+        const uint32_t width = 1u << sh;
+        win.lo = active[1] ? cell(1) : 0u;
+        win.hi = active[0] ? cell(0) + (width - 1) : 0x7FFFFFFFu;  // upper end of the window: rounded up
         if (win.hi < win.lo) win.hi = win.lo;
-        // predicted threshold: middle of its 1024-key cell; never below lo: every pre-zeroed
+        // predicted threshold: middle of its cell; never below lo: every pre-zeroed
         // element must be a listed candidate
-        win.that = active[2] ? (prefix[2] | 0x200u) : 0x7FFFFFFFu;
+        win.that = active[2] ? cell(2) + width / 2 : 0x7FFFFFFFu;
         if (win.that < win.lo) win.that = win.lo;
     }
     return win;

@@ -82,6 +82,18 @@ constexpr uint32_t topk_group_shift_many(uint64_t tiles, uint64_t groups) {
 // 24 of 1.7 M 119.1 / 120.4, four of 13.1 M 133 / 138, 15 of 6,553,600 216.6 / 221.3.
 constexpr bool stream_wide(uint64_t tiles) { return tiles <= kWideTiles; }
 
+// How long the streaming blocks that start together with the sample blocks hold back, in steps of 512 clocks (0.21 us):
+// their loads would bury the samples' few, and they wait for the samples all the same.  A launch whose tiles are loaded
+// before its samples are evaluated gains by waiting longer; one with more, by loading sooner.  us per call at 1 %, 15 / 12.5 / 10 /
+// 7 / 5.5 steps: one bucket of 2.2 M elements 25.9 / 26.1 / 26.3 / 27.2 / 27.1, of 4 M 28.3 / 28.2 / 28.8 / 29.9 / 29.8, of 5 M 30.8 / 30.4 /
+// 30.6 / 31.7 / 32.3, of 6 M 32.7 / 32.2 / 31.9 / 33.1 / 33.8, of 6,553,600 36.7 / 36.6 / 35.3 / 33.8 / 34.1, of 10 M 45.7 / 45.7 / 45.3 /
+// 44.5 / 44.6; two of 2.2 M 29.4 / 28.6 / 27.9 / 29.0 / 29.5, of 3 M 34.2 / 33.8 / 33.0 / 31.6 / 31.5; 24 listed ones of 1001 to 1 M (905
+// tiles) 31.8 / 30.8 / 30.6 / 30.6 / 30.6, to 1.5 M (1343) 36.4 / 36.0 / 35.3 / 33.8 / 33.5; one of 4 M at 5 % 34.3 / 34.7 / 35.7 / 36.6 / 36.2.
+constexpr uint32_t stream_hold(uint64_t tiles, uint32_t nbuckets) {
+    if (nbuckets == 1) return tiles <= 1024 ? 14 : tiles <= 1536 ? 11 : 7;
+    return tiles <= 1152 ? 10 : 7;
+}
+
 // The buckets of a call: consecutive ranges of bucket_elems elements, the last one shorter, or, with
 // counts, nbuckets buffers of those lengths, bucket_elems the longest.
 struct TopkCall {

@@ -1,0 +1,39 @@
+"""Sampled candidate windows whose ends lie in one digit of the key, in neighbouring ones, far apart, or nowhere, on the
+streaming path and on the resident one."""
+import numpy as np
+import pytest
+
+from oracle import F32
+import oracle
+from tests._gpu_util import DEV, to_dev, to_np, bits, student_t
+
+pytestmark = pytest.mark.gpu
+
+
+def _values(kind, n, ratio):
+    rng = np.random.default_rng(n)
+    if kind == "narrow":      # magnitudes of [1, 1.1): one digit
+        return (1.0 + rng.random(n) * 0.1).astype(np.float32) * rng.choice(np.array([1, -1], np.float32), n)
+    g = student_t(rng, n, ties=0.0)
+    if kind == "cliff":       # half of the picks are far above everything else
+        g[rng.random(n) < ratio / 2] *= np.float32(1e30)
+    elif kind == "steps":     # magnitudes of many exponents, infinities on top
+        g *= np.exp2(rng.integers(-60, 60, n)).astype(np.float32)
+        g[rng.integers(0, n, 50)] = np.inf
+    return g
+
+
+@pytest.mark.parametrize("ratio", [0.0001, 0.01, 0.05])
+@pytest.mark.parametrize("kind", ["spread", "narrow", "cliff", "steps"])
+@pytest.mark.parametrize("n", [600_003, 2_200_001])
+def test_windows(n, kind, ratio):
+    from mccl_amd import hip_ops as ops
+    g, res = _values(kind, n, ratio), np.zeros(n, np.float32)
+    dres = to_dev(res, F32)
+    ws = ops.topk_workspace(n, n, ratio, DEV)
+    wire, _ = ops.topk_compress(to_dev(g, F32), dres, ratio, workspace=ws)
+    want, size = oracle.topk_compress(g, res, ratio)
+    if kind in ("spread", "narrow"):
+        assert ops.topk_path_report(ws, n, n, ratio) == (1, 1)   # the window holds the threshold
+    assert wire.cpu().numpy()[:size].tobytes() == want.tobytes()
+    assert np.array_equal(bits(to_np(dres, F32)), bits(res))
