@@ -33,7 +33,8 @@ def test_windows(n, kind, ratio):
     ws = ops.topk_workspace(n, n, ratio, DEV)
     wire, _ = ops.topk_compress(to_dev(g, F32), dres, ratio, workspace=ws)
     want, size = oracle.topk_compress(g, res, ratio)
-    if kind in ("spread", "narrow"):
-        assert ops.topk_path_report(ws, n, n, ratio) == (1, 1)   # the window holds the threshold
+    # the window holds the threshold, and its bin few enough (with a few picks in the sample a window has no upper end)
+    if kind == "spread" or kind == "narrow" and ratio > 0.001:
+        assert ops.topk_path_report(ws, n, n, ratio) == (1, 1)
     assert wire.cpu().numpy()[:size].tobytes() == want.tobytes()
     assert np.array_equal(bits(to_np(dres, F32)), bits(res))
