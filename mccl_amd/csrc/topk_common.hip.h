@@ -237,8 +237,9 @@ __device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v) {
 // 16-byte streaming store written through to memory (agent scope): a later 4-byte
 // repair of the same line by a block on another XCD must not be overwritten by a
 // delayed write-back of this one.  (The wait states: see store16_agent.)
-__device__ __forceinline__ void store_through(float* p, u4a v) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 2" ::"v"(p), "v"(v) : "memory");
+// `base` is the same in every lane, `at` the lane's element behind it.
+__device__ __forceinline__ void store_through(float* base, uint32_t at, u4a v) {
+    asm volatile("global_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 2" ::"v"(at * 4), "v"(v), "s"(base) : "memory");
 }
 
 // A bucket's window is one store16_agent and one load16_agent: the four words change together.
@@ -291,15 +292,16 @@ struct SampleLds {
 // fewer than rank[z] elements or rank[z] == 0.  Called by all threads of the block.  COPIES: the
 // histogram is the sum of that many, STRIDE words apart.
 template <int BINS, int NR, int THREADS, int COPIES = 1, int STRIDE = 0>
-__device__ __forceinline__ void sample_pick(const uint32_t* h, const uint32_t (&rank)[NR], uint32_t* wsum, uint32_t (*res)[2]) {
+__device__ __forceinline__ void sample_pick(const uint32_t* h, const uint32_t (&rank)[NR], uint32_t* wsum, uint32_t (*res)[2],
+                                            uint32_t tid = threadIdx.x) {
     constexpr int PER = BINS / THREADS;
     constexpr int RW = PER % 4 == 0 ? 4 : PER;  // bins per LDS read
     static_assert(PER % RW == 0, "whole vectors");
     typedef uint32_t Row __attribute__((ext_vector_type(RW)));
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+    const int lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(tid / kWave));
     uint32_t c[PER], sum = 0;  // c[j]: bin BINS - 1 - PER t - j
-    const Row* row = (const Row*)&h[BINS - PER * (threadIdx.x + 1)];
+    const Row* row = (const Row*)&h[BINS - PER * (tid + 1)];
 #pragma unroll
     for (int v = 0; v < PER / RW; v++) {
         Row x = row[PER / RW - 1 - v];
@@ -313,7 +315,7 @@ __device__ __forceinline__ void sample_pick(const uint32_t* h, const uint32_t (&
     }
     const uint32_t inc = wave_inclusive_scan(sum);
     if (lane == kWave - 1) wsum[wave] = inc;
-    if (threadIdx.x < NR) { res[threadIdx.x][0] = BINS; res[threadIdx.x][1] = 0; }
+    if (tid < NR) { res[tid][0] = BINS; res[tid][1] = 0; }
     __syncthreads();
     const uint32_t s = lane < THREADS / kWave ? wsum[lane] : 0u;
     uint32_t above = inc - sum + (uint32_t)__builtin_amdgcn_readlane((int)(wave_inclusive_scan(s) - s), wave);
@@ -322,7 +324,7 @@ __device__ __forceinline__ void sample_pick(const uint32_t* h, const uint32_t (&
 #pragma unroll
         for (int z = 0; z < NR; z++) {
             if (above < rank[z] && rank[z] <= above + c[j]) {
-                res[z][0] = (uint32_t)(BINS - 1 - PER * (int)threadIdx.x - j);
+                res[z][0] = (uint32_t)(BINS - 1 - PER * (int)tid - j);
                 res[z][1] = rank[z] - above;
             }
         }
