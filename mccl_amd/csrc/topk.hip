@@ -12,7 +12,8 @@
 //
 // RESIDENT PATH (topk_resident.hip; one launch): buckets of up to 2 M elements, 2 M a call.
 // SINGLE-PASS PATH (one pass over the gradient, 12 B/element of HBM traffic, two launches):
-// larger buckets and many buckets at a time; see the section "single-pass path" below.
+// larger buckets and many buckets at a time; see the section "single-pass path" below.  Lists of middle-sized buckets
+// take it in one launch (topk_whole.hip).
 // EXACT PATH (any input; six launches): ratios above 12 %, many small buckets,
 // and topk_path = 1 (topk_route.h has the rule and its measurements).
 //   [pass A]   residual <- grad + residual, histogram of key[30:20]
@@ -521,7 +522,7 @@ __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_top
     uint32_t b, t;
     bool emit = false;
     if constexpr (LISTED) {
-        b = listed_bucket(bk, j, &t);
+        b = listed_bucket(bk->lfirst, j, &t);
         const uint32_t sblocks = (topk_tiles(bk->lcount[b]) + kTiles - 1) / kTiles;
         if (t >= sblocks) {
             t -= sblocks;
@@ -600,7 +601,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
     const BucketsArg bk = buckets_arg();
     __shared__ SelectLds L;
     uint32_t b = first_bucket + blockIdx.y, grp = blockIdx.x;
-    if (g.listed) b = listed_bucket(bk, blockIdx.x, &grp);
+    if (g.listed) b = listed_bucket(bk->lfirst, blockIdx.x, &grp);
     const FusedGeo fg = fused_geo(g, bk, b);
     if (grp >= fg.ng) return;
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
@@ -1038,7 +1039,12 @@ bool launch_by_path(const Buckets& bk, const Geometry& g, const Workspace& w, co
     const uint64_t limit_ticks = (uint64_t)tuning().topk_barrier_ms * 100000ull;  // of 10 ns
     // (tests of the give-up path: the sample and lead blocks publish a number nobody waits for)
     const auto published = [](uint32_t epoch) { return tuning().topk_stall_test ? ~epoch : epoch; };
-    if (route.path == kPathStream) {
+    const uint32_t shift = most_groups_shift(g);
+    const uint32_t group_tiles = route.path == kPathStream ? whole_tiles(call, shift, whole_limit_on(share)) : 0;
+    if (group_tiles) {
+        const uint32_t epoch = next_epoch();
+        launch_whole(bk, g, w, group_tiles, shift, epoch, published(epoch), limit_ticks, st);
+    } else if (route.path == kPathStream) {
         if (g.listed) (g.many ? launch_single_pass<true, true> : launch_single_pass<true, false>)(bk, g, w, fits, st);
         else (g.many ? launch_single_pass<false, true> : launch_single_pass<false, false>)(bk, g, w, fits, st);
     } else {

@@ -42,7 +42,9 @@ enum {
     S_OK = 11,            // single-pass path: 1 when the window selection succeeded for this bucket
     S_EXACT_HIST = 12,    // 1 when hist round 0 holds the full histogram
     S_TIMEOUT = 13,       // single-pass path: a block gave up waiting (result invalid, payload header poisoned)
-    S_BARF = 16           // 16..19: barriers of the exact selection inside the select launch
+    S_BARF = 16,          // 16..19: barriers of the exact selection inside the select launch
+    S_DONE = 20,          // one launch: lines of select blocks that have arrived
+    S_LEFT = 21           // ... select blocks that are done
 };
 
 struct Geometry {
@@ -132,13 +134,13 @@ __device__ __forceinline__ uint32_t* bucket_wire(const Geometry& g, BucketsArg b
 }
 // Bucket of block j of a list's launch, and which of the bucket's blocks it is.  On the scalar unit: the
 // block's loads wait for it.
-__device__ __forceinline__ uint32_t listed_bucket(BucketsArg bk, uint32_t j, uint32_t* x) {
+__device__ __forceinline__ uint32_t listed_bucket(const __attribute__((address_space(4))) uint32_t* firsts, uint32_t j, uint32_t* x) {
     uint32_t b = 0;
     *x = j;
-    for (uint32_t c = 0; c < kMaxListed && bk->lfirst[c] <= j; c += 16) {
+    for (uint32_t c = 0; c < kMaxListed && firsts[c] <= j; c += 16) {
 #pragma unroll
         for (uint32_t i = 0; i < 16; i++) {
-            const uint32_t first = bk->lfirst[c + i];
+            const uint32_t first = firsts[c + i];
             if (first <= j) {
                 b = c + i;
                 *x = j - first;
@@ -167,6 +169,10 @@ StreamShare stream_share(hipStream_t st);
 uint64_t waiting_limit(const StreamShare& share, uint64_t per_cu);
 // ... of a resident launch.
 uint64_t resident_limit_on(const StreamShare& share);
+// The single-pass path's one launch (topk_whole.hip), for calls that whole_tiles admits.
+uint64_t whole_limit_on(const StreamShare& share);
+void launch_whole(const Buckets& bk, const Geometry& g, const Workspace& w, uint32_t group_tiles, uint32_t groups_shift, uint32_t epoch,
+                  uint32_t published, uint64_t limit_ticks, hipStream_t st);
 // A list of buckets goes in as many launches as keep each under `limit`.
 void launch_resident(const Buckets& bk, const Geometry& g, const Workspace& w, int vecs, uint64_t limit, uint32_t epoch,
                      uint32_t published, uint64_t limit_ticks, hipStream_t st);

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
     if (!lead) {
         const uint32_t j = blockIdx.x - nlead;
         if (g.listed) {
-            b = listed_bucket(bk, j, &x);
+            b = listed_bucket(bk->lfirst, j, &x);
         } else {
             const uint32_t per_bucket = (uint32_t)((g.bucket_elems + PER - 1) / PER);
             b = j / per_bucket;

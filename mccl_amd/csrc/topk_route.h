@@ -172,6 +172,37 @@ inline uint32_t next_launch(const uint32_t* counts, uint32_t* order, uint32_t le
     return taken;
 }
 
+// Tiles of a group where the streaming path takes a list in one launch (topk_whole.hip), an even number, the same for
+// every bucket; 0 where it takes two.  A group is a select block that waits for others, so a call has at most `limit` of
+// them (stream_limit), at most 1 << shift in a bucket, and candidates in it that its block can keep: beyond, a block reads
+// them from memory on each of four passes (24 buckets of 1001 to 1 M at 5 %, 33 and 10 tiles a group: 32.7 us in two
+// launches, 40 / 30 in one).  us per call, two launches / one: 24 buckets of 1001 to 1.5 M elements (1343 tiles) 33.8 / 28.9, at 0.1 %
+// 32.7 / 27.3, to 2.2 M 41.9 / 39.0, to 3 M (2750 tiles) 46.9 / 46.2, 12 of 1000 to 2 M 29.6 / 26.7, 60 of 1000 to 1 M 48.8 / 40.4, 16 of
+// 300,000 32.1 / 28.0, of 1 M 62.2 / 59.8, three of 100 to 6.5 M 35.7 / 34.2, two of 2.5 M 30.8 / 29.4, ten of 1000 to 3 M at 5 % 38.4 / 33.7.  Few large
+// buckets gain nothing: two of 4 M 38.4 / 41.1, five of 2.2 M 47.5 / 48.1; nor do those of one buffer, whose two launches have
+// no table to read: one bucket of 2.2 M 26.1 / 26.7, of 6,553,600 33.7 / 34.6, eight of 2.5 M 65 / 69.
+// Groups of a call: 24 buckets of 1001 to 1.5 M with 64 / 96 / 160 / 224 of them 31.2 / 30.3 / 29.1 / 28.9.
+constexpr uint32_t kWholeMost = 64;      // tiles of a group: a lane each
+constexpr uint32_t kWholeOwn = 2600;     // candidates of its group that a select block keeps in LDS
+constexpr uint32_t kWholeGroups = 256;
+constexpr uint64_t kWholeTiles = 4096;
+inline uint32_t whole_tiles(const TopkCall& c, uint32_t shift, uint64_t limit) {
+    if (!c.counts || limit < c.nbuckets) return 0;
+    uint64_t sum = 0;
+    for (uint32_t b = 0; b < c.nbuckets; b++) sum += topk_tiles(c.counts[b]);
+    if (sum > kWholeTiles || (sum > 1664 && c.nbuckets < 8)) return 0;
+    const uint64_t longest = topk_tiles(c.bucket_elems);
+    const double candidates = window_share((double)c.k_full / (double)c.bucket_elems) * kFTile;  // of a tile
+    uint32_t per = (uint32_t)((sum + kWholeGroups - 1) / kWholeGroups);
+    for (per = per < 8 ? 8 : per + (per & 1); per <= kWholeMost && per * candidates <= 0.92 * kWholeOwn; per += 2) {
+        if ((longest + per - 1) / per > 1u << shift) continue;
+        uint64_t groups = 0;
+        for (uint32_t b = 0; b < c.nbuckets; b++) groups += (topk_tiles(c.counts[b]) + per - 1) / per;
+        if (groups <= limit) return per;
+    }
+    return 0;
+}
+
 struct Route {
     Path path;
     int vecs;  // resident path: vectors per thread

@@ -1,5 +1,6 @@
-// The single-pass top-k path's tiles: their candidate slots and window bins, the streaming blocks, and the exact selection
-// that a bucket's select blocks run together when the window fails.
+// What the kernels of the single-pass top-k path (topk.hip: two launches, topk_whole.hip: one) share: the tiles, their
+// candidate slots and window bins, the streaming blocks, and the exact selection that a bucket's select blocks run together when
+// the window fails.
 #pragma once
 
 #include "topk_common.hip.h"
