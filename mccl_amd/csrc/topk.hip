@@ -561,35 +561,6 @@ __global__ __launch_bounds__(THREADS, StreamShape<THREADS>::kPerSimd) void k_top
     stream_tiles<THREADS, MANY>(bk, g, w, b, t * kTiles, fg, g.gshift, epoch, limit_ticks, L.a);
 }
 
-// The need-th smallest index among the list's entries with key == T: radix select over
-// the index, 11 + 11 + 10 bits.  for_list(f) calls f(index, key) for every entry of the list
-// this thread looks at.  Called by all threads of the block.
-template <class ForList>
-__device__ __forceinline__ uint32_t resolve_ties64(ForList&& for_list, uint32_t T, uint32_t need,
-                                                   uint32_t* lh /* kBins0 words */, uint32_t* scratch) {
-    uint32_t iwant = need, iprefix = 0;
-    const int shifts[3] = {21, 10, 0};
-    const int widths[3] = {11, 11, 10};
-    for (int r = 0; r < 3; r++) {
-        const int bins = 1 << widths[r];
-        for (int i = threadIdx.x; i < kBins0; i += kBlock) lh[i] = 0;
-        __syncthreads();
-        const int hs = shifts[r] + widths[r];
-        for_list([&](uint32_t idx, uint32_t key) {
-            const bool match = hs >= 32 ? true : ((idx >> hs) == (iprefix >> hs));
-            // bins stored reversed, so that pick_bin's top-down scan runs over ascending indices
-            if (key == T && match) atomicAdd(&lh[(bins - 1) - ((idx >> shifts[r]) & (bins - 1))], 1u);
-        });
-        __syncthreads();
-        uint32_t left;
-        const uint32_t rb = pick_bin<kBins0, kBlock>(lh, iwant, 0, &left, scratch);
-        iprefix |= ((uint32_t)(bins - 1) - (rb - (uint32_t)(kBins0 - bins))) << shifts[r];
-        iwant = left;
-    }
-    return iprefix;
-}
-
-
 // ---- the select launch ----------------------------------------------------------------------
 // blockIdx.x = group, blockIdx.y = bucket - first_bucket; of a list, blocks of all its buckets in a row
 // (Buckets::lfirst).  Everything the streaming launch
@@ -603,7 +574,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
     uint32_t b = first_bucket + blockIdx.y, grp = blockIdx.x;
     if (g.listed) b = listed_bucket(bk->lfirst, blockIdx.x, &grp);
     const FusedGeo fg = fused_geo(g, bk, b);
-    if (grp >= fg.ng) return;
+    if (grp * fg.tpg >= fg.ntiles) return;  // (no division on the way to the first loads)
     uint32_t* st = w.state + (uint64_t)b * kStateWords;
     uint32_t* out = bucket_wire(g, bk, b);
     // Every load of the first round trip is issued before the first value is looked at, the small
@@ -619,7 +590,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
     // a replay of a captured launch carries the same epoch: also behind a run that was given up
     if (grp == 0 && threadIdx.x == 0) st[S_READY] = 0u;
     if (gave_up) return;  // the streaming launch gave the bucket up: its payload header says so
-    const uint32_t lo = win[0], that_key = win[2], wmul = window_mul(win[0], win[1]);
+    const uint32_t lo = win[0], that_key = win[2];
     const uint32_t k = fg.k;
     const uint64_t bn = fg.bn;
     const int lane = threadIdx.x & (kWave - 1);
@@ -637,8 +608,9 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
         break;
     }
     const int lstar = __ffsll((long long)reach) - 1;
-    const uint32_t pair_hi = (uint32_t)__shfl((int)tot[1], lstar, kWave), pair_lo = (uint32_t)__shfl((int)tot[0], lstar, kWave);
-    const uint32_t above_pair = (uint32_t)__shfl((int)inc, lstar, kWave) - pair_hi - pair_lo;  // candidates in the bins above the pair
+    auto at_lstar = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, lstar); };
+    const uint32_t pair_hi = at_lstar(tot[1]), pair_lo = at_lstar(tot[0]);
+    const uint32_t above_pair = at_lstar(inc) - pair_hi - pair_lo;  // candidates in the bins above the pair
     const bool in_hi = above_pair + pair_hi >= k;                                     // the upper bin of the pair reaches k
     const uint32_t jstar = (uint32_t)(kCoarse - 1 - 2 * lstar) - (in_hi ? 0u : 1u);
     if (jstar == (uint32_t)(kCoarse - 1)) {  // the threshold lies at or above the window's upper end
@@ -658,82 +630,106 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
 
     // ---- 4: exact threshold from the bin's list ---------------------------------------------
     const uint64_t* l2 = w.blist + ((uint64_t)b * (kCoarse - 1) + jstar) * g.lcapb;
+    // The need-th largest entry by (key, then lower index): rounds of 10 bits over both until few entries share the
+    // prefix, and these are ranked by each wavefront for itself.  Most lists take one round (3500 entries over up to 1024
+    // digits), and ties need no search of their own.  With rounds over the whole key, of 1.3 us each, and searches for ties
+    // and for the group's place behind them a bucket of 6.5 M elements took 32.9 us, and 30.9 this way.
     // the first 4096 entries stay in registers (a bin of the expected width holds about 3500)
     constexpr int kL2Regs = 16;
     uint64_t ent[kL2Regs];
 #pragma unroll
     for (int j = 0; j < kL2Regs; j++) {
         const uint32_t i = (uint32_t)j * kBlock + threadIdx.x;
-        ent[j] = i < n2 ? l2[i] : 0ull;
+        ent[j] = l2[i < n2 ? i : n2 - 1];  // (n2 >= need >= 1)
     }
+    // (the bin's bounds take three divisions: made while the entries are on their way, with the first bound of the
+    // window hidden until here, as the compiler would make them before; 30.9 us -> 30.6)
+    uint32_t wlo = lo;
+    asm volatile("" : "+s"(wlo));
+    const uint32_t wmul = window_mul(wlo, win[1]);
+    const uint32_t bin_lo = window_bin_lo(wlo, wmul, jstar);  // smallest key of the threshold bin
+    const uint32_t bin_span = window_bin_lo(wlo, wmul, jstar + 1) - bin_lo;  // jstar <= kCoarse - 2
+    const uint32_t last = (uint32_t)(bn - 1);
+    const int index_bits = 32 - __clz((int)last);
+    auto order = [&](uint64_t e) { return ((uint64_t)(key64(e) - bin_lo) << index_bits) | (last - (uint32_t)e); };
+    // past the list's end: shares no prefix, and lies before no group
+#pragma unroll
+    for (int j = 0; j < kL2Regs; j++) ent[j] = (uint32_t)j * kBlock + threadIdx.x < n2 ? order(ent[j]) : 1ull << 63;
     auto for_list2 = [&](auto&& body) {
 #pragma unroll
         for (int j = 0; j < kL2Regs; j++)
-            if ((uint32_t)j * kBlock + threadIdx.x < n2) body((uint32_t)ent[j], key64(ent[j]));
+            if ((uint32_t)j * kBlock < n2) body(ent[j]);
 #pragma unroll 1
-        for (uint32_t i = kL2Regs * kBlock + threadIdx.x; i < n2; i += kBlock) {
-            const uint64_t e = l2[i];
-            body((uint32_t)e, key64(e));
-        }
+        for (uint32_t i = kL2Regs * kBlock + threadIdx.x; i < n2; i += kBlock) body(order(l2[i]));
     };
-    uint32_t above_before;
-    block_exclusive_scan(ab, L.scratch, &above_before);
     uint32_t* lh = L.lh;
-    const uint32_t bin_lo = window_bin_lo(lo, wmul, jstar);  // smallest key of the threshold bin
-    const uint32_t bin_span = window_bin_lo(lo, wmul, jstar + 1) - bin_lo;  // jstar <= kCoarse - 2
-    uint32_t vprefix = 0, want = need;              // key - bin_lo: up to 30 bits, selected as 10 + 10 + 10
-    // rounds whose digits lie wholly above the bin's span are skipped
-    const int first_round = bin_span <= (1u << 10) ? 2 : (bin_span <= (1u << 20) ? 1 : 0);
+    uint64_t* const few = (uint64_t*)(lh + kBinsR);  // the entries to rank
+    uint32_t* const nfew = lh + kBinsR + 2 * kWave;
+    int bits = index_bits + (bin_span > 1 ? 32 - __clz((int)(bin_span - 1)) : 0);  // of the entries still open
+    uint64_t prefix = 0;
+    uint32_t want = need, m = n2;
+    if (threadIdx.x == 0) *nfew = 0;
 #pragma unroll 1
-    for (int r = first_round; r < 3; r++) {
-        const int sh = 20 - 10 * r;
-        const int hs = sh + 10;
-        for (int i = threadIdx.x; i < kBinsR; i += kBlock) lh[i] = 0;
+    while (m > (uint32_t)kWave && !failed) {  // block-uniform
+        const int sh = bits > 10 ? bits - 10 : 0;
+        ((u4a*)lh)[threadIdx.x] = u4a{0u, 0u, 0u, 0u};
+        static_assert(kBinsR == 4 * kBlock, "cleared by one store each");
         __syncthreads();
-        for_list2([&](uint32_t, uint32_t key) {
-            const uint32_t v = key - bin_lo;
-            if ((v >> hs) == (vprefix >> hs)) atomicAdd(&lh[(v >> sh) & (kBinsR - 1)], 1u);
+        for_list2([&](uint64_t o) {
+            if ((o >> bits) == (prefix >> bits)) atomicAdd(&lh[(uint32_t)((o ^ prefix) >> sh)], 1u);
         });
         __syncthreads();
-        {
-            const uint32_t wants[1] = {want};
-            sample_pick<kBinsR, 1, kBlock>(lh, wants, L.wsum, L.res);
-        }
-        const uint32_t bin = L.res[0][0], left = L.res[0][1];
-        __syncthreads();  // res is rewritten by the next round
-        if (bin >= (uint32_t)kBinsR) {  // the list holds fewer matching keys than the counts promised
-            failed = true;
-            break;
-        }
-        vprefix |= bin << sh;
-        want = left;
+        const uint32_t wants[1] = {want};
+        sample_pick<kBinsR, 1, kBlock>(lh, wants, L.wsum, L.res);
+        const uint32_t bin = L.res[0][0];
+        want = L.res[0][1];
+        // the list holds fewer entries than the counts promised, or one of them twice
+        failed = bin >= (uint32_t)kBinsR || bits == 0;
+        if (!failed) m = lh[bin];
+        prefix |= (uint64_t)bin << sh;
+        bits = sh;
+        __syncthreads();  // the next round clears and writes what was read here
     }
     if (failed) break;
-    const uint32_t T = bin_lo + vprefix;
-    const uint32_t need2 = want;
-    const uint32_t ties = lh[vprefix & (kBinsR - 1)];
-    __syncthreads();
-    // when only some keys equal to T are taken, they are the need2 lowest indices
-    const uint32_t istar = ties != need2 ? resolve_ties64(for_list2, T, need2, lh, L.scratch) : 0xFFFFFFFFu;
-    auto is_pick = [&](bool valid, uint32_t key, uint32_t idx) {
-        return valid && (key > T || (key == T && idx <= istar));
-    };
-    // the threshold bin's picks at indices below this group's first element
-    uint32_t mine_before = 0, mine_all = 0;
-    const uint64_t first_elem = (uint64_t)G.t0 * kFTile;
-    for_list2([&](uint32_t idx, uint32_t key) {
-        if (is_pick(true, key, idx)) {
-            mine_all++;
-            mine_before += (uint64_t)idx < first_elem ? 1u : 0u;
+    if (m == n2) __syncthreads();  // (no round was taken)
+    for_list2([&](uint64_t o) {
+        if ((o >> bits) == (prefix >> bits)) {
+            const uint32_t i = atomicAdd(nfew, 1u);
+            if (i < (uint32_t)kWave) few[i] = o;
         }
     });
-    uint32_t l2_before, l2_total;
-    block_exclusive_scan(mine_before, L.scratch, &l2_before);
-    block_exclusive_scan(mine_all, L.scratch, &l2_total);
-    if (above_total + l2_total != k) {  // cannot happen with consistent lists
+    __syncthreads();
+    if (*nfew != m) {
         failed = true;
         break;
     }
+    uint64_t cut;  // the last pick
+    {
+        const uint64_t mine = few[lane];
+        uint32_t larger = 0;
+#pragma unroll 4
+        for (uint32_t j = 0; j < m; j++) larger += few[j] > mine ? 1u : 0u;
+        const int at = __ffsll((long long)__ballot((uint32_t)lane < m && larger == want - 1)) - 1;
+        if (at < 0) {  // (an entry twice)
+            failed = true;
+            break;
+        }
+        cut = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(mine >> 32), at) << 32 |
+              (uint32_t)__builtin_amdgcn_readlane((int)mine, at);
+    }
+    const uint32_t T = bin_lo + (uint32_t)(cut >> index_bits);
+    const uint32_t istar = last - (uint32_t)(cut & ((1ull << index_bits) - 1));
+    auto is_pick = [&](bool valid, uint32_t key, uint32_t idx) {
+        return valid && (key > T || (key == T && idx <= istar));
+    };
+    // the picks at indices below this group's first element
+    const uint32_t from_end = last - G.t0 * (uint32_t)kFTile;  // what `last - index` exceeds there
+    uint32_t before = ab;
+    for_list2([&](uint64_t o) {
+        before += o >= cut && (uint32_t)(o & ((1ull << index_bits) - 1)) > from_end ? 1u : 0u;
+    });
+    before = wave_inclusive_scan(before);
+    if (lane == kWave - 1) L.wsum[wave] = before;
     // ---- 5: payload, in index order -----------------------------------------------------------
     // picks per tile first: the register-held tiles' into rcnt, the others' into the total
     uint32_t w_total = 0;
@@ -753,8 +749,12 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
           });
     if (lane == 0) L.wtot[wave] = w_total;
     __syncthreads();
-    uint32_t wave_off = above_before + l2_before;
-    for (int i = 0; i < wave; i++) wave_off += L.wtot[i];
+    uint32_t wave_off = 0;
+#pragma unroll
+    for (int i = 0; i < kFWaves; i++) {
+        wave_off += L.wsum[i];
+        if (i < wave) wave_off += L.wtot[i];
+    }
     auto emit_half = [&](bool valid, uint64_t e, uint32_t pos) {
         const uint32_t key = key64(e), idx = (uint32_t)e, bitsv = (uint32_t)(e >> 32);
         const bool pick = is_pick(valid, key, idx);
@@ -822,7 +822,6 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
     }
     if (grp == 0 && threadIdx.x == 0) {
         st[S_T] = T;
-        st[S_NEED] = need2;
         st[S_ISTAR] = istar;
         st[S_OK] = 1u;
     }
