@@ -24,7 +24,7 @@
 // 5 % 65,537 14.5 / 13.2.  Blocks of 512 threads with twice the vectors are no faster (65,537 12.9, 1 M 21.8), of 256 slower.
 //
 // The blocks of a bucket wait for one another, so they have to be resident together, whatever else the
-// GPU runs.  At 64 registers, 54 KiB of LDS and 1024 threads two blocks fit a CU: 512 the GPU, 64 an XCD.  A
+// GPU runs.  At 64 registers, 49 KiB of LDS and 1024 threads two blocks fit a CU: 512 the GPU, 64 an XCD.  A
 // launch has at most resident_limit of them that wait (topk_route.h): a quarter of those slots, as
 // many launches as a process's four hardware queues can have under way.  They are consecutive in the
 // grid and dealt to the XCDs in turn, at most 16 to each.  So on every XCD, for any launches under way
@@ -424,7 +424,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
                 return (uint32_t)j * kRThreads + threadIdx.x < m && (me[j] - low) >> bits == prefix >> bits;
             };
 #pragma unroll 1
-            while (rm > (uint32_t)kRRank) {  // block-uniform
+            while (rm > (uint32_t)kRRank && bits) {  // block-uniform; ends whatever the scratch memory holds
                 const int at = bits > kRBits ? bits - kRBits : 0;
                 __syncthreads();
                 ((u2a*)L.lh)[threadIdx.x] = u2a{0u, 0u};
@@ -439,6 +439,7 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
                 rm = L.pick[2];
                 bits = at;
             }
+            rm = rm < (uint32_t)kRRank ? rm : (uint32_t)kRRank;
             __syncthreads();
 #pragma unroll
             for (int j = 0; j < 2; j++)

@@ -381,7 +381,7 @@ __device__ __forceinline__ void whole_select(BucketsArg bk, const Geometry& g, c
                     asm volatile("" : "+v"(anew));
                     sample_pick<kBins0, 1, kWThreads>(S.lh, wants, S.wsum, S.res, anew);
                     const uint32_t bin = S.res[0][0];
-                    if (bin >= (uint32_t)kBins0) {  // the list holds fewer entries than the counts promised
+                    if (bin >= (uint32_t)kBins0 || bits == 0) {  // the list holds fewer entries than the counts promised, or one of them twice
                         failed = true;
                         break;
                     }
