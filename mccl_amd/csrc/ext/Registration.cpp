@@ -239,8 +239,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
             mccl::check_single_tensor(t);
             const size_t nbytes = mccl::tensor_nbytes(t);
             const size_t cap = capacity.is_none() ? c.compressed_size(nbytes / sizeof(float)) : capacity.cast<size_t>();
-            at::Tensor out = at::empty({static_cast<int64_t>(cap)},
-                                       at::TensorOptions().dtype(at::kByte).device(t.device()));
+            at::Tensor out = mccl::empty_beside(t, static_cast<int64_t>(cap), at::kByte);
             const uint64_t id = stable_id.is_none() ? stable_id_of(t) : stable_id.cast<uint64_t>();
             const size_t used = c.compress(t.data_ptr(), nbytes, out.data_ptr(), cap, t.scalar_type(), id);
             return first_bytes(out, used);
@@ -248,7 +247,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
            "Top-k payload of a gradient bucket as a uint8 device tensor; error feedback is kept per stable_id")
         .def("decompress", [](mccl::TopKCompressor& c, const at::Tensor& wire, int64_t numel, py::object size) {
             check_payload(wire, size, numel);
-            at::Tensor out = at::empty({numel}, at::TensorOptions().dtype(at::kFloat).device(wire.device()));
+            at::Tensor out = mccl::empty_beside(wire, numel, at::kFloat);
             const size_t sz = size.is_none() ? static_cast<size_t>(wire.numel()) : size.cast<size_t>();
             c.decompress(wire.data_ptr(), sz, out.data_ptr(), static_cast<size_t>(numel) * 4, at::kFloat);
             return out;
@@ -277,8 +276,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
             mccl::check_single_tensor(t);
             const size_t nbytes = mccl::tensor_nbytes(t);
             const size_t cap = capacity.is_none() ? c.max_compressed_size(nbytes) : capacity.cast<size_t>();
-            at::Tensor out = at::empty({static_cast<int64_t>(cap)},
-                                       at::TensorOptions().dtype(at::kByte).device(t.device()));
+            at::Tensor out = mccl::empty_beside(t, static_cast<int64_t>(cap), at::kByte);
             const size_t used = c.compress(t.data_ptr(), nbytes, out.data_ptr(), cap, t.scalar_type());
             return first_bytes(out, used);
         }, py::arg("tensor"), py::arg("capacity") = py::none(),
@@ -286,7 +284,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def("decompress", [](mccl::FP16Compressor& c, const at::Tensor& wire, int64_t numel, py::object size,
                               at::ScalarType dtype) {
             check_payload(wire, size, numel);
-            at::Tensor out = at::empty({numel}, at::TensorOptions().dtype(dtype).device(wire.device()));
+            at::Tensor out = mccl::empty_beside(wire, numel, dtype);
             const size_t sz = size.is_none() ? static_cast<size_t>(wire.numel()) : size.cast<size_t>();
             c.decompress(wire.data_ptr(), sz, out.data_ptr(), static_cast<size_t>(numel) * out.element_size(), dtype);
             return out;
