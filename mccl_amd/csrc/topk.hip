@@ -1039,7 +1039,10 @@ bool launch_by_path(const Buckets& bk, const Geometry& g, const Workspace& w, co
     // (tests of the give-up path: the sample and lead blocks publish a number nobody waits for)
     const auto published = [](uint32_t epoch) { return tuning().topk_stall_test ? ~epoch : epoch; };
     const uint32_t shift = most_groups_shift(g);
-    const uint32_t group_tiles = route.path == kPathStream ? whole_tiles(call, shift, whole_limit_on(share)) : 0;
+    // A recorded list takes two launches, the second of which takes the windows back, also behind a first one that was given up.
+    // (One launch with a kernel in front of it that takes them back: 24 buckets of 1001 to 1.5 M elements replayed in 35.7 us, two
+    // launches 33.1; 16 of 300,000 34.8 / 32.0, 16 of 1 M 62.6 / 62.7, 12 of 1000 to 4 M at 5 % 48.1 / 47.9.)
+    const uint32_t group_tiles = route.path == kPathStream && !is_capturing(st) ? whole_tiles(call, shift, whole_limit_on(share)) : 0;
     if (group_tiles) {
         const uint32_t epoch = next_epoch();
         launch_whole(bk, g, w, group_tiles, shift, epoch, published(epoch), limit_ticks, st);

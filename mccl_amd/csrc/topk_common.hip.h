@@ -34,7 +34,7 @@ enum {
     S_LO_KEY = 0,         // candidates have key >= this
     S_HI_KEY = 1,         // keys >= this fall into the top coarse bin
     S_THAT = 2,           // predicted threshold key; the streaming blocks store 0.0f for keys >= this
-    S_READY = 3,          // the call's epoch number once the other three are valid; 0 after the call
+    S_READY = 3,          // the call's epoch number once the other three are valid; 0 after the call, unless a list went in one launch
     S_P0 = 4, S_R0 = 5,   // exact path: key prefix / picks still to place after round 0
     S_P1 = 6, S_R1 = 7,   // after round 1
     S_T = 8, S_NEED = 9,  // exact threshold key, number of keys == T that are taken
@@ -43,8 +43,7 @@ enum {
     S_EXACT_HIST = 12,    // 1 when hist round 0 holds the full histogram
     S_TIMEOUT = 13,       // single-pass path: a block gave up waiting (result invalid, payload header poisoned)
     S_BARF = 16,          // 16..19: barriers of the exact selection inside the select launch
-    S_DONE = 20,          // one launch: lines of select blocks that have arrived
-    S_LEFT = 21           // ... select blocks that are done
+    S_DONE = 20           // one launch: lines of select blocks that have arrived
 };
 
 struct Geometry {
@@ -166,6 +165,7 @@ inline void place_bucket(Buckets* to, uint32_t i, const Buckets& from, uint32_t 
 // The stream's share of the device, and how many blocks of a launch on it, of which `per_cu` fit a CU, may wait for
 // others (stream_limit).
 StreamShare stream_share(hipStream_t st);
+bool is_capturing(hipStream_t st);
 uint64_t waiting_limit(const StreamShare& share, uint64_t per_cu);
 // ... of a resident launch.
 uint64_t resident_limit_on(const StreamShare& share);

@@ -597,6 +597,8 @@ __global__ __launch_bounds__(kBlock) void k_resident_unpublish(uint32_t* state, 
     if (b < nbuckets) st_agent(state + (uint64_t)b * kStateWords + S_READY, 0u);
 }
 
+}  // namespace
+
 bool is_capturing(hipStream_t st) {
     if (!st) return false;  // the null stream cannot be captured, and asking about it can fail while another one is
     hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
@@ -606,6 +608,8 @@ bool is_capturing(hipStream_t st) {
     }
     return s != hipStreamCaptureStatusNone;
 }
+
+namespace {
 
 // `nlead`: buckets of more than one block, which come first.
 template <int V>

@@ -22,7 +22,9 @@
 // of a bucket wait for each other as well, so a launch has at most as many of them as the resident path has blocks that
 // wait (whole_tiles), a quarter of the GPU's slots where a process has four hardware queues: however many launches are under
 // way, all of theirs find slots on every XCD, and being the last blocks of their grids they keep no other block from one that
-// they wait for.  Every wait has a limit (`limit_ticks`); a bucket that gives up is left as in k_topk_stream.
+// they wait for.  Every wait has a limit (`limit_ticks`); a bucket that gives up is left as in k_topk_stream.  The window
+// stays published behind the launch: blocks that wait for it can leave before the sample block has published, and no count of
+// them survives that.  A replay would carry the same epoch, so a call that is recorded takes two launches (launch_by_path).
 //
 // What bounds it is the chain of round trips behind the last streaming block.  One bucket of 2.2 M elements, us from the
 // first block's start, in a build with stamps: window published 7.9, sums stored 10.7, tiles finished 12.5, a group's candidates in
@@ -110,7 +112,7 @@ __device__ __forceinline__ void whole_sample(BucketsArg bk, const Geometry& g, c
         if (threadIdx.x == 0) {
             st_agent(st + S_OK, 0u);
             st_agent(st + S_TIMEOUT, 0u);
-            st_agent64((uint64_t*)(st + S_DONE), 0ull);  // and S_LEFT
+            st_agent(st + S_DONE, 0u);
             store16_agent(st + S_BARF, z);
         }
         // the histograms of the exact selection, should the select blocks need it
@@ -478,12 +480,6 @@ __global__ __launch_bounds__(kWThreads, 8) void k_topk_whole(WholeBuckets, Geome
     const FusedGeo fg = whole_geo(g, bk, b, h);
     if (select) {
         whole_select<MANY>(bk, g, w, h, b, t, fg, epoch, limit_ticks, L);
-        // a replay of a captured launch carries the same epoch, also behind a run that was given up: the last block that
-        // has waited for the window takes it back
-        if (threadIdx.x == 0) {
-            uint32_t* const st = w.state + (uint64_t)b * kStateWords;
-            if (__hip_atomic_fetch_add(st + S_LEFT, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == fg.ng) st_agent(st + S_READY, 0u);
-        }
         return;
     }
     // the blocks that start together with the sample blocks hold back (stream_hold)

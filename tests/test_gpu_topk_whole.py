@@ -174,3 +174,59 @@ def test_four_streams(ops):
                 assert w.cpu().numpy()[:size].tobytes() == want.tobytes()
         for r, d in zip(want_res, res):
             assert np.array_equal(bits(to_np(d, F32)), bits(r))
+
+
+STATE_WORDS, HIST_WORDS, S_READY = 32, 4096, 3   # per bucket, at the front of a workspace: histograms, then state
+
+
+def _published(ws, count):
+    return ws.view(torch.int32)[count * HIST_WORDS:count * (HIST_WORDS + STATE_WORDS)].view(count, STATE_WORDS)[:, S_READY].tolist()
+
+
+def test_a_recorded_list_takes_its_windows_back(ops):
+    """One launch leaves the windows published under its number.  A replay carries the number of the replay before, so a
+    recorded list has to end with them taken back, also when its blocks gave up."""
+    rng = np.random.default_rng(12)
+    lengths, ratio = [700_001, 300_000, 5_000], 0.01
+    count, longest = len(lengths), max(lengths)
+    grads = [to_dev(student_t(rng, n), F32) for n in lengths]
+    res = [torch.zeros(n, device=DEV) for n in lengths]
+    ws = ops.topk_workspace(longest * count, longest, ratio, DEV)
+    status = torch.zeros(1, dtype=torch.int32, device=DEV)
+    call = lambda: ops.topk_compress_list(grads, res, ratio, workspace=ws, status=status)
+    call()
+    assert all(_published(ws, count))
+    graphs, wires = [], []
+    try:
+        for stall in (1, 0):
+            ops.set_tuning("topk_stall_test", stall)
+            ops.set_tuning("topk_barrier_ms", 1 if stall else 2000)
+            side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side), torch.cuda.graph(graph, stream=side):
+                wires.append(call())
+            torch.cuda.current_stream().wait_stream(side)
+            graphs.append(graph)
+    finally:
+        ops.set_tuning("topk_stall_test", 0)
+        ops.set_tuning("topk_barrier_ms", 2000)
+    for step in range(3):
+        status.zero_()
+        graphs[0].replay()
+        torch.cuda.synchronize()
+        assert int(status) == -9
+        assert _published(ws, count) == [0] * count
+        values = [student_t(rng, n, scale=10.0 ** -step) for n in lengths]
+        for g, r, v in zip(grads, res, values):
+            g.copy_(torch.from_numpy(v))
+            r.zero_()
+        status.zero_()
+        graphs[1].replay()
+        torch.cuda.synchronize()
+        assert int(status) == 0
+        assert _published(ws, count) == [0] * count
+        for v, r, w in zip(values, res, wires[1]):
+            want_r = np.zeros(v.size, np.float32)
+            want, size = oracle.topk_compress(v, want_r, ratio)
+            assert w.cpu().numpy()[:size].tobytes() == want.tobytes(), step
+            assert np.array_equal(bits(to_np(r, F32)), bits(want_r)), step
