@@ -706,10 +706,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_topk_select(Buckets, Geometry g, 
     uint64_t cut;  // the last pick
     {
         const uint64_t mine = few[lane];
-        uint32_t larger = 0;
-#pragma unroll 4
-        for (uint32_t j = 0; j < m; j++) larger += few[j] > mine ? 1u : 0u;
-        const int at = __ffsll((long long)__ballot((uint32_t)lane < m && larger == want - 1)) - 1;
+        const int at = __ffsll((long long)__ballot((uint32_t)lane < m && reaching_entries(few, 0, m, mine) == want)) - 1;
         if (at < 0) {  // (an entry twice)
             failed = true;
             break;

@@ -4,6 +4,7 @@
 
 #include "common.hip.h"
 #include "runtime.h"
+#include "topk_rank.h"
 #include "topk_route.h"
 
 namespace mcclhip {

@@ -407,14 +407,17 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
         }
         if (!tied) {
             // The r-th largest entry: by radix rounds over key and index (entries differ in their index), until few enough
-            // share a prefix to rank them, by counting for each of them the larger ones.
+            // share a prefix to rank them, by counting for each of them those that reach it.
             uint64_t me[2];
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 const uint32_t i = (uint32_t)j * kRThreads + threadIdx.x;
                 me[j] = i >= m ? 0ull : nblk > 1 ? ld_agent64((const uint64_t*)(mem + kRListAt) + i) : L.list[i];
             }
-            if (threadIdx.x == 0) L.count = 0;
+            if (threadIdx.x == 0) {
+                L.count = 0;
+                L.cut = kNoCut;
+            }
             if (threadIdx.x < (uint32_t)kRRank) L.rank[threadIdx.x] = 0;
             const uint64_t low = (uint64_t)base << 32;
             uint32_t rm = m, rr = r;
@@ -454,13 +457,11 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
                 const uint32_t per = (rm + kRWaves - 1) / kRWaves, from = per * wave, to = from + per < rm ? from + per : rm;
                 if (from < to) {
                     const uint64_t mine = L.sub[lane];
-                    uint32_t rank = 0;
-#pragma unroll 4
-                    for (uint32_t j = from; j < to; j++) rank += L.sub[j] > mine ? 1u : 0u;
+                    const uint32_t rank = reaching_entries(L.sub, from, to, mine);
                     if ((uint32_t)lane < rm && rank) atomicAdd(&L.rank[lane], rank);
                 }
                 __syncthreads();
-                if (threadIdx.x < rm && L.rank[threadIdx.x] == rr - 1) L.cut = L.sub[threadIdx.x];
+                if (threadIdx.x < rm && L.rank[threadIdx.x] == rr) L.cut = L.sub[threadIdx.x];
                 __syncthreads();
             }
             const uint64_t cut = L.cut;
@@ -578,7 +579,9 @@ __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometr
         }
         pos0 += (uint32_t)__builtin_amdgcn_readlane((int)up_to, kWave - 1);
     }
-    if (x == 0 && threadIdx.x == 0) {
+    if (x == 0 && threadIdx.x == 0 && T == (uint32_t)(kNoCut >> 32)) {
+        give_up();  // nothing was picked (a branch where the cut is read takes every call 0.15 us)
+    } else if (x == 0 && threadIdx.x == 0) {
         st[S_T] = T;
         st[S_ISTAR] = istar;
         st[S_READY] = 0u;  // a replay of a captured launch carries the same epoch

@@ -172,6 +172,7 @@ __device__ __forceinline__ void whole_select(BucketsArg bk, const Geometry& g, c
     const uint32_t* const tile_cnt = w.tile_cnt + (uint64_t)b * g.ftiles;
     if (threadIdx.x < kCoarse) S.cnt[threadIdx.x] = 0;
     if (threadIdx.x == 0) {
+        S.cut = kNoCut;
         u4a wn = wait_window(st, epoch, limit_ticks);  // (the counters are only meaningful once the sample block has cleared them)
         if (wn[3] && !wait_word<4>(line + G_TILES, tg1 - tg0, limit_ticks)) wn[3] = 0u;
         S.win[0] = wn[0]; S.win[1] = wn[1]; S.win[2] = wn[2]; S.win[3] = wn[3];
@@ -400,16 +401,14 @@ __device__ __forceinline__ void whole_select(BucketsArg bk, const Geometry& g, c
                     }
                     if (tid < m) {
                         const uint64_t me = S.list[tid];
-                        uint32_t rank = 0;
-#pragma unroll 4
-                        for (uint32_t j = 0; j < m; j++) rank += S.list[j] > me ? 1u : 0u;
-                        if (rank == want - 1) S.cut = me;
+                        if (reaching_entries(S.list, 0, m, me) == want) S.cut = me;
                     }
                     __syncthreads();
                     cut = S.cut;
                     step = 2;
                 }
             }
+            failed |= cut == kNoCut;  // (an entry twice)
             if (failed) break;
             T = bin_lo + (uint32_t)(cut >> 32);
             istar = ~(uint32_t)cut;
