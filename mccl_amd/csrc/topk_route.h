@@ -176,16 +176,22 @@ inline uint32_t next_launch(const uint32_t* counts, uint32_t* order, uint32_t le
 // every bucket; 0 where it takes two.  A group is a select block that waits for others, so a call has at most `limit` of
 // them (stream_limit), at most 1 << shift in a bucket, and candidates in it that its block can keep: beyond, a block reads
 // them from memory on each of four passes (24 buckets of 1001 to 1 M at 5 %, 33 and 10 tiles a group: 32.7 us in two
-// launches, 40 / 30 in one).  us per call, two launches / one: 24 buckets of 1001 to 1.5 M elements (1343 tiles) 33.8 / 28.9, at 0.1 %
-// 32.7 / 27.3, to 2.2 M 41.9 / 39.0, to 3 M (2750 tiles) 46.9 / 46.2, 12 of 1000 to 2 M 29.6 / 26.7, 60 of 1000 to 1 M 48.8 / 40.4, 16 of
-// 300,000 32.1 / 28.0, of 1 M 62.2 / 59.8, three of 100 to 6.5 M 35.7 / 34.2, two of 2.5 M 30.8 / 29.4, ten of 1000 to 3 M at 5 % 38.4 / 33.7.  Few large
-// buckets gain nothing: two of 4 M 38.4 / 41.1, five of 2.2 M 47.5 / 48.1; nor do those of one buffer, whose two launches have
-// no table to read: one bucket of 2.2 M 26.1 / 26.7, of 6,553,600 33.7 / 34.6, eight of 2.5 M 65 / 69.
-// Groups of a call: 24 buckets of 1001 to 1.5 M with 64 / 96 / 160 / 224 of them 31.2 / 30.3 / 29.1 / 28.9.
+// launches, 40 / 30 in one).  us per call, two launches / one, both as they stand (two runs of one side differ by 0.2 at 2 % and
+// 5 %, 1 at 1 %): 24 buckets of 1001 to 1.5 M elements (1357 tiles) 30.2 / 28.2, at 0.1 % 28.9 / 25.7, at 2 % 34.6 / 28.7, to 2.2 M 37.3 /
+// 34.0, 12 of 1000 to 2 M 26.6 / 25.5, 60 of 1000 to 1 M 42.1 / 37.6, 16 of 300,000 29.5 / 26.9, of 1 M 58.0 / 54.8, two of 2.5 M 28.1 / 27.8, three
+// of 2.2 M 31.0 / 29.5, one of 2.5 M 25.1 / 24.5, ten of 1000 to 3 M at 5 % 35.4 / 31.9, 12 of 1000 to 4 M 44.6 / 39.7.  Few large buckets gain
+// nothing: two of 4 M 34.9 / 37.4, five of 2.2 M 43.9 / 45.0; nor do those of one buffer, whose two launches have
+// no table to read: one bucket of 2.2 M 24.5 / 24.6, of 6,553,600 30.8 / 32.0, eight of 2.5 M 61.8 / 65.3.
+// A bucket's groups add to the same counters and meet: with many candidates in few tiles a bucket of many groups waits longer
+// than the second launch takes to start.  So above kWholeDenser long buckets go in two launches: three of 100 to 6.5 M 32.7 /
+// 33.2, 24 of 1001 to 3 M (2502 tiles, the longest 733) 42.7 / 43.7, 12 of 1000 to 6.5 M 46.2 / 47.2, eight of 1.3 M (318) 42.3 / 42.5, of 2 M (489)
+// 54.0 / 55.0; 12 of 1 M (2940, 245) 47.9 / 46.8.  Below, 24 of 1001 to 3 M at 0.1 % 40.3 / 38.2, eight of 2 M 51.0 / 49.0.
+// Groups of a call: 24 buckets of 1001 to 1.5 M with 64 / 96 / 160 / 224 of them 29.8 / 28.9 / 28.8 / 27.5.
 constexpr uint32_t kWholeMost = 64;      // tiles of a group: a lane each
 constexpr uint32_t kWholeOwn = 2600;     // candidates of its group that a select block keeps in LDS
 constexpr uint32_t kWholeGroups = 256;
 constexpr uint64_t kWholeTiles = 4096;
+constexpr double kWholeDenser = 68.0;    // candidates of a tile: a ratio of 0.85 %
 inline uint32_t whole_tiles(const TopkCall& c, uint32_t shift, uint64_t limit) {
     if (!c.counts || limit < c.nbuckets) return 0;
     uint64_t sum = 0;
@@ -193,6 +199,7 @@ inline uint32_t whole_tiles(const TopkCall& c, uint32_t shift, uint64_t limit) {
     if (sum > kWholeTiles || (sum > 1664 && c.nbuckets < 8)) return 0;
     const uint64_t longest = topk_tiles(c.bucket_elems);
     const double candidates = window_share((double)c.k_full / (double)c.bucket_elems) * kFTile;  // of a tile
+    if (!c.many && candidates > kWholeDenser && longest > (sum > 2304 ? 320 : 1280)) return 0;
     uint32_t per = (uint32_t)((sum + kWholeGroups - 1) / kWholeGroups);
     for (per = per < 8 ? 8 : per + (per & 1); per <= kWholeMost && per * candidates <= 0.92 * kWholeOwn; per += 2) {
         if ((longest + per - 1) / per > 1u << shift) continue;

@@ -67,3 +67,39 @@ def test_lists_in_one_launch(tmp_path):
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", "-I", os.path.join(ROOT, "mccl_amd", "csrc"), str(src), "-o",
                     str(exe)], check=True)
     assert subprocess.run([str(exe)], capture_output=True, text=True, timeout=120).stdout == "ok\n"
+
+
+LONG_BUCKETS = r"""
+#include "topk_route.h"
+#include <algorithm>
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+using namespace mcclhip;
+static bool one(uint64_t others, uint32_t count, uint64_t longest, double ratio) {   // tiles
+    std::vector<uint64_t> v(count, others * kFTile);
+    v.push_back(longest * kFTile);
+    const uint64_t n = std::max(others, longest) * kFTile;
+    const uint32_t k = (uint32_t)(n * ratio);
+    const TopkCall c = {n * v.size(), n, (uint32_t)v.size(), v.data(), k ? k : 1, topk_many(n, ratio)};
+    return whole_tiles(c, c.many ? 8 : topk_group_shift_few(topk_tiles(n)), 256);
+}
+int main() {
+    for (const double ratio : {0.001, 0.005, 0.008, 0.009, 0.01, 0.011, 0.012, 0.02}) {
+        const bool dense = ratio > 0.0085 && ratio < 0.0115;   // few slots a tile and many candidates in them
+        const bool ok = one(10, 10, 1280, ratio) && one(10, 10, 1281, ratio) != dense &&     // up to 2304 tiles
+                        one(198, 10, 320, ratio) && one(198, 10, 324, ratio) &&              // 2300, 2304
+                        one(199, 10, 320, ratio) && one(199, 10, 321, ratio) != dense;       // more
+        if (!ok) { std::printf("%g\n", ratio); return 1; }
+    }
+    std::puts("ok");
+}
+"""
+
+
+def test_long_buckets_of_dense_tiles_take_two_launches(tmp_path):
+    src, exe = tmp_path / "long.cpp", tmp_path / "long"
+    src.write_text(LONG_BUCKETS)
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", "-I", os.path.join(ROOT, "mccl_amd", "csrc"), str(src), "-o",
+                    str(exe)], check=True)
+    assert subprocess.run([str(exe)], capture_output=True, text=True, timeout=120).stdout == "ok\n"
