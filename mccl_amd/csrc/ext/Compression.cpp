@@ -204,6 +204,7 @@ std::vector<at::Tensor> TopKCompressor::compress_many(const std::vector<at::Tens
     std::vector<at::Tensor*> residuals;
     payloads.reserve(buckets.size());
     residuals.reserve(buckets.size());
+    const bool watched = allocations_are_watched();
     for (size_t i = 0; i < buckets.size(); i++) {
         const at::Tensor& t = buckets[i];
         check_single_tensor(t);
@@ -212,7 +213,7 @@ std::vector<at::Tensor> TopKCompressor::compress_many(const std::vector<at::Tens
         for (size_t j = 0; j < i; j++)
             MCCL_CHECK(stable_ids[j] != stable_ids[i], "compress_many: the same stable id twice in one call");
         // (allocated at its size: a narrowed view of a larger buffer takes the host another 0.6 us per bucket)
-        payloads.push_back(empty_beside(t, static_cast<int64_t>(compressed_size(static_cast<size_t>(t.numel()))), at::kByte));
+        payloads.push_back(empty_beside(t, static_cast<int64_t>(compressed_size(static_cast<size_t>(t.numel()))), at::kByte, watched));
     }
     const uint64_t evictions = evictions_;
     for (size_t i = 0; i < buckets.size(); i++)
