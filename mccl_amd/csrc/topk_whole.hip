@@ -80,6 +80,8 @@ struct WholeLds {
     };
 };
 
+static_assert(sizeof(WholeLds<false>) <= 40 * 1024 && sizeof(WholeLds<true>) <= 40 * 1024, "four blocks to a CU");
+
 __device__ __forceinline__ FusedGeo whole_geo(const Geometry& g, BucketsArg bk, uint32_t b, const Whole& h) {
     FusedGeo f;
     f.bn = bucket_count(g, bk, b);

@@ -1,5 +1,6 @@
 """Lists that go in one launch: one bucket and as many as a list holds, groups of one tile and of several, groups whose
-candidates do not fit LDS or whose tiles are dense, buckets that fall back beside others that don't, a wait that runs out, replays."""
+candidates do not fit LDS or whose tiles are dense, buckets that fall back beside others that don't, a wait that runs out; and
+recorded ones, which go in two.  One launch leaves its windows published, two take them back: that tells the routes apart."""
 import numpy as np
 import pytest
 import torch
@@ -29,7 +30,14 @@ def _misled(rng, n):
     return g
 
 
-def _check(ops, grads, ratio, single_pass=None):
+STATE_WORDS, HIST_WORDS, S_READY = 32, 4096, 3   # per bucket, at the front of a workspace: histograms, then state
+
+
+def _published(ws, count):
+    return ws.view(torch.int32)[count * HIST_WORDS:count * (HIST_WORDS + STATE_WORDS)].view(count, STATE_WORDS)[:, S_READY].tolist()
+
+
+def _check(ops, grads, ratio, single_pass=None, one_launch=True):
     longest, count = max(g.size for g in grads), len(grads)
     rng = np.random.default_rng(count)
     residuals = [(rng.standard_normal(g.size) * 1e-9).astype(np.float32) for g in grads]
@@ -38,6 +46,7 @@ def _check(ops, grads, ratio, single_pass=None):
     ws = ops.topk_workspace(longest * count, longest, ratio, DEV)
     wires = ops.topk_compress_list([to_dev(g, F32, (i + 1) % 3) for i, g in enumerate(grads)], dres, ratio, workspace=ws, status=status)
     assert int(status) == 0
+    assert [w != 0 for w in _published(ws, count)] == [one_launch] * count
     if single_pass is not None:
         assert ops.topk_path_report(ws, longest * count, longest, ratio) == (single_pass, count)
     for g, r, d, w in zip(grads, residuals, dres, wires):
@@ -54,7 +63,9 @@ def _check(ops, grads, ratio, single_pass=None):
     [70_001 + i for i in range(64)]])
 def test_lists(ops, lengths, ratio):
     rng = np.random.default_rng(len(lengths))
-    _check(ops, [student_t(rng, n, ties=0.01) for n in lengths], ratio)
+    # (a group of 8 tiles that may be all candidates, or of 12 at 5 %, has more than a block keeps)
+    two = lengths == [1] or ratio == 0.05 and len(lengths) == 12
+    _check(ops, [student_t(rng, n, ties=0.01) for n in lengths], ratio, one_launch=not two)
 
 
 @pytest.mark.parametrize("ratio", [0.01, 0.05])
@@ -107,6 +118,7 @@ def test_a_wait_that_runs_out(ops):
         ops.set_tuning("topk_stall_test", 0)
         ops.set_tuning("topk_barrier_ms", 2000)
     assert int(status) == -9
+    assert all(_published(ws, 2))
     assert all(int(w[:4].view(torch.int32)) == -1 for w in wires)
     status.zero_()
     for r in res:
@@ -119,7 +131,7 @@ def test_a_wait_that_runs_out(ops):
 
 
 def test_replays(ops):
-    """A recorded list call, replayed with other gradients: every replay carries the same number."""
+    """A recorded list call, which takes two launches, replayed with other gradients: every replay carries the same number."""
     rng = np.random.default_rng(9)
     lengths = [700_001, 300_000, 5_000]
     grads = [torch.empty(n, device=DEV) for n in lengths]
@@ -165,8 +177,8 @@ def test_four_streams(ops):
             with torch.cuda.stream(stream):
                 wires.append(ops.topk_compress_list(grads, res, 0.01, workspace=ws, status=status))
     torch.cuda.synchronize()
-    for s, (_, values, _, res, _, status) in enumerate(calls):
-        assert int(status) == 0
+    for s, (_, values, _, res, ws, status) in enumerate(calls):
+        assert int(status) == 0 and all(_published(ws, len(lengths)))
         want_res = [np.zeros(n, np.float32) for n in lengths]
         for rep in range(3):
             for v, r, w in zip(values, want_res, wires[rep * 4 + s]):
@@ -174,13 +186,6 @@ def test_four_streams(ops):
                 assert w.cpu().numpy()[:size].tobytes() == want.tobytes()
         for r, d in zip(want_res, res):
             assert np.array_equal(bits(to_np(d, F32)), bits(r))
-
-
-STATE_WORDS, HIST_WORDS, S_READY = 32, 4096, 3   # per bucket, at the front of a workspace: histograms, then state
-
-
-def _published(ws, count):
-    return ws.view(torch.int32)[count * HIST_WORDS:count * (HIST_WORDS + STATE_WORDS)].view(count, STATE_WORDS)[:, S_READY].tolist()
 
 
 def test_a_recorded_list_takes_its_windows_back(ops):
