@@ -22,7 +22,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 HERE = os.path.join(ROOT, "mccl_amd")
 OUT = os.path.join(ROOT, "profiles", "hbm_traffic.json")
 SOURCES = ["common.hip.h", "fold.hip", "fold_rows.h", "ring_cut.h", "topk.hip", "topk_common.hip.h", "topk_stream.hip.h",
-           "topk_route.h", "sparse.hip"]
+           "topk_rank.h", "topk_route.h", "sparse.hip"]
 N_GRAD = 96_510_024
 COPY_KIB = N_GRAD * 4 / 1024.0          # bench.py's torch copy_ of one rank buffer
 

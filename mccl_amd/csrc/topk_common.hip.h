@@ -75,10 +75,10 @@ struct Workspace {
     // single-pass path
     uint32_t* tile_cnt;     // [nbuckets][ftiles] candidates in the tile's slots, or kDense
     uint64_t* slots;        // [nbuckets][ftiles][slots] (bits << 32) | index, index order
-    uint32_t* grp_cnt;      // [nbuckets][groups][kCntStride] finished tiles per group (first word of each 256 bytes)
-    uint32_t* gsuf;         // [nbuckets][128 bins][groups] a group's candidates in the bins above bin j
+    uint32_t* grp_cnt;      // [nbuckets][groups][kCntStride] finished tiles per group (first word of each 256 bytes; one launch: see group_line)
+    uint32_t* gsuf;         // [nbuckets][128 bins][groups] a group's candidates in the bins above bin j (one launch: [nbuckets][groups][128 bins])
     uint32_t* bin_fill;     // [nbuckets][128] the bucket's candidates per coarse window bin (= entries of the bin's list)
-    uint64_t* blist;        // [nbuckets][63][lcapb] the window's candidates by coarse bin, any order
+    uint64_t* blist;        // [nbuckets][127][lcapb] the window's candidates by coarse bin, any order
     uint32_t* rmem;         // [nbuckets][kRWords] resident path
     int* status;            // caller's device word (may be null): receives MCCL_HIP_ERR_TIMEOUT when a block gives up
 };
@@ -346,7 +346,7 @@ __device__ __forceinline__ void sample_pick(const uint32_t* h, const uint32_t (&
 // noise away from the expected rank of the k-th largest key, and the predicted threshold - by 11 key
 // bits and then, in one histogram for all three, by 2048 bins over the digits that they lie in.  Zeros are not counted:
 // sparse gradients' would all add to one LDS word (at 99 % zeros the window was published two microseconds later, and a call
-// of 6,553,600 elements at 0.1 % took 31.7 us, so 29.3), and a rank among them would stretch the digits down to zero's.
+// of 6,553,600 elements at 0.1 % took 31.7 us, so 29.1), and a rank among them would stretch the digits down to zero's.
 // Called by all THREADS threads of a block; the result is valid in thread 0.
 // `under_way()` runs while the sample's loads are under way.
 struct SampleWindow {

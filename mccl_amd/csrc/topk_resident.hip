@@ -151,9 +151,11 @@ template <int V>
 __global__ __launch_bounds__(kRThreads, 8) void k_topk_resident(Buckets, Geometry g, Workspace w, uint32_t nlead, uint32_t epoch,
                                                                 uint32_t published, uint64_t limit_ticks) {
     constexpr uint32_t PER = kRThreads * 4 * V;  // elements of a block
-    // Buckets of this many elements start from a sampled window, which costs about 5 us and saves a round.
-    // With a sample and without, us: 8 x 70,000 elements 17.9 / 16.0, 30 x 33,000 20.7 / 18.8, 8 x 262,143 22.0 / 21.9,
-    // 3 x 300,000 18.7 / 17.4, one of 400,000 18.9 / 18.0, of 1 M 21.3 / 23.5, of 2 M 25.4 / 28.1, 2 x 1 M 22.0 / 24.0.
+    // Buckets of this many elements start from a sampled window, which costs about 4 us and saves a round.
+    // With a sample and without, us: one of 262,144 elements 16.4 / 16.0, of 300,000 17.0 / 15.9, of 400,000 17.5 / 16.6, of 450,000 17.7 /
+    // 17.0, of 500,000 17.5 / 17.9, of 700,000 19.1 / 19.8, of 1 M 20.2 / 22.2, of 2 M 24.1 / 27.6, 2 x 1 M 21.6 / 24.5; 8 x 70,000 16.5 / 16.0, 30 x 33,000 18.2 / 18.8,
+    // 3 x 300,000 17.9 / 18.0.  (Several buckets of more cross sooner than one does, 8 x 262,143 20.3 / 22.0, 5 x 400,000 20.4 / 22.1, and go without it
+    // all the same: the rule asks for the bucket alone.)
     constexpr uint32_t kSampleMin = 1u << 19;
     const BucketsArg bk = buckets_arg();
     __shared__ ResidentLds L;

@@ -84,11 +84,14 @@ constexpr bool stream_wide(uint64_t tiles) { return tiles <= kWideTiles; }
 
 // How long the streaming blocks that start together with the sample blocks hold back, in steps of 512 clocks (0.21 us):
 // their loads would bury the samples' few, and they wait for the samples all the same.  A launch whose tiles are loaded
-// before its samples are evaluated gains by waiting longer; one with more, by loading sooner.  us per call at 1 %, 15 / 12.5 / 10 /
-// 7 / 5.5 steps: one bucket of 2.2 M elements 25.9 / 26.1 / 26.3 / 27.2 / 27.1, of 4 M 28.3 / 28.2 / 28.8 / 29.9 / 29.8, of 5 M 30.8 / 30.4 /
-// 30.6 / 31.7 / 32.3, of 6 M 32.7 / 32.2 / 31.9 / 33.1 / 33.8, of 6,553,600 36.7 / 36.6 / 35.3 / 33.8 / 34.1, of 10 M 45.7 / 45.7 / 45.3 /
-// 44.5 / 44.6; two of 2.2 M 29.4 / 28.6 / 27.9 / 29.0 / 29.5, of 3 M 34.2 / 33.8 / 33.0 / 31.6 / 31.5; 24 listed ones of 1001 to 1 M (905
-// tiles) 31.8 / 30.8 / 30.6 / 30.6 / 30.6, to 1.5 M (1343) 36.4 / 36.0 / 35.3 / 33.8 / 33.5; one of 4 M at 5 % 34.3 / 34.7 / 35.7 / 36.6 / 36.2.
+// before its samples are evaluated gains by waiting longer; one with more, by loading sooner.  us per call at 1 %, 7 / 9 / 10 / 11 /
+// 12 / 14 steps: one bucket of 2.2 M elements (538 tiles) 25.4 / 25.2 / 25.1 / 24.5 / 24.3 / 24.3, of 4 M (977) 27.9 / 28.0 / 26.9 / 26.5 / 26.0 /
+// 26.0, of 1100 tiles 29.2 / 28.6 / 28.1 / 27.5 / 27.4 / 27.5, of 1221 29.5 / 28.9 / 28.5 / 28.1 / 27.9 / 28.1, of 1465 30.6 / 29.8 / 29.4 / 29.3 / 29.3 /
+// 29.6, of 1536 30.3 / 29.5 / 29.5 / 29.8 / 29.9 / 30.2, of 1550 30.4 / 31.0 / 30.9 / 31.3 / 31.8 / 32.3, of 1600 31.1 / 30.8 / 31.1 / 32.2 / 32.6 / 33.1, of 8 M (1954)
+// 33.8 / 34.2 / 35.4 / 36.2 / 36.8 / 37.8, of 10 M 42.0 / 41.7 / 41.7 / 42.6 / 42.1 / 43.6; two of 2.2 M (1075) 27.0 / 26.4 / 25.9 / 25.5 / 26.4 / 26.0, as a list 27.0 /
+// 26.5 / 26.2 / 26.5 / 27.0 / 28.6, of 3 M (1465) 29.8 / 30.1 / 30.1 / 31.3 / 31.5 / 31.4; 24 listed ones of 1001 to 1 M (952) 26.0 / 25.6 / 25.4 / 25.0 / 25.0 / 24.9, to
+// 1.5 M (1357) 27.8 / 27.9 / 28.4 / 28.5 / 28.2 / 28.1, 16 of 300,000 (1184) 26.8 / 27.1 / 28.6 / 27.6 / 28.5 / 28.8; one of 4 M at 5 % 33.8 / 33.3 / 32.7 / 32.3 / 31.9 / 31.7.
+// (Two runs of one side differ by 0.2 to 0.6.)
 constexpr uint32_t stream_hold(uint64_t tiles, uint32_t nbuckets) {
     if (nbuckets == 1) return tiles <= 1024 ? 14 : tiles <= 1536 ? 11 : 7;
     return tiles <= 1152 ? 10 : 7;
@@ -217,16 +220,16 @@ struct Route {
 
 // `forced`: the tuning key "topk_path" (1 exact, 2 single-pass, 3 resident where it is admitted).
 // Measured per call, us:
-//   resident where one launch may take the call: 65,536 elements 15 against 28 exact; 1 M 21 against 26
-//     streaming; 8 x 262,144 20 against 30 streaming; 16 x 65,536 18 against 31 exact; 1500 x 16,384, where a
-//     bucket is one block and nobody waits, 63 against 187 exact.
-//   Beyond, several launches are slower than the two of the streaming path (24 buckets of 1001 to 1.5 M, three
-//     launches: 68 against 38) ...
+//   resident where one launch may take the call: 65,536 elements 12.6 against 20.4 streaming and 27.7 exact; 1 M 19.9
+//     against 22.5 streaming; 8 x 262,144 21.7 against 23.3 streaming; 16 x 65,536 15.7 against 21.9 streaming and 31.7 exact; 1500 x
+//     16,384, where a bucket is one block and nobody waits, 62 against 188 exact.
+//   Beyond, several launches are slower than the one or two of the streaming path (24 buckets of 1001 to 1.5 M, three
+//     launches: 66 against 28) ...
 //   ... unless the streaming path's tiles run out of candidate slots (share of a bucket inside the sampled window
 //     times 4096; of 1024 slots 60 % are counted on: ratios up to 0.12).  With slots for many candidates,
-//     at 5 %, several resident launches or the exact path against the streaming path: that list 73 / 43, 30 buckets of
-//     20,000 to 2 M 172 / 65, one bucket of 2.2 M 65 / 31, of 6.5 M 140 / 38, 4 x 2 M 115 / 43, 20 x 300,000 74 / 39,
-//     20 x 1.5 M 291 / 107; one of 6.5 M at 12 % 144 / 51.  Tiles that run out are read again as a whole: with 128 slots
+//     at 5 %, several resident launches or the exact path against the streaming path: that list 69 / 31, 30 buckets of
+//     20,000 to 2 M 163 / 59, one bucket of 2.2 M 63 / 27, of 6.5 M 137 / 38, 4 x 2 M 116 / 40, 20 x 300,000 74 / 36,
+//     20 x 1.5 M 283 / 101; one of 6.5 M at 12 % 144 / 47.  Tiles that run out are read again as a whole: with 128 slots
 //     that list at 5 % 71 against 199, 30 buckets of 20,000 to 2 M in seven launches 169 against 240.
 //   Buckets of one buffer take the exact path then: with 128 slots, at 5 %, one of 6.5 M 144 against 448, 16 x 262,144 57
 //     against 99, 4 x 2 M 117 against 167, 20 x 1.5 M 288 against 320; of many large ones the streaming path shares that

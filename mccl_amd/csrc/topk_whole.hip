@@ -29,7 +29,7 @@
 // What bounds it is the chain of round trips behind the last streaming block.  One bucket of 2.2 M elements, us from the
 // first block's start, in a build with stamps: window published 7.9, sums stored 10.7, tiles finished 12.5, a group's candidates in
 // LDS 13.8, counted and the places known 15.9, listed and met 19.8, the bin found 20.8, threshold 23.7, picks counted 24.3, stored
-// 25.4.  24 buckets of 1001 to 1.5 M elements at 1 %, two launches / this one: 34.0 / 28.9 us.  Also built, and slower: streaming
+// 25.4.  24 buckets of 1001 to 1.5 M elements at 1 %, two launches / this one: 30.2 / 28.2 us.  Also built, and slower: streaming
 // blocks that count and list their candidates themselves, behind one atomic a bin and block (6.5 M elements 52.7 us), and select
 // blocks that add up all groups' rows of counts instead of meeting (31.6 at 2.2 M).
 #include "topk_stream.hip.h"
