@@ -192,7 +192,8 @@ int mccl_hip_topk_compress(const float* grad, float* residual, uint64_t n_total,
 /* TopKCompressor::compress for a LIST of buckets that are separate buffers of
  * their own lengths (the tensor list of a coalesced allreduce,
  * csrc/backend/ProcessGroupMCCL.cpp:2257-2313, compresses bucket by bucket), in
- * one launch or the two of mccl_hip_topk_compress: per-bucket calls are bound
+ * one launch or, also on a stream that is being captured, the two of
+ * mccl_hip_topk_compress: per-bucket calls are bound
  * by launch latency, a list is not.  host_grads[b] / host_residuals[b] hold
  * host_counts[b] fp32 elements; bucket b's payload [u32 k_b][k_b x {u32 index,
  * f32 value}] goes to host_wires[b], which holds host_wire_capacities[b] bytes
